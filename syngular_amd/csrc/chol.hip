@@ -38,15 +38,6 @@ __device__ __forceinline__ double recip_nr(double x) {
     return fma(r, e, r);
 }
 
-// Work-group barrier that orders LDS only: global stores issued before it
-// stay in flight.  For phases whose global writes no thread of the
-// work-group reads back (a plain __syncthreads waits for them to land).
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 __global__ __launch_bounds__(256) void maxdiag_kernel(const double *g, int64_t n, int64_t ld, double *out,
                                                       int *dropped) {
     __shared__ double red[4];

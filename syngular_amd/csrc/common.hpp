@@ -54,6 +54,15 @@ __device__ __forceinline__ int find_item(const Item *items, int n, int64_t b) {
     return lo;
 }
 
+// Work-group barrier that orders LDS only: global stores issued before it
+// stay in flight.  For phases whose global writes no thread of the
+// work-group reads back (a plain __syncthreads waits for them to land).
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Host-side helpers shared by the multi-step routines (gemm.hip).
 int gemm_f64_launch(syn_gemm_item P, hipStream_t s, bool mixed = false);
 int gemm_f64_split_launch(syn_gemm_item P, hipStream_t s, double *ws, int64_t ws_cap);

@@ -1,0 +1,1329 @@
+// Direct phase of the blocked Gram eigen-solver: tridiagonal reduction and
+// divide and conquer.
+//
+// A Gram matrix G is reduced to tridiagonal form T = H^T G H by Householder
+// reflectors (Golub & Van Loan 8.3.1, in the panel form of LAPACK's dlatrd),
+// T is diagonalised by divide and conquer (Cuppen 1981; deflation, secular
+// equation and the recomputed z of Gu & Eisenstat 1995), the eigenvectors of
+// T are transformed back to rt = (H Q)^T with compact WY blocks, and G is
+// replaced by rt G rt^T, diagonal to rounding.  The Jacobi sweeps that follow
+// (tjacobi.hip) start from there: their end-of-sweep test is what accepts the
+// result, and a matrix with an entry that still passes it is rotated until
+// none does, so the phase changes how many sweeps a call takes (usually none)
+// and not what its result satisfies.
+//
+// Why: a block Jacobi sweep rewrites G and rt in every one of its n / 16
+// steps and a call takes 7..14 sweeps, about 4 n^3 flops each; the reduction
+// costs 4/3 n^3, the divide and conquer 8/3 n^3 at most and the products
+// 6 n^3, once.  Calls measured with the sweeps alone and with this phase, in
+// ms: one matrix of order 64 0.78 / 0.48, 128 1.5 / 0.81, 256 3.3 / 1.8, 512
+// 7.1 / 3.8, 1024 21 / 9.7, 2048 80 / 39; 8 of order 512 9.6 / 4.3; 2000 of
+// order 64 5.3 / 2.2, 1000 of 128 15.5 / 3.5, 800 of 256 88 / 12.8.
+// Residuals fall with the number of rotations: rt^T diag(s^2) rt - G from
+// 1e-13 to 1e-15 of the largest eigenvalue.
+//
+// Buffers of a problem: G's strict upper triangle holds the reflectors (row
+// j: v_j from column j + 1; the lower triangle and the diagonal keep G and
+// restore it), x (n x n) the reduced matrix and then the merges' eigenvector
+// matrices U, y (n x n) the permuted rows of a merge and G rt^T, vec the
+// vectors, node records and T factors.
+#include "gemm_tile.hpp"
+#include "prof.hpp"
+#include "tdc.hpp"
+
+#include <algorithm>
+
+namespace syn {
+
+// Vector region of a problem (2048 * half >= 64 n doubles, tjacobi.hpp):
+// rows of n doubles, then the 32 x 32 T factors of the reflector blocks.
+struct Tdc {
+    int n;
+    int64_t ldg, ldr;
+    double *g, *rt, *x, *y;
+    double *d, *e, *tau;       // tridiagonal form and reflector scales
+    double *dd;                // eigenvalues of the current nodes, by row
+    double *dl, *zl, *zh;      // poles, z and recomputed z of the undeflated part
+    double *tr;                // roots relative to their origin pole
+    int *org, *src;            // origin pole of a root; source row of a position
+    int *meta, *nrot;          // undeflated count and rotations of a node (at its first row)
+    int *rp;                   // row pairs of the rotations
+    double *rcs;               // their cosines and sines
+    double *rho;               // rank-one weight of a node (at its first row)
+    int *fail;                 // the direct phase does not apply to this matrix
+    double *tf;                // T factors
+};
+
+__device__ __forceinline__ Tdc tdc_view(const syn_gbj_item &P) {
+    Tdc t;
+    const int64_t n = P.nv, half = tj_dims<16>(n).half;
+    t.n = (int)n;
+    t.ldg = P.ldg;
+    t.ldr = P.ldr;
+    t.g = P.g;
+    t.rt = P.rt;
+    t.x = P.w + tj_g2_off<16>(half, n);
+    t.y = P.w + tj_floor_off<16>(half) + 1;
+    double *w = P.w;
+    t.d = w;
+    t.e = w + n;
+    t.tau = w + 2 * n;
+    t.dd = w + 3 * n;
+    t.dl = w + 4 * n;
+    t.zl = w + 5 * n;
+    t.zh = w + 6 * n;
+    t.tr = w + 7 * n;
+    t.org = (int *)(w + 8 * n);
+    t.src = t.org + n;
+    t.meta = (int *)(w + 9 * n);
+    t.nrot = t.meta + n;
+    t.rp = (int *)(w + 10 * n);
+    t.rcs = w + 11 * n;
+    t.rho = w + 13 * n;
+    t.fail = (int *)(w + 14 * n);
+    t.tf = w + 16 * n;
+    return t;
+}
+
+// Leaves of the divide and conquer (a power of two, at most kLeaf rows each);
+// leaf i starts at row i n / leaves, so sizes differ by one at most.
+constexpr int kLeaf = 16;
+__host__ __device__ __forceinline__ int tdc_leaves(int64_t n) {
+    int l = 1;
+    while ((n + l - 1) / l > kLeaf) l *= 2;
+    return l;
+}
+__device__ __forceinline__ int leaf_start(int n, int leaves, int i) { return (int)((int64_t)i * n / leaves); }
+
+// Rows of node t of a level (level 1 merges pairs of leaves); false when the
+// problem has no such node or takes no direct phase.
+__device__ __forceinline__ bool tdc_node(const Tdc &T, int level, int t, int &lo, int &mid, int &hi) {
+    const int L = tdc_leaves(T.n);
+    if (t >= (L >> level) || *T.fail) return false;
+    lo = leaf_start(T.n, L, t << level);
+    mid = leaf_start(T.n, L, (t << level) + (1 << (level - 1)));
+    hi = leaf_start(T.n, L, (t + 1) << level);
+    return true;
+}
+
+__device__ __forceinline__ double rcp_nr(double x) {
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(r, fma(-x, r, 1.0), r);
+    return fma(r, fma(-x, r, 1.0), r);
+}
+
+__device__ __forceinline__ double rsq_nr(double x) {
+    double y = __builtin_amdgcn_rsq(x);
+    y = fma(0.5 * y, fma(-x * y, y, 1.0), y);
+    return fma(0.5 * y, fma(-x * y, y, 1.0), y);
+}
+
+// Sums over the 16 lanes of a DPP row and over the wave (every lane gets the
+// sum): row rotations in the vector unit and lane reads, a few dozen cycles
+// where a cross-lane exchange through LDS takes about sixty a step.
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, 0xf, 0xf, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, false);
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+__device__ __forceinline__ double row_sum(double v) {
+    v += dpp_f64<0x128>(v);   // row_ror:8, 4, 2, 1
+    v += dpp_f64<0x124>(v);
+    v += dpp_f64<0x122>(v);
+    return v + dpp_f64<0x121>(v);
+}
+__device__ __forceinline__ void opaque(int &x) { asm volatile("" : "+v"(x)); }
+__device__ __forceinline__ double lane_f64(double v, int lane) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, lane);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), lane);
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+__device__ __forceinline__ double all_sum(double v) {
+    v = row_sum(v);
+    return (lane_f64(v, 0) + lane_f64(v, 16)) + (lane_f64(v, 32) + lane_f64(v, 48));
+}
+
+// ---------------------------------------------------------------------------
+// Reduction to tridiagonal form T = H^T G H, the matrix in registers.
+//
+// Step j reflects column j below its diagonal: v (v_j+1 = 1), tau, then
+// p = tau A v, w = p - (tau/2 p.v) v and A <- A - v w^T - w v^T.  A pass over
+// the registers applies step j - 1's v and w and multiplies the result by
+// step j's v at once: column j alone is brought up to date first, from p, v
+// and its value before the pass.  So a step is one exchange of p and of the
+// next column, a few short vector operations that every wave (one
+// work-group) or work-group (several) does for itself, and the pass.
+// ---------------------------------------------------------------------------
+
+// Reflector of a column: alpha = its entry at j + 1, xn2 = the squared norm
+// below.  H alpha = beta e1 (LAPACK's sign), v = column * scal below j + 1.  A
+// column below 1e-145 (the matrix is scaled to order one) counts as zero.
+__device__ __forceinline__ void reflector(double alpha, double xn2, double &beta, double &tau, double &scal) {
+    beta = alpha;
+    tau = scal = 0.0;
+    if (xn2 > 1e-290) {
+        const double h = fma(alpha, alpha, xn2), r = rsq_nr(h), s = h * r, aa = fabs(alpha);
+        beta = -copysign(s, alpha);
+        tau = fma(aa, r, 1.0);
+        scal = copysign(rcp_nr(aa + s), alpha);
+    }
+}
+
+// Power-of-two scale that brings a Gram matrix to order one (its largest
+// entry is on the diagonal); 0 for a zero, tiny, huge or non-finite diagonal,
+// which the Jacobi sweeps take as they did.  Non-finite entries elsewhere end
+// in the leaves' iteration limit.
+__device__ __forceinline__ double gram_scale(const Tdc &T) {
+    double mx = 0.0, bad = 0.0;
+    for (int i = threadIdx.x & 63; i < T.n; i += 64) {
+        const double v = fabs(T.g[i * T.ldg + i]);
+        mx = fmax(mx, v);
+        if (!(v <= 1e280)) bad = 1.0;
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        mx = fmax(mx, __shfl_xor(mx, off, 64));
+        bad = fmax(bad, __shfl_xor(bad, off, 64));
+    }
+    return bad != 0.0 || !(mx > 1e-280) ? 0.0 : ldexp(1.0, -ilogb(mx));
+}
+
+// Orders up to 16 NB, one work-group of NB waves per matrix.  The matrix is
+// symmetric: of its NB x NB tiles of 16 x 16, wave I keeps (I, I - k mod NB),
+// k = 0 .. NB / 2 (the last k in the lower half of the waves only), so each
+// pair of blocks has one tile, every wave the same number, and 256 rows fit
+// the register file of one compute unit.  Lane (li, lk) holds rows lk + 4 r
+// and column li of its tiles.  A tile adds to the product's rows of block I
+// (summed over the wave's tiles, then over li) and, as its transpose, of
+// block J (summed over r and lk, then over the waves by wave 0).  A step is
+// the pass over the tiles by all waves and the short vector work of wave 0,
+// a barrier after each.
+__device__ __forceinline__ double lk_sum(double v) {   // over the four rows of 16 lanes
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const auto l32 = __builtin_amdgcn_permlane32_swap((unsigned)u, (unsigned)u, false, false);
+    const auto h32 = __builtin_amdgcn_permlane32_swap((unsigned)(u >> 32), (unsigned)(u >> 32), false, false);
+    const double s = __builtin_bit_cast(double, (uint64_t)h32[0] << 32 | l32[0]) +
+                     __builtin_bit_cast(double, (uint64_t)h32[1] << 32 | l32[1]);
+    const uint64_t w = __builtin_bit_cast(uint64_t, s);
+    const auto l16 = __builtin_amdgcn_permlane16_swap((unsigned)w, (unsigned)w, false, false);
+    const auto h16 = __builtin_amdgcn_permlane16_swap((unsigned)(w >> 32), (unsigned)(w >> 32), false, false);
+    return __builtin_bit_cast(double, (uint64_t)h16[0] << 32 | l16[0]) +
+           __builtin_bit_cast(double, (uint64_t)h16[1] << 32 | l16[1]);
+}
+
+template <int NB>
+__global__ __launch_bounds__(64 * NB) void td_reduce_kernel(const syn_gbj_item *__restrict__ items, int nlo, int nhi) {
+    constexpr int N = 16 * NB, KT = NB / 2 + 1, E = N / 64;
+    __shared__ double vs[N], ws[N], us[N], colp[NB][KT][16], rowp[N], colx[N];
+    if (items[blockIdx.x].nv <= nlo || items[blockIdx.x].nv > nhi) return;
+    const Tdc T = tdc_view(items[blockIdx.x]);
+    const int n = T.n, tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+    const int I = __builtin_amdgcn_readfirstlane(tid >> 6);   // scalar: tile indices and their tests too
+    const double sc = gram_scale(T);
+    if (tid == 0) *T.fail = sc == 0.0;
+    if (sc == 0.0) return;
+    double a[KT][4];
+#pragma unroll
+    for (int k = 0; k < KT; ++k) {
+        const int J = I >= k ? I - k : I - k + NB;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int i = 16 * I + lk + 4 * r, c = 16 * J + li;
+            a[k][r] = (i < n && c < n && (k < KT - 1 || I < NB / 2)) ? T.g[i * T.ldg + c] * sc : 0.0;
+        }
+    }
+    for (int i = tid; i < N; i += 64 * NB) {
+        vs[i] = ws[i] = us[i] = rowp[i] = 0.0;
+        colx[i] = i < n ? T.g[i] * sc : 0.0;
+    }
+    for (int i = tid; i < NB * KT * 16; i += 64 * NB) (&colp[0][0][0])[i] = 0.0;
+    // every entry is in registers before reflectors overwrite the upper triangle
+    __syncthreads();
+    double tau = 0.0;   // of the previous step, in wave 0
+    for (int j = 0; j < n - 1; ++j) {
+        if (I == 0) {
+            // p of step j - 1 (u still its v), w, column j and its reflector
+            double v[E], p[E], c[E], s = 0.0;
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const int i = lane + 64 * e, B = i >> 4;
+                if (NB > 12) __builtin_amdgcn_sched_barrier(0);
+                double y = rowp[i];
+#pragma unroll
+                for (int k = 1; k < KT; ++k) y += colp[B][k][i & 15];
+                v[e] = us[i];
+                p[e] = i >= j ? tau * y : 0.0;
+                c[e] = colx[i];
+                s = fma(p[e], v[e], s);
+                ws[i] = p[e];
+            }
+            const double kk = 0.5 * tau * all_sum(s);
+            __builtin_amdgcn_wave_barrier();
+            const double vj = us[j], wj = fma(-kk, vj, ws[j]);
+            __builtin_amdgcn_wave_barrier();
+            double xn2 = 0.0;
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const int i = lane + 64 * e;
+                const double w = fma(-kk, v[e], p[e]);
+                c[e] = fma(-w, vj, fma(-v[e], wj, c[e]));
+                if (i > j + 1) xn2 = fma(c[e], c[e], xn2);
+                vs[i] = v[e];
+                ws[i] = w;
+                us[i] = c[e];   // the column: v is its multiple by scal
+            }
+            xn2 = all_sum(xn2);
+            __builtin_amdgcn_wave_barrier();
+            const double dj = us[j], alpha = us[j + 1];
+            __builtin_amdgcn_wave_barrier();
+            double beta, scal;
+            reflector(alpha, xn2, beta, tau, scal);
+            if (lane == 0) {
+                T.d[j] = dj;
+                T.e[j] = j < n - 2 ? beta : alpha;
+                T.tau[j] = tau;
+            }
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const int i = lane + 64 * e;
+                const double x = i <= j ? 0.0 : i == j + 1 ? 1.0 : c[e] * scal;
+                us[i] = x;
+                if (i > j && i < n) T.g[j * T.ldg + i] = x;
+            }
+        }
+        lds_barrier();
+        if (j == n - 2) break;
+        const int jb = (j + 1) >> 4, jl = (j + 1) & 15;
+        // the lane's coordinates anew in every step: the tiles' LDS addresses
+        // are an addition each, and kept across steps they would not fit
+        int li = lane & 15, lk = lane >> 4;
+        opaque(li);
+        opaque(lk);
+        const bool row_live = 16 * I + 15 > j;
+        // A <- A - v w^T - w v^T
+        if (row_live) {
+            double vi[4], wi[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                vi[r] = vs[16 * I + lk + 4 * r];
+                wi[r] = ws[16 * I + lk + 4 * r];
+            }
+#pragma unroll
+            for (int k = 0; k < KT; ++k) {
+                const int J = I >= k ? I - k : I - k + NB;
+                if (NB > 12 && k % 2 == 0) __builtin_amdgcn_sched_barrier(0);   // 1024 threads: loads kept few
+                if (16 * J + 15 <= j || (k == KT - 1 && I >= NB / 2)) continue;
+                const double vj = vs[16 * J + li], wj = ws[16 * J + li];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) a[k][r] = fma(-wi[r], vj, fma(-vi[r], wj, a[k][r]));
+                // the next column, or the row that is its transpose
+                if (J == jb) {
+                    if (li == jl)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) colx[16 * I + lk + 4 * r] = a[k][r];
+                } else if (I == jb) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (lk + 4 * r == jl) colx[16 * J + li] = a[k][r];
+                }
+            }
+        }
+        // y = A u
+        double ui[4], s[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            ui[r] = us[16 * I + lk + 4 * r];
+            s[r] = 0.0;
+        }
+#pragma unroll
+        for (int k = 0; k < KT; ++k) {
+            const int J = I >= k ? I - k : I - k + NB;
+            if (NB > 12 && k % 2 == 0) __builtin_amdgcn_sched_barrier(0);
+            if (16 * J + 15 <= j || (k == KT - 1 && I >= NB / 2)) continue;
+            double t = 0.0;
+            if (row_live) {
+                const double uj = us[16 * J + li];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    s[r] = fma(a[k][r], uj, s[r]);
+                    t = fma(a[k][r], ui[r], t);
+                }
+            }
+            if (k > 0) {
+                t = lk_sum(t);
+                if (lk == 0) colp[J][k][li] = t;
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const double y = row_sum(s[r]);
+            if (li == 0) rowp[16 * I + lk + 4 * r] = y;
+        }
+        lds_barrier();
+    }
+    // the last diagonal entry takes the last step's v and w
+    if (I == (n - 1) >> 4 && li == ((n - 1) & 15)) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (16 * I + lk + 4 * r == n - 1) T.d[n - 1] = fma(-2.0 * ws[n - 1], vs[n - 1], a[0][r]);
+    }
+}
+
+// Orders up to 64 P, several work-groups per matrix: work-group g of S holds
+// columns S (8 q + wave) + g, lane l of a wave rows l + 64 p, so a column's
+// sum stays within its wave.  p and the next column travel through global
+// memory as self-validating words (half of a double beside the step's
+// number, one 64-bit relaxed atomic each): a reader polls the word itself,
+// and no fence or flag orders anything.  Two buffers by step parity: a
+// work-group publishes step j + 1 only after it has read all of step j, so
+// nobody overwrites what is still to be read.  Every wait is bounded: past
+// the limit (another work-group never got a compute unit) the work-group
+// gives up, the matrix counts as failed and the Jacobi sweeps take it.
+constexpr int kMultiThreads = 512;
+constexpr int kMultiWaves = kMultiThreads / 64;
+constexpr int kSpin = 1 << 15;
+constexpr unsigned kGroupedMax = 16;
+
+// words of the exchange: parity, vector (p, column), entry, half; in x, which
+// the reduction does not use otherwise
+__device__ __forceinline__ uint64_t *xword(const Tdc &T, int par, int which, int i) {
+    return (uint64_t *)T.x + ((((int64_t)par * 2 + which) * T.n + i) << 1);
+}
+__device__ __forceinline__ void publish(uint64_t *w, double v, unsigned tag) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v), t = (uint64_t)tag << 32;
+    __hip_atomic_store(w, t | (uint32_t)u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(w + 1, t | (u >> 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint64_t peek(const uint64_t *w) {
+    return __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// work-groups of a matrix
+template <int Q>
+__host__ __device__ __forceinline__ int multi_groups(int64_t n) {
+    return (int)((n + kMultiWaves * Q - 1) / (kMultiWaves * Q));
+}
+
+__global__ __launch_bounds__(256) void td_clear_kernel(const syn_gbj_item *__restrict__ items, int nlo, int nhi) {
+    if (items[blockIdx.x].nv <= nlo || items[blockIdx.x].nv > nhi) return;
+    const Tdc T = tdc_view(items[blockIdx.x]);
+    for (int i = blockIdx.y * 256 + threadIdx.x; i < 8 * T.n; i += gridDim.y * 256) T.x[i] = 0.0;
+    if (blockIdx.y == 0 && threadIdx.x == 0) *T.fail = 0;
+}
+
+template <int P, int Q>
+__global__ __launch_bounds__(kMultiThreads) void td_reduce_multi_kernel(const syn_gbj_item *__restrict__ items,
+                                                                        int n_items, int nlo, int nhi, int S, int grouped) {
+    constexpr int N = 64 * P, NW = kMultiWaves, E = (N + kMultiThreads - 1) / kMultiThreads;
+    __shared__ double v0[2][N], w0[2][N], v1[2][N], red[2][NW], red2[2][NW];
+    __shared__ int gone;
+    // a matrix's work-groups follow each other in the launch, on one XCD
+    // (every eighth work-group) when grouped: those already running never
+    // wait for one behind another matrix's
+    const int k = grouped ? blockIdx.x >> 3 : blockIdx.x, item = grouped ? k / S * 8 + (blockIdx.x & 7) : k / S;
+    const int g = k % S;
+    if (item >= n_items || items[item].nv <= nlo || items[item].nv > nhi) return;
+    const Tdc T = tdc_view(items[item]);
+    const int n = T.n;
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const double sc = gram_scale(T);
+    if (sc == 0.0) {
+        if (g == 0 && tid == 0) *T.fail = 1;
+        return;
+    }
+    double a[P][Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+            const int i = lane + 64 * p, c = S * (NW * q + wv) + g;
+            a[p][q] = (i < n && c < n) ? T.g[c * T.ldg + i] * sc : 0.0;
+        }
+    double v[E], c[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = 0.0;
+    double tau = 0.0;
+    int budget = kSpin;
+    if (tid == 0) gone = 0;
+    for (int i = tid; i < N; i += kMultiThreads) {
+        v1[1][i] = 0.0;
+        v1[0][i] = 0.0;
+    }
+    lds_barrier();
+    for (int j = 0; j < n - 1; ++j) {
+        const int par = j & 1;
+        // p of step j - 1 and column j before it (entries from j on)
+        double p[E], s = 0.0;
+        bool ok = true;
+        if (j == 0) {
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const int i = tid + kMultiThreads * e;
+                p[e] = 0.0;
+                c[e] = i < n ? T.g[i * T.ldg] * sc : 0.0;   // row 0's owner may be past this step
+            }
+        } else {
+            // the words of all entries are asked for together until each is there
+            do {
+                ok = true;
+#pragma unroll
+                for (int e = 0; e < E; ++e) {
+                    const int i = tid + kMultiThreads * e;
+                    p[e] = c[e] = 0.0;
+                    if (i < n && i >= j) {
+                        const uint64_t *wp = xword(T, par, 0, i), *wc = xword(T, par, 1, i);
+                        const uint64_t a0 = peek(wp), a1 = peek(wp + 1), b0 = peek(wc), b1 = peek(wc + 1);
+                        ok = ok && (unsigned)(a0 >> 32) == (unsigned)j && (unsigned)(a1 >> 32) == (unsigned)j &&
+                             (unsigned)(b0 >> 32) == (unsigned)j && (unsigned)(b1 >> 32) == (unsigned)j;
+                        p[e] = __builtin_bit_cast(double, a1 << 32 | (uint32_t)a0);
+                        c[e] = __builtin_bit_cast(double, b1 << 32 | (uint32_t)b0);
+                    }
+                }
+            } while (!ok && --budget > 0);
+        }
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const int i = tid + kMultiThreads * e;
+            s = fma(p[e], v[e], s);
+            if (i < N) w0[par][i] = p[e];   // w below
+        }
+        if (!ok) gone = 1;
+        s = all_sum(s);
+        if (lane == 0) red[par][wv] = s;
+        lds_barrier();
+        if (gone) {
+            if (tid == 0) *T.fail = 1;
+            return;
+        }
+        double kk = 0.0;
+#pragma unroll
+        for (int q = 0; q < NW; ++q) kk += red[par][q];
+        kk *= 0.5 * tau;
+        // v1 of the other parity holds step j - 1's v
+        const double vj = v1[par ^ 1][j], wj = fma(-kk, vj, w0[par][j]);
+        double xn2 = 0.0;
+        lds_barrier();   // w0[par][j] is read as p before it becomes w
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const int i = tid + kMultiThreads * e;
+            const double w = fma(-kk, v[e], p[e]);
+            c[e] = fma(-w, vj, fma(-v[e], wj, c[e]));
+            if (i > j + 1) xn2 = fma(c[e], c[e], xn2);
+            if (i < N) {
+                v0[par][i] = v[e];
+                w0[par][i] = w;
+                v1[par][i] = c[e];   // the column: v is its multiple by scal
+            }
+        }
+        xn2 = all_sum(xn2);
+        if (lane == 0) red2[par][wv] = xn2;
+        lds_barrier();
+        xn2 = 0.0;
+#pragma unroll
+        for (int q = 0; q < NW; ++q) xn2 += red2[par][q];
+        const double dj = v1[par][j], alpha = v1[par][j + 1];
+        double beta, scal;
+        reflector(alpha, xn2, beta, tau, scal);
+        if (tid == 0 && g == 0) {
+            T.d[j] = dj;
+            T.e[j] = j < n - 2 ? beta : alpha;
+            T.tau[j] = tau;
+        }
+        if (j == n - 2) {
+            // the last diagonal entry takes the last step's v and w
+#pragma unroll
+            for (int q = 0; q < Q; ++q)
+#pragma unroll
+                for (int p2 = 0; p2 < P; ++p2)
+                    if (lane + 64 * p2 == n - 1 && S * (NW * q + wv) + g == n - 1)
+                        T.d[n - 1] = fma(-2.0 * w0[par][n - 1], v0[par][n - 1], a[p2][q]);
+            break;
+        }
+        lds_barrier();   // the column has been read: it becomes v
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const int i = tid + kMultiThreads * e;
+            v[e] = i <= j ? 0.0 : i == j + 1 ? 1.0 : c[e] * scal;
+            if (i < N) v1[par][i] = v[e];
+            // row j of the upper triangle was read by its owner alone
+            if (j % S == g && i > j && i < n) T.g[j * T.ldg + i] = v[e];
+        }
+        lds_barrier();
+        double y[Q], vc[Q], wc[Q];
+        int lane = tid & 63;   // addresses of the pass anew in every step, as above
+        opaque(lane);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int cc = S * (NW * q + wv) + g;
+            y[q] = 0.0;
+            vc[q] = cc < n ? v0[par][cc] : 0.0;
+            wc[q] = cc < n ? w0[par][cc] : 0.0;
+        }
+#pragma unroll
+        for (int p2 = 0; p2 < P; ++p2) {
+            if (P > 8 && (p2 & 1) == 0) __builtin_amdgcn_sched_barrier(0);   // row loads not all in flight at once
+            if (64 * p2 + 63 <= j) continue;
+            const int i = lane + 64 * p2;
+            const double vi = v0[par][i], wi = w0[par][i], ui = v1[par][i];
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                a[p2][q] = fma(-wi, vc[q], fma(-vi, wc[q], a[p2][q]));
+                y[q] = fma(a[p2][q], ui, y[q]);
+            }
+        }
+        const unsigned tag = j + 1;
+        uint64_t *xcol = xword(T, par ^ 1, 1, lane);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            if (S * (NW * q + wv) + g != j + 1) continue;
+#pragma unroll
+            for (int p2 = 0; p2 < P; ++p2)
+                if (lane + 64 * p2 > j && lane + 64 * p2 < n) publish(xcol + 128 * p2, a[p2][q], tag);
+        }
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int cc = S * (NW * q + wv) + g;
+            const double t = tau * all_sum(y[q]);
+            if (lane == 0 && cc > j && cc < n) publish(xword(T, par ^ 1, 0, cc), t, tag);
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Leaves: implicit QL (Golub & Van Loan 8.3.3) of the tridiagonal block of at
+// most kLeaf rows, one wave each.  Lane c carries component c of every
+// eigenvector and a copy of the diagonals of its own (no exchange between
+// lanes); the eigenvectors leave as the rows of rt, eigenvalues ascending.
+// The split points' rank-one terms are subtracted here: node boundaries take
+// |e| off the diagonal on both sides.
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(64) void td_leaf_kernel(const syn_gbj_item *__restrict__ items) {
+    __shared__ double sd[kLeaf][64], se[kLeaf][64], q[kLeaf][64];
+    const Tdc T = tdc_view(items[blockIdx.x]);
+    const int L = tdc_leaves(T.n), t = blockIdx.y, c = threadIdx.x;
+    if (t >= L || *T.fail) return;
+    const int lo = leaf_start(T.n, L, t), hi = leaf_start(T.n, L, t + 1), m = hi - lo;
+    for (int i = 0; i < m; ++i) {
+        sd[i][c] = T.d[lo + i];
+        se[i][c] = i + 1 < m ? T.e[lo + i] : 0.0;
+        q[i][c] = i == c ? 1.0 : 0.0;
+    }
+    if (lo > 0) sd[0][c] -= fabs(T.e[lo - 1]);
+    if (hi < T.n) sd[m - 1][c] -= fabs(T.e[hi - 1]);
+    bool ok = true;
+    for (int l = 0; l < m; ++l) {
+        for (int it = 0;; ++it) {
+            int mm = l;
+            for (; mm < m - 1; ++mm)
+                if (fabs(se[mm][c]) <= 1.2e-16 * (fabs(sd[mm][c]) + fabs(sd[mm + 1][c])) + 1e-22) break;
+            if (mm == l) break;
+            if (it == 60) {
+                ok = false;
+                break;
+            }
+            double g = (sd[l + 1][c] - sd[l][c]) / (2.0 * se[l][c]);
+            double r = sqrt(fma(g, g, 1.0));
+            g = sd[mm][c] - sd[l][c] + se[l][c] / (g + copysign(r, g));
+            double s = 1.0, co = 1.0, p = 0.0;
+            int i = mm - 1;
+            for (; i >= l; --i) {
+                const double f = s * se[i][c], b = co * se[i][c], r2 = fma(f, f, g * g);
+                if (!(r2 > 1e-290)) {   // both vanish: the block splits here
+                    sd[i + 1][c] -= p;
+                    se[i + 1][c] = 0.0;
+                    se[mm][c] = 0.0;
+                    break;
+                }
+                const double ir = rsq_nr(r2);
+                se[i + 1][c] = r2 * ir;
+                s = f * ir;
+                co = g * ir;
+                g = sd[i + 1][c] - p;
+                r = fma(sd[i][c] - g, s, 2.0 * co * b);
+                p = s * r;
+                sd[i + 1][c] = g + p;
+                g = fma(co, r, -b);
+                const double z1 = q[i + 1][c], z0 = q[i][c];
+                q[i + 1][c] = fma(s, z0, co * z1);
+                q[i][c] = fma(co, z0, -s * z1);
+            }
+            if (i >= l) continue;
+            sd[l][c] -= p;
+            se[l][c] = g;
+            se[mm][c] = 0.0;
+        }
+    }
+    if (!ok && c == 0) *T.fail = 1;
+    // ascending order, ties by index
+    for (int i = 0; i < m; ++i) {
+        int rk = 0;
+        for (int k = 0; k < m; ++k) rk += (sd[k][c] < sd[i][c]) || (sd[k][c] == sd[i][c] && k < i);
+        if (c < m) T.rt[(int64_t)(lo + rk) * T.ldr + lo + c] = q[i][c];
+        if (c == 0) T.dd[lo + rk] = sd[i][c];
+    }
+    if (c == 0) T.meta[lo] = m;
+}
+
+// ---------------------------------------------------------------------------
+// Merge of two solved halves: D + rho z z^T with z the last row of the first
+// half's Q and the first row of the second's.  This kernel orders the poles
+// (each half brings its roots and its deflated values, two ascending lists
+// each), deflates (a negligible z entry, or two poles whose rotation would
+// leave a negligible off-diagonal entry), and writes the row order, the
+// rotations, the undeflated poles and z.
+// ---------------------------------------------------------------------------
+constexpr int kPrepThreads = 256;
+__host__ __device__ constexpr int64_t prep_lds(int64_t k) { return 2 * k + 3 * ((k + 1) / 2) + 16; }   // doubles
+
+__device__ __forceinline__ int lower_count(const double *a, int lo, int hi, double v, bool with_equal) {
+    const int base = lo;
+    while (lo < hi) {
+        const int m = (lo + hi) >> 1;
+        if (a[m] < v || (with_equal && a[m] == v))
+            lo = m + 1;
+        else
+            hi = m;
+    }
+    return lo - base;
+}
+
+__global__ __launch_bounds__(kPrepThreads) void td_prep_kernel(const syn_gbj_item *__restrict__ items, int level) {
+    extern __shared__ double sm[];
+    __shared__ double red[2][kPrepThreads / 64];
+    __shared__ int scan[kPrepThreads], sh[4];
+    const Tdc T = tdc_view(items[blockIdx.x]);
+    int lo, mid, hi;
+    if (!tdc_node(T, level, blockIdx.y, lo, mid, hi)) return;
+    const int k = hi - lo, n1 = mid - lo, tid = threadIdx.x;
+    double *ds = sm, *zs = sm + k;
+    int *sidx = (int *)(zs + k), *nt = sidx + k, *dfl = nt + k;   // 3 k ints
+    const int K1 = T.meta[lo], K2 = T.meta[mid];
+    const double e = T.e[mid - 1], rho = 2.0 * fabs(e);
+    const int b[5] = {0, K1, n1, n1 + K2, k};
+    for (int i = tid; i < k; i += kPrepThreads) zs[i] = T.dd[lo + i];
+    __syncthreads();
+    double zmax = 0.0, dmax = 0.0;
+    // ranks among the four lists (their values staged in zs)
+    for (int i = tid; i < k; i += kPrepThreads) {
+        const double v = zs[i];
+        const int own = i < b[1] ? 0 : i < b[2] ? 1 : i < b[3] ? 2 : 3;
+        int rk = 0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) rk += q == own ? i - b[q] : lower_count(zs, b[q], b[q + 1], v, q < own);
+        ds[rk] = v;
+        sidx[rk] = i;
+        dmax = fmax(dmax, fabs(v));
+    }
+    __syncthreads();
+    for (int i = tid; i < k; i += kPrepThreads) {
+        const int r = sidx[i];
+        const double z = r < n1 ? T.rt[(int64_t)(lo + r) * T.ldr + mid - 1]
+                                : copysign(1.0, e) * T.rt[(int64_t)(lo + r) * T.ldr + mid];
+        zs[i] = z * 0.70710678118654752440;
+        zmax = fmax(zmax, fabs(zs[i]));
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        zmax = fmax(zmax, __shfl_xor(zmax, off, 64));
+        dmax = fmax(dmax, __shfl_xor(dmax, off, 64));
+    }
+    if ((tid & 63) == 0) {
+        red[0][tid >> 6] = zmax;
+        red[1][tid >> 6] = dmax;
+    }
+    if (tid < 4) sh[tid] = 0;
+    __syncthreads();
+    for (int q = 0; q < kPrepThreads / 64; ++q) {
+        zmax = fmax(zmax, red[0][q]);
+        dmax = fmax(dmax, red[1][q]);
+    }
+    const double tol = 8.0 * 1.1102230246251565e-16 * fmax(dmax, zmax);
+    // the entries that stay, in order (nt), and the negligible ones (dfl)
+    const int per = (k + kPrepThreads - 1) / kPrepThreads, i0 = tid * per, i1 = i0 + per < k ? i0 + per : k;
+    int cnt = 0;
+    for (int i = i0; i < i1; ++i) cnt += rho * fabs(zs[i]) > tol;
+    scan[tid] = cnt;
+    __syncthreads();
+    for (int off = 1; off < kPrepThreads; off <<= 1) {
+        const int a = tid >= off ? scan[tid - off] : 0;
+        __syncthreads();
+        scan[tid] += a;
+        __syncthreads();
+    }
+    const int n_nt = scan[kPrepThreads - 1];
+    int at = scan[tid] - cnt;
+    for (int i = i0; i < i1; ++i) {
+        if (rho * fabs(zs[i]) > tol)
+            nt[at++] = i;
+        else
+            dfl[i - at] = i;
+    }
+    __syncthreads();
+    // two neighbouring poles so close that a rotation deflates one of them
+    for (int q = tid; q + 1 < n_nt; q += kPrepThreads) {
+        const double s = zs[nt[q]], c = zs[nt[q + 1]], t = ds[nt[q + 1]] - ds[nt[q]];
+        if (fabs(t * c * s) <= tol * fma(c, c, s * s)) sh[0] = 1;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        int K = n_nt, nr = 0, nd = k - n_nt;
+        if (sh[0]) {
+            K = 0;
+            int pj = nt[0];
+            for (int q = 1; q < n_nt; ++q) {
+                const int j = nt[q];
+                const double s0 = zs[pj], c0 = zs[j], t = ds[j] - ds[pj], h2 = fma(c0, c0, s0 * s0);
+                if (fabs(t * c0 * s0) <= tol * h2) {
+                    const double ih = 1.0 / sqrt(h2), c = c0 * ih, s = -s0 * ih;
+                    zs[j] = h2 * ih;
+                    zs[pj] = 0.0;
+                    const double dp = ds[pj], dj = ds[j];
+                    ds[j] = fma(dp * s, s, dj * c * c);
+                    ds[pj] = fma(dp * c, c, dj * s * s);
+                    T.rp[2 * (lo + nr)] = pj;
+                    T.rp[2 * (lo + nr) + 1] = j;
+                    T.rcs[2 * (lo + nr)] = c;
+                    T.rcs[2 * (lo + nr) + 1] = s;
+                    ++nr;
+                    dfl[nd++] = pj;
+                } else {
+                    nt[K++] = pj;   // K <= q: behind the entries still to come
+                }
+                pj = j;
+            }
+            nt[K++] = pj;
+        }
+        sh[1] = K;
+        sh[2] = nr;
+    }
+    __syncthreads();
+    const int K = sh[1], nr = sh[2], nd = k - K;
+    // positions: undeflated first, then the deflated ones ascending
+    for (int q = tid; q < K; q += kPrepThreads) {
+        T.dl[lo + q] = ds[nt[q]];
+        T.zl[lo + q] = zs[nt[q]];
+        T.src[lo + q] = sidx[nt[q]];
+    }
+    for (int q = tid; q < nd; q += kPrepThreads) {
+        const double v = ds[dfl[q]];
+        int rk = 0;
+        for (int u = 0; u < nd; ++u) {
+            const double o = ds[dfl[u]];
+            rk += o < v || (o == v && u < q);
+        }
+        T.dd[lo + K + rk] = v;
+        T.src[lo + K + rk] = sidx[dfl[q]];
+    }
+    __syncthreads();
+    // the rotations act on source rows
+    for (int q = tid; q < nr; q += kPrepThreads) {
+        T.rp[2 * (lo + q)] = sidx[T.rp[2 * (lo + q)]];
+        T.rp[2 * (lo + q) + 1] = sidx[T.rp[2 * (lo + q) + 1]];
+    }
+    if (tid == 0) {
+        T.meta[lo] = K;
+        T.nrot[lo] = nr;
+        T.rho[lo] = rho;
+    }
+}
+
+// Rows of a node into their merge order (rt -> y, the half a row does not
+// reach zero), after the deflating rotations.  A work-group takes 64 columns
+// of the node: the rotations act on rows, so its columns are its own.
+__global__ __launch_bounds__(256) void td_copy_kernel(const syn_gbj_item *__restrict__ items, int level) {
+    const Tdc T = tdc_view(items[blockIdx.x]);
+    int lo, mid, hi;
+    if (!tdc_node(T, level, blockIdx.z, lo, mid, hi)) return;
+    const int k = hi - lo, n = T.n, c = blockIdx.y * 64 + (threadIdx.x & 63), rg = threadIdx.x >> 6;
+    const int nr = T.nrot[lo];
+    if ((int)blockIdx.y * 64 >= k) return;
+    double *rt = T.rt + (int64_t)lo * T.ldr + lo;
+    if (nr) {
+        // the halves' zero blocks become rows that the rotations fill
+        if (c < k)
+            for (int i = rg; i < k; i += 4)
+                if ((i < mid - lo) != (c < mid - lo)) rt[i * T.ldr + c] = 0.0;
+        __syncthreads();
+        if (rg == 0 && c < k) {
+            for (int q = 0; q < nr; ++q) {
+                double *p = rt + T.rp[2 * (lo + q)] * T.ldr + c, *r = rt + T.rp[2 * (lo + q) + 1] * T.ldr + c;
+                const double co = T.rcs[2 * (lo + q)], s = T.rcs[2 * (lo + q) + 1], xv = *p, yv = *r;
+                *p = fma(co, xv, s * yv);
+                *r = fma(co, yv, -s * xv);
+            }
+        }
+        __syncthreads();
+    }
+    if (c >= k) return;
+    double *y = T.y + (int64_t)lo * n + lo;
+    for (int i = rg; i < k; i += 4) {
+        const int s = T.src[lo + i];
+        const bool in = nr || (s < mid - lo) == (c < mid - lo);
+        y[(int64_t)i * n + c] = in ? rt[s * T.ldr + c] : 0.0;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Secular equation 1 + sum_i a_i / (d_i - lambda) = 0, a_i = rho z_i^2, one
+// thread per root, poles in LDS.  A root is kept as its distance tau to the
+// nearer pole (its origin), so d_i - lambda = (d_i - d_origin) - tau has no
+// cancellation.  Iteration: the rational interpolation through the two poles
+// around the root (Li 1993, the middle way), safeguarded by a bracket that
+// every evaluation shrinks; it stops at the rounding level of the sum or of
+// the bracket.
+// ---------------------------------------------------------------------------
+constexpr int kSecThreads = 64;
+
+__device__ __forceinline__ void secular_sums(const double *dl, const double *a, int K, int j, double dorg, double tau,
+                                             double &psi, double &dpsi, double &phi, double &dphi) {
+    psi = dpsi = phi = dphi = 0.0;
+    for (int i = 0; i < K; ++i) {
+        const double r = rcp_nr((dl[i] - dorg) - tau), t = a[i] * r, tt = t * r;
+        const bool left = i <= j;
+        psi += left ? t : 0.0;
+        dpsi += left ? tt : 0.0;
+        phi += left ? 0.0 : t;
+        dphi += left ? 0.0 : tt;
+    }
+}
+
+__device__ __forceinline__ bool secular_root(const double *dl, const double *a, int K, int j, double asum, int &org,
+                                             double &tau) {
+    org = j;
+    if (K == 1) {
+        tau = a[0];
+        return true;
+    }
+    const bool last = j == K - 1;
+    const int jl = last ? K - 2 : j, jr = jl + 1;   // the poles of the interpolation
+    double lo, hi, psi, dpsi, phi, dphi;
+    if (last) {
+        lo = 0.0;
+        hi = asum;
+        tau = 0.5 * hi;
+    } else {
+        const double gap = dl[j + 1] - dl[j], mid = 0.5 * gap;
+        secular_sums(dl, a, K, jl, dl[j], mid, psi, dpsi, phi, dphi);
+        const double f = 1.0 + psi + phi, aj = a[j], ar = a[j + 1];
+        // the two poles' model with the other terms at their midpoint value
+        const double c = f + (aj - ar) / mid;
+        if (f >= 0.0) {
+            lo = 0.0;
+            hi = mid;
+            const double b = fma(c, gap, aj + ar), q = aj * gap, ds = sqrt(fmax(fma(b, b, -4.0 * c * q), 0.0));
+            tau = b > 0.0 ? 2.0 * q / (b + ds) : (b - ds) / (2.0 * c);
+        } else {
+            org = j + 1;
+            lo = -mid;
+            hi = 0.0;
+            const double b = fma(-c, gap, aj + ar), q = ar * gap, ds = sqrt(fmax(fma(b, b, 4.0 * c * q), 0.0));
+            tau = b > 0.0 ? -2.0 * q / (b + ds) : (b - ds) / (2.0 * c);
+        }
+        if (!(tau > lo && tau < hi)) tau = 0.5 * (lo + hi);
+    }
+    const double dorg = dl[org], eps = 1.1102230246251565e-16;
+    for (int it = 0; it < 200; ++it) {
+        secular_sums(dl, a, K, jl, dorg, tau, psi, dpsi, phi, dphi);
+        const double f = 1.0 + psi + phi;
+        if (fabs(f) <= eps * (8.0 * (fabs(psi) + fabs(phi)) + 2.0 + fabs(tau) * (dpsi + dphi))) return true;
+        if (f < 0.0)
+            lo = tau;
+        else
+            hi = tau;
+        if (hi - lo <= 2.0 * eps * fmax(fabs(lo), fabs(hi))) return true;
+        const double d1 = (dl[jl] - dorg) - tau, d2 = (dl[jr] - dorg) - tau;
+        const double c = f - d1 * dpsi - d2 * dphi, am = (d1 + d2) * f - d1 * d2 * (dpsi + dphi), b = d1 * d2 * f;
+        const double ds = sqrt(fmax(fma(am, am, -4.0 * b * c), 0.0));
+        double eta;
+        if (last)
+            eta = am >= 0.0 ? (am + ds) / (2.0 * c) : 2.0 * b / (am - ds);
+        else
+            eta = am <= 0.0 ? (am - ds) / (2.0 * c) : 2.0 * b / (am + ds);
+        if (!(f * eta < 0.0)) eta = -f / (dpsi + dphi);
+        double nx = tau + eta;
+        if (!(nx > lo && nx < hi) || (it > 12 && (it & 1)))
+            nx = lo == 0.0 ? 0.0625 * hi : hi == 0.0 ? 0.0625 * lo : 0.5 * (lo + hi);
+        if (nx == tau) return true;
+        tau = nx;
+    }
+    return false;
+}
+
+__global__ __launch_bounds__(kSecThreads) void td_secular_kernel(const syn_gbj_item *__restrict__ items, int level) {
+    extern __shared__ double sm[];
+    const Tdc T = tdc_view(items[blockIdx.x]);
+    int lo, mid, hi;
+    if (!tdc_node(T, level, blockIdx.z, lo, mid, hi)) return;
+    const int K = T.meta[lo], tid = threadIdx.x, j = blockIdx.y * kSecThreads + tid;
+    if ((int)blockIdx.y * kSecThreads >= K) return;
+    double *dl = sm, *a = sm + K;
+    const double rho = T.rho[lo];
+    double asum = 0.0;
+    for (int i = tid; i < K; i += kSecThreads) {
+        dl[i] = T.dl[lo + i];
+        const double z = T.zl[lo + i];
+        a[i] = rho * z * z;
+        asum += a[i];
+    }
+    asum = wave_sum(asum);
+    __syncthreads();
+    if (j >= K) return;
+    int org;
+    double tau;
+    const bool ok = secular_root(dl, a, K, j, asum * (1.0 + 1e-15), org, tau);
+    if (!ok) *T.fail = 1;
+    T.org[lo + j] = org;
+    T.tr[lo + j] = tau;
+    T.dd[lo + j] = dl[org] + tau;
+}
+
+// z recomputed from the roots (the z whose secular equation has exactly
+// these roots), one thread per entry: z_i^2 = prod_j (lambda_j - d_i) over
+// prod_{j != i} (d_j - d_i), up to a constant factor.
+__global__ __launch_bounds__(kSecThreads) void td_zhat_kernel(const syn_gbj_item *__restrict__ items, int level) {
+    extern __shared__ double sm[];
+    const Tdc T = tdc_view(items[blockIdx.x]);
+    int lo, mid, hi;
+    if (!tdc_node(T, level, blockIdx.z, lo, mid, hi)) return;
+    const int K = T.meta[lo], tid = threadIdx.x, i = blockIdx.y * kSecThreads + tid;
+    if ((int)blockIdx.y * kSecThreads >= K) return;
+    double *dl = sm, *od = sm + K, *tr = od + K;
+    for (int q = tid; q < K; q += kSecThreads) {
+        dl[q] = T.dl[lo + q];
+        od[q] = T.dl[lo + T.org[lo + q]];
+        tr[q] = T.tr[lo + q];
+    }
+    __syncthreads();
+    if (i >= K) return;
+    const double di = dl[i];
+    double prod = (od[i] - di) + tr[i];
+    for (int j = 0; j < K; ++j)
+        if (j != i) prod *= ((od[j] - di) + tr[j]) * rcp_nr(dl[j] - di);
+    T.zh[lo + i] = copysign(sqrt(fabs(prod)), T.zl[lo + i]);
+}
+
+// Rows of U^T (eigenvectors of D + rho z z^T, unit norm) into x, a wave per
+// root; the deflated rows go back from y to rt as they are.
+__global__ __launch_bounds__(256) void td_vec_kernel(const syn_gbj_item *__restrict__ items, int level) {
+    const Tdc T = tdc_view(items[blockIdx.x]);
+    int lo, mid, hi;
+    if (!tdc_node(T, level, blockIdx.z, lo, mid, hi)) return;
+    const int K = T.meta[lo], k = hi - lo, n = T.n, lane = threadIdx.x & 63;
+    const int j = blockIdx.y * 4 + (threadIdx.x >> 6);
+    if (j >= k) return;
+    if (j >= K) {
+        const double *y = T.y + (int64_t)(lo + j) * n + lo;
+        double *r = T.rt + (int64_t)(lo + j) * T.ldr + lo;
+        for (int c = lane; c < k; c += 64) r[c] = y[c];
+        return;
+    }
+    const double od = T.dl[lo + T.org[lo + j]], tr = T.tr[lo + j];
+    double s = 0.0;
+    for (int i = lane; i < K; i += 64) {
+        const double u = T.zh[lo + i] * rcp_nr((T.dl[lo + i] - od) - tr);
+        s = fma(u, u, s);
+    }
+    s = rsq_nr(wave_sum(s));
+    double *x = T.x + (int64_t)(lo + j) * n + lo;
+    for (int i = lane; i < K; i += 64) x[i] = T.zh[lo + i] * rcp_nr((T.dl[lo + i] - od) - tr) * s;
+}
+
+// ---------------------------------------------------------------------------
+// Products on the 64 x 64 MFMA tile: the merge's rt = U^T y (what 0), and
+// with the back-transformed rt: y = G rt^T (1), G = rt y (2).  blockIdx.y
+// is the tile, blockIdx.z the node.
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(256, 2) void td_gemm_kernel(const syn_gbj_item *__restrict__ items, int what,
+                                                         int level) {
+    const Tdc T = tdc_view(items[blockIdx.x]);
+    const int n = T.n;
+    syn_gemm_item P;
+    P.alpha = 1.0;
+    P.beta = 0.0;
+    P.transA = P.transB = 0;
+    P.tri = 0;
+    P.block_start = 0;
+    if (what == 0) {
+        int lo, mid, hi;
+        if (!tdc_node(T, level, blockIdx.z, lo, mid, hi)) return;
+        const int K = T.meta[lo];
+        P.A = T.x + (int64_t)lo * n + lo;
+        P.B = T.y + (int64_t)lo * n + lo;
+        P.C = T.rt + (int64_t)lo * T.ldr + lo;
+        P.lda = P.ldb = n;
+        P.ldc = T.ldr;
+        P.m = P.k = K;
+        P.n = hi - lo;
+    } else {
+        if (*T.fail) return;
+        P.m = P.n = P.k = n;
+        if (what == 1) {
+            P.A = T.g;
+            P.lda = T.ldg;
+            P.B = T.rt;
+            P.ldb = T.ldr;
+            P.transB = 1;
+            P.C = T.y;
+            P.ldc = n;
+        } else {
+            P.A = T.rt;
+            P.lda = T.ldr;
+            P.B = T.y;
+            P.ldb = n;
+            P.C = T.g;
+            P.ldc = T.ldg;
+        }
+    }
+    P.tiles_n = (P.n + 63) / 64;
+    if (blockIdx.y >= P.tiles_n * ((P.m + 63) / 64)) return;
+    __shared__ GemmSmem<64, 64, 16, double> smem;
+    if (what == 1)
+        gemm_f64_tile_t<64, 64, 16, 32, 32, false, true, double>(P, blockIdx.y, smem, 0, INT64_MAX);
+    else
+        gemm_f64_tile_t<64, 64, 16, 32, 32, false, false, double>(P, blockIdx.y, smem, 0, INT64_MAX);
+}
+
+// ---------------------------------------------------------------------------
+// Back-transformation rt <- rt (I - V T^T V^T) block by block from the last:
+// the T factor of each block of 32 reflectors (LAPACK dlarft, forward,
+// columnwise), then one work-group per 32 rows of rt walks the blocks.
+// ---------------------------------------------------------------------------
+constexpr int kBlk = 32;
+__host__ __device__ __forceinline__ int refl_blocks(int n) { return (n - 2 + kBlk - 1) / kBlk; }
+
+__global__ __launch_bounds__(256) void td_tfac_kernel(const syn_gbj_item *__restrict__ items) {
+    __shared__ double vs[kBlk][65], S[kBlk][kBlk + 1], F[kBlk][kBlk + 1];
+    const Tdc T = tdc_view(items[blockIdx.x]);
+    const int n = T.n, j0 = blockIdx.y * kBlk, nb = n - 2 - j0 < kBlk ? n - 2 - j0 : kBlk, tid = threadIdx.x;
+    if (nb <= 0 || *T.fail) return;
+    const int a = tid >> 3, c0 = (tid & 7) * 4;
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int k0 = j0 + 1; k0 < n; k0 += 64) {
+        __syncthreads();
+        for (int e = tid; e < kBlk * 64; e += 256) {
+            const int r = e >> 6, k = k0 + (e & 63);
+            vs[r][e & 63] = (r < nb && k > j0 + r && k < n) ? T.g[(int64_t)(j0 + r) * T.ldg + k] : 0.0;
+        }
+        __syncthreads();
+        for (int k = 0; k < 64; ++k)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) acc[q] = fma(vs[a][k], vs[c0 + q][k], acc[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) S[a][c0 + q] = acc[q];
+    for (int e = tid; e < kBlk * kBlk; e += 256) F[e / kBlk][e % kBlk] = 0.0;
+    __syncthreads();
+    for (int j = 0; j < nb; ++j) {
+        const double tau = T.tau[j0 + j];
+        if (tid < j) {
+            double s = 0.0;
+            for (int l = tid; l < j; ++l) s = fma(F[tid][l], S[l][j], s);
+            F[tid][j] = -tau * s;
+        } else if (tid == j) {
+            F[j][j] = tau;
+        }
+        __syncthreads();
+    }
+    double *tf = T.tf + (int64_t)blockIdx.y * kBlk * kBlk;
+    for (int e = tid; e < kBlk * kBlk; e += 256) tf[e] = F[e / kBlk][e % kBlk];
+}
+
+__global__ __launch_bounds__(256) void td_back_kernel(const syn_gbj_item *__restrict__ items) {
+    __shared__ double Yp[4][kBlk][kBlk + 1], Z[kBlk][kBlk + 1], F[kBlk][kBlk + 1];
+    const Tdc T = tdc_view(items[blockIdx.x]);
+    const int n = T.n, r0 = blockIdx.y * 32;
+    if (r0 >= n || *T.fail) return;
+    const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+    for (int b = refl_blocks(n) - 1; b >= 0; --b) {
+        const int j0 = b * kBlk, nb = n - 2 - j0 < kBlk ? n - 2 - j0 : kBlk, cs = j0 + 1;
+        __syncthreads();   // Yp, Z and F of the previous block are free
+        const double *tf = T.tf + (int64_t)b * kBlk * kBlk;
+        for (int e = tid; e < kBlk * kBlk; e += 256) F[e / kBlk][e % kBlk] = tf[e];
+        // Y = rt V^T-rows over this wave's chunks of 16 columns: lane lk
+        // takes four consecutive columns of each chunk, element s of every
+        // lane in the s-th MFMA (the same columns in both operands)
+        v4d acc[2][2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
+        for (int k0 = cs + 16 * wv; k0 < n; k0 += 64) {
+            const int k = k0 + 4 * lk;
+            double q[2][4], v[2][4];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int row = r0 + 16 * i + li, ref = 16 * i + li;
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    const bool in = k + s < n;
+                    q[i][s] = (in && row < n) ? T.rt[(int64_t)row * T.ldr + k + s] : 0.0;
+                    v[i][s] = (in && ref < nb && k + s > j0 + ref) ? T.g[(int64_t)(j0 + ref) * T.ldg + k + s] : 0.0;
+                }
+            }
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(q[i][s], v[j][s], acc[i][j], 0, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) Yp[wv][16 * i + lk + 4 * r][16 * j + li] = acc[i][j][r];
+        __syncthreads();
+        for (int e = tid; e < kBlk * kBlk; e += 256) {
+            const int i = e / kBlk, j = e % kBlk;
+            Yp[0][i][j] = (Yp[0][i][j] + Yp[1][i][j]) + (Yp[2][i][j] + Yp[3][i][j]);
+        }
+        __syncthreads();
+        // Z = Y T^T, T upper triangular
+        for (int e = tid; e < kBlk * kBlk; e += 256) {
+            const int i = e / kBlk, a = e % kBlk;
+            double s = 0.0;
+            for (int c = a; c < kBlk; ++c) s = fma(Yp[0][i][c], F[a][c], s);
+            Z[i][a] = s;
+        }
+        __syncthreads();
+        // rt -= Z V, 16 columns of both row tiles at a time
+        for (int c0 = cs + 16 * wv; c0 < n; c0 += 64) {
+            const int col = c0 + li;
+            v4d o[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int row = r0 + 16 * i + lk + 4 * r;
+                    o[i][r] = (row < n && col < n) ? T.rt[(int64_t)row * T.ldr + col] : 0.0;
+                }
+#pragma unroll
+            for (int k0 = 0; k0 < kBlk; k0 += 4) {
+                const int ref = k0 + lk;
+                const double v =
+                    (ref < nb && col < n && col > j0 + ref) ? T.g[(int64_t)(j0 + ref) * T.ldg + col] : 0.0;
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    o[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(-Z[16 * i + li][k0 + lk], v, o[i], 0, 0, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int row = r0 + 16 * i + lk + 4 * r;
+                    if (row < n && col < n) T.rt[(int64_t)row * T.ldr + col] = o[i][r];
+                }
+        }
+    }
+}
+
+// G's upper triangle back from the lower one (the reflectors are used up),
+// a 32 x 32 tile pair per work-group; where the phase does not apply, rt is
+// the identity the Jacobi sweeps start from.
+__global__ __launch_bounds__(256) void td_restore_kernel(const syn_gbj_item *__restrict__ items) {
+    __shared__ double s[32][33];
+    const Tdc T = tdc_view(items[blockIdx.x]);
+    const int n = T.n, nt = (n + 31) / 32;
+    int bi = 0, t = blockIdx.y;
+    if (t >= nt * (nt + 1) / 2) return;
+    while (t > bi) t -= ++bi;   // tile (bi, t), t <= bi
+    const int r0 = 32 * bi, c0 = 32 * t, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    for (int i = ty; i < 32; i += 8)
+        s[i][tx] = (r0 + i < n && c0 + tx < n) ? T.g[(int64_t)(r0 + i) * T.ldg + c0 + tx] : 0.0;
+    __syncthreads();
+    for (int i = ty; i < 32; i += 8) {
+        const int r = c0 + i, c = r0 + tx;
+        if (r < n && c < n && c > r) T.g[(int64_t)r * T.ldg + c] = s[tx][i];
+    }
+    if (*T.fail) {
+        for (int i = ty; i < 32; i += 8) {
+            if (r0 + i < n && c0 + tx < n) T.rt[(int64_t)(r0 + i) * T.ldr + c0 + tx] = (r0 + i == c0 + tx) ? 1.0 : 0.0;
+            if (c0 + i < n && r0 + tx < n) T.rt[(int64_t)(c0 + i) * T.ldr + r0 + tx] = (c0 + i == r0 + tx) ? 1.0 : 0.0;
+        }
+    }
+}
+
+// largest order of the class (nlo, nhi], 0 if it has none
+static int64_t class_max(const std::vector<syn_gbj_item> &host, int nlo, int nhi) {
+    int64_t m = 0;
+    for (const syn_gbj_item &it : host)
+        if (it.nv > nlo && it.nv <= nhi) m = std::max(m, it.nv);
+    return m;
+}
+
+template <int NB>
+static int reduce_single(const syn_gbj_item *items, const std::vector<syn_gbj_item> &host, int nlo, hipStream_t st) {
+    if (!class_max(host, nlo, 16 * NB)) return SYN_OK;
+    hipLaunchKernelGGL(td_reduce_kernel<NB>, dim3((unsigned)host.size()), dim3(64 * NB), 0, st, items, nlo, 16 * NB);
+    SYN_LAUNCH_CHECK("tridiagonal reduction");
+    return SYN_OK;
+}
+
+template <int P, int Q>
+static int reduce_multi(const syn_gbj_item *items, const std::vector<syn_gbj_item> &host, int nlo, hipStream_t st) {
+    const int nhi = 64 * P;
+    const int64_t nmax = class_max(host, nlo, nhi);
+    if (!nmax) return SYN_OK;
+    const unsigned ni = (unsigned)host.size(), S = (unsigned)multi_groups<Q>(nmax);
+    hipLaunchKernelGGL(td_clear_kernel, dim3(ni, (unsigned)((8 * nmax + 255) / 256)), dim3(256), 0, st, items, nlo, nhi);
+    // up to 16 work-groups of a matrix on one XCD, more over all of them
+    const int grouped = S <= kGroupedMax;
+    const unsigned grid = (grouped ? (ni + 7) / 8 * 8 : ni) * S;
+    hipLaunchKernelGGL((td_reduce_multi_kernel<P, Q>), dim3(grid), dim3(kMultiThreads), 0, st, items, (int)ni, nlo, nhi,
+                       (int)S, grouped);
+    SYN_LAUNCH_CHECK("tridiagonal reduction over work-groups");
+    return SYN_OK;
+}
+
+bool tdc_takes(int64_t nv) { return nv >= kTdcMin && nv <= kTdcMax; }
+
+int tdc_launch(const syn_gbj_item *items, const std::vector<syn_gbj_item> &host, hipStream_t st) {
+    const unsigned ni = (unsigned)host.size();
+    int64_t nmax = 0;
+    int levels = 0, lmax = 1;
+    for (const syn_gbj_item &it : host) {
+        nmax = std::max(nmax, it.nv);
+        const int L = tdc_leaves(it.nv);
+        lmax = std::max(lmax, L);
+    }
+    while ((1 << levels) < lmax) ++levels;
+    if (int rc = reduce_single<4>(items, host, 0, st)) return rc;
+    if (int rc = reduce_single<8>(items, host, 64, st)) return rc;
+    if (int rc = reduce_single<12>(items, host, 128, st)) return rc;
+    if (int rc = reduce_single<16>(items, host, 192, st)) return rc;
+    if (int rc = reduce_multi<8, 4>(items, host, 256, st)) return rc;
+    if (int rc = reduce_multi<16, 2>(items, host, 512, st)) return rc;
+    if (int rc = reduce_multi<32, 2>(items, host, 1024, st)) return rc;
+    const unsigned nblk = (unsigned)refl_blocks((int)nmax);
+    hipLaunchKernelGGL(td_tfac_kernel, dim3(ni, nblk), dim3(256), 0, st, items);
+    hipLaunchKernelGGL(td_leaf_kernel, dim3(ni, (unsigned)lmax), dim3(64), 0, st, items);
+    for (int l = 1; l <= levels; ++l) {
+        // the largest node of the level and how many the largest problem has
+        int64_t k = 0;
+        for (const syn_gbj_item &it : host) {
+            const int64_t L = tdc_leaves(it.nv);
+            if ((L >> l) > 0) k = std::max(k, ((it.nv << l) + L - 1) / L);
+        }
+        const unsigned nodes = (unsigned)(lmax >> l), c64 = (unsigned)((k + 63) / 64);
+        const size_t plds = (size_t)prep_lds(k) * sizeof(double), slds = (size_t)k * 2 * sizeof(double);
+        hipLaunchKernelGGL(td_prep_kernel, dim3(ni, nodes), dim3(kPrepThreads), plds, st, items, l);
+        hipLaunchKernelGGL(td_copy_kernel, dim3(ni, c64, nodes), dim3(256), 0, st, items, l);
+        hipLaunchKernelGGL(td_secular_kernel, dim3(ni, c64, nodes), dim3(kSecThreads), slds, st, items, l);
+        hipLaunchKernelGGL(td_zhat_kernel, dim3(ni, c64, nodes), dim3(kSecThreads), slds + slds / 2, st, items, l);
+        hipLaunchKernelGGL(td_vec_kernel, dim3(ni, (unsigned)((k + 3) / 4), nodes), dim3(256), 0, st, items, l);
+        hipLaunchKernelGGL(td_gemm_kernel, dim3(ni, c64 * c64, nodes), dim3(256), 0, st, items, 0, l);
+        SYN_LAUNCH_CHECK("divide and conquer");
+    }
+    const unsigned t32 = (unsigned)((nmax + 31) / 32), t64 = (unsigned)((nmax + 63) / 64);
+    hipLaunchKernelGGL(td_back_kernel, dim3(ni, t32), dim3(256), 0, st, items);
+    hipLaunchKernelGGL(td_restore_kernel, dim3(ni, t32 * (t32 + 1) / 2), dim3(256), 0, st, items);
+    hipLaunchKernelGGL(td_gemm_kernel, dim3(ni, t64 * t64), dim3(256), 0, st, items, 1, 0);
+    hipLaunchKernelGGL(td_gemm_kernel, dim3(ni, t64 * t64), dim3(256), 0, st, items, 2, 0);
+    SYN_LAUNCH_CHECK("direct phase");
+    return SYN_OK;
+}
+
+}  // namespace syn

@@ -16,6 +16,10 @@
 //           slab of the accumulated eigenvector rows, on the f64 MFMA with
 //           the operands in registers.
 //
+// Matrices of an order that the direct phase takes (tdc.hip) come to the
+// sweeps already diagonal to rounding, and mostly pass the test below at once;
+// the sweeps are for the rest.
+//
 // A step is one launch, the solves of step s beside the updates of step
 // s - 1, and several problems share every launch.  A pair whose tile has no
 // |G_ik| > max(tol sqrt(|G_ii G_kk|), eps max_j G_jj) among the planes it
@@ -27,6 +31,7 @@
 // form, with the planes in the cyclic-by-blocks order.
 #include "common.hpp"
 #include "prof.hpp"
+#include "tdc.hpp"
 
 #include <algorithm>
 #include <cstring>
@@ -39,7 +44,6 @@ namespace syn {
 // has TP = 2 TB rows.  The pair solve uses one thread per 2 x 2 block of a
 // round, (TP/2)^2 threads; an update work-group four waves.
 constexpr int kTUpdThreads = 256;    // four waves per update work-group
-constexpr int kTCol = 64;            // columns of an rt slab
 
 typedef double v4d __attribute__((ext_vector_type(4)));
 typedef double v2d __attribute__((ext_vector_type(2)));
@@ -143,28 +147,6 @@ __device__ __forceinline__ void rotation(double apq, double app, double aqq, dou
     s = c * t;
 }
 
-struct TjDims {
-    int64_t nblk, np, half, ncs;
-};
-
-// rt slab width: the fused 16-row steps give each wave two groups of 16
-// columns (fewer, fuller work-groups, so a launch of a few large problems
-// fits one round of resident work-groups); the 32-row updates one
-template <int TB>
-__host__ __device__ constexpr int tj_slab_cols() {
-    return TB == 16 ? 2 * kTCol : kTCol;
-}
-
-template <int TB>
-__host__ __device__ __forceinline__ TjDims tj_dims(int64_t nv) {
-    TjDims d;
-    d.nblk = (nv + TB - 1) / TB;
-    d.np = d.nblk + (d.nblk & 1);
-    d.half = d.np / 2;
-    d.ncs = (nv + tj_slab_cols<TB>() - 1) / tj_slab_cols<TB>();
-    return d;
-}
-
 // Update work of a problem at a step: the upper-triangle G tiles (a, b),
 // a <= b, two per work-group (each by two waves, one per 16-column half),
 // then one work-group per rt slab of tj_slab_cols columns.
@@ -211,21 +193,6 @@ __device__ __forceinline__ double *tj_wset(const syn_gbj_item &P, int64_t half, 
 template <int TB>
 __device__ __forceinline__ int *tj_flags(const syn_gbj_item &P, int64_t half, int par = 0) {
     return (int *)(P.w + 2 * half * (2 * TB) * (2 * TB)) + par * half;
-}
-
-// Absolute rotation floor eps * max_i G_ii (set by the init kernel): Gram
-// entries below it are at the rounding level of forming G, so rotating them
-// changes nothing that the Gram route can resolve, and in a rank-deficient G
-// (a null space at noise level) a purely relative test would never settle.
-template <int TB>
-__host__ __device__ __forceinline__ int64_t tj_floor_off(int64_t half) {
-    return 2 * half * (2 * TB) * (2 * TB) + half;
-}
-
-// the second Gram buffer (ld nv), after the sort scratch
-template <int TB>
-__host__ __device__ __forceinline__ int64_t tj_g2_off(int64_t half, int64_t nv) {
-    return tj_floor_off<TB>(half) + 1 + nv * nv + nv + 4;
 }
 
 // The pair solve on a tile S already in LDS: W <- I, the rotation test of
@@ -892,11 +859,13 @@ __global__ __launch_bounds__(256) void tjf_copyback_kernel(const syn_gbj_item *_
     }
 }
 
+// rt <- I for the problems without a direct phase (P.active 1, not 2), and
+// the rotation floor.
 template <int TB>
 __global__ __launch_bounds__(256) void tj_init_kernel(const syn_gbj_item *__restrict__ items) {
     __shared__ double red[4];
     const syn_gbj_item &P = items[blockIdx.x];
-    const int64_t nel = P.nv * P.nv;
+    const int64_t nel = P.active == 2 ? 0 : P.nv * P.nv;
     for (int64_t e = threadIdx.x; e < nel; e += 256) {
         const int64_t i = e / P.nv, j = e - i * P.nv;
         P.rt[i * P.ldr + j] = (i == j) ? 1.0 : 0.0;
@@ -1009,14 +978,6 @@ __global__ __launch_bounds__(256) void tj_zero_kernel(int32_t *c, int n) {
     for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) c[i] = 0;
 }
 
-// per-problem workspace: W tiles and flags (two sets), floor, the sort
-// scratch (rt copy, s) and the second Gram buffer
-template <int TB>
-static int64_t tj_work(int64_t nv) {
-    const int64_t half = tj_dims<TB>(nv).half;
-    return tj_g2_off<TB>(half, nv) + nv * nv;
-}
-
 // Gram entries from which a call counts as many problems: its launches are
 // bound by the tile updates' bytes rather than by the pair solves' latency.
 constexpr int64_t kManyEntries = int64_t(1) << 23;
@@ -1081,9 +1042,28 @@ class PinnedLease {
     int rc_ = 0;
 };
 
+// The direct phase (tdc.hip) of the problems it takes.
+static int gram_direct(syn_gbj_item *items, const syn_gbj_item *items_host, int n_items, double *work,
+                       const PinnedLease &pin, hipStream_t st) {
+    std::vector<syn_gbj_item> host;
+    int64_t off = 0;
+    for (int i = 0; i < n_items; ++i) {
+        if (!tdc_takes(items_host[i].nv)) continue;
+        host.push_back(items_host[i]);
+        host.back().w = work + off;
+        off += tj_work<16>(host.back().nv);
+    }
+    if (host.empty()) return SYN_OK;
+    const size_t bytes = host.size() * sizeof(syn_gbj_item);
+    memcpy(pin.data(), host.data(), bytes);
+    if (int rc = hip_check(hipMemcpyAsync(items, pin.data(), bytes, hipMemcpyHostToDevice, st), "gram direct table"))
+        return rc;
+    return tdc_launch(items, host, st);
+}
+
 template <int TB>
 static int gram_blocked(syn_gbj_item *items, std::vector<syn_gbj_item> &all, int n_items, double *work,
-                        int32_t *counters, double tol, int max_sweeps, int *sweeps, hipStream_t st) {
+                        int32_t *counters, double tol, int max_sweeps, int *sweeps, hipStream_t st, bool direct) {
     // passes of the pair solves' rounds (while they rotate): a launch of many
     // problems is bound by its tile updates, beside which a second pass costs
     // little and saves sweeps (batch of 4096 chains: 7272 -> 5996 launches a
@@ -1099,7 +1079,7 @@ static int gram_blocked(syn_gbj_item *items, std::vector<syn_gbj_item> &all, int
         all[i].w = work + tot_w;
         tot_w += tj_work<TB>(all[i].nv);
         all[i].counter = counters + i;
-        all[i].active = all[i].nv > 1;
+        all[i].active = direct && tdc_takes(all[i].nv) ? 2 : all[i].nv > 1;
         all[i].solve_start = all[i].tile_start = 0;
     }
     // pinned regions, one per kind of transfer: the item table (first and
@@ -1164,6 +1144,23 @@ static int gram_blocked(syn_gbj_item *items, std::vector<syn_gbj_item> &all, int
     for (int i = 0; i < n_items; ++i)
         if (all[i].active) idx.push_back(i);
     int used = 0;
+    if (direct && std::any_of(all.begin(), all.end(), [](const syn_gbj_item &it) { return it.active == 2; })) {
+        // the direct phase counts as the first sweep; of its problems only
+        // those with an entry that still passes the rotation test go on
+        hipLaunchKernelGGL(tj_zero_kernel, dim3(1), dim3(256), 0, st, chk, n_items);
+        hipLaunchKernelGGL(tj_check_kernel<TB>, dim3((unsigned)n_items, 64), dim3(256), 0, st, items, 0, tol, counters,
+                           chk);
+        SYN_LAUNCH_CHECK("gram direct test");
+        if (int rc = hip_check(hipMemcpyAsync((void *)hk, chk, n * sizeof(int32_t), hipMemcpyDeviceToHost, st),
+                               "gram direct test flags"))
+            return rc;
+        if (int rc = hip_check(hipStreamSynchronize(st), "gram direct sync")) return rc;
+        used = 1;
+        std::vector<int> next;
+        for (int i : idx)
+            if (all[i].active != 2 || hk[i] != 0) next.push_back(i);
+        idx.swap(next);
+    }
     // the table of a sweep's active problems and its owner table are built
     // again only when the active set changed (a sweep that ends with every
     // problem still going leaves both as they are)
@@ -1320,14 +1317,20 @@ extern "C" int syn_jacobi_gram_blocked_f64(syn_gbj_item *items, const syn_gbj_it
         narrow.swap(all);
         wide.clear();
     }
+    const bool direct = max_sweeps > 0;
+    // its table's staging is held until the sweeps' last wait on the stream
+    PinnedLease pin((size_t)n_items * sizeof(syn_gbj_item), (hipStream_t)stream);
+    if (pin.rc()) return pin.rc();
+    if (direct)
+        if (int rc = gram_direct(items, items_host, n_items, work, pin, (hipStream_t)stream)) return rc;
     int sw_w = 0, sw_n = 0;
     if (!wide.empty())
         if (int rc = gram_blocked<32>(items, wide, (int)wide.size(), work, counters, tol, max_sweeps, &sw_w,
-                                      (hipStream_t)stream))
+                                      (hipStream_t)stream, direct))
             return rc;
     if (!narrow.empty())
         if (int rc = gram_blocked<16>(items, narrow, (int)narrow.size(), work, counters, tol, max_sweeps, &sw_n,
-                                      (hipStream_t)stream))
+                                      (hipStream_t)stream, direct))
             return rc;
     if (sweeps) *sweeps = std::max(sw_w, sw_n);
     return SYN_OK;
