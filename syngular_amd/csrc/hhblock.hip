@@ -10,6 +10,7 @@
 // diagonal, zeros above) and T (LAPACK dlarft, forward, columnwise:
 // T[0:j, j] = -tau_j T[0:j, 0:j] V[:, 0:j]^T v_j, T[j, j] = tau_j).
 #include "common.hpp"
+#include "hh_tile.hpp"
 #include "prof.hpp"
 
 namespace syn {
@@ -164,6 +165,38 @@ __global__ __launch_bounds__(kPanelThreads) void hh_panel_kernel(double *__restr
     }
 }
 
+// Panels of up to 1024 rows below and with their first: in registers
+// (hh_tile.hpp), 16 waves.  A whole 600 x 600 QR with 300 columns kept: 5.75 ->
+// 2.53 ms, 1024 x 1024 with 512: 14.6 -> 5.2 ms.  Taller panels keep the kernel
+// above, which streams them from L2.
+template <int RT>
+__global__ __launch_bounds__(kPanelThreads) void hh_panel_reg_kernel(double *W, int64_t ldw, double *V, int64_t ldv,
+                                                                     double *tau, double *T, int64_t ldt, int64_t m,
+                                                                     int64_t j0, int b) {
+    extern __shared__ double dyn[];
+    HhSmem<kPanelWaves> &sm = *(HhSmem<kPanelWaves> *)dyn;
+    hh_panel_regs<RT, kPanelWaves>(W + j0 * ldw + j0, ldw, (int)(m - j0), b, T, ldt, tau + j0, V + j0 * ldv + j0, ldv,
+                                   sm);
+}
+
+template <int RT>
+static int panel_regs(double *w, int64_t ldw, double *v, int64_t ldv, double *tau, double *t, int64_t ldt, int64_t m,
+                      int64_t j0, int b, hipStream_t s) {
+    constexpr size_t lds = sizeof(HhSmem<kPanelWaves>);
+    static bool attr_set = false;
+    if (!attr_set) {
+        if (int rc = hip_check(hipFuncSetAttribute((const void *)hh_panel_reg_kernel<RT>,
+                                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
+                               "syn_hh_panel_f64: hipFuncSetAttribute"))
+            return rc;
+        attr_set = true;
+    }
+    hipLaunchKernelGGL(hh_panel_reg_kernel<RT>, dim3(1), dim3(kPanelThreads), lds, s, w, ldw, v, ldv, tau, t, ldt, m,
+                       j0, b);
+    SYN_LAUNCH_CHECK("syn_hh_panel_f64 launch");
+    return SYN_OK;
+}
+
 }  // namespace syn
 
 extern "C" int syn_hh_panel_f64(double *w, int64_t ldw, double *v, int64_t ldv, double *tau, double *t, int64_t ldt,
@@ -177,6 +210,10 @@ extern "C" int syn_hh_panel_f64(double *w, int64_t ldw, double *v, int64_t ldv, 
     }
     hipStream_t s = (hipStream_t)stream;
     ProfScope ps(kTagQr, 0.0, s);
+    const int64_t rows = m - j0;
+    if (rows <= 256) return panel_regs<1>(w, ldw, v, ldv, tau, t, ldt, m, j0, (int)b, s);
+    if (rows <= 512) return panel_regs<2>(w, ldw, v, ldv, tau, t, ldt, m, j0, (int)b, s);
+    if (rows <= 1024) return panel_regs<4>(w, ldw, v, ldv, tau, t, ldt, m, j0, (int)b, s);
     hipLaunchKernelGGL(hh_panel_kernel, dim3(1), dim3(kPanelThreads), 0, s, w, ldw, v, ldv, tau, t, ldt, m, j0,
                        (int)b);
     SYN_LAUNCH_CHECK("syn_hh_panel_f64 launch");

@@ -8,17 +8,24 @@
 // Q = H_0 H_1 ... H_{p-1} [I; 0]  (Golub & Van Loan, Alg. 5.1.2 / 5.2.1).
 //
 // Parallel layout: the 64 lanes of a wave own 64 consecutive columns and the
-// 4 waves own 4 contiguous row segments, so every global access of the
+// 8 waves own 8 contiguous row segments, so every global access of the
 // row-major W and Q is coalesced along a row; the per-column partial dot
-// products of the 4 segments are combined through LDS.  The working copy of
+// products of the segments are combined through LDS.  The working copy of
 // the leading block lives in LDS when it fits and in the caller's workspace
 // (L2-resident at these sizes) otherwise.
+//
+// That column-by-column form is for matrices of more than 512 rows or 96
+// factored columns; the others go by panels of 32 columns in registers
+// (hh_tile.hpp) with the compact WY products on the MFMA.
 #include "common.hpp"
+#include "hh_tile.hpp"
 #include "prof.hpp"
+
+#include <algorithm>
 
 namespace syn {
 
-constexpr int kQrThreads = 256;
+constexpr int kQrThreads = 512;
 constexpr int kQrWaves = kQrThreads / 64;
 constexpr int64_t kQrLdsDoubles = (96 * 1024) / 8;
 
@@ -135,6 +142,60 @@ __device__ void qr_one(const syn_qr_item &P, double *lds_w) {
     }
 }
 
+// Panels of kHhCols columns factored in registers, W (the leading block) in
+// the workspace: each panel's reflectors are applied to the columns right of
+// it, and at the end, from the last panel back, to [I; 0], 16 columns per
+// wave.  A column costs about a microsecond of dependent steps (two barriers)
+// instead of a pass over the matrix by rows.  One matrix through ops.qr_many,
+// before and after: 64 x 32 198 / 74 us, 128 x 64 656 / 181, 256 x 64 2018 /
+// 282, 96 x 90 772 / 226, 512 x 24 1086 / 172.
+constexpr int64_t kTileRows = 512, kTileCols = 96;
+constexpr int kTilePanels = (int)kTileCols / kHhCols;
+struct QrTileSmem {
+    HhSmem<kQrWaves> hh;
+    double T[kTilePanels][kHhCols * kHhCols];
+};
+
+template <int RT>
+__device__ void qr_tile(const syn_qr_item &P, QrTileSmem &sm) {
+    const int m = (int)P.m, nb = (int)(P.n < P.keep ? P.n : P.keep), kq = (int)(P.keep < P.m ? P.keep : P.m);
+    const int p = m < nb ? m : nb, tid = threadIdx.x, wv = tid >> 6;
+    double *W = P.work;
+    for (int e = tid; e < m * nb; e += kQrThreads) {
+        const int i = e / nb, j = e - i * nb;
+        W[e] = P.a[i * P.rs + j * P.cs];
+    }
+    __syncthreads();
+    for (int j0 = 0; j0 < p; j0 += kHhCols) {
+        const int b = p - j0 < kHhCols ? p - j0 : kHhCols;
+        double *Wp = W + (int64_t)j0 * nb + j0, *T = sm.T[j0 / kHhCols];
+        hh_panel_regs<RT, kQrWaves>(Wp, nb, m - j0, b, T, kHhCols, P.tau + j0, nullptr, 0, sm.hh);
+        for (int c = j0 + b + 16 * wv; c < p; c += 16 * kQrWaves)
+            hh_apply_wave(Wp, nb, m - j0, b, T, kHhCols, true, W + (int64_t)j0 * nb + c, nb, p - c < 16 ? p - c : 16);
+        __syncthreads();
+    }
+    double *Q = P.q_trans ? P.work + (int64_t)m * nb : P.q;
+    const int64_t ldq = P.q_trans ? kq : P.ldq;
+    for (int e = tid; e < m * kq; e += kQrThreads) {
+        const int i = e / kq, c = e - i * kq;
+        Q[i * ldq + c] = (i == c) ? 1.0 : 0.0;
+    }
+    __syncthreads();
+    for (int j0 = (p - 1) / kHhCols * kHhCols; j0 >= 0; j0 -= kHhCols) {
+        const int b = p - j0 < kHhCols ? p - j0 : kHhCols;
+        for (int c = j0 + 16 * wv; c < kq; c += 16 * kQrWaves)
+            hh_apply_wave(W + (int64_t)j0 * nb + j0, nb, m - j0, b, sm.T[j0 / kHhCols], kHhCols, false,
+                          Q + j0 * ldq + c, ldq, kq - c < 16 ? kq - c : 16);
+        __syncthreads();
+    }
+    if (P.q_trans) {
+        for (int e = tid; e < m * kq; e += kQrThreads) {
+            const int c = e / m, i = e - c * m;
+            P.q[c * P.ldq + i] = Q[i * ldq + c];
+        }
+    }
+}
+
 // lds_cap: doubles of dynamic LDS the launch holds; a matrix whose leading
 // block fits works in LDS, a larger one in its workspace.
 __global__ __launch_bounds__(kQrThreads) void qr_kernel(const syn_qr_item *__restrict__ items, int n_items,
@@ -142,10 +203,36 @@ __global__ __launch_bounds__(kQrThreads) void qr_kernel(const syn_qr_item *__res
     extern __shared__ double lds_w[];
     const syn_qr_item &P = items[blockIdx.x];
     const int64_t nb = P.n < P.keep ? P.n : P.keep;
-    if (P.m * nb <= lds_cap)
+    if (P.m <= kTileRows && nb <= kTileCols) {
+        QrTileSmem &sm = *(QrTileSmem *)lds_w;
+        if (P.m <= 128)
+            qr_tile<1>(P, sm);
+        else if (P.m <= 256)
+            qr_tile<2>(P, sm);
+        else
+            qr_tile<4>(P, sm);
+    } else if (P.m * nb <= lds_cap)
         qr_one<true>(P, lds_w);
     else
         qr_one<false>(P, lds_w);
+}
+
+// every launch holds what the panel form needs; the other form its lds_cap
+static int qr_launch(const syn_qr_item *items, int n_items, int64_t lds_doubles, hipStream_t s) {
+    static bool attr_set = false;
+    const size_t most = std::max(sizeof(QrTileSmem), (size_t)kQrLdsDoubles * sizeof(double));
+    if (!attr_set) {
+        if (int rc = hip_check(hipFuncSetAttribute((const void *)qr_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                   (int)most),
+                               "syn_qr_f64: hipFuncSetAttribute"))
+            return rc;
+        attr_set = true;
+    }
+    const size_t lds = std::max(sizeof(QrTileSmem), (size_t)lds_doubles * sizeof(double));
+    ProfScope ps(kTagQr, 0.0, s);
+    hipLaunchKernelGGL(qr_kernel, dim3(n_items), dim3(kQrThreads), lds, s, items, n_items, lds_doubles);
+    SYN_LAUNCH_CHECK("syn_qr_f64 launch");
+    return SYN_OK;
 }
 
 }  // namespace syn
@@ -157,19 +244,7 @@ extern "C" int syn_qr_f64(const syn_qr_item *items, int n_items, void *stream) {
         return SYN_EINVAL;
     }
     if (n_items == 0) return SYN_OK;
-    static bool attr_set = false;
-    if (!attr_set) {
-        if (int rc = hip_check(hipFuncSetAttribute((const void *)qr_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                   (int)(kQrLdsDoubles * sizeof(double))),
-                               "syn_qr_f64: hipFuncSetAttribute"))
-            return rc;
-        attr_set = true;
-    }
-    ProfScope ps(kTagQr, 0.0, (hipStream_t)stream);
-    hipLaunchKernelGGL(qr_kernel, dim3(n_items), dim3(kQrThreads), kQrLdsDoubles * sizeof(double),
-                       (hipStream_t)stream, items, n_items, kQrLdsDoubles);
-    SYN_LAUNCH_CHECK("syn_qr_f64 launch");
-    return SYN_OK;
+    return qr_launch(items, n_items, kQrLdsDoubles, (hipStream_t)stream);
 }
 
 extern "C" int syn_qr_sized_f64(const syn_qr_item *items, int n_items, int64_t lds_doubles, void *stream) {
@@ -180,17 +255,5 @@ extern "C" int syn_qr_sized_f64(const syn_qr_item *items, int n_items, int64_t l
         return SYN_EINVAL;
     }
     if (n_items == 0) return SYN_OK;
-    static bool attr_set = false;
-    if (!attr_set) {
-        if (int rc = hip_check(hipFuncSetAttribute((const void *)qr_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                   (int)(kQrLdsDoubles * sizeof(double))),
-                               "syn_qr_sized_f64: hipFuncSetAttribute"))
-            return rc;
-        attr_set = true;
-    }
-    ProfScope ps(kTagQr, 0.0, (hipStream_t)stream);
-    hipLaunchKernelGGL(qr_kernel, dim3(n_items), dim3(kQrThreads), (size_t)lds_doubles * sizeof(double),
-                       (hipStream_t)stream, items, n_items, lds_doubles);
-    SYN_LAUNCH_CHECK("syn_qr_sized_f64 launch");
-    return SYN_OK;
+    return qr_launch(items, n_items, lds_doubles, (hipStream_t)stream);
 }

@@ -28,6 +28,7 @@
 // matrices U, y (n x n) the permuted rows of a merge and G rt^T, vec the
 // vectors, node records and T factors.
 #include "gemm_tile.hpp"
+#include "hh_tile.hpp"
 #include "prof.hpp"
 #include "tdc.hpp"
 
@@ -200,19 +201,6 @@ __device__ __forceinline__ double gram_scale(const Tdc &T) {
 // block J (summed over r and lk, then over the waves by wave 0).  A step is
 // the pass over the tiles by all waves and the short vector work of wave 0,
 // a barrier after each.
-__device__ __forceinline__ double lk_sum(double v) {   // over the four rows of 16 lanes
-    const uint64_t u = __builtin_bit_cast(uint64_t, v);
-    const auto l32 = __builtin_amdgcn_permlane32_swap((unsigned)u, (unsigned)u, false, false);
-    const auto h32 = __builtin_amdgcn_permlane32_swap((unsigned)(u >> 32), (unsigned)(u >> 32), false, false);
-    const double s = __builtin_bit_cast(double, (uint64_t)h32[0] << 32 | l32[0]) +
-                     __builtin_bit_cast(double, (uint64_t)h32[1] << 32 | l32[1]);
-    const uint64_t w = __builtin_bit_cast(uint64_t, s);
-    const auto l16 = __builtin_amdgcn_permlane16_swap((unsigned)w, (unsigned)w, false, false);
-    const auto h16 = __builtin_amdgcn_permlane16_swap((unsigned)(w >> 32), (unsigned)(w >> 32), false, false);
-    return __builtin_bit_cast(double, (uint64_t)h16[0] << 32 | l16[0]) +
-           __builtin_bit_cast(double, (uint64_t)h16[1] << 32 | l16[1]);
-}
-
 template <int NB>
 __global__ __launch_bounds__(64 * NB) void td_reduce_kernel(const syn_gbj_item *__restrict__ items, int nlo, int nhi) {
     constexpr int N = 16 * NB, KT = NB / 2 + 1, E = N / 64;
