@@ -14,6 +14,7 @@
 // by decreasing norm with in-place swaps.
 #include "common.hpp"
 #include "prof.hpp"
+#include "rotation.hpp"
 
 namespace syn {
 
@@ -259,11 +260,8 @@ __global__ __launch_bounds__(NT) void jacobi_gram_kernel(const syn_jacobi_item *
                 double c = 1.0, sn = 0.0;
                 if (q < g) {
                     const double apq = A[p * ld + q], app = A[p * ld + p], aqq = A[q * ld + q];
-                    if (fabs(apq) > fmax(tol * sqrt(fabs(app) * fabs(aqq)), floor_abs)) {
-                        const double zeta = (aqq - app) / (2.0 * apq);
-                        const double t = copysign(1.0, zeta) / (fabs(zeta) + hypot(1.0, zeta));
-                        c = 1.0 / sqrt(fma(t, t, 1.0));
-                        sn = c * t;
+                    if (rotates(apq, app, aqq, tol, floor_abs)) {
+                        rotation(apq, app, aqq, c, sn);
                         rotated = 1;
                     }
                 } else {

@@ -581,76 +581,86 @@ __global__ __launch_bounds__(kMultiThreads) void td_reduce_multi_kernel(const sy
 
 // ---------------------------------------------------------------------------
 // Leaves: implicit QL (Golub & Van Loan 8.3.3) of the tridiagonal block of at
-// most kLeaf rows, one wave each.  Lane c carries component c of every
-// eigenvector and a copy of the diagonals of its own (no exchange between
-// lanes); the eigenvectors leave as the rows of rt, eigenvalues ascending.
-// The split points' rank-one terms are subtracted here: node boundaries take
-// |e| off the diagonal on both sides.
+// most kLeaf rows, one wave each; the eigenvectors leave as the rows of rt,
+// eigenvalues ascending.  The rotations form one serial chain of about 200
+// for 16 rows: the diagonals live in two registers, entry i in lane i of each
+// row of lanes, read and written by lane number, so a link is its dozen
+// dependent operations and one reciprocal square root (with the diagonals in
+// LDS, a round trip each, the leaf took 120 us); lane c carries component c
+// of the vector the chain is at, the others are in LDS off the chain.  The
+// split points' rank-one terms are subtracted here: node boundaries take |e|
+// off the diagonal on both sides.
 // ---------------------------------------------------------------------------
+__device__ __forceinline__ void set_entry(double &v, int i, double x) {
+    if ((int)(threadIdx.x & 15) == i) v = x;
+}
+
 __global__ __launch_bounds__(64) void td_leaf_kernel(const syn_gbj_item *__restrict__ items) {
-    __shared__ double sd[kLeaf][64], se[kLeaf][64], q[kLeaf][64];
+    __shared__ double q[kLeaf][64];
     const Tdc T = tdc_view(items[blockIdx.x]);
-    const int L = tdc_leaves(T.n), t = blockIdx.y, c = threadIdx.x;
+    const int L = tdc_leaves(T.n), t = blockIdx.y, c = threadIdx.x, i = c & 15;
     if (t >= L || *T.fail) return;
     const int lo = leaf_start(T.n, L, t), hi = leaf_start(T.n, L, t + 1), m = hi - lo;
-    for (int i = 0; i < m; ++i) {
-        sd[i][c] = T.d[lo + i];
-        se[i][c] = i + 1 < m ? T.e[lo + i] : 0.0;
-        q[i][c] = i == c ? 1.0 : 0.0;
-    }
-    if (lo > 0) sd[0][c] -= fabs(T.e[lo - 1]);
-    if (hi < T.n) sd[m - 1][c] -= fabs(T.e[hi - 1]);
+    double dv = i < m ? T.d[lo + i] : 0.0, ev = i + 1 < m ? T.e[lo + i] : 0.0;
+    if (lo > 0 && i == 0) dv -= fabs(T.e[lo - 1]);
+    if (hi < T.n && i == m - 1) dv -= fabs(T.e[hi - 1]);
+    for (int k = 0; k < kLeaf; ++k) q[k][c] = k == c ? 1.0 : 0.0;
     bool ok = true;
-    for (int l = 0; l < m; ++l) {
+    for (int l = 0; l < m && ok; ++l) {
         for (int it = 0;; ++it) {
-            int mm = l;
-            for (; mm < m - 1; ++mm)
-                if (fabs(se[mm][c]) <= 1.2e-16 * (fabs(sd[mm][c]) + fabs(sd[mm + 1][c])) + 1e-22) break;
+            // the first negligible off-diagonal entry from l on (the last
+            // entry is zero, so there is one)
+            const double dn = dpp_f64<0x101>(dv);   // row_shl:1, the next entry
+            const bool small = fabs(ev) <= 1.2e-16 * (fabs(dv) + fabs(dn)) + 1e-22 || i >= m - 1;
+            const int mm = __builtin_ctz((unsigned)(__ballot(small) & 0xffffu) >> l << l);
             if (mm == l) break;
             if (it == 60) {
                 ok = false;
                 break;
             }
-            double g = (sd[l + 1][c] - sd[l][c]) / (2.0 * se[l][c]);
-            double r = sqrt(fma(g, g, 1.0));
-            g = sd[mm][c] - sd[l][c] + se[l][c] / (g + copysign(r, g));
-            double s = 1.0, co = 1.0, p = 0.0;
-            int i = mm - 1;
-            for (; i >= l; --i) {
-                const double f = s * se[i][c], b = co * se[i][c], r2 = fma(f, f, g * g);
-                if (!(r2 > 1e-290)) {   // both vanish: the block splits here
-                    sd[i + 1][c] -= p;
-                    se[i + 1][c] = 0.0;
-                    se[mm][c] = 0.0;
-                    break;
-                }
+            const double dl = lane_f64(dv, l), el = lane_f64(ev, l);
+            double g = (lane_f64(dv, l + 1) - dl) / (2.0 * el);
+            const double r0 = sqrt(fma(g, g, 1.0));
+            double dnext = lane_f64(dv, mm);
+            g = dnext - dl + el / (g + copysign(r0, g));
+            double s = 1.0, co = 1.0, p = 0.0, z1 = q[mm][c];
+            int k = mm - 1;
+            for (; k >= l; --k) {
+                const double ek = lane_f64(ev, k), dk = lane_f64(dv, k), z0 = q[k][c];
+                const double f = s * ek, b = co * ek, r2 = fma(f, f, g * g);
+                if (!(r2 > 1e-290)) break;   // both vanish: the block splits here
                 const double ir = rsq_nr(r2);
-                se[i + 1][c] = r2 * ir;
+                set_entry(ev, k + 1, r2 * ir);
                 s = f * ir;
                 co = g * ir;
-                g = sd[i + 1][c] - p;
-                r = fma(sd[i][c] - g, s, 2.0 * co * b);
+                g = dnext - p;
+                const double r = fma(dk - g, s, 2.0 * co * b);
                 p = s * r;
-                sd[i + 1][c] = g + p;
+                set_entry(dv, k + 1, g + p);
                 g = fma(co, r, -b);
-                const double z1 = q[i + 1][c], z0 = q[i][c];
-                q[i + 1][c] = fma(s, z0, co * z1);
-                q[i][c] = fma(co, z0, -s * z1);
+                q[k + 1][c] = fma(s, z0, co * z1);
+                z1 = fma(co, z0, -s * z1);
+                dnext = dk;
             }
-            if (i >= l) continue;
-            sd[l][c] -= p;
-            se[l][c] = g;
-            se[mm][c] = 0.0;
+            // the entry the chain stopped at: l, or where it split
+            q[k + 1][c] = z1;
+            set_entry(dv, k + 1, dnext - p);
+            set_entry(ev, k + 1, k >= l ? 0.0 : g);
+            set_entry(ev, mm, 0.0);
         }
     }
     if (!ok && c == 0) *T.fail = 1;
     // ascending order, ties by index
-    for (int i = 0; i < m; ++i) {
-        int rk = 0;
-        for (int k = 0; k < m; ++k) rk += (sd[k][c] < sd[i][c]) || (sd[k][c] == sd[i][c] && k < i);
-        if (c < m) T.rt[(int64_t)(lo + rk) * T.ldr + lo + c] = q[i][c];
-        if (c == 0) T.dd[lo + rk] = sd[i][c];
+    int rk = 0;
+    for (int k = 0; k < m; ++k) {
+        const double o = lane_f64(dv, k);
+        rk += o < dv || (o == dv && k < i);
     }
+    for (int k = 0; k < m; ++k) {
+        const int r = __builtin_amdgcn_readlane(rk, k);
+        if (c < m) T.rt[(int64_t)(lo + r) * T.ldr + lo + c] = q[k][c];
+    }
+    if (c < m) T.dd[lo + rk] = dv;
     if (c == 0) T.meta[lo] = m;
 }
 
