@@ -16,9 +16,9 @@
 // steps and a call takes 7..14 sweeps, about 4 n^3 flops each; the reduction
 // costs 4/3 n^3, the divide and conquer 8/3 n^3 at most and the products
 // 6 n^3, once.  Calls measured with the sweeps alone and with this phase, in
-// ms: one matrix of order 64 0.78 / 0.48, 128 1.5 / 0.81, 256 3.3 / 1.8, 512
-// 7.1 / 3.8, 1024 21 / 9.7, 2048 80 / 39; 8 of order 512 9.6 / 4.3; 2000 of
-// order 64 5.3 / 2.2, 1000 of 128 15.5 / 3.5, 800 of 256 88 / 12.8.
+// ms: one matrix of order 64 0.78 / 0.45, 128 1.5 / 0.72, 256 3.3 / 1.6, 512
+// 7.1 / 3.5, 1024 21 / 9.4, 2048 80 / 37; 8 of order 512 9.6 / 4.1; 2000 of
+// order 64 5.3 / 2.0, 1000 of 128 15.5 / 3.2, 800 of 256 88 / 12.1.
 // Residuals fall with the number of rotations: rt^T diag(s^2) rt - G from
 // 1e-13 to 1e-15 of the largest eigenvalue.
 //
@@ -35,6 +35,8 @@
 #include <algorithm>
 
 namespace syn {
+
+typedef double v2du __attribute__((ext_vector_type(2), aligned(8)));
 
 // Vector region of a problem (2048 * half >= 64 n doubles, tjacobi.hpp):
 // rows of n doubles, then the 32 x 32 T factors of the reflector blocks.
@@ -864,19 +866,33 @@ __global__ __launch_bounds__(256) void td_copy_kernel(const syn_gbj_item *__rest
 
 // ---------------------------------------------------------------------------
 // Secular equation 1 + sum_i a_i / (d_i - lambda) = 0, a_i = rho z_i^2, one
-// thread per root, poles in LDS.  A root is kept as its distance tau to the
+// four lanes per root, poles in LDS.  A root is kept as its distance tau to the
 // nearer pole (its origin), so d_i - lambda = (d_i - d_origin) - tau has no
 // cancellation.  Iteration: the rational interpolation through the two poles
 // around the root (Li 1993, the middle way), safeguarded by a bracket that
 // every evaluation shrinks; it stops at the rounding level of the sum or of
 // the bracket.
 // ---------------------------------------------------------------------------
-constexpr int kSecThreads = 64;
+constexpr int kSecThreads = 256;
+constexpr int kSecRoots = kSecThreads / 4;   // roots of a work-group
 
-__device__ __forceinline__ void secular_sums(const double *dl, const double *a, int K, int j, double dorg, double tau,
-                                             double &psi, double &dpsi, double &phi, double &dphi) {
+// Four lanes (lk) share a root and take every fourth term each; j0 is the
+// first root of the wave's 16, so the terms before it are left of every root
+// of the wave and those from j0 + 16 on right of it, and only the 16 between
+// need a selection.
+__device__ __forceinline__ void secular_sums(const double *dl, const double *a, int K, int j0, int j, int lk,
+                                             double dorg, double tau, double &psi, double &dpsi, double &phi,
+                                             double &dphi) {
     psi = dpsi = phi = dphi = 0.0;
-    for (int i = 0; i < K; ++i) {
+    int i = lk;
+#pragma unroll 2
+    for (; i < j0; i += 4) {
+        const double r = rcp_nr((dl[i] - dorg) - tau), t = a[i] * r;
+        psi += t;
+        dpsi = fma(t, r, dpsi);
+    }
+    const int mid = j0 + 16 < K ? j0 + 16 : K;
+    for (; i < mid; i += 4) {
         const double r = rcp_nr((dl[i] - dorg) - tau), t = a[i] * r, tt = t * r;
         const bool left = i <= j;
         psi += left ? t : 0.0;
@@ -884,10 +900,20 @@ __device__ __forceinline__ void secular_sums(const double *dl, const double *a, 
         phi += left ? 0.0 : t;
         dphi += left ? 0.0 : tt;
     }
+#pragma unroll 2
+    for (; i < K; i += 4) {
+        const double r = rcp_nr((dl[i] - dorg) - tau), t = a[i] * r;
+        phi += t;
+        dphi = fma(t, r, dphi);
+    }
+    psi = lk_sum(psi);
+    dpsi = lk_sum(dpsi);
+    phi = lk_sum(phi);
+    dphi = lk_sum(dphi);
 }
 
-__device__ __forceinline__ bool secular_root(const double *dl, const double *a, int K, int j, double asum, int &org,
-                                             double &tau) {
+__device__ __forceinline__ bool secular_root(const double *dl, const double *a, int K, int j0, int j, int lk,
+                                             double asum, int &org, double &tau) {
     org = j;
     if (K == 1) {
         tau = a[0];
@@ -902,7 +928,7 @@ __device__ __forceinline__ bool secular_root(const double *dl, const double *a, 
         tau = 0.5 * hi;
     } else {
         const double gap = dl[j + 1] - dl[j], mid = 0.5 * gap;
-        secular_sums(dl, a, K, jl, dl[j], mid, psi, dpsi, phi, dphi);
+        secular_sums(dl, a, K, j0, jl, lk, dl[j], mid, psi, dpsi, phi, dphi);
         const double f = 1.0 + psi + phi, aj = a[j], ar = a[j + 1];
         // the two poles' model with the other terms at their midpoint value
         const double c = f + (aj - ar) / mid;
@@ -922,7 +948,7 @@ __device__ __forceinline__ bool secular_root(const double *dl, const double *a, 
     }
     const double dorg = dl[org], eps = 1.1102230246251565e-16;
     for (int it = 0; it < 200; ++it) {
-        secular_sums(dl, a, K, jl, dorg, tau, psi, dpsi, phi, dphi);
+        secular_sums(dl, a, K, j0, jl, lk, dorg, tau, psi, dpsi, phi, dphi);
         const double f = 1.0 + psi + phi;
         if (fabs(f) <= eps * (8.0 * (fabs(psi) + fabs(phi)) + 2.0 + fabs(tau) * (dpsi + dphi))) return true;
         if (f < 0.0)
@@ -953,41 +979,46 @@ __global__ __launch_bounds__(kSecThreads) void td_secular_kernel(const syn_gbj_i
     const Tdc T = tdc_view(items[blockIdx.x]);
     int lo, mid, hi;
     if (!tdc_node(T, level, blockIdx.z, lo, mid, hi)) return;
-    const int K = T.meta[lo], tid = threadIdx.x, j = blockIdx.y * kSecThreads + tid;
-    if ((int)blockIdx.y * kSecThreads >= K) return;
+    const int K = T.meta[lo], tid = threadIdx.x, lane = tid & 63;
+    if ((int)blockIdx.y * kSecRoots >= K) return;
     double *dl = sm, *a = sm + K;
     const double rho = T.rho[lo];
-    double asum = 0.0;
     for (int i = tid; i < K; i += kSecThreads) {
         dl[i] = T.dl[lo + i];
         const double z = T.zl[lo + i];
         a[i] = rho * z * z;
-        asum += a[i];
     }
-    asum = wave_sum(asum);
     __syncthreads();
-    if (j >= K) return;
+    const int j0 = blockIdx.y * kSecRoots + 16 * (tid >> 6), li = lane & 15, lk = lane >> 4;
+    if (j0 >= K) return;
+    double asum = 0.0;
+    for (int i = lane; i < K; i += 64) asum += a[i];
+    asum = all_sum(asum);
+    const int j = j0 + li < K ? j0 + li : K - 1;   // lanes past the last root repeat it
     int org;
     double tau;
-    const bool ok = secular_root(dl, a, K, j, asum * (1.0 + 1e-15), org, tau);
+    const bool ok = secular_root(dl, a, K, j0, j, lk, asum * (1.0 + 1e-15), org, tau);
     if (!ok) *T.fail = 1;
-    T.org[lo + j] = org;
-    T.tr[lo + j] = tau;
-    T.dd[lo + j] = dl[org] + tau;
+    if (lk == 0 && j0 + li < K) {
+        T.org[lo + j] = org;
+        T.tr[lo + j] = tau;
+        T.dd[lo + j] = dl[org] + tau;
+    }
 }
 
 // z recomputed from the roots (the z whose secular equation has exactly
 // these roots), one thread per entry: z_i^2 = prod_j (lambda_j - d_i) over
 // prod_{j != i} (d_j - d_i), up to a constant factor.
-__global__ __launch_bounds__(kSecThreads) void td_zhat_kernel(const syn_gbj_item *__restrict__ items, int level) {
+constexpr int kZhatThreads = 64;
+__global__ __launch_bounds__(kZhatThreads) void td_zhat_kernel(const syn_gbj_item *__restrict__ items, int level) {
     extern __shared__ double sm[];
     const Tdc T = tdc_view(items[blockIdx.x]);
     int lo, mid, hi;
     if (!tdc_node(T, level, blockIdx.z, lo, mid, hi)) return;
-    const int K = T.meta[lo], tid = threadIdx.x, i = blockIdx.y * kSecThreads + tid;
-    if ((int)blockIdx.y * kSecThreads >= K) return;
+    const int K = T.meta[lo], tid = threadIdx.x, i = blockIdx.y * kZhatThreads + tid;
+    if ((int)blockIdx.y * kZhatThreads >= K) return;
     double *dl = sm, *od = sm + K, *tr = od + K;
-    for (int q = tid; q < K; q += kSecThreads) {
+    for (int q = tid; q < K; q += kZhatThreads) {
         dl[q] = T.dl[lo + q];
         od[q] = T.dl[lo + T.org[lo + q]];
         tr[q] = T.tr[lo + q];
@@ -1149,14 +1180,28 @@ __global__ __launch_bounds__(256) void td_back_kernel(const syn_gbj_item *__rest
         for (int k0 = cs + 16 * wv; k0 < n; k0 += 64) {
             const int k = k0 + 4 * lk;
             double q[2][4], v[2][4];
+            if (nb == kBlk && k0 >= j0 + kBlk && k0 + 16 <= n) {
+                // right of the block's triangle: whole rows of V; rows of rt
+                // past the last repeat it (their results are not stored)
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int row = r0 + 16 * i + li, ref = 16 * i + li;
+                for (int i = 0; i < 2; ++i) {
+                    const int row = r0 + 16 * i + li < n ? r0 + 16 * i + li : n - 1;
+                    const double *qp = T.rt + (int64_t)row * T.ldr + k, *vp = T.g + (int64_t)(j0 + 16 * i + li) * T.ldg + k;
+                    const v2du q0 = *(const v2du *)qp, q1 = *(const v2du *)(qp + 2);
+                    const v2du v0 = *(const v2du *)vp, v1 = *(const v2du *)(vp + 2);
+                    q[i][0] = q0.x, q[i][1] = q0.y, q[i][2] = q1.x, q[i][3] = q1.y;
+                    v[i][0] = v0.x, v[i][1] = v0.y, v[i][2] = v1.x, v[i][3] = v1.y;
+                }
+            } else {
 #pragma unroll
-                for (int s = 0; s < 4; ++s) {
-                    const bool in = k + s < n;
-                    q[i][s] = (in && row < n) ? T.rt[(int64_t)row * T.ldr + k + s] : 0.0;
-                    v[i][s] = (in && ref < nb && k + s > j0 + ref) ? T.g[(int64_t)(j0 + ref) * T.ldg + k + s] : 0.0;
+                for (int i = 0; i < 2; ++i) {
+                    const int row = r0 + 16 * i + li, ref = 16 * i + li;
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) {
+                        const bool in = k + s < n;
+                        q[i][s] = (in && row < n) ? T.rt[(int64_t)row * T.ldr + k + s] : 0.0;
+                        v[i][s] = (in && ref < nb && k + s > j0 + ref) ? T.g[(int64_t)(j0 + ref) * T.ldg + k + s] : 0.0;
+                    }
                 }
             }
 #pragma unroll
@@ -1310,7 +1355,7 @@ int tdc_launch(const syn_gbj_item *items, const std::vector<syn_gbj_item> &host,
         hipLaunchKernelGGL(td_prep_kernel, dim3(ni, nodes), dim3(kPrepThreads), plds, st, items, l);
         hipLaunchKernelGGL(td_copy_kernel, dim3(ni, c64, nodes), dim3(256), 0, st, items, l);
         hipLaunchKernelGGL(td_secular_kernel, dim3(ni, c64, nodes), dim3(kSecThreads), slds, st, items, l);
-        hipLaunchKernelGGL(td_zhat_kernel, dim3(ni, c64, nodes), dim3(kSecThreads), slds + slds / 2, st, items, l);
+        hipLaunchKernelGGL(td_zhat_kernel, dim3(ni, c64, nodes), dim3(kZhatThreads), slds + slds / 2, st, items, l);
         hipLaunchKernelGGL(td_vec_kernel, dim3(ni, (unsigned)((k + 3) / 4), nodes), dim3(256), 0, st, items, l);
         hipLaunchKernelGGL(td_gemm_kernel, dim3(ni, c64 * c64, nodes), dim3(256), 0, st, items, 0, l);
         SYN_LAUNCH_CHECK("divide and conquer");
