@@ -75,6 +75,37 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, 2) void gemm_f64_pair(s
         gemm_f64_tile<BM, BN, BK, WM, WN, double>(P1, tile_of_block(bid - tiles0, tiles1, P1.tiles_n, P1.tri));
 }
 
+// Launches of few 64 x 64 tiles, four work-groups a tile (gemm_f64_quad).
+// Up to half of the 256 compute units busy with 64 x 64 tiles the quadrants
+// are faster at every K (us, 64 x 64 tiles / quadrants): 1 tile K = 16 4.7 /
+// 4.6, 256 16.9 / 8.0, 1024 57 / 24; 64 tiles of 256 18.3 / 9.5, 128 of 64
+// 8.0 / 6.5, of 256 19.4 / 12.8.  256 tiles: 16 6.2 / 7.8, 64 9.1 / 9.2, 256
+// 21.6 / 19.9; 512 of 256 29.5 / 33.2.
+constexpr int kQuadK = 32;
+constexpr int64_t kQuadMax = 128;
+
+template <typename CT>
+__global__ __launch_bounds__(256, 2) void gemm_quad_grouped(const syn_gemm_item *__restrict__ items, int n_items,
+                                                              int64_t total) {
+    const int64_t b = xcd_remap(blockIdx.x, 4 * total), t = b >> 2;
+    const syn_gemm_item &P = items[find_item(items, n_items, t)];
+    gemm_f64_quad<kQuadK, CT>(P, t - P.block_start, (int)(b & 3));
+}
+
+template <typename CT>
+__global__ __launch_bounds__(256, 2) void gemm_quad_single(syn_gemm_item P) {
+    const int64_t b = xcd_remap(blockIdx.x, (int64_t)gridDim.x);
+    gemm_f64_quad<kQuadK, CT>(P, b >> 2, (int)(b & 3));
+}
+
+__global__ __launch_bounds__(256, 2) void gemm_quad_pair(syn_gemm_item P0, int64_t tiles0, syn_gemm_item P1) {
+    const int64_t b = xcd_remap(blockIdx.x, (int64_t)gridDim.x), t = b >> 2;
+    if (t < tiles0)
+        gemm_f64_quad<kQuadK, double>(P0, t, (int)(b & 3));
+    else
+        gemm_f64_quad<kQuadK, double>(P1, t - tiles0, (int)(b & 3));
+}
+
 // Split-K form of a single problem: work-group b computes K slice
 // b / tiles of tile b % tiles; slice 0 writes C (with beta), slice s > 0
 // writes the partial product into ws + (s - 1) m ws_ld, and
@@ -137,7 +168,9 @@ int gemm_f64_pair_launch(syn_gemm_item P0, syn_gemm_item P1, hipStream_t s) {
         fl += f;
     }
     ProfScope ps(tile ? kTagGemmPair128 : kTagGemmPair64, fl, s);
-    if (tile)
+    if (!tile && t0 + t1 <= kQuadMax)
+        hipLaunchKernelGGL(gemm_quad_pair, dim3((unsigned)(4 * (t0 + t1))), dim3(256), 0, s, P0, t0, P1);
+    else if (tile)
         hipLaunchKernelGGL((gemm_f64_pair<128, 128, 16, 64, 64>), dim3((unsigned)(t0 + t1)), dim3(256), 0, s, P0, t0,
                            P1, t1);
     else
@@ -163,7 +196,9 @@ int gemm_f64_launch(syn_gemm_item P, hipStream_t s, bool mixed) {
     if (nbits >= 2) fl /= 3.0;
     if (mixed) {
         ProfScope ps(tile ? kTagGemmMixed128 : kTagGemmMixed64, fl, s);
-        if (tile)
+        if (!tile && tiles <= kQuadMax)
+            hipLaunchKernelGGL(gemm_quad_single<float>, dim3((unsigned)(4 * tiles)), dim3(256), 0, s, P);
+        else if (tile)
             hipLaunchKernelGGL((gemm_f64_single<128, 128, 16, 64, 64, float>), dim3((unsigned)tiles), dim3(256), 0,
                                s, P);
         else
@@ -173,7 +208,9 @@ int gemm_f64_launch(syn_gemm_item P, hipStream_t s, bool mixed) {
         return SYN_OK;
     }
     ProfScope ps(tile ? kTagGemmSingle128 : kTagGemmSingle64, fl, s);
-    if (tile)
+    if (!tile && tiles <= kQuadMax)
+        hipLaunchKernelGGL(gemm_quad_single<double>, dim3((unsigned)(4 * tiles)), dim3(256), 0, s, P);
+    else if (tile)
         hipLaunchKernelGGL((gemm_f64_single<128, 128, 16, 64, 64>), dim3((unsigned)tiles), dim3(256), 0, s, P);
     else
         hipLaunchKernelGGL((gemm_f64_single<64, 64, 16, 32, 32>), dim3((unsigned)tiles), dim3(256), 0, s, P);
@@ -279,6 +316,13 @@ template <typename CT>
 static void launch_grouped(const syn_gemm_item *items, int n_items, int64_t total, int tile, hipStream_t s) {
     const bool pers = total >= kPersistentMin && n_items > 1;
     const unsigned grid = (unsigned)(pers ? kPersistentGrid : total);
+    if constexpr (!__is_same(CT, bf16s)) {
+        if (tile == 0 && total <= kQuadMax) {
+            hipLaunchKernelGGL(gemm_quad_grouped<CT>, dim3((unsigned)(4 * total)), dim3(256), 0, s, items, n_items,
+                               total);
+            return;
+        }
+    }
     if (tile == 0) {
         if (pers)
             hipLaunchKernelGGL((gemm_f64_grouped_persistent<64, 64, 16, 32, 32, CT>), dim3(grid), dim3(256), 0, s,

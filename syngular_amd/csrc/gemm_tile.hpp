@@ -90,8 +90,8 @@ struct GemmSmem {
 };
 
 template <int BM, int BN, int BK, int WM, int WN, bool TA, bool TB, typename CT>
-__device__ __forceinline__ void gemm_f64_tile_t(const syn_gemm_item &P, int64_t t, GemmSmem<BM, BN, BK, CT> &sm,
-                                                int64_t klo, int64_t khi) {
+__device__ __forceinline__ void gemm_f64_tile_at(const syn_gemm_item &P, int64_t row0, int64_t col0,
+                                                 GemmSmem<BM, BN, BK, CT> &sm, int64_t klo, int64_t khi) {
     constexpr int NW = (BM / WM) * (BN / WN);
     constexpr int NT = NW * 64;
     constexpr int TI = WM / 16, TJ = WN / 16;
@@ -100,11 +100,9 @@ __device__ __forceinline__ void gemm_f64_tile_t(const syn_gemm_item &P, int64_t 
     auto &As = sm.As;
     auto &Bs = sm.Bs;
 
-    const int64_t row0 = (t / P.tiles_n) * BM, col0 = (t % P.tiles_n) * BN;
     const int tri = P.tri;
-    if ((tri & 1) && col0 >= row0 + BM) return;  // tile strictly above the diagonal of C
     const int64_t m = P.m, n = P.n, lda = P.lda, ldb = P.ldb;
-    if (row0 >= m) return;  // a size known on the device only: the launch covers its largest
+    if (row0 >= m || col0 >= n) return;  // a size known on the device only: the launch covers its largest
     // K band of the structurally non-zero products for this tile
     int64_t kmin = 0, k = P.k;
     if (tri & 2) k = k < row0 + BM ? k : row0 + BM;
@@ -272,6 +270,14 @@ __device__ __forceinline__ void gemm_f64_tile_t(const syn_gemm_item &P, int64_t 
             }
 }
 
+template <int BM, int BN, int BK, int WM, int WN, bool TA, bool TB, typename CT>
+__device__ __forceinline__ void gemm_f64_tile_t(const syn_gemm_item &P, int64_t t, GemmSmem<BM, BN, BK, CT> &sm,
+                                                int64_t klo, int64_t khi) {
+    const int64_t row0 = (t / P.tiles_n) * BM, col0 = (t % P.tiles_n) * BN;
+    if ((P.tri & 1) && col0 >= row0 + BM) return;  // tile strictly above the diagonal of C
+    gemm_f64_tile_at<BM, BN, BK, WM, WN, TA, TB, CT>(P, row0, col0, sm, klo, khi);
+}
+
 // The operand orientation is fixed at compile time in each instance, so the
 // loads carry no per-element branches and the register budget fits two
 // work-groups per compute unit.
@@ -289,6 +295,33 @@ __device__ __forceinline__ void gemm_f64_tile(const syn_gemm_item &P, int64_t t,
             gemm_f64_tile_t<BM, BN, BK, WM, WN, true, false, CT>(P, t, sm, klo, khi);
         else
             gemm_f64_tile_t<BM, BN, BK, WM, WN, true, true, CT>(P, t, sm, klo, khi);
+    }
+}
+
+// Quadrant quad (0..3) of 64 x 64 tile t as a 32 x 32 tile of its own, one
+// 16 x 16 block a wave, 32 of K a step.  For launches whose tiles leave compute
+// units idle: a wave of the 64 x 64 tile runs 16 MFMAs and a barrier every 16
+// of K (0.8 us measured), a wave of the quadrant 8 every 32 (0.65 us).  The
+// MFMAs of an output element are the same in the same order, so a launch may
+// take either form and gives the same bits.  (A third form that loads the
+// MFMA operands from global memory without LDS measured the same up to 64
+// tiles and less beyond; a second K tile in flight changed nothing.)
+template <int BK, typename CT>
+__device__ __forceinline__ void gemm_f64_quad(const syn_gemm_item &P, int64_t t, int quad) {
+    __shared__ GemmSmem<32, 32, BK, CT> sm;
+    const int64_t row64 = (t / P.tiles_n) * 64, col64 = (t % P.tiles_n) * 64;
+    if ((P.tri & 1) && col64 >= row64 + 64) return;
+    const int64_t row0 = row64 + 32 * (quad >> 1), col0 = col64 + 32 * (quad & 1);
+    if (!P.transA) {
+        if (!P.transB)
+            gemm_f64_tile_at<32, 32, BK, 16, 16, false, false, CT>(P, row0, col0, sm, 0, INT64_MAX);
+        else
+            gemm_f64_tile_at<32, 32, BK, 16, 16, false, true, CT>(P, row0, col0, sm, 0, INT64_MAX);
+    } else {
+        if (!P.transB)
+            gemm_f64_tile_at<32, 32, BK, 16, 16, true, false, CT>(P, row0, col0, sm, 0, INT64_MAX);
+        else
+            gemm_f64_tile_at<32, 32, BK, 16, 16, true, true, CT>(P, row0, col0, sm, 0, INT64_MAX);
     }
 }
 
