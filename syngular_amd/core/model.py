@@ -14,8 +14,47 @@ from __future__ import annotations
 import numpy as np
 import torch
 
-from .. import linalg, ops
+from .. import _lib, ops
 from ..tensor import MatrixProductOperator, MatrixProductState
+
+
+def _arena(sizes):
+    """One float64 device tensor with a 256-byte aligned sub-buffer per size:
+    (tensor, offsets in doubles, addresses)."""
+    padded = (sizes + 31) // 32 * 32
+    off = np.cumsum(padded) - padded
+    t = torch.empty(int(padded.sum()), dtype=torch.float64, device=ops.device())
+    return t, off, np.uint64(t.data_ptr()) + (8 * off).astype(np.uint64)
+
+
+def _views(t, off, first, count, shape):
+    """The tensors of `count` equally shaped neighbours of an arena."""
+    l, d, r = (int(v) for v in shape)
+    step = (l * d * r + 31) // 32 * 32
+    return t.as_strided((count, l, d, r), (step, d * r, r, 1), int(off[first])).unbind(0)
+
+
+def _state(sites, shape, input_shape, bond_shape, params):
+    """A MatrixProductState of device cores of known shapes."""
+    mp = MatrixProductState()
+    mp.sites, mp.shape, mp.sites_number = sites, shape, len(sites)
+    mp.decomposed = True
+    mp.parameters_number, mp.real_parameters_number = params, None
+    mp.input_shape, mp.bond_shape = input_shape, bond_shape
+    return mp
+
+
+def _gemm_items(it, A, B, C, m, n, k, lda, ta):
+    """Fill a grouped GEMM table: C (m x n) = op(A) B, B row-major.  Returns
+    (tile, work-groups, flops)."""
+    tile = 1 if int((m * n).sum()) >= 256 * 128 * 128 else 0
+    bm = 128 if tile else 64
+    tn = (n + bm - 1) // bm
+    blocks = (m + bm - 1) // bm * tn
+    it["A"], it["B"], it["C"], it["m"], it["n"], it["k"] = A, B, C, m, n, k
+    it["lda"], it["ldb"], it["ldc"], it["alpha"], it["transA"] = lda, n, n, 1.0, ta
+    it["block_start"], it["tiles_n"] = np.cumsum(blocks) - blocks, tn
+    return tile, int(blocks.sum()), float((2.0 * m * n * k).sum())
 
 
 def matmul_batch(weight, states):
@@ -23,40 +62,126 @@ def matmul_batch(weight, states):
     per state) in grouped launches: one MPO x MPS apply launch for every site
     of every state, then the QR truncation to each state's min bond
     (tensor/matrix_product_state.py:432-468), bond by bond, with one QR launch
-    and two GEMM launches per bond over all the states that need it.  States
-    whose site count differs from the operator's, or a non-default matmul /
-    rounding mode, go through ``weight @ x`` one by one."""
+    and two GEMM launches per bond over all the states that need it.  Every
+    buffer's address is known before the first launch, so the tables of all
+    launches are filled by array operations over the states and go to the
+    device in one copy (64 states of 6 cores spent 12 ms on the host in one
+    tensor and one table row at a time, against 0.5 ms of kernels).  States
+    whose site count differs from the operator's or whose shapes do not chain,
+    or a non-default matmul / rounding mode, go through ``weight @ x`` one by
+    one."""
     states = list(states)
     n = weight.sites_number
     if (MatrixProductOperator.MATMUL_MODE != "standard" or MatrixProductState.ROUNDING != "qr"
             or any(x.sites_number != n for x in states)):
         return [weight @ x for x in states]
+    if not states:
+        return []
     dims = [min(min(weight.bond_shape), min(x.bond_shape)) for x in states]
-    flat = ops.apply_many([(weight.sites[k], x.sites[k]) for x in states for k in range(n)])
-    outs = [MatrixProductState.from_sites(flat[i * n:(i + 1) * n]) for i in range(len(states))]
-    if not MatrixProductOperator.COMPRESS:
-        return outs
-    todo = [i for i, o in enumerate(outs) if dims[i] < min(o.bond_shape)]
-    work = {i: outs[i].copy() for i in todo}
-    params = {i: 0 for i in todo}
-    for k in range(n - 1):
-        Ls = [linalg.left_unfold(work[i].sites[k], work[i].shape[k]) for i in todo]
-        Rs = [linalg.right_unfold(work[i].sites[k + 1], work[i].shape[k + 1]) for i in todo]
-        Qs = ops.qr_many([(L, dims[i]) for L, i in zip(Ls, todo)])
-        Ss = [torch.empty((Q.shape[1], L.shape[1]), dtype=torch.float64, device=L.device) for Q, L in zip(Qs, Ls)]
-        ops.gemm_many([(Q.t(), L, S, 1.0, 0.0) for Q, L, S in zip(Qs, Ls, Ss)])
-        Ws = [torch.empty((S.shape[0], Rm.shape[1]), dtype=torch.float64, device=S.device) for S, Rm in zip(Ss, Rs)]
-        ops.gemm_many([(S, Rm, W, 1.0, 0.0) for S, Rm, W in zip(Ss, Rs, Ws)])
-        for i, Q, W in zip(todo, Qs, Ws):
-            t = work[i]
-            t.shape[k] = tuple(t.shape[k][:-1]) + (dims[i],)
-            t.shape[k + 1] = (dims[i],) + tuple(t.shape[k + 1][1:])
-            t.sites[k] = linalg.reshape(Q, t.shape[k])
-            t.sites[k + 1] = linalg.reshape(W, t.shape[k + 1])
-            params[i] += t.sites[k].numel()
-    for i in todo:
-        work[i].parameters_number = params[i] + work[i].sites[-1].numel()
-        outs[i] = work[i]
+    # states of equal shapes next to each other
+    members = {}
+    for i, x in enumerate(states):
+        members.setdefault((dims[i], *(s.shape for s in x.sites)), []).append(i)
+    keys = list(members)
+    if any(len(s) != 3 for key in keys for s in key[1:]):
+        return [weight @ x for x in states]
+    X = np.array([key[1:] for key in keys], dtype=np.int64)               # group, site, (l, d, r)
+    D = np.array([key[0] for key in keys], dtype=np.int64)
+    O = np.array([s.shape for s in weight.sites], dtype=np.int64)         # site, (l, in, out, r)
+    P = np.stack([X[:, :, 0] * O[:, 0], np.broadcast_to(O[:, 2], X.shape[:2]), X[:, :, 2] * O[:, 3]], axis=2)
+    cut = D < P[:, :-1, 2].min(axis=1) if MatrixProductOperator.COMPRESS else np.zeros(len(keys), bool)
+    rows = P[:, :, 0] * P[:, :, 1]                                        # rows of the left unfoldings
+    rows[:, 1:] = np.where(cut[:, None], D[:, None] * P[:, 1:, 1], rows[:, 1:])
+    if ((X[:, :, 1] != O[:, 1]).any() or P.min() <= 0 or (cut & (D <= 0)).any()
+            or (P[cut, :-1, 2] != P[cut, 1:, 0]).any() or (rows[cut, :-1] < D[cut, None]).any()):
+        return [weight @ x for x in states]
+
+    order = [i for g in members.values() for i in g]
+    count = np.array([len(g) for g in members.values()])
+    first = np.cumsum(count) - count
+    rep = np.repeat(np.arange(len(keys)), count)
+    hold = [[s.contiguous() for s in states[i].sites] for i in order]     # inputs, alive until the launch
+    ws = [w.contiguous() for w in weight.sites]
+    cores = [_arena(P[rep, k].prod(axis=1)) for k in range(n)]
+
+    # the tables, one after the other in one buffer
+    J = len(order)
+    todo = cut[rep]
+    T = int(todo.sum())
+    ap, qr = np.dtype(_lib.APPLY_ITEM), np.dtype(_lib.QR_ITEM)
+    ge = np.dtype(_lib.GEMM_ITEM)
+    nbytes = J * n * ap.itemsize + (n - 1) * T * (qr.itemsize + 2 * ge.itemsize)
+    table, at = np.zeros(nbytes, dtype=np.uint8), 0
+
+    def take(dtype, cnt):
+        nonlocal at
+        o, at = at, at + cnt * dtype.itemsize
+        return o, table[o:at].view(dtype)
+
+    _, it = take(ap, J * n)
+    it = it.reshape(J, n)
+    it["x"] = [[s.data_ptr() for s in h] for h in hold]
+    it["o"] = [w.data_ptr() for w in ws]
+    it["p"] = np.stack([c[2] for c in cores], axis=1)
+    it["chil"], it["din"], it["chir"] = X[rep, :, 0], X[rep, :, 1], X[rep, :, 2]
+    it["dl"], it["dout"], it["dr"] = O[:, 0], O[:, 2], O[:, 3]
+    nel = P[rep].prod(axis=2)
+    blocks = ((nel + _lib.APPLY_BLOCK - 1) // _lib.APPLY_BLOCK).reshape(-1)
+    it["block_start"] = (np.cumsum(blocks) - blocks).reshape(J, n)
+    apply_bytes = 8.0 * float(nel.sum() + X[rep].prod(axis=2).sum() + J * O.prod(axis=1).sum())
+
+    steps, done, carry = [], [], []
+    if T:
+        sel = rep[todo]                                                   # group of each truncated state
+        Dt = D[sel]
+        core = cores[0][2][todo]
+        for k in range(n - 1):
+            m, r = rows[sel, k], P[sel, k, 2]
+            cols = P[sel, k + 1, 1] * P[sel, k + 1, 2]
+            nb = np.minimum(r, Dt)
+            Q, S, W = _arena(m * Dt), _arena(Dt * r), _arena(Dt * cols)
+            work, tau = _arena(m * nb), _arena(nb)
+            oq, it = take(qr, T)
+            it["a"], it["rs"], it["cs"], it["m"], it["n"], it["keep"] = core, r, 1, m, r, Dt
+            it["q"], it["ldq"], it["work"], it["tau"] = Q[2], Dt, work[2], tau[2]
+            o1, it = take(ge, T)
+            g1 = _gemm_items(it, Q[2], core, S[2], Dt, r, m, Dt, 1)
+            o2, it = take(ge, T)
+            g2 = _gemm_items(it, S[2], cores[k + 1][2][todo], W[2], Dt, cols, r, r, 0)
+            steps.append((oq, o1, g1, o2, g2))
+            done.append(Q)
+            carry.append((S, W, work, tau))
+            core = W[2]
+
+    dev = ops._upload(table)
+    base, stream = dev.data_ptr(), ops._stream()
+    if ops._profiling[0]:
+        _lib.call("syn_prof_note_flops", apply_bytes)
+    _lib.call("syn_mpo_apply_f64", base, J * n, int(blocks.sum()), stream)
+    for oq, o1, g1, o2, g2 in steps:
+        _lib.call("syn_qr_f64", base + oq, T, stream)
+        for o, (tile, total, flops) in ((o1, g1), (o2, g2)):
+            if ops._profiling[0]:
+                _lib.call("syn_prof_note_flops", flops)
+            _lib.call("syn_gemm_f64", base + o, T, total, tile, stream)
+
+    outs = [None] * J
+    at = 0                                                                # first truncated state of the group
+    for g, key in enumerate(keys):
+        c = int(count[g])
+        input_shape, bond_shape = tuple(P[g, :, 1].tolist()), tuple(P[g, :-1, 2].tolist())
+        shape = [tuple(v) for v in P[g].tolist()]
+        if cut[g]:
+            d = int(D[g])
+            shape = [(shape[k][0] if k == 0 else d, shape[k][1], d if k < n - 1 else shape[k][2]) for k in range(n)]
+            held = [(*done[k][:2], at) for k in range(n - 1)] + [(*carry[-1][1][:2], at)]
+            at += c
+        else:
+            held = [(*cores[k][:2], int(first[g])) for k in range(n)]
+        params = sum(l * d * r for l, d, r in shape)
+        per_site = [_views(t, off, f, c, sh) for (t, off, f), sh in zip(held, shape)]
+        for i, sites in zip(members[key], zip(*per_site)):
+            outs[i] = _state(list(sites), list(shape), input_shape, bond_shape, params)
     return outs
 
 
