@@ -167,6 +167,7 @@ typedef struct {
     double *q;
     int64_t ldq;
     int32_t q_trans;  /* 1: store Q^T (kq x m, row-major, ldq) instead of Q */
+    int32_t columns;  /* 1: column by column, in one order of sums whatever the shape */
     double *work;
     double *tau;
 } syn_qr_item;
@@ -489,6 +490,31 @@ typedef struct {
     int64_t block_start;
 } syn_rowscale_item;
 int syn_rowscale_f64(const syn_rowscale_item *items, int n_items, int64_t total_blocks, void *stream);
+
+/* ------------------------------------------------------------------ */
+/* Small tables by value                                                 */
+/* Each of these is the entry point of the same name without _host, with  */
+/* the items in host memory: at most SYN_INLINE_BYTES of them, copied      */
+/* into the kernel's arguments before the call returns (SYN_EINVAL        */
+/* beyond).  No device table, no copy on the stream; the results have     */
+/* the same bits.                                                         */
+/* ------------------------------------------------------------------ */
+#define SYN_INLINE_BYTES 3840
+int syn_gemm_f64_host(const syn_gemm_item *items, int n_items, int64_t total_blocks, int tile, void *stream);
+int syn_gemm_mixed_f64_host(const syn_gemm_item *items, int n_items, int64_t total_blocks, int tile, void *stream);
+int syn_gemm_bf16_f64_host(const syn_gemm_item *items, int n_items, int64_t total_blocks, int tile, void *stream);
+int syn_mpo_apply_f64_host(const syn_apply_item *items, int n_items, int64_t total_blocks, void *stream);
+int syn_rowscale_f64_host(const syn_rowscale_item *items, int n_items, int64_t total_blocks, void *stream);
+int syn_eye_f64_host(const syn_eye_item *items, int n_items, int64_t total_blocks, void *stream);
+int syn_copy_f64_host(const syn_copy_item *items, int n_items, int64_t total_blocks, void *stream);
+int syn_vecnorms_f64_host(const syn_vecnorm_item *items, int n_items, int64_t total_blocks, void *stream);
+int syn_qr_f64_host(const syn_qr_item *items, int n_items, void *stream);
+int syn_qr_sized_f64_host(const syn_qr_item *items, int n_items, int64_t lds_doubles, void *stream);
+int syn_jacobi_f64_host(const syn_jacobi_item *items, int n_items, double tol, int max_sweeps, void *stream);
+int syn_jacobi_gram_f64_host(const syn_jacobi_item *items, int n_items, int64_t nv_max, double tol, int max_sweeps, void *stream);
+int syn_truncate_f64_host(const syn_trunc_item *items, int n_items, void *stream);
+int syn_diagmax_f64_host(const syn_diagmax_item *items, int n_items, void *stream);
+int syn_chol_leaf_f64_host(const syn_chol_item *items, int n_items, void *stream);
 
 /* ------------------------------------------------------------------ */
 /* Live per-kernel timing (HIP events on the launch stream).             */

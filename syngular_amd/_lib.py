@@ -40,7 +40,7 @@ DSUM_ITEM = np.dtype(
      ("lo", _I), ("ro", _I), ("edge", np.int32), ("block_start", _I)], align=True)
 QR_ITEM = np.dtype(
     [("a", _P), ("rs", _I), ("cs", _I), ("m", _I), ("n", _I), ("keep", _I), ("q", _P), ("ldq", _I),
-     ("q_trans", np.int32), ("work", _P), ("tau", _P)], align=True)
+     ("q_trans", np.int32), ("columns", np.int32), ("work", _P), ("tau", _P)], align=True)
 JACOBI_ITEM = np.dtype(
     [("x", _P), ("ldx", _I), ("nv", _I), ("len", _I), ("rt", _P), ("ldr", _I), ("s", _P), ("sweeps", _P),
      ("gram", np.int32)], align=True)
@@ -128,6 +128,17 @@ SIGNATURES = {
     "syn_prof_end": (_I32, [ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_double),
                             ctypes.POINTER(ctypes.c_double), _I32]),
 }
+
+# entry points that also take their table from host memory, by value (as
+# name + "_host"), and the item types they are found by
+INLINE_BYTES = 3840  # SYN_INLINE_BYTES
+HOST_ENTRIES = {name: name + "_host" for name in (
+    "syn_gemm_f64", "syn_gemm_mixed_f64", "syn_gemm_bf16_f64", "syn_mpo_apply_f64", "syn_rowscale_f64", "syn_eye_f64",
+    "syn_copy_f64", "syn_vecnorms_f64", "syn_qr_f64", "syn_qr_sized_f64", "syn_jacobi_f64", "syn_jacobi_gram_f64",
+    "syn_truncate_f64", "syn_diagmax_f64", "syn_chol_leaf_f64")}
+SIGNATURES.update({host: SIGNATURES[name] for name, host in HOST_ENTRIES.items()})
+INLINE_ITEMS = frozenset([GEMM_ITEM, APPLY_ITEM, ROWSCALE_ITEM, EYE_ITEM, COPY_ITEM, VECNORM_ITEM, QR_ITEM, JACOBI_ITEM,
+                          TRUNC_ITEM, DIAGMAX_ITEM, CHOL_ITEM])
 
 PROF_NTAGS = 20
 PROF_TAGS = {

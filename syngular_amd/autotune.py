@@ -130,7 +130,7 @@ def tune(max_bytes=4 << 30, reps=3):
             it["alpha"], it["beta"] = 1.0, 0.0
             st = np.concatenate([[0], np.cumsum(tm * tn)])
             it["block_start"], it["tiles_n"] = st[:-1], tn
-            d_it = ops._upload(it)
+            d_it = ops._device_table(it)
             fn = ops.gemm_fn(kind)
             total = int(st[-1])
             call(fn, d_it.data_ptr(), cnt, total, t, ops._stream())

@@ -145,7 +145,7 @@ def gemm_table(A, B, C, m, n, k, lda, ldb, ldc, ta=0, tb=0, alpha=1.0, beta=0.0,
     dev = ops._upload(it)
     if ops._profiling[0]:
         call("syn_prof_note_flops", float((2.0 * m * n * k).sum()))
-    call(ops.gemm_fn(mixed), dev.data_ptr(), cnt, total, tile, ops._stream())
+    call(ops.entry(ops.gemm_fn(mixed), dev), dev.data_ptr(), cnt, total, tile, ops._stream())
 
 
 def _launch_blocks(fn, it, nel):
@@ -157,7 +157,7 @@ def _launch_blocks(fn, it, nel):
     if total == 0:
         return
     dev = ops._upload(it)
-    call(fn, dev.data_ptr(), len(it), total, ops._stream())
+    call(ops.entry(fn, dev), dev.data_ptr(), len(it), total, ops._stream())
 
 
 def eye_table(x, n):
@@ -192,7 +192,7 @@ def vecnorm_table(x, rows, cols, ld, axis, out):
     it["block_start"] = st
     if total:
         dev = ops._upload(it)
-        call("syn_vecnorms_f64", dev.data_ptr(), cnt, total, ops._stream())
+        call(ops.entry("syn_vecnorms_f64", dev), dev.data_ptr(), cnt, total, ops._stream())
 
 
 def apply_table(x, o, p, chil, din, chir, dl, dout, dr):
@@ -210,14 +210,16 @@ def apply_table(x, o, p, chil, din, chir, dl, dout, dr):
 QR_LDS_CLASSES = (2048, 6144, 12288)
 
 
-def qr_table(a, m, n, q, work, tau):
+def qr_table(a, m, n, q, work, tau, columns=False):
     """Householder QR of every row-major m x n (m > n) matrix: q (m x n) gets
-    the thin orthogonal factor."""
+    the thin orthogonal factor.  columns: column by column, in one order of
+    sums (the mixed sweep rounds the factors to FP32, which would turn another
+    order's last bits into differences of an FP32 ulp)."""
     it = np.zeros(len(a), dtype=_lib.QR_ITEM)
     it["a"], it["rs"], it["cs"] = a, n, 1
     it["m"], it["n"], it["keep"] = m, n, n
     it["q"], it["ldq"], it["q_trans"] = q, n, 0
-    it["work"], it["tau"] = work, tau
+    it["work"], it["tau"], it["columns"] = work, tau, columns
     # one launch per LDS class of the matrices, each with the dynamic LDS its
     # largest matrix needs: small matrices do not hold a compute unit's LDS
     # for the large ones
@@ -229,7 +231,7 @@ def qr_table(a, m, n, q, work, tau):
             continue
         dev = ops._upload(it[sel])
         lds = int(need[sel].max()) if c < len(QR_LDS_CLASSES) else 0
-        call("syn_qr_sized_f64", dev.data_ptr(), len(sel), lds, ops._stream())
+        call(ops.entry("syn_qr_sized_f64", dev), dev.data_ptr(), len(sel), lds, ops._stream())
 
 
 # size classes (matrix order) of the LDS Jacobi launches
@@ -254,7 +256,7 @@ def jacobi_table(x, g, rt, s):
         if len(sel) == 0:
             continue
         dev = ops._upload(it[sel])
-        call("syn_jacobi_gram_f64", dev.data_ptr(), len(sel), int(g[sel].max()), TOL_LDS, ops.JACOBI_SWEEPS,
+        call(ops.entry("syn_jacobi_gram_f64", dev), dev.data_ptr(), len(sel), int(g[sel].max()), TOL_LDS, ops.JACOBI_SWEEPS,
              ops._stream())
 
 
@@ -286,7 +288,7 @@ def diagmax_table(g, n, ld, out, dropped):
     it["g"], it["n"], it["ld"], it["out"], it["dropped"] = g, n, ld, out, dropped
     if len(it):
         dev = ops._upload(it)
-        call("syn_diagmax_f64", dev.data_ptr(), len(it), ops._stream())
+        call(ops.entry("syn_diagmax_f64", dev), dev.data_ptr(), len(it), ops._stream())
 
 
 def chol_leaf_table(g, l, x, ld, n, maxdiag, tolrel, dropped):
@@ -295,7 +297,7 @@ def chol_leaf_table(g, l, x, ld, n, maxdiag, tolrel, dropped):
     it["n"], it["maxdiag"], it["tolrel"], it["dropped"] = n, maxdiag, tolrel, dropped
     if len(it):
         dev = ops._upload(it)
-        call("syn_chol_leaf_f64", dev.data_ptr(), len(it), ops._stream())
+        call(ops.entry("syn_chol_leaf_f64", dev), dev.data_ptr(), len(it), ops._stream())
 
 
 CHOL_LEAF = 64
@@ -434,7 +436,7 @@ def truncate_table(s, g, chi_max, cutoff, keep, disc):
     it["keep"], it["discarded"] = keep, disc
     if len(it):
         dev = ops._upload(it)
-        call("syn_truncate_f64", dev.data_ptr(), len(it), ops._stream())
+        call(ops.entry("syn_truncate_f64", dev), dev.data_ptr(), len(it), ops._stream())
 
 
 # --------------------------------------------------------------------------
@@ -664,7 +666,7 @@ class ChainBatch:
                 mt, rt = m[ti], r[ti]
                 wk, wp = arena(mt * rt)
                 tk, tp = arena(rt)
-                qr_table(ptr[a[ti], k], mt, rt, q[ti], wp, tp)
+                qr_table(ptr[a[ti], k], mt, rt, q[ti], wp, tp, columns=mixed)
                 st, sp = arena(rt * rt)
                 gemm_table(q[ti], ptr[a[ti], k], sp, rt, rt, mt, rt, rt, rt, ta=1)
                 S[ti] = sp

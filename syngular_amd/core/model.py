@@ -153,7 +153,7 @@ def matmul_batch(weight, states):
             carry.append((S, W, work, tau))
             core = W[2]
 
-    dev = ops._upload(table)
+    dev = ops._device_table(table)
     base, stream = dev.data_ptr(), ops._stream()
     if ops._profiling[0]:
         _lib.call("syn_prof_note_flops", apply_bytes)

@@ -295,9 +295,10 @@ __global__ __launch_bounds__(kCholThreads) void chol_diag_kernel(const double *G
 }
 
 // One leaf (n <= 64) per work-group, for many problems at once.
-__global__ __launch_bounds__(kCholThreads) void chol_leaf_many_kernel(const syn_chol_item *__restrict__ items) {
+template <typename Tab>
+__global__ __launch_bounds__(kCholThreads) void chol_leaf_many_kernel(Tab tab) {
     __shared__ double a[kNb][kNb + 1], lo[kNb][kNb + 1];
-    const syn_chol_item &P = items[blockIdx.x];
+    const syn_chol_item &P = tab.get()[blockIdx.x];
     chol_diag_body<kCholTG>(P.g, P.ldg, P.l, P.ldl, P.n, 0, P.x, P.ldx, P.maxdiag, P.tolrel, P.dropped, a, lo);
 }
 
@@ -396,8 +397,9 @@ __global__ __launch_bounds__(kCholThreads) void chol_node_kernel(double *G, int6
     node_gemm(X21 + kNb, ldx, T, kNb, false, X21, ldx, n2, kNb, n2, -1.0, 0.0, false, a, lo);
 }
 
-__global__ __launch_bounds__(256) void diagmax_many_kernel(const syn_diagmax_item *__restrict__ items) {
-    const syn_diagmax_item &P = items[blockIdx.x];
+template <typename Tab>
+__global__ __launch_bounds__(256) void diagmax_many_kernel(Tab tab) {
+    const syn_diagmax_item &P = tab.get()[blockIdx.x];
     __shared__ double red[4];
     double m = 0.0;
     for (int64_t i = threadIdx.x; i < P.n; i += 256) m = fmax(m, P.g[i * P.ld + i]);
@@ -617,6 +619,24 @@ extern "C" int syn_cholqr_f64(double *A, int64_t m, int64_t n, int64_t lda, doub
     return gemm_f64_launch(make_gemm(A, lda, 0, X, n, 1, Q, ldq, m, n, n, 1.0, 0.0, 8), s, mixed != 0);
 }
 
+namespace syn {
+template <typename Tab>
+static int chol_leaf_launch(Tab tab, int n_items, void *stream) {
+    hipStream_t s = (hipStream_t)stream;
+    ProfScope ps(kTagCholDiag, 0.0, s);
+    hipLaunchKernelGGL(chol_leaf_many_kernel<Tab>, dim3(n_items), dim3(kCholThreads), 0, s, tab);
+    SYN_LAUNCH_CHECK("syn_chol_leaf_f64 launch");
+    return SYN_OK;
+}
+
+template <typename Tab>
+static int diagmax_launch(Tab tab, int n_items, void *stream) {
+    hipLaunchKernelGGL(diagmax_many_kernel<Tab>, dim3(n_items), dim3(256), 0, (hipStream_t)stream, tab);
+    SYN_LAUNCH_CHECK("syn_diagmax_f64 launch");
+    return SYN_OK;
+}
+}  // namespace syn
+
 extern "C" int syn_chol_leaf_f64(const syn_chol_item *items, int n_items, void *stream) {
     using namespace syn;
     if (n_items < 0 || (n_items && !items)) {
@@ -624,11 +644,14 @@ extern "C" int syn_chol_leaf_f64(const syn_chol_item *items, int n_items, void *
         return SYN_EINVAL;
     }
     if (n_items == 0) return SYN_OK;
-    hipStream_t s = (hipStream_t)stream;
-    ProfScope ps(kTagCholDiag, 0.0, s);
-    hipLaunchKernelGGL(chol_leaf_many_kernel, dim3(n_items), dim3(kCholThreads), 0, s, items);
-    SYN_LAUNCH_CHECK("syn_chol_leaf_f64 launch");
-    return SYN_OK;
+    return chol_leaf_launch(DeviceTable<syn_chol_item>{items}, n_items, stream);
+}
+
+extern "C" int syn_chol_leaf_f64_host(const syn_chol_item *items, int n_items, void *stream) {
+    using namespace syn;
+    if (int rc = inline_check(items, n_items, "syn_chol_leaf_f64_host")) return rc;
+    if (n_items == 0) return SYN_OK;
+    return launch_inline(items, n_items, [&](const auto &tab) { return chol_leaf_launch(tab, n_items, stream); });
 }
 
 extern "C" int syn_diagmax_f64(const syn_diagmax_item *items, int n_items, void *stream) {
@@ -638,9 +661,14 @@ extern "C" int syn_diagmax_f64(const syn_diagmax_item *items, int n_items, void 
         return SYN_EINVAL;
     }
     if (n_items == 0) return SYN_OK;
-    hipLaunchKernelGGL(diagmax_many_kernel, dim3(n_items), dim3(256), 0, (hipStream_t)stream, items);
-    SYN_LAUNCH_CHECK("syn_diagmax_f64 launch");
-    return SYN_OK;
+    return diagmax_launch(DeviceTable<syn_diagmax_item>{items}, n_items, stream);
+}
+
+extern "C" int syn_diagmax_f64_host(const syn_diagmax_item *items, int n_items, void *stream) {
+    using namespace syn;
+    if (int rc = inline_check(items, n_items, "syn_diagmax_f64_host")) return rc;
+    if (n_items == 0) return SYN_OK;
+    return launch_inline(items, n_items, [&](const auto &tab) { return diagmax_launch(tab, n_items, stream); });
 }
 
 extern "C" int syn_cholqr_refine_f64(const double *Q1, int64_t m, int64_t n, int64_t ldq1, double *Q, int64_t ldq,

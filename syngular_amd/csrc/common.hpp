@@ -54,6 +54,48 @@ __device__ __forceinline__ int find_item(const Item *items, int n, int64_t b) {
     return lo;
 }
 
+// Item table of a launch: in device memory, or by value in the kernel's
+// arguments when it comes from the host and has few items.  A table of one to a
+// few dozen items otherwise costs a pinned allocation, a copy command of 3 us
+// on the stream and the gap before the kernel that waits for it.  Two sizes, so
+// that a single item does not carry kInlineBytes of arguments.
+constexpr size_t kInlineBytes = SYN_INLINE_BYTES;
+template <typename Item>
+struct DeviceTable {
+    const Item *p;
+    __device__ __forceinline__ const Item *get() const { return p; }
+};
+template <typename Item, int N>
+struct InlineTable {
+    Item it[N];
+    __device__ __forceinline__ const Item *get() const { return it; }
+};
+template <typename Item>
+constexpr int kInlineItems = (int)(kInlineBytes / sizeof(Item));
+
+// launch(table) with the items as an InlineTable; the caller has checked n
+template <typename Item, typename F>
+inline int launch_inline(const Item *items, int n, F launch) {
+    if (n == 1) {
+        InlineTable<Item, 1> t;
+        memcpy(t.it, items, sizeof(Item));
+        return launch(t);
+    }
+    InlineTable<Item, kInlineItems<Item>> t;
+    memcpy(t.it, items, (size_t)n * sizeof(Item));
+    memset((void *)(t.it + n), 0, (kInlineItems<Item> - n) * sizeof(Item));
+    return launch(t);
+}
+// SYN_EINVAL when a host table cannot go by value
+template <typename Item>
+inline int inline_check(const Item *items, int n, const char *who) {
+    if (n < 0 || n > kInlineItems<Item> || (n && !items)) {
+        set_error("%s: %d items (a host table holds at most %d)", who, n, kInlineItems<Item>);
+        return SYN_EINVAL;
+    }
+    return SYN_OK;
+}
+
 // Work-group barrier that orders LDS only: global stores issued before it
 // stay in flight.  For phases whose global writes no thread of the
 // work-group reads back (a plain __syncthreads waits for them to land).

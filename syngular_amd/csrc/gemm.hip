@@ -25,9 +25,9 @@ __device__ __forceinline__ int64_t tile_of_block(int64_t bid, int64_t total, int
     return by_col ? pos * tiles_n + line : line * tiles_n + pos;
 }
 
-template <int BM, int BN, int BK, int WM, int WN, typename CT = double>
-__global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, 2) void gemm_f64_grouped(
-    const syn_gemm_item *__restrict__ items, int n_items, int64_t total) {
+template <int BM, int BN, int BK, int WM, int WN, typename CT, typename Tab>
+__global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, 2) void gemm_f64_grouped(Tab tab, int n_items, int64_t total) {
+    const syn_gemm_item *__restrict__ items = tab.get();
     if (n_items == 1) {
         gemm_f64_tile<BM, BN, BK, WM, WN, CT>(items[0],
                                               tile_of_block(blockIdx.x, total, items[0].tiles_n, items[0].tri));
@@ -84,9 +84,9 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, 2) void gemm_f64_pair(s
 constexpr int kQuadK = 32;
 constexpr int64_t kQuadMax = 128;
 
-template <typename CT>
-__global__ __launch_bounds__(256, 2) void gemm_quad_grouped(const syn_gemm_item *__restrict__ items, int n_items,
-                                                              int64_t total) {
+template <typename CT, typename Tab>
+__global__ __launch_bounds__(256, 2) void gemm_quad_grouped(Tab tab, int n_items, int64_t total) {
+    const syn_gemm_item *__restrict__ items = tab.get();
     const int64_t b = xcd_remap(blockIdx.x, 4 * total), t = b >> 2;
     const syn_gemm_item &P = items[find_item(items, n_items, t)];
     gemm_f64_quad<kQuadK, CT>(P, t - P.block_start, (int)(b & 3));
@@ -312,102 +312,96 @@ namespace syn {
 constexpr int64_t kPersistentMin = 4096;
 constexpr int64_t kPersistentGrid = 1024;
 
-template <typename CT>
-static void launch_grouped(const syn_gemm_item *items, int n_items, int64_t total, int tile, hipStream_t s) {
-    const bool pers = total >= kPersistentMin && n_items > 1;
+// A table by value has few items: its launches of 4096 tiles and more are of
+// large problems, whose tiles gain nothing from the persistent form.
+template <typename CT, typename Tab>
+static int launch_grouped(Tab tab, int n_items, int64_t total, int tile, hipStream_t s, const char *who) {
+    constexpr bool kDevice = __is_same(Tab, DeviceTable<syn_gemm_item>);
+    const bool pers = kDevice && total >= kPersistentMin && n_items > 1;
     const unsigned grid = (unsigned)(pers ? kPersistentGrid : total);
+    bool quad = false;
     if constexpr (!__is_same(CT, bf16s)) {
-        if (tile == 0 && total <= kQuadMax) {
-            hipLaunchKernelGGL(gemm_quad_grouped<CT>, dim3((unsigned)(4 * total)), dim3(256), 0, s, items, n_items,
+        quad = tile == 0 && total <= kQuadMax;
+        if (quad)
+            hipLaunchKernelGGL((gemm_quad_grouped<CT, Tab>), dim3((unsigned)(4 * total)), dim3(256), 0, s, tab, n_items,
                                total);
-            return;
-        }
     }
-    if (tile == 0) {
-        if (pers)
+    if constexpr (kDevice) {
+        if (pers && tile == 0)
             hipLaunchKernelGGL((gemm_f64_grouped_persistent<64, 64, 16, 32, 32, CT>), dim3(grid), dim3(256), 0, s,
-                               items, n_items, total);
-        else
-            hipLaunchKernelGGL((gemm_f64_grouped<64, 64, 16, 32, 32, CT>), dim3(grid), dim3(256), 0, s, items, n_items,
-                               total);
-    } else {
-        if (pers)
+                               tab.p, n_items, total);
+        else if (pers)
             hipLaunchKernelGGL((gemm_f64_grouped_persistent<128, 128, 16, 64, 64, CT>), dim3(grid), dim3(256), 0, s,
-                               items, n_items, total);
+                               tab.p, n_items, total);
+    }
+    if (!pers && !quad) {
+        if (tile == 0)
+            hipLaunchKernelGGL((gemm_f64_grouped<64, 64, 16, 32, 32, CT, Tab>), dim3(grid), dim3(256), 0, s, tab,
+                               n_items, total);
         else
-            hipLaunchKernelGGL((gemm_f64_grouped<128, 128, 16, 64, 64, CT>), dim3(grid), dim3(256), 0, s, items,
+            hipLaunchKernelGGL((gemm_f64_grouped<128, 128, 16, 64, 64, CT, Tab>), dim3(grid), dim3(256), 0, s, tab,
                                n_items, total);
     }
+    SYN_LAUNCH_CHECK(who);
+    return SYN_OK;
+}
+
+// the three compute types' entry points: items on the device, or on the host
+// and passed by value
+template <typename CT>
+static int gemm_entry(const syn_gemm_item *items, int n_items, int64_t total_blocks, int tile, void *stream, int tag64,
+                      int tag128, bool host, const char *who) {
+    if (n_items < 0 || total_blocks < 0) {
+        set_error("%s: negative item or block count", who);
+        return SYN_EINVAL;
+    }
+    if (host)
+        if (int rc = inline_check(items, n_items, who)) return rc;
+    if (n_items == 0 || total_blocks == 0) return SYN_OK;
+    if (total_blocks > 0x7fffffffLL) {
+        set_error("%s: %lld tiles exceed the grid limit", who, (long long)total_blocks);
+        return SYN_EINVAL;
+    }
+    hipStream_t s = (hipStream_t)stream;
+    if (tile != 0 && tile != 1) {
+        set_error("%s: unknown tile configuration %d", who, tile);
+        return SYN_EINVAL;
+    }
+    ProfScope ps(tile == 1 ? tag128 : tag64, -1.0, s);
+    if (!host) return launch_grouped<CT>(DeviceTable<syn_gemm_item>{items}, n_items, total_blocks, tile, s, who);
+    return launch_inline(items, n_items, [&](const auto &tab) {
+        return launch_grouped<CT>(tab, n_items, total_blocks, tile, s, who);
+    });
 }
 
 }  // namespace syn
 
-extern "C" int syn_gemm_f64(const syn_gemm_item *items, int n_items, int64_t total_blocks, int tile,
-                            void *stream) {
+extern "C" int syn_gemm_f64(const syn_gemm_item *items, int n_items, int64_t total_blocks, int tile, void *stream) {
     using namespace syn;
-    if (n_items < 0 || total_blocks < 0) {
-        set_error("syn_gemm_f64: negative item or block count");
-        return SYN_EINVAL;
-    }
-    if (n_items == 0 || total_blocks == 0) return SYN_OK;
-    if (total_blocks > 0x7fffffffLL) {
-        set_error("syn_gemm_f64: %lld tiles exceed the grid limit", (long long)total_blocks);
-        return SYN_EINVAL;
-    }
-    hipStream_t s = (hipStream_t)stream;
-    if (tile != 0 && tile != 1) {
-        set_error("syn_gemm_f64: unknown tile configuration %d", tile);
-        return SYN_EINVAL;
-    }
-    ProfScope ps(tile == 1 ? kTagGemmGrouped128 : kTagGemmGrouped64, -1.0, s);
-    launch_grouped<double>(items, n_items, total_blocks, tile, s);
-    SYN_LAUNCH_CHECK("syn_gemm_f64 launch");
-    return SYN_OK;
+    return gemm_entry<double>(items, n_items, total_blocks, tile, stream, kTagGemmGrouped64, kTagGemmGrouped128, false, "syn_gemm_f64");
 }
 
-
-extern "C" int syn_gemm_bf16_f64(const syn_gemm_item *items, int n_items, int64_t total_blocks, int tile,
-                                 void *stream) {
+extern "C" int syn_gemm_f64_host(const syn_gemm_item *items, int n_items, int64_t total_blocks, int tile, void *stream) {
     using namespace syn;
-    if (n_items < 0 || total_blocks < 0) {
-        set_error("syn_gemm_bf16_f64: negative item or block count");
-        return SYN_EINVAL;
-    }
-    if (n_items == 0 || total_blocks == 0) return SYN_OK;
-    if (total_blocks > 0x7fffffffLL) {
-        set_error("syn_gemm_bf16_f64: %lld tiles exceed the grid limit", (long long)total_blocks);
-        return SYN_EINVAL;
-    }
-    hipStream_t s = (hipStream_t)stream;
-    if (tile != 0 && tile != 1) {
-        set_error("syn_gemm_bf16_f64: unknown tile configuration %d", tile);
-        return SYN_EINVAL;
-    }
-    ProfScope ps(tile == 1 ? kTagGemmBf16128 : kTagGemmBf1664, -1.0, s);
-    launch_grouped<bf16s>(items, n_items, total_blocks, tile, s);
-    SYN_LAUNCH_CHECK("syn_gemm_bf16_f64 launch");
-    return SYN_OK;
+    return gemm_entry<double>(items, n_items, total_blocks, tile, stream, kTagGemmGrouped64, kTagGemmGrouped128, true, "syn_gemm_f64_host");
 }
 
-extern "C" int syn_gemm_mixed_f64(const syn_gemm_item *items, int n_items, int64_t total_blocks, int tile,
-                                  void *stream) {
+extern "C" int syn_gemm_mixed_f64(const syn_gemm_item *items, int n_items, int64_t total_blocks, int tile, void *stream) {
     using namespace syn;
-    if (n_items < 0 || total_blocks < 0) {
-        set_error("syn_gemm_mixed_f64: negative item or block count");
-        return SYN_EINVAL;
-    }
-    if (n_items == 0 || total_blocks == 0) return SYN_OK;
-    if (total_blocks > 0x7fffffffLL) {
-        set_error("syn_gemm_mixed_f64: %lld tiles exceed the grid limit", (long long)total_blocks);
-        return SYN_EINVAL;
-    }
-    hipStream_t s = (hipStream_t)stream;
-    if (tile != 0 && tile != 1) {
-        set_error("syn_gemm_mixed_f64: unknown tile configuration %d", tile);
-        return SYN_EINVAL;
-    }
-    ProfScope ps(tile == 1 ? kTagGemmMixed128 : kTagGemmMixed64, -1.0, s);
-    launch_grouped<float>(items, n_items, total_blocks, tile, s);
-    SYN_LAUNCH_CHECK("syn_gemm_mixed_f64 launch");
-    return SYN_OK;
+    return gemm_entry<float>(items, n_items, total_blocks, tile, stream, kTagGemmMixed64, kTagGemmMixed128, false, "syn_gemm_mixed_f64");
+}
+
+extern "C" int syn_gemm_mixed_f64_host(const syn_gemm_item *items, int n_items, int64_t total_blocks, int tile, void *stream) {
+    using namespace syn;
+    return gemm_entry<float>(items, n_items, total_blocks, tile, stream, kTagGemmMixed64, kTagGemmMixed128, true, "syn_gemm_mixed_f64_host");
+}
+
+extern "C" int syn_gemm_bf16_f64(const syn_gemm_item *items, int n_items, int64_t total_blocks, int tile, void *stream) {
+    using namespace syn;
+    return gemm_entry<bf16s>(items, n_items, total_blocks, tile, stream, kTagGemmBf1664, kTagGemmBf16128, false, "syn_gemm_bf16_f64");
+}
+
+extern "C" int syn_gemm_bf16_f64_host(const syn_gemm_item *items, int n_items, int64_t total_blocks, int tile, void *stream) {
+    using namespace syn;
+    return gemm_entry<bf16s>(items, n_items, total_blocks, tile, stream, kTagGemmBf1664, kTagGemmBf16128, true, "syn_gemm_bf16_f64_host");
 }

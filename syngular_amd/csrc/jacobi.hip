@@ -176,10 +176,10 @@ __device__ void jacobi_one(const syn_jacobi_item &P, double *lds, double tol, in
     if (tid == 0 && P.sweeps) *P.sweeps = sweep;
 }
 
-__global__ __launch_bounds__(kJacThreads) void jacobi_kernel(const syn_jacobi_item *__restrict__ items, double tol,
-                                                             int max_sweeps) {
+template <typename Tab>
+__global__ __launch_bounds__(kJacThreads) void jacobi_kernel(Tab tab, double tol, int max_sweeps) {
     extern __shared__ double lds[];
-    const syn_jacobi_item &P = items[blockIdx.x];
+    const syn_jacobi_item &P = tab.get()[blockIdx.x];
     if (P.nv * P.len + P.nv * P.nv <= kJacLdsDoubles)
         jacobi_one<true>(P, lds, tol, max_sweeps);
     else
@@ -207,15 +207,14 @@ __global__ __launch_bounds__(kJacThreads) void jacobi_kernel(const syn_jacobi_it
 constexpr int kGramThreads = 256;
 constexpr int kGramMax = 64;
 
-template <int NT>
-__global__ __launch_bounds__(NT) void jacobi_gram_kernel(const syn_jacobi_item *__restrict__ items,
-                                                                   int nv_max, double tol, int max_sweeps) {
+template <int NT, typename Tab>
+__global__ __launch_bounds__(NT) void jacobi_gram_kernel(Tab tab, int nv_max, double tol, int max_sweeps) {
     extern __shared__ double lds[];
     __shared__ double cs[kGramMax / 2][2];
     __shared__ int pp[kGramMax / 2], qq[kGramMax / 2];
     __shared__ int rank[kGramMax];
     __shared__ int rotated;
-    const syn_jacobi_item &P = items[blockIdx.x];
+    const syn_jacobi_item &P = tab.get()[blockIdx.x];
     const int tid = threadIdx.x;
     if (P.nv < 1 || P.nv > nv_max || P.len != P.nv) {
         // not a problem this kernel takes: flag it in s and leave the rest
@@ -333,17 +332,13 @@ __global__ __launch_bounds__(NT) void jacobi_gram_kernel(const syn_jacobi_item *
 
 }  // namespace syn
 
-extern "C" int syn_jacobi_gram_f64(const syn_jacobi_item *items, int n_items, int64_t nv_max, double tol,
-                                   int max_sweeps, void *stream) {
-    using namespace syn;
-    if (n_items < 0 || nv_max < 1 || nv_max > kGramMax || max_sweeps < 0 || !(tol >= 0.0)) {
-        set_error("syn_jacobi_gram_f64: bad arguments (nv_max=%lld, limit %d)", (long long)nv_max, kGramMax);
-        return SYN_EINVAL;
-    }
-    if (n_items == 0) return SYN_OK;
+namespace syn {
+
+template <typename Tab>
+static int jacobi_gram_launch(Tab tab, int n_items, int64_t nv_max, double tol, int max_sweeps, void *stream) {
     static bool attr_set = false;
     if (!attr_set) {   // orders above 32 take more than 64 KiB of LDS
-        if (int rc = hip_check(hipFuncSetAttribute((const void *)jacobi_gram_kernel<kGramThreads>,
+        if (int rc = hip_check(hipFuncSetAttribute((const void *)jacobi_gram_kernel<kGramThreads, Tab>,
                                                    hipFuncAttributeMaxDynamicSharedMemorySize,
                                                    (int)(2 * kGramMax * (kGramMax + 1) * sizeof(double))),
                                "syn_jacobi_gram_f64: hipFuncSetAttribute"))
@@ -352,32 +347,80 @@ extern "C" int syn_jacobi_gram_f64(const syn_jacobi_item *items, int n_items, in
     }
     const size_t shm = 2 * (size_t)nv_max * (size_t)(nv_max + 1) * sizeof(double);
     ProfScope ps(kTagJacobi, 0.0, (hipStream_t)stream);
-    auto kern = nv_max <= 16 ? jacobi_gram_kernel<64>
-                             : (nv_max <= 32 ? jacobi_gram_kernel<128> : jacobi_gram_kernel<kGramThreads>);
+    auto kern = nv_max <= 16 ? jacobi_gram_kernel<64, Tab>
+                             : (nv_max <= 32 ? jacobi_gram_kernel<128, Tab> : jacobi_gram_kernel<kGramThreads, Tab>);
     const int nt = nv_max <= 16 ? 64 : (nv_max <= 32 ? 128 : kGramThreads);
-    hipLaunchKernelGGL(kern, dim3(n_items), dim3(nt), shm, (hipStream_t)stream, items,
-                       (int)nv_max, tol, max_sweeps);
+    hipLaunchKernelGGL(kern, dim3(n_items), dim3(nt), shm, (hipStream_t)stream, tab, (int)nv_max, tol, max_sweeps);
     SYN_LAUNCH_CHECK("syn_jacobi_gram_f64 launch");
     return SYN_OK;
+}
+
+static int gram_args(int n_items, int64_t nv_max, double tol, int max_sweeps) {
+    if (n_items < 0 || nv_max < 1 || nv_max > kGramMax || max_sweeps < 0 || !(tol >= 0.0)) {
+        set_error("syn_jacobi_gram_f64: bad arguments (nv_max=%lld, limit %d)", (long long)nv_max, kGramMax);
+        return SYN_EINVAL;
+    }
+    return SYN_OK;
+}
+
+template <typename Tab>
+static int jacobi_launch(Tab tab, int n_items, double tol, int max_sweeps, void *stream) {
+    static bool attr_set = false;
+    if (!attr_set) {
+        (void)hipFuncSetAttribute((const void *)jacobi_kernel<Tab>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)(kJacLdsDoubles * sizeof(double)));
+        attr_set = true;
+    }
+    ProfScope ps(kTagJacobi, 0.0, (hipStream_t)stream);
+    hipLaunchKernelGGL(jacobi_kernel<Tab>, dim3(n_items), dim3(kJacThreads), kJacLdsDoubles * sizeof(double),
+                       (hipStream_t)stream, tab, tol, max_sweeps);
+    SYN_LAUNCH_CHECK("syn_jacobi_f64 launch");
+    return SYN_OK;
+}
+
+static int jacobi_args(int n_items, double tol, int max_sweeps) {
+    if (n_items < 0 || max_sweeps < 0 || !(tol >= 0.0)) {
+        set_error("syn_jacobi_f64: bad arguments");
+        return SYN_EINVAL;
+    }
+    return SYN_OK;
+}
+
+}  // namespace syn
+
+extern "C" int syn_jacobi_gram_f64(const syn_jacobi_item *items, int n_items, int64_t nv_max, double tol,
+                                   int max_sweeps, void *stream) {
+    using namespace syn;
+    if (int rc = gram_args(n_items, nv_max, tol, max_sweeps)) return rc;
+    if (n_items == 0) return SYN_OK;
+    return jacobi_gram_launch(DeviceTable<syn_jacobi_item>{items}, n_items, nv_max, tol, max_sweeps, stream);
+}
+
+extern "C" int syn_jacobi_gram_f64_host(const syn_jacobi_item *items, int n_items, int64_t nv_max, double tol,
+                                        int max_sweeps, void *stream) {
+    using namespace syn;
+    if (int rc = gram_args(n_items, nv_max, tol, max_sweeps)) return rc;
+    if (int rc = inline_check(items, n_items, "syn_jacobi_gram_f64_host")) return rc;
+    if (n_items == 0) return SYN_OK;
+    return launch_inline(items, n_items, [&](const auto &tab) {
+        return jacobi_gram_launch(tab, n_items, nv_max, tol, max_sweeps, stream);
+    });
 }
 
 extern "C" int syn_jacobi_f64(const syn_jacobi_item *items, int n_items, double tol, int max_sweeps,
                               void *stream) {
     using namespace syn;
-    if (n_items < 0 || max_sweeps < 0 || !(tol >= 0.0)) {
-        set_error("syn_jacobi_f64: bad arguments");
-        return SYN_EINVAL;
-    }
+    if (int rc = jacobi_args(n_items, tol, max_sweeps)) return rc;
     if (n_items == 0) return SYN_OK;
-    static bool attr_set = false;
-    if (!attr_set) {
-        (void)hipFuncSetAttribute((const void *)jacobi_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)(kJacLdsDoubles * sizeof(double)));
-        attr_set = true;
-    }
-    ProfScope ps(kTagJacobi, 0.0, (hipStream_t)stream);
-    hipLaunchKernelGGL(jacobi_kernel, dim3(n_items), dim3(kJacThreads), kJacLdsDoubles * sizeof(double),
-                       (hipStream_t)stream, items, tol, max_sweeps);
-    SYN_LAUNCH_CHECK("syn_jacobi_f64 launch");
-    return SYN_OK;
+    return jacobi_launch(DeviceTable<syn_jacobi_item>{items}, n_items, tol, max_sweeps, stream);
+}
+
+extern "C" int syn_jacobi_f64_host(const syn_jacobi_item *items, int n_items, double tol, int max_sweeps,
+                                   void *stream) {
+    using namespace syn;
+    if (int rc = jacobi_args(n_items, tol, max_sweeps)) return rc;
+    if (int rc = inline_check(items, n_items, "syn_jacobi_f64_host")) return rc;
+    if (n_items == 0) return SYN_OK;
+    return launch_inline(items, n_items,
+                         [&](const auto &tab) { return jacobi_launch(tab, n_items, tol, max_sweeps, stream); });
 }

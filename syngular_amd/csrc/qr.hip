@@ -27,11 +27,13 @@ namespace syn {
 
 constexpr int kQrThreads = 512;
 constexpr int kQrWaves = kQrThreads / 64;
+constexpr int kColWaves = 4;
 constexpr int64_t kQrLdsDoubles = (96 * 1024) / 8;
 
+template <int NW>
 __device__ __forceinline__ void seg_bounds(int64_t lo, int64_t hi, int w, int64_t &a, int64_t &b) {
     const int64_t len = hi > lo ? hi - lo : 0;
-    const int64_t per = (len + kQrWaves - 1) / kQrWaves;
+    const int64_t per = (len + NW - 1) / NW;
     a = lo + per * w;
     b = a + per;
     if (a > hi) a = hi;
@@ -40,38 +42,65 @@ __device__ __forceinline__ void seg_bounds(int64_t lo, int64_t hi, int w, int64_
 
 // Apply H = I - tau v v^T (v = [1; M[j+1:, j]] taken from V) to columns
 // [c_lo, c_hi) of M (rows j..m-1).  V and M may alias (factorisation step).
+template <int NW>
 __device__ __forceinline__ void apply_reflector(const double *V, int64_t ldv, int64_t j, double tau, double *M,
                                                 int64_t ldm, int64_t m, int64_t c_lo, int64_t c_hi,
                                                 double (*red)[64]) {
+    // rows loaded together: column j is not among those written, but the
+    // compiler cannot know, and row by row each would wait for the last store
+    constexpr int U = 8;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     int64_t r0, r1;
-    seg_bounds(j + 1, m, w, r0, r1);
+    seg_bounds<NW>(j + 1, m, w, r0, r1);
     for (int64_t c0 = c_lo; c0 < c_hi; c0 += 64) {
         const int64_t c = c0 + lane;
         const bool act = c < c_hi;
         double part = 0.0;
-        if (act)
-            for (int64_t i = r0; i < r1; ++i) part = fma(V[i * ldv + j], M[i * ldm + c], part);
+        if (act) {
+            int64_t i = r0;
+            for (; i + U <= r1; i += U) {
+                double v[U], x[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    v[u] = V[(i + u) * ldv + j];
+                    x[u] = M[(i + u) * ldm + c];
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u) part = fma(v[u], x[u], part);
+            }
+            for (; i < r1; ++i) part = fma(V[i * ldv + j], M[i * ldm + c], part);
+        }
         red[w][lane] = part;
         __syncthreads();
         double dot = 0.0;
         if (act) {
             dot = M[j * ldm + c];
 #pragma unroll
-            for (int q = 0; q < kQrWaves; ++q) dot += red[q][lane];
+            for (int q = 0; q < NW; ++q) dot += red[q][lane];
         }
         const double f = tau * dot;
         __syncthreads();  // every wave has read red[] and M[j, c] before row j changes
         if (act) {
             if (w == 0) M[j * ldm + c] -= f;
-            for (int64_t i = r0; i < r1; ++i) M[i * ldm + c] = fma(-f, V[i * ldv + j], M[i * ldm + c]);
+            int64_t i = r0;
+            for (; i + U <= r1; i += U) {
+                double v[U], x[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    v[u] = V[(i + u) * ldv + j];
+                    x[u] = M[(i + u) * ldm + c];
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u) M[(i + u) * ldm + c] = fma(-f, v[u], x[u]);
+            }
+            for (; i < r1; ++i) M[i * ldm + c] = fma(-f, V[i * ldv + j], M[i * ldm + c]);
         }
     }
 }
 
-template <bool IN_LDS>
-__device__ void qr_one(const syn_qr_item &P, double *lds_w) {
-    __shared__ double red[kQrWaves][64];
+template <int NW, bool IN_LDS>
+__device__ __forceinline__ void qr_one(const syn_qr_item &P, double *lds_w) {
+    __shared__ double red[NW][64];
     __shared__ double shv[4];
     const int64_t m = P.m, n = P.n, keep = P.keep;
     const int64_t nb = n < keep ? n : keep;
@@ -80,7 +109,7 @@ __device__ void qr_one(const syn_qr_item &P, double *lds_w) {
     double *W = IN_LDS ? lds_w : P.work;
     const int tid = threadIdx.x;
 
-    for (int64_t e = tid; e < m * nb; e += kQrThreads) {
+    for (int64_t e = tid; e < m * nb; e += (64 * NW)) {
         const int64_t i = e / nb, j = e - i * nb;
         W[e] = P.a[i * P.rs + j * P.cs];
     }
@@ -88,7 +117,7 @@ __device__ void qr_one(const syn_qr_item &P, double *lds_w) {
 
     for (int64_t j = 0; j < p; ++j) {
         double part = 0.0;
-        for (int64_t i = j + 1 + tid; i < m; i += kQrThreads) {
+        for (int64_t i = j + 1 + tid; i < m; i += (64 * NW)) {
             const double v = W[i * nb + j];
             part = fma(v, v, part);
         }
@@ -97,7 +126,7 @@ __device__ void qr_one(const syn_qr_item &P, double *lds_w) {
         __syncthreads();
         if (tid == 0) {
             double xn2 = 0.0;
-            for (int q = 0; q < kQrWaves; ++q) xn2 += red[q][0];
+            for (int q = 0; q < NW; ++q) xn2 += red[q][0];
             const double alpha = W[j * nb + j];
             double tau = 0.0, scal = 0.0;
             if (xn2 > 0.0) {
@@ -113,9 +142,9 @@ __device__ void qr_one(const syn_qr_item &P, double *lds_w) {
         __syncthreads();
         const double tau = shv[0], scal = shv[1];
         if (tau != 0.0) {
-            for (int64_t i = j + 1 + tid; i < m; i += kQrThreads) W[i * nb + j] *= scal;
+            for (int64_t i = j + 1 + tid; i < m; i += (64 * NW)) W[i * nb + j] *= scal;
             __syncthreads();
-            apply_reflector(W, nb, j, tau, W, nb, m, j + 1, nb, red);
+            apply_reflector<NW>(W, nb, j, tau, W, nb, m, j + 1, nb, red);
         }
         __syncthreads();
     }
@@ -124,18 +153,18 @@ __device__ void qr_one(const syn_qr_item &P, double *lds_w) {
     // tail and transposed on the way out).
     double *Q = P.q_trans ? P.work + m * nb : P.q;
     const int64_t ldq = P.q_trans ? kq : P.ldq;
-    for (int64_t e = tid; e < m * kq; e += kQrThreads) {
+    for (int64_t e = tid; e < m * kq; e += (64 * NW)) {
         const int64_t i = e / kq, c = e - i * kq;
         Q[i * ldq + c] = (i == c) ? 1.0 : 0.0;
     }
     __syncthreads();
     for (int64_t j = p - 1; j >= 0; --j) {
         const double tau = P.tau[j];
-        if (tau != 0.0) apply_reflector(W, nb, j, tau, Q, ldq, m, j, kq, red);
+        if (tau != 0.0) apply_reflector<NW>(W, nb, j, tau, Q, ldq, m, j, kq, red);
         __syncthreads();
     }
     if (P.q_trans) {
-        for (int64_t e = tid; e < m * kq; e += kQrThreads) {
+        for (int64_t e = tid; e < m * kq; e += (64 * NW)) {
             const int64_t c = e / m, i = e - c * m;
             P.q[c * P.ldq + i] = Q[i * ldq + c];
         }
@@ -157,7 +186,7 @@ struct QrTileSmem {
 };
 
 template <int RT>
-__device__ void qr_tile(const syn_qr_item &P, QrTileSmem &sm) {
+__device__ __forceinline__ void qr_tile(const syn_qr_item &P, QrTileSmem &sm) {
     const int m = (int)P.m, nb = (int)(P.n < P.keep ? P.n : P.keep), kq = (int)(P.keep < P.m ? P.keep : P.m);
     const int p = m < nb ? m : nb, tid = threadIdx.x, wv = tid >> 6;
     double *W = P.work;
@@ -198,12 +227,22 @@ __device__ void qr_tile(const syn_qr_item &P, QrTileSmem &sm) {
 
 // lds_cap: doubles of dynamic LDS the launch holds; a matrix whose leading
 // block fits works in LDS, a larger one in its workspace.
-__global__ __launch_bounds__(kQrThreads) void qr_kernel(const syn_qr_item *__restrict__ items, int n_items,
-                                                         int64_t lds_cap) {
+template <typename Tab>
+__global__ __launch_bounds__(kQrThreads) void qr_kernel(Tab tab, int64_t lds_cap) {
     extern __shared__ double lds_w[];
-    const syn_qr_item &P = items[blockIdx.x];
+    const syn_qr_item &P = tab.get()[blockIdx.x];
     const int64_t nb = P.n < P.keep ? P.n : P.keep;
-    if (P.m <= kTileRows && nb <= kTileCols) {
+    if (P.columns) {
+        // The column-by-column form by four waves, whatever the shape.  The mixed
+        // sweep asks for it: it rounds its factors to FP32, where another order of
+        // the FP64 sums, no less exact, now and then ends on the neighbouring FP32
+        // number, so this order is part of that form's results.
+        if (threadIdx.x >= 64 * kColWaves) return;   // whole waves: the others' barriers do not wait for them
+        if (P.m * nb <= lds_cap)
+            qr_one<kColWaves, true>(P, lds_w);
+        else
+            qr_one<kColWaves, false>(P, lds_w);
+    } else if (P.m <= kTileRows && nb <= kTileCols) {
         QrTileSmem &sm = *(QrTileSmem *)lds_w;
         if (P.m <= 128)
             qr_tile<1>(P, sm);
@@ -212,17 +251,18 @@ __global__ __launch_bounds__(kQrThreads) void qr_kernel(const syn_qr_item *__res
         else
             qr_tile<4>(P, sm);
     } else if (P.m * nb <= lds_cap)
-        qr_one<true>(P, lds_w);
+        qr_one<kQrWaves, true>(P, lds_w);
     else
-        qr_one<false>(P, lds_w);
+        qr_one<kQrWaves, false>(P, lds_w);
 }
 
 // every launch holds what the panel form needs; the other form its lds_cap
-static int qr_launch(const syn_qr_item *items, int n_items, int64_t lds_doubles, hipStream_t s) {
+template <typename Tab>
+static int qr_launch(Tab tab, int n_items, int64_t lds_doubles, hipStream_t s) {
     static bool attr_set = false;
     const size_t most = std::max(sizeof(QrTileSmem), (size_t)kQrLdsDoubles * sizeof(double));
     if (!attr_set) {
-        if (int rc = hip_check(hipFuncSetAttribute((const void *)qr_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+        if (int rc = hip_check(hipFuncSetAttribute((const void *)qr_kernel<Tab>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                                    (int)most),
                                "syn_qr_f64: hipFuncSetAttribute"))
             return rc;
@@ -230,7 +270,7 @@ static int qr_launch(const syn_qr_item *items, int n_items, int64_t lds_doubles,
     }
     const size_t lds = std::max(sizeof(QrTileSmem), (size_t)lds_doubles * sizeof(double));
     ProfScope ps(kTagQr, 0.0, s);
-    hipLaunchKernelGGL(qr_kernel, dim3(n_items), dim3(kQrThreads), lds, s, items, n_items, lds_doubles);
+    hipLaunchKernelGGL(qr_kernel<Tab>, dim3(n_items), dim3(kQrThreads), lds, s, tab, lds_doubles);
     SYN_LAUNCH_CHECK("syn_qr_f64 launch");
     return SYN_OK;
 }
@@ -244,7 +284,11 @@ extern "C" int syn_qr_f64(const syn_qr_item *items, int n_items, void *stream) {
         return SYN_EINVAL;
     }
     if (n_items == 0) return SYN_OK;
-    return qr_launch(items, n_items, kQrLdsDoubles, (hipStream_t)stream);
+    return qr_launch(DeviceTable<syn_qr_item>{items}, n_items, kQrLdsDoubles, (hipStream_t)stream);
+}
+
+extern "C" int syn_qr_f64_host(const syn_qr_item *items, int n_items, void *stream) {
+    return syn_qr_sized_f64_host(items, n_items, syn::kQrLdsDoubles, stream);
 }
 
 extern "C" int syn_qr_sized_f64(const syn_qr_item *items, int n_items, int64_t lds_doubles, void *stream) {
@@ -255,5 +299,18 @@ extern "C" int syn_qr_sized_f64(const syn_qr_item *items, int n_items, int64_t l
         return SYN_EINVAL;
     }
     if (n_items == 0) return SYN_OK;
-    return qr_launch(items, n_items, lds_doubles, (hipStream_t)stream);
+    return qr_launch(DeviceTable<syn_qr_item>{items}, n_items, lds_doubles, (hipStream_t)stream);
+}
+
+extern "C" int syn_qr_sized_f64_host(const syn_qr_item *items, int n_items, int64_t lds_doubles, void *stream) {
+    using namespace syn;
+    if (int rc = inline_check(items, n_items, "syn_qr_sized_f64_host")) return rc;
+    if (lds_doubles < 0 || lds_doubles > kQrLdsDoubles) {
+        set_error("syn_qr_sized_f64_host: bad LDS size %lld (at most %lld doubles)", (long long)lds_doubles,
+                  (long long)kQrLdsDoubles);
+        return SYN_EINVAL;
+    }
+    if (n_items == 0) return SYN_OK;
+    return launch_inline(items, n_items,
+                         [&](const auto &tab) { return qr_launch(tab, n_items, lds_doubles, (hipStream_t)stream); });
 }

@@ -39,8 +39,9 @@ __device__ __forceinline__ void apply_block(const syn_apply_item &P, int64_t loc
     }
 }
 
-__global__ __launch_bounds__(kSiteThreads) void apply_kernel(const syn_apply_item *__restrict__ items, int n,
-                                                             int64_t total) {
+template <typename Tab>
+__global__ __launch_bounds__(kSiteThreads) void apply_kernel(Tab tab, int n) {
+    const syn_apply_item *__restrict__ items = tab.get();
     const int64_t bid = blockIdx.x;
     const syn_apply_item &P = items[find_item(items, n, bid)];
     const int64_t nel = P.chil * P.dl * P.dout * P.chir * P.dr;
@@ -135,8 +136,9 @@ __global__ __launch_bounds__(kSiteThreads) void dsum_kernel(const syn_dsum_item 
     }
 }
 
-__global__ __launch_bounds__(kSiteThreads) void rowscale_kernel(const syn_rowscale_item *__restrict__ items,
-                                                                int n, int64_t total) {
+template <typename Tab>
+__global__ __launch_bounds__(kSiteThreads) void rowscale_kernel(Tab tab, int n) {
+    const syn_rowscale_item *__restrict__ items = tab.get();
     const int64_t bid = blockIdx.x;
     const syn_rowscale_item &P = items[find_item(items, n, bid)];
     const int64_t nel = P.rows * P.cols;
@@ -154,8 +156,9 @@ __global__ __launch_bounds__(kSiteThreads) void rowscale_kernel(const syn_rowsca
     }
 }
 
-__global__ __launch_bounds__(kSiteThreads) void eye_kernel(const syn_eye_item *__restrict__ items, int n,
-                                                           int64_t total) {
+template <typename Tab>
+__global__ __launch_bounds__(kSiteThreads) void eye_kernel(Tab tab, int n) {
+    const syn_eye_item *__restrict__ items = tab.get();
     const int64_t bid = blockIdx.x;
     const syn_eye_item &P = items[find_item(items, n, bid)];
     const int64_t nel = P.n * P.n;
@@ -168,8 +171,9 @@ __global__ __launch_bounds__(kSiteThreads) void eye_kernel(const syn_eye_item *_
     }
 }
 
-__global__ __launch_bounds__(kSiteThreads) void copy_kernel(const syn_copy_item *__restrict__ items, int n,
-                                                            int64_t total) {
+template <typename Tab>
+__global__ __launch_bounds__(kSiteThreads) void copy_kernel(Tab tab, int n) {
+    const syn_copy_item *__restrict__ items = tab.get();
     const int64_t bid = blockIdx.x;
     const syn_copy_item &P = items[find_item(items, n, bid)];
     const int64_t base = (bid - P.block_start) * SYN_APPLY_BLOCK + threadIdx.x;
@@ -189,15 +193,30 @@ static int grid_check(int n_items, int64_t total_blocks, const char *who) {
 
 }  // namespace syn
 
+namespace syn {
+template <typename Tab>
+static int apply_launch(Tab tab, int n_items, int64_t total_blocks, void *stream) {
+    hipStream_t s = (hipStream_t)stream;
+    ProfScope ps(kTagApply, -1.0, s);
+    hipLaunchKernelGGL(apply_kernel<Tab>, dim3((unsigned)total_blocks), dim3(kSiteThreads), 0, s, tab, n_items);
+    SYN_LAUNCH_CHECK("syn_mpo_apply_f64 launch");
+    return SYN_OK;
+}
+}  // namespace syn
+
 extern "C" int syn_mpo_apply_f64(const syn_apply_item *items, int n_items, int64_t total_blocks, void *stream) {
     using namespace syn;
     if (int rc = grid_check(n_items, total_blocks, "syn_mpo_apply_f64")) return rc;
     if (n_items == 0 || total_blocks == 0) return SYN_OK;
-    ProfScope ps(kTagApply, -1.0, (hipStream_t)stream);
-    hipLaunchKernelGGL(apply_kernel, dim3((unsigned)total_blocks), dim3(kSiteThreads), 0, (hipStream_t)stream,
-                       items, n_items, total_blocks);
-    SYN_LAUNCH_CHECK("syn_mpo_apply_f64 launch");
-    return SYN_OK;
+    return apply_launch(DeviceTable<syn_apply_item>{items}, n_items, total_blocks, stream);
+}
+
+extern "C" int syn_mpo_apply_f64_host(const syn_apply_item *items, int n_items, int64_t total_blocks, void *stream) {
+    using namespace syn;
+    if (int rc = grid_check(n_items, total_blocks, "syn_mpo_apply_f64_host")) return rc;
+    if (int rc = inline_check(items, n_items, "syn_mpo_apply_f64_host")) return rc;
+    if (n_items == 0 || total_blocks == 0) return SYN_OK;
+    return launch_inline(items, n_items, [&](const auto &tab) { return apply_launch(tab, n_items, total_blocks, stream); });
 }
 
 extern "C" int syn_mpo_mpo_f64(const syn_mpo_mpo_item *items, int n_items, int64_t total_blocks, void *stream) {
@@ -220,14 +239,29 @@ extern "C" int syn_direct_sum_f64(const syn_dsum_item *items, int n_items, int64
     return SYN_OK;
 }
 
+namespace syn {
+template <typename Tab>
+static int rowscale_launch(Tab tab, int n_items, int64_t total_blocks, void *stream) {
+    hipStream_t s = (hipStream_t)stream;
+    hipLaunchKernelGGL(rowscale_kernel<Tab>, dim3((unsigned)total_blocks), dim3(kSiteThreads), 0, s, tab, n_items);
+    SYN_LAUNCH_CHECK("syn_rowscale_f64 launch");
+    return SYN_OK;
+}
+}  // namespace syn
+
 extern "C" int syn_rowscale_f64(const syn_rowscale_item *items, int n_items, int64_t total_blocks, void *stream) {
     using namespace syn;
     if (int rc = grid_check(n_items, total_blocks, "syn_rowscale_f64")) return rc;
     if (n_items == 0 || total_blocks == 0) return SYN_OK;
-    hipLaunchKernelGGL(rowscale_kernel, dim3((unsigned)total_blocks), dim3(kSiteThreads), 0, (hipStream_t)stream,
-                       items, n_items, total_blocks);
-    SYN_LAUNCH_CHECK("syn_rowscale_f64 launch");
-    return SYN_OK;
+    return rowscale_launch(DeviceTable<syn_rowscale_item>{items}, n_items, total_blocks, stream);
+}
+
+extern "C" int syn_rowscale_f64_host(const syn_rowscale_item *items, int n_items, int64_t total_blocks, void *stream) {
+    using namespace syn;
+    if (int rc = grid_check(n_items, total_blocks, "syn_rowscale_f64_host")) return rc;
+    if (int rc = inline_check(items, n_items, "syn_rowscale_f64_host")) return rc;
+    if (n_items == 0 || total_blocks == 0) return SYN_OK;
+    return launch_inline(items, n_items, [&](const auto &tab) { return rowscale_launch(tab, n_items, total_blocks, stream); });
 }
 
 extern "C" int syn_kron_bonds_f64(const syn_mpo_mpo_item *items, int n_items, int64_t total_blocks, void *stream) {
@@ -240,22 +274,52 @@ extern "C" int syn_kron_bonds_f64(const syn_mpo_mpo_item *items, int n_items, in
     return SYN_OK;
 }
 
+namespace syn {
+template <typename Tab>
+static int eye_launch(Tab tab, int n_items, int64_t total_blocks, void *stream) {
+    hipStream_t s = (hipStream_t)stream;
+    hipLaunchKernelGGL(eye_kernel<Tab>, dim3((unsigned)total_blocks), dim3(kSiteThreads), 0, s, tab, n_items);
+    SYN_LAUNCH_CHECK("syn_eye_f64 launch");
+    return SYN_OK;
+}
+}  // namespace syn
+
 extern "C" int syn_eye_f64(const syn_eye_item *items, int n_items, int64_t total_blocks, void *stream) {
     using namespace syn;
     if (int rc = grid_check(n_items, total_blocks, "syn_eye_f64")) return rc;
     if (n_items == 0 || total_blocks == 0) return SYN_OK;
-    hipLaunchKernelGGL(eye_kernel, dim3((unsigned)total_blocks), dim3(kSiteThreads), 0, (hipStream_t)stream, items,
-                       n_items, total_blocks);
-    SYN_LAUNCH_CHECK("syn_eye_f64 launch");
+    return eye_launch(DeviceTable<syn_eye_item>{items}, n_items, total_blocks, stream);
+}
+
+extern "C" int syn_eye_f64_host(const syn_eye_item *items, int n_items, int64_t total_blocks, void *stream) {
+    using namespace syn;
+    if (int rc = grid_check(n_items, total_blocks, "syn_eye_f64_host")) return rc;
+    if (int rc = inline_check(items, n_items, "syn_eye_f64_host")) return rc;
+    if (n_items == 0 || total_blocks == 0) return SYN_OK;
+    return launch_inline(items, n_items, [&](const auto &tab) { return eye_launch(tab, n_items, total_blocks, stream); });
+}
+
+namespace syn {
+template <typename Tab>
+static int copy_launch(Tab tab, int n_items, int64_t total_blocks, void *stream) {
+    hipStream_t s = (hipStream_t)stream;
+    hipLaunchKernelGGL(copy_kernel<Tab>, dim3((unsigned)total_blocks), dim3(kSiteThreads), 0, s, tab, n_items);
+    SYN_LAUNCH_CHECK("syn_copy_f64 launch");
     return SYN_OK;
 }
+}  // namespace syn
 
 extern "C" int syn_copy_f64(const syn_copy_item *items, int n_items, int64_t total_blocks, void *stream) {
     using namespace syn;
     if (int rc = grid_check(n_items, total_blocks, "syn_copy_f64")) return rc;
     if (n_items == 0 || total_blocks == 0) return SYN_OK;
-    hipLaunchKernelGGL(copy_kernel, dim3((unsigned)total_blocks), dim3(kSiteThreads), 0, (hipStream_t)stream, items,
-                       n_items, total_blocks);
-    SYN_LAUNCH_CHECK("syn_copy_f64 launch");
-    return SYN_OK;
+    return copy_launch(DeviceTable<syn_copy_item>{items}, n_items, total_blocks, stream);
+}
+
+extern "C" int syn_copy_f64_host(const syn_copy_item *items, int n_items, int64_t total_blocks, void *stream) {
+    using namespace syn;
+    if (int rc = grid_check(n_items, total_blocks, "syn_copy_f64_host")) return rc;
+    if (int rc = inline_check(items, n_items, "syn_copy_f64_host")) return rc;
+    if (n_items == 0 || total_blocks == 0) return SYN_OK;
+    return launch_inline(items, n_items, [&](const auto &tab) { return copy_launch(tab, n_items, total_blocks, stream); });
 }

@@ -18,8 +18,9 @@ __device__ __forceinline__ double wave_suffix_incl(double v, int lane) {
     return v;
 }
 
-__global__ __launch_bounds__(64) void trunc_kernel(const syn_trunc_item *__restrict__ items) {
-    const syn_trunc_item &P = items[blockIdx.x];
+template <typename Tab>
+__global__ __launch_bounds__(64) void trunc_kernel(Tab tab) {
+    const syn_trunc_item &P = tab.get()[blockIdx.x];
     const int lane = threadIdx.x;
     const int64_t n = P.n;
     const double *s = P.s;
@@ -57,6 +58,15 @@ __global__ __launch_bounds__(64) void trunc_kernel(const syn_trunc_item *__restr
 
 }  // namespace syn
 
+namespace syn {
+template <typename Tab>
+static int trunc_launch(Tab tab, int n_items, void *stream) {
+    hipLaunchKernelGGL(trunc_kernel<Tab>, dim3(n_items), dim3(64), 0, (hipStream_t)stream, tab);
+    SYN_LAUNCH_CHECK("syn_truncate_f64 launch");
+    return SYN_OK;
+}
+}  // namespace syn
+
 extern "C" int syn_truncate_f64(const syn_trunc_item *items, int n_items, void *stream) {
     using namespace syn;
     if (n_items < 0) {
@@ -64,9 +74,14 @@ extern "C" int syn_truncate_f64(const syn_trunc_item *items, int n_items, void *
         return SYN_EINVAL;
     }
     if (n_items == 0) return SYN_OK;
-    hipLaunchKernelGGL(trunc_kernel, dim3(n_items), dim3(64), 0, (hipStream_t)stream, items);
-    SYN_LAUNCH_CHECK("syn_truncate_f64 launch");
-    return SYN_OK;
+    return trunc_launch(DeviceTable<syn_trunc_item>{items}, n_items, stream);
+}
+
+extern "C" int syn_truncate_f64_host(const syn_trunc_item *items, int n_items, void *stream) {
+    using namespace syn;
+    if (int rc = inline_check(items, n_items, "syn_truncate_f64_host")) return rc;
+    if (n_items == 0) return SYN_OK;
+    return launch_inline(items, n_items, [&](const auto &tab) { return trunc_launch(tab, n_items, stream); });
 }
 
 // ---------------------------------------------------------------------------
@@ -83,8 +98,9 @@ namespace syn {
 
 constexpr int kNormThreads = 256;
 
-__global__ __launch_bounds__(kNormThreads) void vecnorm_kernel(const syn_vecnorm_item *__restrict__ items, int n,
-                                                               int64_t total) {
+template <typename Tab>
+__global__ __launch_bounds__(kNormThreads) void vecnorm_kernel(Tab tab, int n) {
+    const syn_vecnorm_item *__restrict__ items = tab.get();
     __shared__ double part[kNormThreads];
     const int64_t bid = blockIdx.x;
     const syn_vecnorm_item &P = items[find_item(items, n, bid)];
@@ -121,6 +137,14 @@ __global__ __launch_bounds__(kNormThreads) void vecnorm_kernel(const syn_vecnorm
     if (lane == 0) P.out[i] = sqrt(a);
 }
 
+template <typename Tab>
+static int vecnorm_launch(Tab tab, int n_items, int64_t total_blocks, void *stream) {
+    hipLaunchKernelGGL(vecnorm_kernel<Tab>, dim3((unsigned)total_blocks), dim3(kNormThreads), 0, (hipStream_t)stream,
+                       tab, n_items);
+    SYN_LAUNCH_CHECK("syn_vecnorms_f64 launch");
+    return SYN_OK;
+}
+
 }  // namespace syn
 
 extern "C" int syn_vecnorms_f64(const syn_vecnorm_item *items, int n_items, int64_t total_blocks, void *stream) {
@@ -130,8 +154,17 @@ extern "C" int syn_vecnorms_f64(const syn_vecnorm_item *items, int n_items, int6
         return SYN_EINVAL;
     }
     if (n_items == 0 || total_blocks == 0) return SYN_OK;
-    hipLaunchKernelGGL(vecnorm_kernel, dim3((unsigned)total_blocks), dim3(kNormThreads), 0, (hipStream_t)stream,
-                       items, n_items, total_blocks);
-    SYN_LAUNCH_CHECK("syn_vecnorms_f64 launch");
-    return SYN_OK;
+    return vecnorm_launch(DeviceTable<syn_vecnorm_item>{items}, n_items, total_blocks, stream);
+}
+
+extern "C" int syn_vecnorms_f64_host(const syn_vecnorm_item *items, int n_items, int64_t total_blocks, void *stream) {
+    using namespace syn;
+    if (int rc = inline_check(items, n_items, "syn_vecnorms_f64_host")) return rc;
+    if (total_blocks < 0 || total_blocks > 0x7fffffffLL) {
+        set_error("syn_vecnorms_f64_host: bad block count %lld", (long long)total_blocks);
+        return SYN_EINVAL;
+    }
+    if (n_items == 0 || total_blocks == 0) return SYN_OK;
+    return launch_inline(items, n_items,
+                         [&](const auto &tab) { return vecnorm_launch(tab, n_items, total_blocks, stream); });
 }

@@ -82,7 +82,36 @@ def count_uploads(on=True):
     return n
 
 
-def _upload(items: np.ndarray) -> torch.Tensor:
+class HostTable:
+    """A small item table that goes to its kernel by value (``entry``): no
+    device copy, no copy command on the stream."""
+
+    __slots__ = ("items",)
+
+    def __init__(self, items):
+        self.items = items
+
+    def data_ptr(self):
+        return self.items.__array_interface__["data"][0]
+
+
+def entry(fn, table):
+    """The library's entry point of a launch for the table `_upload` gave."""
+    return _lib.HOST_ENTRIES[fn] if isinstance(table, HostTable) else fn
+
+
+def _upload(items: np.ndarray):
+    """The item table of one launch: by value when it is small and its entry
+    point takes it so, else a device copy.  Under graph capture (and in the
+    eager run that measures one) every table is a copy from the capture's
+    StagingPool."""
+    if (items.nbytes <= _lib.INLINE_BYTES and items.dtype in _lib.INLINE_ITEMS and _staging[0] is None
+            and _upload_count[0] is None):
+        return HostTable(np.ascontiguousarray(items))
+    return _device_table(items)
+
+
+def _device_table(items: np.ndarray) -> torch.Tensor:
     """Copy an item table to the device without blocking the host: the bytes
     go through torch's cached pinned-host allocator, which keeps the staging
     buffer alive until the asynchronous copy on the current stream is done;
@@ -180,7 +209,7 @@ def gemm_many(problems, tile=None, mixed=False):
         fl = sum(2.0 * p[0].shape[0] * p[0].shape[1] * p[1].shape[1] * frac.get(bin(p[5]).count("1"), 1.0 / 3.0)
                  for p in problems)
         call("syn_prof_note_flops", fl)
-    call(gemm_fn(mixed), _ptr(dev), len(problems), start, tile, _stream())
+    call(entry(gemm_fn(mixed), dev), _ptr(dev), len(problems), start, tile, _stream())
     return dev
 
 
@@ -241,7 +270,7 @@ def apply_many(pairs):
             # bytes moved: every output element written once, operands read once
             byt = sum(8.0 * (o[0].numel() + o[1].numel() + o[2].numel()) for o in outs)
             call("syn_prof_note_flops", byt)
-        call("syn_mpo_apply_f64", _ptr(dev), len(pairs), start, _stream())
+        call(entry("syn_mpo_apply_f64", dev), _ptr(dev), len(pairs), start, _stream())
     return [o[0] for o in outs]
 
 
@@ -343,7 +372,7 @@ def rowscale_many(problems):
         start += _blocks(X.numel())
     if start:
         dev = _upload(items)
-        call("syn_rowscale_f64", _ptr(dev), len(problems), start, _stream())
+        call(entry("syn_rowscale_f64", dev), _ptr(dev), len(problems), start, _stream())
 
 
 def vecnorms_many(problems):
@@ -365,7 +394,7 @@ def vecnorms_many(problems):
         start += (cols + 63) // 64 if axis == 0 else (rows + 3) // 4
     if start:
         dev = _upload(items)
-        call("syn_vecnorms_f64", _ptr(dev), len(problems), start, _stream())
+        call(entry("syn_vecnorms_f64", dev), _ptr(dev), len(problems), start, _stream())
 
 
 def copy_many(pairs):
@@ -380,7 +409,7 @@ def copy_many(pairs):
         start += _blocks(src.numel())
     if start:
         dev = _upload(items)
-        call("syn_copy_f64", _ptr(dev), len(pairs), start, _stream())
+        call(entry("syn_copy_f64", dev), _ptr(dev), len(pairs), start, _stream())
 
 
 def eye_many(views):
@@ -396,7 +425,7 @@ def eye_many(views):
         start += _blocks(X.shape[0] * X.shape[0])
     if start:
         dev = _upload(items)
-        call("syn_eye_f64", _ptr(dev), len(views), start, _stream())
+        call(entry("syn_eye_f64", dev), _ptr(dev), len(views), start, _stream())
 
 
 # --------------------------------------------------------------------------
@@ -428,7 +457,7 @@ def qr_many(problems, q_trans=False):
         it["work"], it["tau"] = _ptr(work), _ptr(tau)
     if len(problems):
         dev = _upload(items)
-        call("syn_qr_f64", _ptr(dev), len(problems), _stream())
+        call(entry("syn_qr_f64", dev), _ptr(dev), len(problems), _stream())
     return [o[0] for o in outs]
 
 
@@ -658,7 +687,7 @@ def jacobi_many(mats, tol=None, max_sweeps=JACOBI_SWEEPS, gram=False):
         it["gram"] = int(gram)
     if len(mats):
         dev = _upload(items)
-        call("syn_jacobi_f64", _ptr(dev), len(mats), float(tol), int(max_sweeps), _stream())
+        call(entry("syn_jacobi_f64", dev), _ptr(dev), len(mats), float(tol), int(max_sweeps), _stream())
     return outs
 
 
@@ -693,7 +722,7 @@ def jacobi_gram_many(mats, tol=None, max_sweeps=JACOBI_SWEEPS):
         it["gram"] = 1
     if len(mats):
         dev = _upload(items)
-        call("syn_jacobi_gram_f64", _ptr(dev), len(mats), nv_max, float(tol), int(max_sweeps), _stream())
+        call(entry("syn_jacobi_gram_f64", dev), _ptr(dev), len(mats), nv_max, float(tol), int(max_sweeps), _stream())
     return outs
 
 
@@ -714,7 +743,7 @@ def truncate_many(problems):
         it["discarded"] = _ptr(disc) + 8 * i
     if n:
         dev = _upload(items)
-        call("syn_truncate_f64", _ptr(dev), n, _stream())
+        call(entry("syn_truncate_f64", dev), _ptr(dev), n, _stream())
     return keep, disc
 
 
