@@ -36,6 +36,7 @@
 
 namespace syn {
 
+typedef double v2d __attribute__((ext_vector_type(2)));
 typedef double v2du __attribute__((ext_vector_type(2), aligned(8)));
 
 // Vector region of a problem (2048 * half >= 64 n doubles, tjacobi.hpp):
@@ -194,19 +195,84 @@ __device__ __forceinline__ double gram_scale(const Tdc &T) {
 }
 
 // Orders up to 16 NB, one work-group of NB waves per matrix.  The matrix is
-// symmetric: of its NB x NB tiles of 16 x 16, wave I keeps (I, I - k mod NB),
-// k = 0 .. NB / 2 (the last k in the lower half of the waves only), so each
-// pair of blocks has one tile, every wave the same number, and 256 rows fit
-// the register file of one compute unit.  Lane (li, lk) holds rows lk + 4 r
-// and column li of its tiles.  A tile adds to the product's rows of block I
-// (summed over the wave's tiles, then over li) and, as its transpose, of
-// block J (summed over r and lk, then over the waves by wave 0).  A step is
-// the pass over the tiles by all waves and the short vector work of wave 0,
-// a barrier after each.
+// symmetric: of its NB x NB tiles of 16 x 16, wave I keeps the diagonal one,
+// those an even distance left of it and those an odd distance right of it, so
+// each pair of blocks has one tile and 256 rows fit the register file of one
+// compute unit.  Blocks die from the first on, and this deal leaves every live
+// wave half of the live blocks at any time (the NB / 2 blocks before a wave's
+// own, dealt first, kept the last wave at all its tiles for half of the
+// steps).  Lane (li, lk) holds rows lk + 4 r and column li of its tiles.  A
+// tile adds to the product's rows of block I (summed over the wave's tiles,
+// then over li) and, as its transpose, of block J (summed over r, then over lk
+// for four tiles at once, then over the waves by wave 0).
+//
+// A step is wave 0's short vector work and the pass over the tiles by all.
+// Wave 0 publishes v and w as soon as it has them, and the others update their
+// tiles while it works out the next column and its reflector.  Tiles go four at
+// a time without a branch between them, so that their loads overlap, and the
+// sums over lanes are taken for four values at once.  Bound by latency and, at
+// 16 waves, by LDS reads and vector issue about equally (cycles of a step of
+// order 256: 600 for p, 1900 for the reflector beside the update, 2800 for the
+// product).  Against tiles one by one, dealt as the NB / 2 blocks before a
+// wave's own, and wave 0's work ahead of the whole pass: one matrix of order
+// 256 870 -> 663 us, 192 444 -> 382, 128 222 -> 188.  The update on the MFMA
+// (one 16 x 16 x 4, half of its contraction zeros) measured 762 and 198 at 256
+// and 128 without the wave sums below, two block rows a wave 1020 and 270.
+template <int NB>
+struct TdTiles {
+    static constexpr int KT = NB / 2 + 1, KS = NB / 2, KG = (KT + 2) / 4;
+    // block of tile k of wave I: its own, those right of it, then from the
+    // nearest on those left of it, so the dead ones are the last (NB, whose
+    // entries stay zero: the wave has no such tile)
+    static __device__ __forceinline__ int block(int I, int k) {
+        const int right = (NB - I) / 2, J = k <= right ? I + 2 * k - 1 : I - 2 * (k - right);
+        return k == 0 ? I : J < 0 ? NB : J;
+    }
+    // tiles of wave I beside its own with a block from jb on
+    static __device__ __forceinline__ int live(int I, int jb) { return (NB - I) / 2 + (I - jb) / 2; }
+    // place of wave I among those that add to block J
+    static __device__ __forceinline__ int slot(int I, int J) {
+        return I > J ? (I - J) / 2 - 1 : (NB - 1 - J) / 2 + (J - I - 1) / 2;
+    }
+};
+
+// Half of a sum over the four rows of 16 lanes, of two values at once: the
+// partners of a pair of halves (or of rows) add what both hold of value a in
+// the first of them and of value b in the second.
+template <bool HALVES>
+__device__ __forceinline__ double swap_add(double a, double b) {
+    const uint64_t ua = __builtin_bit_cast(uint64_t, a), ub = __builtin_bit_cast(uint64_t, b);
+    if constexpr (HALVES) {
+        const auto l = __builtin_amdgcn_permlane32_swap((unsigned)ua, (unsigned)ub, false, false);
+        const auto h = __builtin_amdgcn_permlane32_swap((unsigned)(ua >> 32), (unsigned)(ub >> 32), false, false);
+        return __builtin_bit_cast(double, (uint64_t)h[0] << 32 | l[0]) +
+               __builtin_bit_cast(double, (uint64_t)h[1] << 32 | l[1]);
+    } else {
+        const auto l = __builtin_amdgcn_permlane16_swap((unsigned)ua, (unsigned)ub, false, false);
+        const auto h = __builtin_amdgcn_permlane16_swap((unsigned)(ua >> 32), (unsigned)(ub >> 32), false, false);
+        return __builtin_bit_cast(double, (uint64_t)h[0] << 32 | l[0]) +
+               __builtin_bit_cast(double, (uint64_t)h[1] << 32 | l[1]);
+    }
+}
+
+// Sums over the 16 lanes of a row of four values at once, value li / 4 in
+// lane li.
+__device__ __forceinline__ double row_sum4(double s0, double s1, double s2, double s3) {
+    const bool up = (threadIdx.x & 8) != 0, hi = (threadIdx.x & 4) != 0;
+    const double a = (up ? s2 : s0) + dpp_f64<0x128>(up ? s0 : s2);   // row_ror:8
+    const double b = (up ? s3 : s1) + dpp_f64<0x128>(up ? s1 : s3);
+    double y = (hi ? b : a) + dpp_f64<0x141>(hi ? a : b);             // row_half_mirror
+    y += dpp_f64<0xb1>(y);                                            // quad_perm:[1,0,3,2]
+    return y + dpp_f64<0x4e>(y);                                      // quad_perm:[2,3,0,1]
+}
+
 template <int NB>
 __global__ __launch_bounds__(64 * NB) void td_reduce_kernel(const syn_gbj_item *__restrict__ items, int nlo, int nhi) {
-    constexpr int N = 16 * NB, KT = NB / 2 + 1, E = N / 64;
-    __shared__ double vs[N], ws[N], us[N], colp[NB][KT][16], rowp[N], colx[N];
+    typedef TdTiles<NB> Tl;
+    constexpr int N = 16 * NB, KT = Tl::KT, KS = Tl::KS, KG = Tl::KG, E = N / 64;
+    __shared__ v2d vw[N + 16];                  // v and w of the step before
+    __shared__ double us[N + 16], rowp[N], colx[N];
+    __shared__ double colp[NB][KS][16];
     if (items[blockIdx.x].nv <= nlo || items[blockIdx.x].nv > nhi) return;
     const Tdc T = tdc_view(items[blockIdx.x]);
     const int n = T.n, tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4;
@@ -217,57 +283,69 @@ __global__ __launch_bounds__(64 * NB) void td_reduce_kernel(const syn_gbj_item *
     double a[KT][4];
 #pragma unroll
     for (int k = 0; k < KT; ++k) {
-        const int J = I >= k ? I - k : I - k + NB;
+        const int J = Tl::block(I, k);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int i = 16 * I + lk + 4 * r, c = 16 * J + li;
-            a[k][r] = (i < n && c < n && (k < KT - 1 || I < NB / 2)) ? T.g[i * T.ldg + c] * sc : 0.0;
+            a[k][r] = (J < NB && i < n && c < n) ? T.g[i * T.ldg + c] * sc : 0.0;
         }
     }
-    for (int i = tid; i < N; i += 64 * NB) {
-        vs[i] = ws[i] = us[i] = rowp[i] = 0.0;
+    for (int i = tid; i < N + 16; i += 64 * NB) {
+        vw[i] = v2d{0.0, 0.0};
+        us[i] = 0.0;
+        if (i >= N) continue;
+        rowp[i] = 0.0;
         colx[i] = i < n ? T.g[i] * sc : 0.0;
     }
-    for (int i = tid; i < NB * KT * 16; i += 64 * NB) (&colp[0][0][0])[i] = 0.0;
+    for (int i = tid; i < NB * KS * 16; i += 64 * NB) (&colp[0][0][0])[i] = 0.0;
     // every entry is in registers before reflectors overwrite the upper triangle
     __syncthreads();
-    double tau = 0.0;   // of the previous step, in wave 0
+    double tau = 0.0;   // in wave 0: of the previous step
     for (int j = 0; j < n - 1; ++j) {
+        double c[E];
+        // the lane's coordinates anew in every step: the LDS addresses are an
+        // addition each, and kept across steps they would not fit
+        int lane = tid & 63, li = lane & 15, lk = lane >> 4;
+        opaque(lane);
+        opaque(li);
+        opaque(lk);
         if (I == 0) {
-            // p of step j - 1 (u still its v), w, column j and its reflector
-            double v[E], p[E], c[E], s = 0.0;
+            // p of step j - 1 (u still its v) and w
+            double p[E], u[E], s = 0.0;
 #pragma unroll
             for (int e = 0; e < E; ++e) {
                 const int i = lane + 64 * e, B = i >> 4;
-                if (NB > 12) __builtin_amdgcn_sched_barrier(0);
+                if (NB > 12) __builtin_amdgcn_sched_barrier(0);   // 1024 threads: loads kept few
                 double y = rowp[i];
+                if (NB <= 12)
 #pragma unroll
-                for (int k = 1; k < KT; ++k) y += colp[B][k][i & 15];
-                v[e] = us[i];
+                    for (int k = 0; k < KS; ++k) y += colp[B][k][i & 15];
                 p[e] = i >= j ? tau * y : 0.0;
                 c[e] = colx[i];
-                s = fma(p[e], v[e], s);
-                ws[i] = p[e];
+                u[e] = us[i];
+                s = fma(p[e], u[e], s);
             }
             const double kk = 0.5 * tau * all_sum(s);
-            __builtin_amdgcn_wave_barrier();
-            const double vj = us[j], wj = fma(-kk, vj, ws[j]);
-            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int e = 0; e < E; ++e) vw[lane + 64 * e] = v2d{u[e], fma(-kk, u[e], p[e])};
+        }
+        lds_barrier();
+        if (I == 0) {
+            __builtin_amdgcn_s_setprio(3);   // the others have a pass to hide in
+            // column j and its reflector
+            const v2d xj = vw[j];
             double xn2 = 0.0;
 #pragma unroll
             for (int e = 0; e < E; ++e) {
-                const int i = lane + 64 * e;
-                const double w = fma(-kk, v[e], p[e]);
-                c[e] = fma(-w, vj, fma(-v[e], wj, c[e]));
-                if (i > j + 1) xn2 = fma(c[e], c[e], xn2);
-                vs[i] = v[e];
-                ws[i] = w;
-                us[i] = c[e];   // the column: v is its multiple by scal
+                const v2d x = vw[lane + 64 * e];
+                c[e] = fma(-x[1], xj[0], fma(-x[0], xj[1], c[e]));
+                if (lane + 64 * e > j + 1) xn2 = fma(c[e], c[e], xn2);
+                us[lane + 64 * e] = c[e];   // the column: v is its multiple by scal
             }
-            xn2 = all_sum(xn2);
             __builtin_amdgcn_wave_barrier();
             const double dj = us[j], alpha = us[j + 1];
             __builtin_amdgcn_wave_barrier();
+            xn2 = all_sum(xn2);
             double beta, scal;
             reflector(alpha, xn2, beta, tau, scal);
             if (lane == 0) {
@@ -283,81 +361,124 @@ __global__ __launch_bounds__(64 * NB) void td_reduce_kernel(const syn_gbj_item *
                 if (i > j && i < n) T.g[j * T.ldg + i] = x;
             }
         }
-        lds_barrier();
+        if (I == 0) __builtin_amdgcn_s_setprio(0);
         if (j == n - 2) break;
         const int jb = (j + 1) >> 4, jl = (j + 1) & 15;
-        // the lane's coordinates anew in every step: the tiles' LDS addresses
-        // are an addition each, and kept across steps they would not fit
-        int li = lane & 15, lk = lane >> 4;
-        opaque(li);
-        opaque(lk);
         const bool row_live = 16 * I + 15 > j;
-        // A <- A - v w^T - w v^T
+        const int live = Tl::live(I, jb);   // of the tiles beside the own one
+        // A <- A - v w^T - w v^T.  Four tiles at a time without a branch between
+        // them (dead ones among them meet zeros), so that their loads overlap.
         if (row_live) {
-            double vi[4], wi[4];
+            v2d x[4];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                vi[r] = vs[16 * I + lk + 4 * r];
-                wi[r] = ws[16 * I + lk + 4 * r];
+            for (int r = 0; r < 4; ++r) x[r] = vw[16 * I + lk + 4 * r];
+            const v2d y0 = vw[16 * I + li];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) a[0][r] = fma(-x[r][1], y0[0], fma(-x[r][0], y0[1], a[0][r]));
+#pragma unroll
+            for (int g = 0; g < KG; ++g) {
+                if (live <= 4 * g) continue;
+#pragma unroll
+                for (int h = 0; h < 4; h += 2) {
+                    if (NB > 12) __builtin_amdgcn_sched_barrier(0);
+                    v2d y[2];
+#pragma unroll
+                    for (int q = 0; q < 2; ++q)
+                        if (1 + 4 * g + h + q < KT) y[q] = vw[16 * Tl::block(I, 1 + 4 * g + h + q) + li];
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) {
+                        const int k = 1 + 4 * g + h + q;
+                        if (k >= KT) continue;
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            a[k][r] = fma(-x[r][1], y[q][0], fma(-x[r][0], y[q][1], a[k][r]));
+                    }
+                }
             }
+            // the next column: a tile's column, or the row that is its transpose
+            if (I == jb) {
 #pragma unroll
-            for (int k = 0; k < KT; ++k) {
-                const int J = I >= k ? I - k : I - k + NB;
-                if (NB > 12 && k % 2 == 0) __builtin_amdgcn_sched_barrier(0);   // 1024 threads: loads kept few
-                if (16 * J + 15 <= j || (k == KT - 1 && I >= NB / 2)) continue;
-                const double vj = vs[16 * J + li], wj = ws[16 * J + li];
+                for (int k = 0; k < KT; ++k) {
+                    const int J = Tl::block(I, k);
+                    if (J >= NB) continue;
+                    if (k == 0) {
+                        if (li == jl)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) a[k][r] = fma(-wi[r], vj, fma(-vi[r], wj, a[k][r]));
-                // the next column, or the row that is its transpose
-                if (J == jb) {
-                    if (li == jl)
+                            for (int r = 0; r < 4; ++r) colx[16 * I + lk + 4 * r] = a[k][r];
+                    } else {
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            if (lk + 4 * r == jl) colx[16 * J + li] = a[k][r];
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int k = 1; k < KT; ++k)
+                    if (Tl::block(I, k) == jb && li == jl)
 #pragma unroll
                         for (int r = 0; r < 4; ++r) colx[16 * I + lk + 4 * r] = a[k][r];
-                } else if (I == jb) {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        if (lk + 4 * r == jl) colx[16 * J + li] = a[k][r];
-                }
             }
-        }
-        // y = A u
-        double ui[4], s[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            ui[r] = us[16 * I + lk + 4 * r];
-            s[r] = 0.0;
-        }
-#pragma unroll
-        for (int k = 0; k < KT; ++k) {
-            const int J = I >= k ? I - k : I - k + NB;
-            if (NB > 12 && k % 2 == 0) __builtin_amdgcn_sched_barrier(0);
-            if (16 * J + 15 <= j || (k == KT - 1 && I >= NB / 2)) continue;
-            double t = 0.0;
-            if (row_live) {
-                const double uj = us[16 * J + li];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    s[r] = fma(a[k][r], uj, s[r]);
-                    t = fma(a[k][r], ui[r], t);
-                }
-            }
-            if (k > 0) {
-                t = lk_sum(t);
-                if (lk == 0) colp[J][k][li] = t;
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const double y = row_sum(s[r]);
-            if (li == 0) rowp[16 * I + lk + 4 * r] = y;
         }
         lds_barrier();
+        // y = A u; a wave whose rows have just died clears what it added
+        if (row_live || 16 * I + 15 == j) {
+            double ui[4], s[4];
+            const double u0 = us[16 * I + li];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                ui[r] = us[16 * I + lk + 4 * r];
+                s[r] = a[0][r] * u0;
+            }
+#pragma unroll
+            for (int g = 0; g < KG; ++g) {
+                if (row_live && live <= 4 * g) continue;   // its blocks need no sums any more
+                double sum[2];
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {   // tiles h and h + 2 of the four
+                    if (NB > 12) __builtin_amdgcn_sched_barrier(0);
+                    double t[2] = {0.0, 0.0}, uj[2];
+#pragma unroll
+                    for (int q = 0; q < 2; ++q)
+                        if (1 + 4 * g + h + 2 * q < KT) uj[q] = us[16 * Tl::block(I, 1 + 4 * g + h + 2 * q) + li];
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) {
+                        const int k = 1 + 4 * g + h + 2 * q < KT ? 1 + 4 * g + h + 2 * q : 0;
+                        if (k == 0) continue;
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            s[r] = fma(a[k][r], uj[q], s[r]);
+                            t[q] = fma(a[k][r], ui[r], t[q]);
+                        }
+                    }
+                    sum[h] = swap_add<true>(t[0], t[1]);   // lane rows 0, 1: tile h; 2, 3: tile h + 2
+                }
+                // lane row lk holds the sums of tile 1 + 4 g + lk
+                const double y = swap_add<false>(sum[0], sum[1]);
+                const int kl = 1 + 4 * g + lk, Jl = Tl::block(I, kl);
+                if (kl < KT && Jl < NB) colp[Jl][Tl::slot(I, Jl)][li] = y;
+            }
+            const double y = row_sum4(s[0], s[1], s[2], s[3]);   // of s[li / 4]
+            if ((li & 3) == 0) rowp[16 * I + lk + li] = y;
+        }
+        lds_barrier();
+        // the largest orders: a wave sums its own block's parts, wave 0 would
+        // read all of them one block after the other
+        if (NB > 12) {
+            if (row_live) {
+                double y = lk == 0 ? rowp[16 * I + li] : 0.0;
+#pragma unroll
+                for (int k = 0; k < KS; k += 4) y += colp[I][k + lk][li];
+                y = lk_sum(y);
+                if (lk == 0) rowp[16 * I + li] = y;
+            }
+            lds_barrier();
+        }
     }
     // the last diagonal entry takes the last step's v and w
     if (I == (n - 1) >> 4 && li == ((n - 1) & 15)) {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-            if (16 * I + lk + 4 * r == n - 1) T.d[n - 1] = fma(-2.0 * ws[n - 1], vs[n - 1], a[0][r]);
+            if (16 * I + lk + 4 * r == n - 1) T.d[n - 1] = fma(-2.0 * vw[n - 1][1], vw[n - 1][0], a[0][r]);
     }
 }
 
