@@ -92,7 +92,7 @@ class HostTable:
         self.items = items
 
     def data_ptr(self):
-        return self.items.__array_interface__["data"][0]
+        return self.items.ctypes.data
 
 
 def entry(fn, table):
