@@ -16,9 +16,10 @@
 // steps and a call takes 7..14 sweeps, about 4 n^3 flops each; the reduction
 // costs 4/3 n^3, the divide and conquer 8/3 n^3 at most and the products
 // 6 n^3, once.  Calls measured with the sweeps alone and with this phase, in
-// ms: one matrix of order 64 0.78 / 0.45, 128 1.5 / 0.72, 256 3.3 / 1.6, 512
-// 7.1 / 3.5, 1024 21 / 9.4, 2048 80 / 37; 8 of order 512 9.6 / 4.1; 2000 of
-// order 64 5.3 / 2.0, 1000 of 128 15.5 / 3.2, 800 of 256 88 / 12.1.
+// ms: one matrix of order 64 0.78 / 0.39, 128 1.5 / 0.62, 256 3.3 / 1.32, 512
+// 7.1 / 2.9, 1024 21 / 7.2, 2048 80 / 22; before the reductions below had their
+// present form, 8 of order 512 9.6 / 4.1; 2000 of order 64 5.3 / 2.0, 1000 of
+// 128 15.5 / 3.2, 800 of 256 88 / 12.1.
 // Residuals fall with the number of rotations: rt^T diag(s^2) rt - G from
 // 1e-13 to 1e-15 of the largest eigenvalue.
 //
@@ -485,27 +486,44 @@ __global__ __launch_bounds__(64 * NB) void td_reduce_kernel(const syn_gbj_item *
 // Orders up to 64 P, several work-groups per matrix: work-group g of S holds
 // columns S (8 q + wave) + g, lane l of a wave rows l + 64 p, so a column's
 // sum stays within its wave.  p and the next column travel through global
-// memory as self-validating words (half of a double beside the step's
-// number, one 64-bit relaxed atomic each): a reader polls the word itself,
-// and no fence or flag orders anything.  Two buffers by step parity: a
-// work-group publishes step j + 1 only after it has read all of step j, so
-// nobody overwrites what is still to be read.  Every wait is bounded: past
-// the limit (another work-group never got a compute unit) the work-group
-// gives up, the matrix counts as failed and the Jacobi sweeps take it.
+// memory as the doubles themselves, in words that hold kEmpty until they are
+// written (one 64-bit relaxed atomic each): a reader polls the word itself,
+// and no fence or flag orders anything.  Three buffers by step: whoever has
+// read all of step j knows that all others have read all of step j - 1 (they
+// published step j after it), and empties its own words of step j - 1's buffer
+// before it publishes step j + 1, so they are empty when anyone polls them for
+// step j + 2.  For that every work-group publishes in every step: the last S
+// columns, one of each, go on when their rows are dead.  Every wait is
+// bounded: past the limit (another work-group never got a compute unit) the
+// work-group gives up, the matrix counts as failed and the Jacobi sweeps take
+// it.
+//
+// Order 2048 (128 work-groups) is bound by the exchange, 128 readers of every
+// word (3.0 of a step's 6.6 us; the vectors 1.5, the pass 0.8), the smaller
+// ones by the chain of poll, sums and barriers (order 512: 0.7, 1.0, 0.5 and
+// 0.6 to publish).  With halves of doubles beside a step number (twice the
+// bytes, four loads an entry, all repeated until the last was there), five
+// barriers a step, the pass two rows at a time and the last diagonal entry
+// taken from the registers inside the loop (which kept a second copy of the
+// matrix alive: 250 bytes of scratch a lane), one matrix of order 300, 512,
+// 1024 and 2048 took 1.31, 2.16, 5.5 and 28.1 ms; now 1.01, 1.7, 4.6, 13.5.
 constexpr int kMultiThreads = 512;
 constexpr int kMultiWaves = kMultiThreads / 64;
-constexpr int kSpin = 1 << 15;
+constexpr int kSpin = 1 << 14;   // polls of one step
 constexpr unsigned kGroupedMax = 16;
+constexpr uint64_t kEmpty = ~(uint64_t)0;   // a NaN no operation makes
 
-// words of the exchange: parity, vector (p, column), entry, half; in x, which
-// the reduction does not use otherwise
-__device__ __forceinline__ uint64_t *xword(const Tdc &T, int par, int which, int i) {
-    return (uint64_t *)T.x + ((((int64_t)par * 2 + which) * T.n + i) << 1);
+// words of the exchange: buffer, vector (p, column), entry; in x, which the
+// reduction does not use otherwise
+__device__ __forceinline__ uint64_t *xword(const Tdc &T, int buf, int which, int i) {
+    return (uint64_t *)T.x + (int64_t)(buf * 2 + which) * T.n + i;
 }
-__device__ __forceinline__ void publish(uint64_t *w, double v, unsigned tag) {
-    const uint64_t u = __builtin_bit_cast(uint64_t, v), t = (uint64_t)tag << 32;
-    __hip_atomic_store(w, t | (uint32_t)u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(w + 1, t | (u >> 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+__device__ __forceinline__ void put_word(uint64_t *w, uint64_t u) {
+    __hip_atomic_store(w, u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void publish(uint64_t *w, double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    put_word(w, u == kEmpty ? u >> 1 : u);   // an input's NaN may look like that
 }
 __device__ __forceinline__ uint64_t peek(const uint64_t *w) {
     return __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -520,7 +538,7 @@ __host__ __device__ __forceinline__ int multi_groups(int64_t n) {
 __global__ __launch_bounds__(256) void td_clear_kernel(const syn_gbj_item *__restrict__ items, int nlo, int nhi) {
     if (items[blockIdx.x].nv <= nlo || items[blockIdx.x].nv > nhi) return;
     const Tdc T = tdc_view(items[blockIdx.x]);
-    for (int i = blockIdx.y * 256 + threadIdx.x; i < 8 * T.n; i += gridDim.y * 256) T.x[i] = 0.0;
+    for (int i = blockIdx.y * 256 + threadIdx.x; i < 6 * T.n; i += gridDim.y * 256) ((uint64_t *)T.x)[i] = kEmpty;
     if (blockIdx.y == 0 && threadIdx.x == 0) *T.fail = 0;
 }
 
@@ -528,7 +546,8 @@ template <int P, int Q>
 __global__ __launch_bounds__(kMultiThreads) void td_reduce_multi_kernel(const syn_gbj_item *__restrict__ items,
                                                                         int n_items, int nlo, int nhi, int S, int grouped) {
     constexpr int N = 64 * P, NW = kMultiWaves, E = (N + kMultiThreads - 1) / kMultiThreads;
-    __shared__ double v0[2][N], w0[2][N], v1[2][N], red[2][NW], red2[2][NW];
+    __shared__ v2d vw[N];                         // v and w of the step before
+    __shared__ double us[N], red[NW], red2[NW], sp, sd, sa;
     __shared__ int gone;
     // a matrix's work-groups follow each other in the launch, on one XCD
     // (every eighth work-group) when grouped: those already running never
@@ -539,6 +558,7 @@ __global__ __launch_bounds__(kMultiThreads) void td_reduce_multi_kernel(const sy
     const Tdc T = tdc_view(items[item]);
     const int n = T.n;
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tail = n - S;   // the columns that are published to the end
     const double sc = gram_scale(T);
     if (sc == 0.0) {
         if (g == 0 && tid == 0) *T.fail = 1;
@@ -556,149 +576,168 @@ __global__ __launch_bounds__(kMultiThreads) void td_reduce_multi_kernel(const sy
 #pragma unroll
     for (int e = 0; e < E; ++e) v[e] = 0.0;
     double tau = 0.0;
-    int budget = kSpin;
     if (tid == 0) gone = 0;
-    for (int i = tid; i < N; i += kMultiThreads) {
-        v1[1][i] = 0.0;
-        v1[0][i] = 0.0;
-    }
+    for (int i = tid; i < N; i += kMultiThreads) us[i] = 0.0;
     lds_barrier();
-    for (int j = 0; j < n - 1; ++j) {
-        const int par = j & 1;
+    int buf = 0;
+    for (int j = 0; j < n - 1; ++j, buf = buf == 2 ? 0 : buf + 1) {
+        const int next = buf == 2 ? 0 : buf + 1, before = buf == 0 ? 2 : buf - 1;   // steps j + 1, j - 1
+        // the thread's place anew in every step: addresses kept across steps
+        // would not fit
+        int me = tid;
+        opaque(me);
         // p of step j - 1 and column j before it (entries from j on)
         double p[E], s = 0.0;
         bool ok = true;
         if (j == 0) {
 #pragma unroll
             for (int e = 0; e < E; ++e) {
-                const int i = tid + kMultiThreads * e;
+                const int i = me + kMultiThreads * e;
                 p[e] = 0.0;
                 c[e] = i < n ? T.g[i * T.ldg] * sc : 0.0;   // row 0's owner may be past this step
             }
         } else {
-            // the words of all entries are asked for together until each is there
-            do {
+            // every entry that is not there is asked for again, together
+            uint64_t wp[E], wc[E];
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const int i = me + kMultiThreads * e;
+                wp[e] = i < n && (i >= j || i >= tail) ? kEmpty : 0;
+                wc[e] = i < n && i >= j ? kEmpty : 0;
+            }
+            for (int left = kSpin;;) {
                 ok = true;
 #pragma unroll
                 for (int e = 0; e < E; ++e) {
-                    const int i = tid + kMultiThreads * e;
-                    p[e] = c[e] = 0.0;
-                    if (i < n && i >= j) {
-                        const uint64_t *wp = xword(T, par, 0, i), *wc = xword(T, par, 1, i);
-                        const uint64_t a0 = peek(wp), a1 = peek(wp + 1), b0 = peek(wc), b1 = peek(wc + 1);
-                        ok = ok && (unsigned)(a0 >> 32) == (unsigned)j && (unsigned)(a1 >> 32) == (unsigned)j &&
-                             (unsigned)(b0 >> 32) == (unsigned)j && (unsigned)(b1 >> 32) == (unsigned)j;
-                        p[e] = __builtin_bit_cast(double, a1 << 32 | (uint32_t)a0);
-                        c[e] = __builtin_bit_cast(double, b1 << 32 | (uint32_t)b0);
-                    }
+                    const int i = me + kMultiThreads * e;
+                    if (wp[e] == kEmpty) wp[e] = peek(xword(T, buf, 0, i));
+                    if (wc[e] == kEmpty) wc[e] = peek(xword(T, buf, 1, i));
                 }
-            } while (!ok && --budget > 0);
+#pragma unroll
+                for (int e = 0; e < E; ++e) ok = ok && wp[e] != kEmpty && wc[e] != kEmpty;
+                if (ok || --left == 0) break;
+            }
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                p[e] = me + kMultiThreads * e >= j ? __builtin_bit_cast(double, wp[e]) : 0.0;
+                c[e] = __builtin_bit_cast(double, wc[e]);
+            }
         }
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-            const int i = tid + kMultiThreads * e;
             s = fma(p[e], v[e], s);
-            if (i < N) w0[par][i] = p[e];   // w below
+            if (me + kMultiThreads * e == j) sp = p[e];
         }
         if (!ok) gone = 1;
         s = all_sum(s);
-        if (lane == 0) red[par][wv] = s;
+        if (lane == 0) red[wv] = s;
         lds_barrier();
         if (gone) {
             if (tid == 0) *T.fail = 1;
             return;
         }
+        // all have read step j - 1's words: the wave's own are empty again
+        if (lane < Q) {
+            const int cc = S * (NW * lane + wv) + g;
+            if (cc < n) {
+                put_word(xword(T, before, 0, cc), kEmpty);
+                put_word(xword(T, before, 1, cc), kEmpty);
+            }
+        }
         double kk = 0.0;
 #pragma unroll
-        for (int q = 0; q < NW; ++q) kk += red[par][q];
+        for (int q = 0; q < NW; ++q) kk += red[q];
         kk *= 0.5 * tau;
-        // v1 of the other parity holds step j - 1's v
-        const double vj = v1[par ^ 1][j], wj = fma(-kk, vj, w0[par][j]);
+        const double vj = us[j], wj = fma(-kk, vj, sp);   // us: still step j - 1's v
         double xn2 = 0.0;
-        lds_barrier();   // w0[par][j] is read as p before it becomes w
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-            const int i = tid + kMultiThreads * e;
+            const int i = me + kMultiThreads * e;
             const double w = fma(-kk, v[e], p[e]);
             c[e] = fma(-w, vj, fma(-v[e], wj, c[e]));
             if (i > j + 1) xn2 = fma(c[e], c[e], xn2);
-            if (i < N) {
-                v0[par][i] = v[e];
-                w0[par][i] = w;
-                v1[par][i] = c[e];   // the column: v is its multiple by scal
-            }
+            if (i < N) vw[i] = v2d{v[e], w};
+            if (i == j) sd = c[e];
+            if (i == j + 1) sa = c[e];
         }
         xn2 = all_sum(xn2);
-        if (lane == 0) red2[par][wv] = xn2;
+        if (lane == 0) red2[wv] = xn2;
         lds_barrier();
         xn2 = 0.0;
 #pragma unroll
-        for (int q = 0; q < NW; ++q) xn2 += red2[par][q];
-        const double dj = v1[par][j], alpha = v1[par][j + 1];
+        for (int q = 0; q < NW; ++q) xn2 += red2[q];
+        const double alpha = sa;
         double beta, scal;
         reflector(alpha, xn2, beta, tau, scal);
         if (tid == 0 && g == 0) {
-            T.d[j] = dj;
+            T.d[j] = sd;
             T.e[j] = j < n - 2 ? beta : alpha;
             T.tau[j] = tau;
         }
-        if (j == n - 2) {
-            // the last diagonal entry takes the last step's v and w
-#pragma unroll
-            for (int q = 0; q < Q; ++q)
-#pragma unroll
-                for (int p2 = 0; p2 < P; ++p2)
-                    if (lane + 64 * p2 == n - 1 && S * (NW * q + wv) + g == n - 1)
-                        T.d[n - 1] = fma(-2.0 * w0[par][n - 1], v0[par][n - 1], a[p2][q]);
-            break;
-        }
-        lds_barrier();   // the column has been read: it becomes v
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-            const int i = tid + kMultiThreads * e;
+            const int i = me + kMultiThreads * e;
             v[e] = i <= j ? 0.0 : i == j + 1 ? 1.0 : c[e] * scal;
-            if (i < N) v1[par][i] = v[e];
+            if (i < N) us[i] = v[e];
             // row j of the upper triangle was read by its owner alone
             if (j % S == g && i > j && i < n) T.g[j * T.ldg + i] = v[e];
         }
         lds_barrier();
-        double y[Q], vc[Q], wc[Q];
-        int lane = tid & 63;   // addresses of the pass anew in every step, as above
-        opaque(lane);
+        // 64s of rows loaded together (order 512: 1.34 ms one by one, 1.42 by
+        // four; 2048: 14.6 and 13.5)
+        constexpr int G = P > 8 ? 4 : 1;
+        double y[Q];
+        v2d x[Q];
+        const int lane = me & 63;
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
             const int cc = S * (NW * q + wv) + g;
             y[q] = 0.0;
-            vc[q] = cc < n ? v0[par][cc] : 0.0;
-            wc[q] = cc < n ? w0[par][cc] : 0.0;
+            x[q] = cc < n ? vw[cc] : v2d{0.0, 0.0};
         }
 #pragma unroll
-        for (int p2 = 0; p2 < P; ++p2) {
-            if (P > 8 && (p2 & 1) == 0) __builtin_amdgcn_sched_barrier(0);   // row loads not all in flight at once
-            if (64 * p2 + 63 <= j) continue;
-            const int i = lane + 64 * p2;
-            const double vi = v0[par][i], wi = w0[par][i], ui = v1[par][i];
+        for (int p0 = 0; p0 < P; p0 += G) {
+            if (P > 8) __builtin_amdgcn_sched_barrier(0);   // row loads not all in flight at once
+            if (64 * (p0 + G) <= j + 1) continue;
+            v2d r[G];
+            double u[G];
 #pragma unroll
-            for (int q = 0; q < Q; ++q) {
-                a[p2][q] = fma(-wi, vc[q], fma(-vi, wc[q], a[p2][q]));
-                y[q] = fma(a[p2][q], ui, y[q]);
+            for (int h = 0; h < G; ++h) {
+                r[h] = vw[lane + 64 * (p0 + h)];
+                u[h] = us[lane + 64 * (p0 + h)];
             }
+#pragma unroll
+            for (int h = 0; h < G; ++h)
+#pragma unroll
+                for (int q = 0; q < Q; ++q) {
+                    a[p0 + h][q] = fma(-r[h][1], x[q][0], fma(-r[h][0], x[q][1], a[p0 + h][q]));
+                    y[q] = fma(a[p0 + h][q], u[h], y[q]);
+                }
         }
-        const unsigned tag = j + 1;
-        uint64_t *xcol = xword(T, par ^ 1, 1, lane);
+        // the words emptied above are there before anything of step j + 1 is
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        uint64_t *xcol = xword(T, next, 1, lane);
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
             if (S * (NW * q + wv) + g != j + 1) continue;
 #pragma unroll
             for (int p2 = 0; p2 < P; ++p2)
-                if (lane + 64 * p2 > j && lane + 64 * p2 < n) publish(xcol + 128 * p2, a[p2][q], tag);
+                if (lane + 64 * p2 > j && lane + 64 * p2 < n) publish(xcol + 64 * p2, a[p2][q]);
         }
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
             const int cc = S * (NW * q + wv) + g;
             const double t = tau * all_sum(y[q]);
-            if (lane == 0 && cc > j && cc < n) publish(xword(T, par ^ 1, 0, cc), t, tag);
+            if (lane == 0 && (cc > j || cc >= tail) && cc < n) publish(xword(T, next, 0, cc), t);
         }
+    }
+    // the last diagonal entry is the column that step n - 1 would take (its v
+    // and w are zero)
+    if (g == 0 && tid == 0) {
+        uint64_t u = kEmpty;
+        for (int left = kSpin; u == kEmpty && left > 0; --left) u = peek(xword(T, buf, 1, n - 1));
+        T.d[n - 1] = __builtin_bit_cast(double, u);
+        if (u == kEmpty) *T.fail = 1;
     }
 }
 
@@ -1432,7 +1471,7 @@ static int reduce_multi(const syn_gbj_item *items, const std::vector<syn_gbj_ite
     const int64_t nmax = class_max(host, nlo, nhi);
     if (!nmax) return SYN_OK;
     const unsigned ni = (unsigned)host.size(), S = (unsigned)multi_groups<Q>(nmax);
-    hipLaunchKernelGGL(td_clear_kernel, dim3(ni, (unsigned)((8 * nmax + 255) / 256)), dim3(256), 0, st, items, nlo, nhi);
+    hipLaunchKernelGGL(td_clear_kernel, dim3(ni, (unsigned)((6 * nmax + 255) / 256)), dim3(256), 0, st, items, nlo, nhi);
     // up to 16 work-groups of a matrix on one XCD, more over all of them
     const int grouped = S <= kGroupedMax;
     const unsigned grid = (grouped ? (ni + 7) / 8 * 8 : ni) * S;
