@@ -16,8 +16,8 @@
 // steps and a call takes 7..14 sweeps, about 4 n^3 flops each; the reduction
 // costs 4/3 n^3, the divide and conquer 8/3 n^3 at most and the products
 // 6 n^3, once.  Calls measured with the sweeps alone and with this phase, in
-// ms: one matrix of order 64 0.78 / 0.39, 128 1.5 / 0.62, 256 3.3 / 1.32, 512
-// 7.1 / 2.9, 1024 21 / 7.2, 2048 80 / 22; before the reductions below had their
+// ms: one matrix of order 64 0.78 / 0.39, 128 1.5 / 0.60, 256 3.3 / 1.25, 512
+// 7.1 / 2.7, 1024 21 / 6.7, 2048 80 / 19; before the reductions below had their
 // present form, 8 of order 512 9.6 / 4.1; 2000 of order 64 5.3 / 2.0, 1000 of
 // 128 15.5 / 3.2, 800 of 256 88 / 12.1.
 // Residuals fall with the number of rotations: rt^T diag(s^2) rt - G from
@@ -1276,80 +1276,116 @@ __global__ __launch_bounds__(256, 2) void td_gemm_kernel(const syn_gbj_item *__r
 // ---------------------------------------------------------------------------
 // Back-transformation rt <- rt (I - V T^T V^T) block by block from the last:
 // the T factor of each block of 32 reflectors (LAPACK dlarft, forward,
-// columnwise), then one work-group per 32 rows of rt walks the blocks.
+// columnwise; V V^T on the MFMA, a row of T per lane: order 256 49 -> 14 us),
+// then work-groups of 16 or 32 rows of rt walk the blocks.
 // ---------------------------------------------------------------------------
 constexpr int kBlk = 32;
 __host__ __device__ __forceinline__ int refl_blocks(int n) { return (n - 2 + kBlk - 1) / kBlk; }
 
 __global__ __launch_bounds__(256) void td_tfac_kernel(const syn_gbj_item *__restrict__ items) {
-    __shared__ double vs[kBlk][65], S[kBlk][kBlk + 1], F[kBlk][kBlk + 1];
+    __shared__ double Sp[4][3][256], S[3][16][17];
     const Tdc T = tdc_view(items[blockIdx.x]);
     const int n = T.n, j0 = blockIdx.y * kBlk, nb = n - 2 - j0 < kBlk ? n - 2 - j0 : kBlk, tid = threadIdx.x;
     if (nb <= 0 || *T.fail) return;
-    const int a = tid >> 3, c0 = (tid & 7) * 4;
-    double acc[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int k0 = j0 + 1; k0 < n; k0 += 64) {
-        __syncthreads();
-        for (int e = tid; e < kBlk * 64; e += 256) {
-            const int r = e >> 6, k = k0 + (e & 63);
-            vs[r][e & 63] = (r < nb && k > j0 + r && k < n) ? T.g[(int64_t)(j0 + r) * T.ldg + k] : 0.0;
-        }
-        __syncthreads();
-        for (int k = 0; k < 64; ++k)
+    const int wv = tid >> 6, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+    // S = V V^T, upper tiles, on the MFMA: lane lk takes four consecutive
+    // columns of each 16, the same in both operands
+    v4d s00 = {0.0, 0.0, 0.0, 0.0}, s01 = s00, s11 = s00;
+    for (int k0 = j0 + 1 + 16 * wv; k0 < n; k0 += 64) {
+        const int k = k0 + 4 * lk;
+        double v[2][4];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) acc[q] = fma(vs[a][k], vs[c0 + q][k], acc[q]);
+        for (int i = 0; i < 2; ++i) {
+            const int ref = 16 * i + li;
+            const double *vp = T.g + (int64_t)(j0 + ref) * T.ldg + k;
+            if (nb == kBlk && k0 >= j0 + kBlk && k0 + 16 <= n) {   // right of the block's triangle
+                const v2du v0 = *(const v2du *)vp, v1 = *(const v2du *)(vp + 2);
+                v[i][0] = v0.x, v[i][1] = v0.y, v[i][2] = v1.x, v[i][3] = v1.y;
+            } else {
+#pragma unroll
+                for (int s = 0; s < 4; ++s) v[i][s] = (ref < nb && k + s > j0 + ref && k + s < n) ? vp[s] : 0.0;
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            s00 = __builtin_amdgcn_mfma_f64_16x16x4f64(v[0][s], v[0][s], s00, 0, 0, 0);
+            s01 = __builtin_amdgcn_mfma_f64_16x16x4f64(v[0][s], v[1][s], s01, 0, 0, 0);
+            s11 = __builtin_amdgcn_mfma_f64_16x16x4f64(v[1][s], v[1][s], s11, 0, 0, 0);
+        }
     }
 #pragma unroll
-    for (int q = 0; q < 4; ++q) S[a][c0 + q] = acc[q];
-    for (int e = tid; e < kBlk * kBlk; e += 256) F[e / kBlk][e % kBlk] = 0.0;
+    for (int r = 0; r < 4; ++r) {
+        const int e = (lk + 4 * r) * 16 + li;
+        Sp[wv][0][e] = s00[r];
+        Sp[wv][1][e] = s01[r];
+        Sp[wv][2][e] = s11[r];
+    }
     __syncthreads();
-    for (int j = 0; j < nb; ++j) {
-        const double tau = T.tau[j0 + j];
-        if (tid < j) {
+    for (int e = tid; e < 768; e += 256)
+        S[e >> 8][(e & 255) >> 4][e & 15] = (Sp[0][e >> 8][e & 255] + Sp[1][e >> 8][e & 255]) +
+                                            (Sp[2][e >> 8][e & 255] + Sp[3][e >> 8][e & 255]);
+    __syncthreads();
+    // T[a][j] = -tau_j sum_{a <= l < j} T[a][l] S[l][j], T[j][j] = tau_j: a row
+    // depends on itself only, one lane each
+    if (tid < kBlk) {
+        double *tf = T.tf + (int64_t)blockIdx.y * kBlk * kBlk + tid * kBlk;
+        double row[kBlk];
+#pragma unroll
+        for (int j = 0; j < kBlk; ++j) {
+            const double tj = j < nb ? T.tau[j0 + j] : 0.0;
             double s = 0.0;
-            for (int l = tid; l < j; ++l) s = fma(F[tid][l], S[l][j], s);
-            F[tid][j] = -tau * s;
-        } else if (tid == j) {
-            F[j][j] = tau;
+#pragma unroll
+            for (int l = 0; l < j; ++l)
+                s = fma(row[l], l < 16 ? (j < 16 ? S[0][l][j] : S[1][l][j - 16]) : S[2][l - 16][j - 16], s);
+            row[j] = tid == j ? tj : tid < j ? -tj * s : 0.0;
+            tf[j] = row[j];
         }
-        __syncthreads();
     }
-    double *tf = T.tf + (int64_t)blockIdx.y * kBlk * kBlk;
-    for (int e = tid; e < kBlk * kBlk; e += 256) tf[e] = F[e / kBlk][e % kBlk];
 }
 
-__global__ __launch_bounds__(256) void td_back_kernel(const syn_gbj_item *__restrict__ items) {
-    __shared__ double Yp[4][kBlk][kBlk + 1], Z[kBlk][kBlk + 1], F[kBlk][kBlk + 1];
+// A work-group takes 16 RT rows of rt, its NW waves the columns.  Few
+// work-groups are bound by the chain of blocks: 16 rows and eight waves take
+// half of the time of 32 rows and four (one matrix of order 64 11 / 24 us, 256
+// 56 / 126, 2048 1.94 / 4.05 ms; 30 of 256 85 / 129), many by the reads of V,
+// which 32 rows share (60 of 256 167 / 168, 150 436 / 402, 800 2.5 / 2.0 ms).
+constexpr int64_t kBackFew = 384;   // work-groups of 32 rows
+template <int RT, int NW>
+__global__ __launch_bounds__(64 * NW) void td_back_kernel(const syn_gbj_item *__restrict__ items) {
+    __shared__ double Yp[NW][16 * RT][kBlk + 1], Z[16 * RT][kBlk + 1], F[kBlk][kBlk + 1];
     const Tdc T = tdc_view(items[blockIdx.x]);
-    const int n = T.n, r0 = blockIdx.y * 32;
+    const int n = T.n, r0 = blockIdx.y * 16 * RT;
     if (r0 >= n || *T.fail) return;
     const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63, li = lane & 15, lk = lane >> 4;
     for (int b = refl_blocks(n) - 1; b >= 0; --b) {
         const int j0 = b * kBlk, nb = n - 2 - j0 < kBlk ? n - 2 - j0 : kBlk, cs = j0 + 1;
         __syncthreads();   // Yp, Z and F of the previous block are free
         const double *tf = T.tf + (int64_t)b * kBlk * kBlk;
-        for (int e = tid; e < kBlk * kBlk; e += 256) F[e / kBlk][e % kBlk] = tf[e];
+        for (int e = tid; e < kBlk * kBlk; e += 64 * NW) F[e / kBlk][e % kBlk] = tf[e];
         // Y = rt V^T-rows over this wave's chunks of 16 columns: lane lk
         // takes four consecutive columns of each chunk, element s of every
         // lane in the s-th MFMA (the same columns in both operands)
-        v4d acc[2][2];
+        v4d acc[RT][2];
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < RT; ++i)
 #pragma unroll
             for (int j = 0; j < 2; ++j) acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
-        for (int k0 = cs + 16 * wv; k0 < n; k0 += 64) {
+        for (int k0 = cs + 16 * wv; k0 < n; k0 += 16 * NW) {
             const int k = k0 + 4 * lk;
-            double q[2][4], v[2][4];
+            double q[RT][4], v[2][4];
             if (nb == kBlk && k0 >= j0 + kBlk && k0 + 16 <= n) {
                 // right of the block's triangle: whole rows of V; rows of rt
                 // past the last repeat it (their results are not stored)
 #pragma unroll
-                for (int i = 0; i < 2; ++i) {
+                for (int i = 0; i < RT; ++i) {
                     const int row = r0 + 16 * i + li < n ? r0 + 16 * i + li : n - 1;
-                    const double *qp = T.rt + (int64_t)row * T.ldr + k, *vp = T.g + (int64_t)(j0 + 16 * i + li) * T.ldg + k;
+                    const double *qp = T.rt + (int64_t)row * T.ldr + k;
                     const v2du q0 = *(const v2du *)qp, q1 = *(const v2du *)(qp + 2);
-                    const v2du v0 = *(const v2du *)vp, v1 = *(const v2du *)(vp + 2);
                     q[i][0] = q0.x, q[i][1] = q0.y, q[i][2] = q1.x, q[i][3] = q1.y;
+                }
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const double *vp = T.g + (int64_t)(j0 + 16 * i + li) * T.ldg + k;
+                    const v2du v0 = *(const v2du *)vp, v1 = *(const v2du *)(vp + 2);
                     v[i][0] = v0.x, v[i][1] = v0.y, v[i][2] = v1.x, v[i][3] = v1.y;
                 }
             } else {
@@ -1359,7 +1395,7 @@ __global__ __launch_bounds__(256) void td_back_kernel(const syn_gbj_item *__rest
 #pragma unroll
                     for (int s = 0; s < 4; ++s) {
                         const bool in = k + s < n;
-                        q[i][s] = (in && row < n) ? T.rt[(int64_t)row * T.ldr + k + s] : 0.0;
+                        if (i < RT) q[i < RT ? i : 0][s] = (in && row < n) ? T.rt[(int64_t)row * T.ldr + k + s] : 0.0;
                         v[i][s] = (in && ref < nb && k + s > j0 + ref) ? T.g[(int64_t)(j0 + ref) * T.ldg + k + s] : 0.0;
                     }
                 }
@@ -1367,25 +1403,28 @@ __global__ __launch_bounds__(256) void td_back_kernel(const syn_gbj_item *__rest
 #pragma unroll
             for (int s = 0; s < 4; ++s)
 #pragma unroll
-                for (int i = 0; i < 2; ++i)
+                for (int i = 0; i < RT; ++i)
 #pragma unroll
                     for (int j = 0; j < 2; ++j)
                         acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(q[i][s], v[j][s], acc[i][j], 0, 0, 0);
         }
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < RT; ++i)
 #pragma unroll
             for (int j = 0; j < 2; ++j)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) Yp[wv][16 * i + lk + 4 * r][16 * j + li] = acc[i][j][r];
         __syncthreads();
-        for (int e = tid; e < kBlk * kBlk; e += 256) {
+        for (int e = tid; e < 16 * RT * kBlk; e += 64 * NW) {
             const int i = e / kBlk, j = e % kBlk;
-            Yp[0][i][j] = (Yp[0][i][j] + Yp[1][i][j]) + (Yp[2][i][j] + Yp[3][i][j]);
+            double y = 0.0;
+#pragma unroll
+            for (int w = 0; w < NW; w += 4) y += (Yp[w][i][j] + Yp[w + 1][i][j]) + (Yp[w + 2][i][j] + Yp[w + 3][i][j]);
+            Yp[0][i][j] = y;
         }
         __syncthreads();
         // Z = Y T^T, T upper triangular
-        for (int e = tid; e < kBlk * kBlk; e += 256) {
+        for (int e = tid; e < 16 * RT * kBlk; e += 64 * NW) {
             const int i = e / kBlk, a = e % kBlk;
             double s = 0.0;
             for (int c = a; c < kBlk; ++c) s = fma(Yp[0][i][c], F[a][c], s);
@@ -1393,11 +1432,11 @@ __global__ __launch_bounds__(256) void td_back_kernel(const syn_gbj_item *__rest
         }
         __syncthreads();
         // rt -= Z V, 16 columns of both row tiles at a time
-        for (int c0 = cs + 16 * wv; c0 < n; c0 += 64) {
+        for (int c0 = cs + 16 * wv; c0 < n; c0 += 16 * NW) {
             const int col = c0 + li;
-            v4d o[2];
+            v4d o[RT];
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < RT; ++i)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int row = r0 + 16 * i + lk + 4 * r;
@@ -1409,11 +1448,11 @@ __global__ __launch_bounds__(256) void td_back_kernel(const syn_gbj_item *__rest
                 const double v =
                     (ref < nb && col < n && col > j0 + ref) ? T.g[(int64_t)(j0 + ref) * T.ldg + col] : 0.0;
 #pragma unroll
-                for (int i = 0; i < 2; ++i)
+                for (int i = 0; i < RT; ++i)
                     o[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(-Z[16 * i + li][k0 + lk], v, o[i], 0, 0, 0);
             }
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < RT; ++i)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int row = r0 + 16 * i + lk + 4 * r;
@@ -1521,7 +1560,10 @@ int tdc_launch(const syn_gbj_item *items, const std::vector<syn_gbj_item> &host,
         SYN_LAUNCH_CHECK("divide and conquer");
     }
     const unsigned t32 = (unsigned)((nmax + 31) / 32), t64 = (unsigned)((nmax + 63) / 64);
-    hipLaunchKernelGGL(td_back_kernel, dim3(ni, t32), dim3(256), 0, st, items);
+    if ((int64_t)ni * t32 <= kBackFew)
+        hipLaunchKernelGGL((td_back_kernel<1, 8>), dim3(ni, (unsigned)((nmax + 15) / 16)), dim3(512), 0, st, items);
+    else
+        hipLaunchKernelGGL((td_back_kernel<2, 4>), dim3(ni, t32), dim3(256), 0, st, items);
     hipLaunchKernelGGL(td_restore_kernel, dim3(ni, t32 * (t32 + 1) / 2), dim3(256), 0, st, items);
     hipLaunchKernelGGL(td_gemm_kernel, dim3(ni, t64 * t64), dim3(256), 0, st, items, 1, 0);
     hipLaunchKernelGGL(td_gemm_kernel, dim3(ni, t64 * t64), dim3(256), 0, st, items, 2, 0);

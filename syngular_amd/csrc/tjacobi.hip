@@ -892,35 +892,40 @@ __global__ __launch_bounds__(256) void tj_permute_kernel(const syn_gbj_item *__r
 
 // Decreasing order of each problem's s (ties by index, as a stable sort):
 // rank[i] = #{j : s_j > s_i or (s_j == s_i and j < i)}, perm[rank[i]] = i.
-// s is staged through LDS in chunks of kRankChunk values.
+// s is staged through LDS in chunks of kRankChunk values; a work-group ranks
+// 64 values, a quarter of the comparisons each wave (one work-group for all of
+// them took 1.1 ms at order 2048, 25 us at 256).
 constexpr int kRankChunk = 2048;
 __global__ __launch_bounds__(256) void tj_rank_kernel(const syn_gbj_item *__restrict__ items,
                                                       const int64_t *__restrict__ poff, int64_t *__restrict__ perm) {
     __shared__ double sv[kRankChunk];
     const syn_gbj_item &P = items[blockIdx.x];
-    const int64_t nv = P.nv;
-    int64_t *pm = perm + poff[blockIdx.x];
-    for (int64_t i0 = 0; i0 < nv; i0 += 256) {
-        const int64_t i = i0 + threadIdx.x;
-        // a NaN orders last (as -inf), so the ranks always form a permutation
-        const double s0 = i < nv ? P.s[i] : 0.0, si = s0 == s0 ? s0 : -__builtin_huge_val();
-        int64_t rk = 0;
-        for (int64_t c0 = 0; c0 < nv; c0 += kRankChunk) {
-            const int64_t cn = nv - c0 < kRankChunk ? nv - c0 : kRankChunk;
-            __syncthreads();
-            for (int64_t e = threadIdx.x; e < cn; e += 256) {
-                const double x = P.s[c0 + e];
-                sv[e] = x == x ? x : -__builtin_huge_val();
-            }
-            __syncthreads();
-            if (i < nv)
-                for (int64_t e = 0; e < cn; ++e) {
-                    const double sj = sv[e];
-                    rk += (sj > si) || (sj == si && c0 + e < i);
-                }
+    const int64_t nv = P.nv, i = (int64_t)blockIdx.y * 64 + (threadIdx.x & 63);
+    if ((int64_t)blockIdx.y * 64 >= nv) return;
+    const int part = threadIdx.x >> 6;
+    // a NaN orders last (as -inf), so the ranks always form a permutation
+    const double s0 = i < nv ? P.s[i] : 0.0, si = s0 == s0 ? s0 : -__builtin_huge_val();
+    int rk = 0;
+    for (int64_t c0 = 0; c0 < nv; c0 += kRankChunk) {
+        const int cn = (int)(nv - c0 < kRankChunk ? nv - c0 : kRankChunk);
+        __syncthreads();
+        for (int e = threadIdx.x; e < cn; e += 256) {
+            const double x = P.s[c0 + e];
+            sv[e] = x == x ? x : -__builtin_huge_val();
         }
-        if (i < nv) pm[rk] = i;
+        __syncthreads();
+#pragma unroll 4
+        for (int e = part; e < cn; e += 4) {
+            const double sj = sv[e];
+            rk += (sj > si) || (sj == si && c0 + e < i);
+        }
     }
+    // the four waves' counts
+    __shared__ int cnt[4][64];
+    cnt[part][threadIdx.x & 63] = rk;
+    __syncthreads();
+    if (part == 0 && i < nv)
+        perm[poff[blockIdx.x] + ((cnt[0][threadIdx.x] + cnt[1][threadIdx.x]) + (cnt[2][threadIdx.x] + cnt[3][threadIdx.x]))] = i;
 }
 
 __global__ __launch_bounds__(256) void tj_zero_kernel(int32_t *c, int n) {
@@ -1202,7 +1207,9 @@ static int gram_blocked(syn_gbj_item *items, std::vector<syn_gbj_item> &all, int
     SYN_LAUNCH_CHECK("gram copy back");
     hipLaunchKernelGGL(tj_diag_kernel, dim3(n_items), dim3(256), 0, st, items);
     SYN_LAUNCH_CHECK("gram diag");
-    hipLaunchKernelGGL(tj_rank_kernel, dim3(n_items), dim3(256), 0, st, items, dpoff, dperm);
+    int64_t nv_most = 0;
+    for (const syn_gbj_item &it : all) nv_most = std::max(nv_most, it.nv);
+    hipLaunchKernelGGL(tj_rank_kernel, dim3(n_items, (unsigned)((nv_most + 63) / 64)), dim3(256), 0, st, items, dpoff, dperm);
     SYN_LAUNCH_CHECK("gram order");
     // grid.y spreads each problem's rows over 64 work-groups
     hipLaunchKernelGGL(tj_permute_kernel, dim3(n_items, 64), dim3(256), 0, st, items, dperm, dpoff, work, dtoff, 0);
