@@ -417,7 +417,7 @@ def jacobi_gram_blocked_table(x, g, rt, s, tol=None):
     lib = _lib.load()
     wsz = int(lib.syn_jacobi_gram_blocked_workspace(g.ctypes.data_as(ctypes.c_void_p), cnt))
     work = _empty(wsz)
-    counters = _empty(cnt, torch.int32, zero=True)
+    counters = _empty(cnt, torch.int32)     # the call clears them
     dev_items = _empty(it.nbytes, torch.uint8)
     sweeps = ctypes.c_int(0)
     call("syn_jacobi_gram_blocked_f64", dev_items.data_ptr(), it.ctypes.data_as(ctypes.c_void_p), cnt,
@@ -747,8 +747,8 @@ class ChainBatch:
                 jacobi_table(gp[small], g[small], rtp[small], sp[small])
             if (~small).any():
                 jacobi_gram_blocked_table(gp[~small], g[~small], rtp[~small], sp[~small], jacobi_tol)
-            keep = _empty(len(a), torch.int32, zero=True)
-            disc = _empty(len(a), F64, zero=True)
+            keep = _empty(len(a), torch.int32)     # the truncation writes every entry
+            disc = _empty(len(a), F64)
             kb, db = np.uint64(keep.data_ptr()), np.uint64(disc.data_ptr())
             idx = np.arange(len(a), dtype=np.uint64)
             truncate_table(sp, g, chi_max[a], cutoff[a], kb + 4 * idx, db + 8 * idx)

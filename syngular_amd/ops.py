@@ -274,6 +274,40 @@ def apply_many(pairs):
     return [o[0] for o in outs]
 
 
+# doubles of the product cores that one launch of product_cores forms ahead
+PRODUCT_AHEAD = 1 << 23
+
+
+def product_cores(pairs):
+    """One callable per (O, X) of `pairs` that returns its product core
+    (apply_many).  Neighbours whose cores together hold at most PRODUCT_AHEAD
+    doubles are formed in one launch, by the first of them that is called; a
+    larger one is formed alone, when it is called."""
+    out, group, held = [], [], 0
+
+    def close(group):
+        formed = []
+
+        def take(i):
+            if not formed:
+                formed.extend(apply_many(group))
+            core, formed[i] = formed[i], None
+            return core
+
+        out.extend([lambda i=i: take(i) for i in range(len(group))])
+
+    for O, X in pairs:
+        din = X.shape[1] if X.dim() == 3 else 1
+        nel = O.numel() * X.numel() // max(din * din, 1)
+        if group and held + nel > PRODUCT_AHEAD:
+            close(group)
+            group, held = [], 0
+        group.append((O, X))
+        held += nel
+    close(group)
+    return out
+
+
 def mpo_mpo_many(pairs):
     """pairs: list of (A (al,din,dmid,ar), B (bl,dmid,dout,br)); returns
     P (al*bl, din, dout, ar*br) with P[a*bl+c, i, p, b*br+e] = sum_j A[a,i,j,b] B[c,j,p,e]."""
@@ -731,8 +765,8 @@ def truncate_many(problems):
     (keep int32 (n,), discarded f64 (n,)) device tensors."""
     n = len(problems)
     dev_ = device()
-    keep = torch.zeros(n, dtype=torch.int32, device=dev_)
-    disc = torch.zeros(n, dtype=F64, device=dev_)
+    keep = torch.empty(n, dtype=torch.int32, device=dev_)     # every entry is written
+    disc = torch.empty(n, dtype=F64, device=dev_)
     items = np.zeros(n, dtype=_lib.TRUNC_ITEM)
     for i, (s, chi_max, cutoff) in enumerate(problems):
         it = items[i]
@@ -920,7 +954,7 @@ def jacobi_gram_blocked(G, tol=None, max_sweeps=JACOBI_SWEEPS):
     nva = np.array([nv], dtype=np.int64)
     work = torch.empty(int(_lib.load().syn_jacobi_gram_blocked_workspace(nva.ctypes.data_as(ctypes.c_void_p), 1)),
                        dtype=F64, device=G.device)
-    counters = torch.zeros(1, dtype=torch.int32, device=G.device)
+    counters = torch.empty(1, dtype=torch.int32, device=G.device)   # the call clears it
     dev_items = torch.empty(it.nbytes, dtype=torch.uint8, device=G.device)
     sweeps = ctypes.c_int(0)
     call("syn_jacobi_gram_blocked_f64", _ptr(dev_items), it.ctypes.data_as(ctypes.c_void_p), 1, _ptr(work),

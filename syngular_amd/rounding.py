@@ -102,7 +102,8 @@ def left_orthonormalize(cores, own=False, mixed=False, reorth_budget=None, contr
         m = L.shape[0]
         if m <= r:
             # a wide unfolding: Q = I_m and R = L, no factorisation needed
-            Q, S, tri = torch.eye(m, dtype=F64, device=L.device), L, 0
+            Q, S, tri = torch.empty((m, m), dtype=F64, device=L.device), L, 0
+            ops.eye_many([Q])
         elif r >= CHOLQR_MIN_COLS:
             if reorth_budget is None or mixed:
                 Q, S = ops.cholqr2(L, mixed=mixed)
@@ -174,8 +175,7 @@ def right_svd_sweep(cores, chi_max=None, cutoff=0.0, report=None, mixed=False):
             newc = ops.gemm(Ut, C, mixed=mixed)        # U^T C = S V^T (cc x ncol)
             if not mixed:
                 ops.vecnorms_many([(newc, 1, s[:cc])])  # s_i = ||(S V^T)[i, :]||
-            ops.rowscale_many([(newc, s, 1)])          # -> V^T
-            ops.rowscale_many([(Ut, s, 0)])            # -> (U S)^T
+            ops.rowscale_many([(newc, s, 1), (Ut, s, 0)])   # -> V^T, (U S)^T
             M = Ut.t()
         cores[k] = reshape(newc, (cc, *mid, r))
         cores[k - 1] = reshape(ops.gemm(Pl, M, mixed=mixed), (*prev.shape[:-1], cc))
@@ -199,9 +199,10 @@ def tt_round(cores, chi_max=None, cutoff=0.0, report=None, own=False, precision=
 
 def apply_and_round(mpo_sites, mps_sites, chi_max=None, cutoff=0.0, report=None, precision="fp64"):
     """One apply+round step: MPO x MPS product cores, then tt_round.  Each
-    product core is formed when the left sweep reaches it and dropped once
-    its QR factor replaces it, so at most two product cores (P_k, P_k+1)
-    exist at a time instead of the whole product (133 GB at N=64, d=4,
-    chi=1024, D_w=8, against 2.1 GB per core)."""
-    prod = [(lambda o=o, x=x: ops.apply_many([(o, x)])[0]) for o, x in zip(mpo_sites, mps_sites)]
+    product core is formed when the left sweep reaches it (small ones with
+    their neighbours, ops.product_cores) and dropped once its QR factor
+    replaces it, so at most two large product cores (P_k, P_k+1) exist at a
+    time instead of the whole product (133 GB at N=64, d=4, chi=1024, D_w=8,
+    against 2.1 GB per core)."""
+    prod = ops.product_cores(list(zip(mpo_sites, mps_sites)))
     return tt_round(prod, chi_max, cutoff, report, own=True, precision=precision)

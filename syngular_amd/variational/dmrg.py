@@ -30,16 +30,19 @@ from .. import linalg, ops
 F64 = torch.float64
 
 
-def _sandwich_core(X, W):
-    """Z[(c,e), s, (d,f)] = sum_t W[c,t,s,d] X[e,t,f] as ((c,e) s, (d,f))."""
-    c, t, s, d = W.shape
-    e, t2, f = X.shape
-    if t != t2 or s != t:
-        raise ValueError(f"operands could not be broadcast: operator legs {tuple(W.shape)} vs state {tuple(X.shape)}")
-    Wc = W.contiguous().reshape(c, t, s * d)
-    Xo = X.contiguous().reshape(e, t, 1, f)
-    Z = ops.apply_many([(Xo, Wc)])[0]                # (c*e, 1, s*d*f)
-    return Z.reshape(c * e * s, d * f)
+def _sandwich_cores(state, operator, sites):
+    """One callable per site for Z[(c,e), s, (d,f)] = sum_t W[c,t,s,d] X[e,t,f]
+    as ((c,e) s, (d,f)), formed with its neighbours where small."""
+    pairs, shapes = [], []
+    for k in sites:
+        X, W = state.sites[k], operator.sites[k]
+        c, t, s, d = W.shape
+        e, t2, f = X.shape
+        if t != t2 or s != t:
+            raise ValueError(f"operands could not be broadcast: operator legs {tuple(W.shape)} vs state {tuple(X.shape)}")
+        pairs.append((X.contiguous().reshape(e, t, 1, f), W.contiguous().reshape(c, t, s * d)))
+        shapes.append((c * e * s, d * f))
+    return [lambda f=f, shape=shape: f().reshape(shape) for f, shape in zip(ops.product_cores(pairs), shapes)]
 
 
 def right_blocks(operator, state):
@@ -47,11 +50,12 @@ def right_blocks(operator, state):
     k = n-1 .. 2 as (ket, operator, bra) device tensors, None elsewhere."""
     n = operator.sites_number
     blocks = [None] * n
-    for k in range(n - 1, 1, -1):
+    sites = range(n - 1, 1, -1)
+    for k, core in zip(sites, _sandwich_cores(state, operator, sites)):
         X, W = state.sites[k], operator.sites[k]
         a, s, b = X.shape
         c, d = W.shape[0], W.shape[3]
-        Z = _sandwich_core(X, W)
+        Z = core()
         if k == n - 1:
             R = torch.ones((b, d * b), dtype=F64, device=X.device)
         else:
@@ -67,11 +71,12 @@ def left_blocks(operator, state):
     k = 0 .. n-3 as (ket, operator, bra) device tensors, None elsewhere."""
     n = operator.sites_number
     blocks = [None] * n
-    for k in range(n - 2):
+    sites = range(n - 2)
+    for k, core in zip(sites, _sandwich_cores(state, operator, sites)):
         X, W = state.sites[k], operator.sites[k]
         a, s, b = X.shape
         c, d = W.shape[0], W.shape[3]
-        Z = _sandwich_core(X, W)
+        Z = core()
         if k == 0:
             L = torch.ones((a, c * a), dtype=F64, device=X.device)
         else:
