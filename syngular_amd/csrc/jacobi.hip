@@ -201,8 +201,8 @@ __global__ __launch_bounds__(kJacThreads) void jacobi_kernel(Tab tab, double tol
 // sqrt(max(lambda_i, 0)) are the singular values of C when G = C^T C, and the
 // rows of rt are the matching eigenvectors.
 // ---------------------------------------------------------------------------
-// threads per problem by the largest order of the launch: one wave up to
-// 16 (at most 8 planes a round), two up to 32, four up to 64, so small
+// threads per problem by the largest order of the launch: one wave up to 16,
+// with its matrix in registers (below), two up to 32, four up to 64, so small
 // problems do not wait at four-wave barriers and more of them share a CU
 constexpr int kGramThreads = 256;
 constexpr int kGramMax = 64;
@@ -334,6 +334,139 @@ __global__ __launch_bounds__(NT) void jacobi_gram_kernel(Tab tab, int nv_max, do
 
 namespace syn {
 
+// Orders up to 16, one wave: the matrix stays in registers.  The indices sit in
+// h = ceil(g / 2) slots of two, x and y; lane 8 k + k' holds the 2 x 2 block of
+// slots k and k', so a round's planes are the blocks of the diagonal lanes, and
+// its 2 x 2 updates need the rotations of two slots only.  Between rounds the
+// indices move on by one place of the circle x_1 .. x_h-1, y_h-1 .. y_0 (x_0
+// stays): columns by lane shifts within a row of lanes, rows by a lane
+// permutation.  After 2 h - 1 rounds all planes have met and every index is back
+// where it was.  R stays in LDS, off the chain.  A round is the test, the
+// rotation (about 25 dependent operations), one LDS round trip for c and s and
+// one for the rows; without a plane to rotate the test and the move.  With the
+// matrix in LDS a round was five round trips.  A call of one matrix of order 4,
+// 8 and 16 30, 55 and 127 us, now 24, 37 and 66; 800 of 16 229 and 131.
+constexpr int kReg = 16;
+typedef double jv2d __attribute__((ext_vector_type(2)));
+
+template <int CTRL>
+__device__ __forceinline__ double lane_shift(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, 0xf, 0xf, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, false);
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+__device__ __forceinline__ double from_lane(double v, int lane) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute(4 * lane, (int)(uint32_t)u);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_ds_bpermute(4 * lane, (int)(uint32_t)(u >> 32));
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+
+template <typename Tab>
+__global__ __launch_bounds__(64) void jacobi_gram16_kernel(Tab tab, int nv_max, double tol, int max_sweeps) {
+    __shared__ __attribute__((aligned(16))) double R[kReg][kReg + 2];
+    __shared__ jv2d cs[8];
+    __shared__ double lam[kReg];
+    __shared__ int rank[kReg];
+    const syn_jacobi_item &P = tab.get()[blockIdx.x];
+    const int lane = threadIdx.x;
+    if (P.nv < 1 || P.nv > nv_max || P.len != P.nv) {
+        // not a problem this kernel takes: flag it in s and leave the rest
+        for (int64_t i = lane; i < P.nv; i += 64) P.s[i] = __builtin_nan("");
+        return;
+    }
+    const int g = (int)P.nv, h = (g + 1) / 2, M = 2 * h - 1;
+    const int k = lane >> 3, kc = lane & 7;
+    auto at = [&](int i, int j) { return i < g && j < g && k < h && kc < h ? P.x[i * P.ldx + j] : 0.0; };
+    double a00 = at(k, kc), a01 = at(k, h + kc), a10 = at(h + k, kc), a11 = at(h + k, h + kc);
+    for (int e = lane; e < kReg * kReg; e += 64) R[e / kReg][e % kReg] = e / kReg == e % kReg ? 1.0 : 0.0;
+    const bool diag = k == kc && k < h;
+    // absolute rotation floor, as in the other kernel
+    double m = diag ? fmax(fabs(a00), fabs(a11)) : 0.0;
+    for (int off = 32; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off, 64));
+    const double floor_abs = __DBL_EPSILON__ * m;
+    lds_barrier();
+    int sweep = 0;
+    for (; sweep < max_sweeps && g > 1; ++sweep) {
+        bool any = false;
+        // circle places of the row indices: x_k at k - 1, y_k at 2 h - 2 - k
+        int sx = k - 1, sy = 2 * h - 2 - k;
+        for (int r = 0; r < M; ++r) {
+            const bool rot = diag && rotates(a01, a00, a11, tol, floor_abs);
+            if (__ballot(rot)) {
+                any = true;
+                double c = 1.0, sn = 0.0;
+                if (rot) rotation(a01, a00, a11, c, sn);
+                if (k == kc) cs[k] = jv2d{c, sn};
+                lds_barrier();
+                const jv2d u = cs[k], v = cs[kc];
+                // row indices of the slot (idle slots hold the identity rotation)
+                const int ix = k == 0 ? 0 : sx <= h - 2 ? sx + 1 : 3 * h - 2 - sx;
+                const int iy = sy <= h - 2 ? sy + 1 : 3 * h - 2 - sy;
+                if (u.y != 0.0) {
+                    jv2d *px = (jv2d *)&R[ix][2 * kc], *py = (jv2d *)&R[iy][2 * kc];
+                    const jv2d x = *px, y = *py;
+                    *px = jv2d{u.x * x.x - u.y * y.x, u.x * x.y - u.y * y.y};
+                    *py = jv2d{u.y * x.x + u.x * y.x, u.y * x.y + u.x * y.y};
+                }
+                const double r00 = u.x * a00 - u.y * a10, r01 = u.x * a01 - u.y * a11;
+                const double r10 = u.y * a00 + u.x * a10, r11 = u.y * a01 + u.x * a11;
+                a00 = v.x * r00 - v.y * r01;
+                a01 = v.y * r00 + v.x * r01;
+                a10 = v.x * r10 - v.y * r11;
+                a11 = v.y * r10 + v.x * r11;
+                if (rot) a01 = a10 = 0.0;   // the annihilated pair
+                lds_barrier();
+            }
+            if (h > 1) {
+                // columns: x_1 <- y_0, x_k <- x_k-1, y_h-1 <- x_h-1, y_k <- y_k+1
+                const bool first = kc == 0, last = kc == h - 1;
+                const double s0 = lane_shift<0x111>(first ? a01 : a00), s1 = lane_shift<0x111>(first ? a11 : a10);
+                const double t0 = lane_shift<0x101>(a01), t1 = lane_shift<0x101>(a11);
+                a01 = last ? a00 : t0;
+                a11 = last ? a10 : t1;
+                a00 = first ? a00 : s0;
+                a10 = first ? a10 : s1;
+                // rows alike
+                const bool top = k == 0, end = k == h - 1;
+                const int up = (lane - 8) & 63, down = (lane + 8) & 63;
+                const double p0 = from_lane(top ? a10 : a00, up), p1 = from_lane(top ? a11 : a01, up);
+                const double q0 = from_lane(a10, down), q1 = from_lane(a11, down);
+                a10 = end ? a00 : q0;
+                a11 = end ? a01 : q1;
+                a00 = top ? a00 : p0;
+                a01 = top ? a01 : p1;
+                sx = sx == 0 ? M - 1 : sx - 1;
+                sy = sy == 0 ? M - 1 : sy - 1;
+            }
+        }
+        if (!any) break;
+    }
+    if (diag) {
+        lam[k] = a00;
+        lam[h + k] = a11;
+    }
+    lds_barrier();
+    // decreasing order by eigenvalue (ties by index): rank of each row
+    if (lane < g) {
+        const double li = lam[lane];
+        int rk = 0;
+        for (int j = 0; j < g; ++j) {
+            const double lj = lam[j];
+            rk += (lj > li) || (lj == li && j < lane);
+        }
+        rank[lane] = rk;
+        P.s[rk] = sqrt(fmax(li, 0.0));
+    }
+    lds_barrier();
+    for (int e = lane; e < g * g; e += 64) {
+        const int i = e / g, j = e - i * g;
+        P.rt[(int64_t)rank[i] * P.ldr + j] = R[i][j];
+    }
+    if (lane == 0 && P.sweeps) *P.sweeps = sweep;
+}
+
 template <typename Tab>
 static int jacobi_gram_launch(Tab tab, int n_items, int64_t nv_max, double tol, int max_sweeps, void *stream) {
     static bool attr_set = false;
@@ -347,10 +480,11 @@ static int jacobi_gram_launch(Tab tab, int n_items, int64_t nv_max, double tol, 
     }
     const size_t shm = 2 * (size_t)nv_max * (size_t)(nv_max + 1) * sizeof(double);
     ProfScope ps(kTagJacobi, 0.0, (hipStream_t)stream);
-    auto kern = nv_max <= 16 ? jacobi_gram_kernel<64, Tab>
-                             : (nv_max <= 32 ? jacobi_gram_kernel<128, Tab> : jacobi_gram_kernel<kGramThreads, Tab>);
-    const int nt = nv_max <= 16 ? 64 : (nv_max <= 32 ? 128 : kGramThreads);
-    hipLaunchKernelGGL(kern, dim3(n_items), dim3(nt), shm, (hipStream_t)stream, tab, (int)nv_max, tol, max_sweeps);
+    auto kern = nv_max <= kReg ? jacobi_gram16_kernel<Tab>
+                               : (nv_max <= 32 ? jacobi_gram_kernel<128, Tab> : jacobi_gram_kernel<kGramThreads, Tab>);
+    const int nt = nv_max <= kReg ? 64 : (nv_max <= 32 ? 128 : kGramThreads);
+    hipLaunchKernelGGL(kern, dim3(n_items), dim3(nt), nv_max <= kReg ? 0 : shm, (hipStream_t)stream, tab, (int)nv_max,
+                       tol, max_sweeps);
     SYN_LAUNCH_CHECK("syn_jacobi_gram_f64 launch");
     return SYN_OK;
 }
