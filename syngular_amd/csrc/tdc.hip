@@ -1223,6 +1223,7 @@ __global__ __launch_bounds__(256) void td_vec_kernel(const syn_gbj_item *__restr
 // with the back-transformed rt: y = G rt^T (1), G = rt y (2).  blockIdx.y
 // is the tile, blockIdx.z the node.
 // ---------------------------------------------------------------------------
+template <bool QUAD>
 __global__ __launch_bounds__(256, 2) void td_gemm_kernel(const syn_gbj_item *__restrict__ items, int what,
                                                          int level) {
     const Tdc T = tdc_view(items[blockIdx.x]);
@@ -1265,12 +1266,17 @@ __global__ __launch_bounds__(256, 2) void td_gemm_kernel(const syn_gbj_item *__r
         }
     }
     P.tiles_n = (P.n + 63) / 64;
-    if (blockIdx.y >= P.tiles_n * ((P.m + 63) / 64)) return;
+    const unsigned tile = QUAD ? blockIdx.y >> 2 : blockIdx.y;
+    if (tile >= P.tiles_n * ((P.m + 63) / 64)) return;
+    if constexpr (QUAD) {
+        gemm_f64_quad<32, double>(P, tile, blockIdx.y & 3);
+        return;
+    }
     __shared__ GemmSmem<64, 64, 16, double> smem;
     if (what == 1)
-        gemm_f64_tile_t<64, 64, 16, 32, 32, false, true, double>(P, blockIdx.y, smem, 0, INT64_MAX);
+        gemm_f64_tile_t<64, 64, 16, 32, 32, false, true, double>(P, tile, smem, 0, INT64_MAX);
     else
-        gemm_f64_tile_t<64, 64, 16, 32, 32, false, false, double>(P, blockIdx.y, smem, 0, INT64_MAX);
+        gemm_f64_tile_t<64, 64, 16, 32, 32, false, false, double>(P, tile, smem, 0, INT64_MAX);
 }
 
 // ---------------------------------------------------------------------------
@@ -1520,6 +1526,17 @@ static int reduce_multi(const syn_gbj_item *items, const std::vector<syn_gbj_ite
     return SYN_OK;
 }
 
+// The products of a phase; up to 128 tiles as quadrants, the same bits (the
+// line of gemm.hip; one matrix of order 64 7.2 / 4.8 us a launch, 256 13.5 /
+// 7.6, 512 20.5 / 11.0).
+static void td_gemm(const syn_gbj_item *items, unsigned ni, unsigned tiles, unsigned nodes, int what, int level,
+                    hipStream_t st) {
+    if ((int64_t)ni * tiles * nodes <= 128)
+        hipLaunchKernelGGL(td_gemm_kernel<true>, dim3(ni, 4 * tiles, nodes), dim3(256), 0, st, items, what, level);
+    else
+        hipLaunchKernelGGL(td_gemm_kernel<false>, dim3(ni, tiles, nodes), dim3(256), 0, st, items, what, level);
+}
+
 bool tdc_takes(int64_t nv) { return nv >= kTdcMin && nv <= kTdcMax; }
 
 int tdc_launch(const syn_gbj_item *items, const std::vector<syn_gbj_item> &host, hipStream_t st) {
@@ -1556,7 +1573,7 @@ int tdc_launch(const syn_gbj_item *items, const std::vector<syn_gbj_item> &host,
         hipLaunchKernelGGL(td_secular_kernel, dim3(ni, c64, nodes), dim3(kSecThreads), slds, st, items, l);
         hipLaunchKernelGGL(td_zhat_kernel, dim3(ni, c64, nodes), dim3(kZhatThreads), slds + slds / 2, st, items, l);
         hipLaunchKernelGGL(td_vec_kernel, dim3(ni, (unsigned)((k + 3) / 4), nodes), dim3(256), 0, st, items, l);
-        hipLaunchKernelGGL(td_gemm_kernel, dim3(ni, c64 * c64, nodes), dim3(256), 0, st, items, 0, l);
+        td_gemm(items, ni, c64 * c64, nodes, 0, l, st);
         SYN_LAUNCH_CHECK("divide and conquer");
     }
     const unsigned t32 = (unsigned)((nmax + 31) / 32), t64 = (unsigned)((nmax + 63) / 64);
@@ -1565,8 +1582,8 @@ int tdc_launch(const syn_gbj_item *items, const std::vector<syn_gbj_item> &host,
     else
         hipLaunchKernelGGL((td_back_kernel<2, 4>), dim3(ni, t32), dim3(256), 0, st, items);
     hipLaunchKernelGGL(td_restore_kernel, dim3(ni, t32 * (t32 + 1) / 2), dim3(256), 0, st, items);
-    hipLaunchKernelGGL(td_gemm_kernel, dim3(ni, t64 * t64), dim3(256), 0, st, items, 1, 0);
-    hipLaunchKernelGGL(td_gemm_kernel, dim3(ni, t64 * t64), dim3(256), 0, st, items, 2, 0);
+    td_gemm(items, ni, t64 * t64, 1, 1, 0, st);
+    td_gemm(items, ni, t64 * t64, 1, 2, 0, st);
     SYN_LAUNCH_CHECK("direct phase");
     return SYN_OK;
 }
