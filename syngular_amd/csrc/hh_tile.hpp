@@ -7,7 +7,9 @@
 // column costs two barriers: its entries and partial norms go through LDS,
 // then each wave's partial dot products with every column.  What bounds it is
 // that chain (LDS round trips, one square root and two divisions), about a
-// microsecond a column, not the arithmetic.
+// microsecond a column, not the arithmetic.  (Sums over the waves are shared
+// out over the lanes: 600 x 600 keeping 300 1.72 -> 1.52 ms, 256 x 64 275 ->
+// 245 us.)
 #pragma once
 #include "common.hpp"
 
@@ -29,6 +31,23 @@ __device__ __forceinline__ double lk_sum(double v) {
     const auto h16 = __builtin_amdgcn_permlane16_swap((unsigned)(w >> 32), (unsigned)(w >> 32), false, false);
     return __builtin_bit_cast(double, (uint64_t)h16[0] << 32 | l16[0]) +
            __builtin_bit_cast(double, (uint64_t)h16[1] << 32 | l16[1]);
+}
+
+// Sum over the 16 lanes of a DPP row, in every lane: row rotations in the
+// vector unit, a few dozen cycles where a cross-lane exchange through LDS takes
+// about sixty a step.
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, 0xf, 0xf, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, false);
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+__device__ __forceinline__ double row_sum(double v) {
+    v += dpp_f64<0x128>(v);   // row_ror:8, 4, 2, 1
+    v += dpp_f64<0x124>(v);
+    v += dpp_f64<0x122>(v);
+    return v + dpp_f64<0x121>(v);
 }
 
 template <int NW>
@@ -79,9 +98,7 @@ __device__ __forceinline__ void hh_panel_regs(double *A, int64_t lda, int m, int
             sq = lk_sum(sq);
             if (lane == jl) sm.red[wv] = sq;
             lds_barrier();
-            double xn2 = 0.0;
-#pragma unroll
-            for (int q = 0; q < NW; ++q) xn2 += sm.red[q];
+            const double xn2 = row_sum(li < NW ? sm.red[li & (NW - 1)] : 0.0);
             const double alpha = sm.xs[j];
             double tau = 0.0, scal = 0.0, beta = alpha;
             if (xn2 > 0.0) {
@@ -109,12 +126,16 @@ __device__ __forceinline__ void hh_panel_regs(double *A, int64_t lda, int m, int
                 sm.part[wv][16 + li] = d1;
             }
             lds_barrier();
+            // a quarter of the waves' parts per row of lanes: all of them in
+            // every lane made LDS reads a third of a column of 16 waves
             double f0 = 0.0, f1 = 0.0;
 #pragma unroll
-            for (int q = 0; q < NW; ++q) {
-                f0 += sm.part[q][li];
-                f1 += sm.part[q][16 + li];
+            for (int q = 0; q < NW; q += 4) {
+                f0 += sm.part[q + lk][li];
+                f1 += sm.part[q + lk][16 + li];
             }
+            f0 = lk_sum(f0);
+            f1 = lk_sum(f1);
             f0 = li > j ? tau * f0 : 0.0;
             f1 = 16 + li > j ? tau * f1 : 0.0;
 #pragma unroll

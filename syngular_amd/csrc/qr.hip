@@ -177,7 +177,7 @@ __device__ __forceinline__ void qr_one(const syn_qr_item &P, double *lds_w) {
 // wave.  A column costs about a microsecond of dependent steps (two barriers)
 // instead of a pass over the matrix by rows.  One matrix through ops.qr_many,
 // before and after: 64 x 32 198 / 74 us, 128 x 64 656 / 181, 256 x 64 2018 /
-// 282, 96 x 90 772 / 226, 512 x 24 1086 / 172.
+// 245, 96 x 90 772 / 226, 512 x 24 1086 / 172.
 constexpr int64_t kTileRows = 512, kTileCols = 96;
 constexpr int kTilePanels = (int)kTileCols / kHhCols;
 struct QrTileSmem {

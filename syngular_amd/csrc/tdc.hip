@@ -123,22 +123,6 @@ __device__ __forceinline__ double rsq_nr(double x) {
     return fma(0.5 * y, fma(-x * y, y, 1.0), y);
 }
 
-// Sums over the 16 lanes of a DPP row and over the wave (every lane gets the
-// sum): row rotations in the vector unit and lane reads, a few dozen cycles
-// where a cross-lane exchange through LDS takes about sixty a step.
-template <int CTRL>
-__device__ __forceinline__ double dpp_f64(double v) {
-    const uint64_t u = __builtin_bit_cast(uint64_t, v);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, 0xf, 0xf, false);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, false);
-    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
-}
-__device__ __forceinline__ double row_sum(double v) {
-    v += dpp_f64<0x128>(v);   // row_ror:8, 4, 2, 1
-    v += dpp_f64<0x124>(v);
-    v += dpp_f64<0x122>(v);
-    return v + dpp_f64<0x121>(v);
-}
 __device__ __forceinline__ void opaque(int &x) { asm volatile("" : "+v"(x)); }
 __device__ __forceinline__ double lane_f64(double v, int lane) {
     const uint64_t u = __builtin_bit_cast(uint64_t, v);
@@ -146,6 +130,7 @@ __device__ __forceinline__ double lane_f64(double v, int lane) {
     const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), lane);
     return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
 }
+// sum over the wave, in every lane
 __device__ __forceinline__ double all_sum(double v) {
     v = row_sum(v);
     return (lane_f64(v, 0) + lane_f64(v, 16)) + (lane_f64(v, 32) + lane_f64(v, 48));
