@@ -47,8 +47,10 @@ __device__ __forceinline__ void apply_reflector(const double *V, int64_t ldv, in
                                                 int64_t ldm, int64_t m, int64_t c_lo, int64_t c_hi,
                                                 double (*red)[64]) {
     // rows loaded together: column j is not among those written, but the
-    // compiler cannot know, and row by row each would wait for the last store
-    constexpr int U = 8;
+    // compiler cannot know, and row by row each would wait for the last store (a
+    // segment has 30 rows at most where this form is used: 8 x 128 x 64 409 us
+    // by four, 437 by eight, more by sixteen)
+    constexpr int U = 4;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     int64_t r0, r1;
     seg_bounds<NW>(j + 1, m, w, r0, r1);
@@ -57,18 +59,19 @@ __device__ __forceinline__ void apply_reflector(const double *V, int64_t ldv, in
         const bool act = c < c_hi;
         double part = 0.0;
         if (act) {
-            int64_t i = r0;
-            for (; i + U <= r1; i += U) {
+            const double *vp = V + r0 * ldv + j, *mp = M + r0 * ldm + c;
+            int left = (int)(r1 - r0);
+            for (; left >= U; left -= U, vp += U * ldv, mp += U * ldm) {
                 double v[U], x[U];
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
-                    v[u] = V[(i + u) * ldv + j];
-                    x[u] = M[(i + u) * ldm + c];
+                    v[u] = vp[u * ldv];
+                    x[u] = mp[u * ldm];
                 }
 #pragma unroll
                 for (int u = 0; u < U; ++u) part = fma(v[u], x[u], part);
             }
-            for (; i < r1; ++i) part = fma(V[i * ldv + j], M[i * ldm + c], part);
+            for (; left > 0; --left, vp += ldv, mp += ldm) part = fma(*vp, *mp, part);
         }
         red[w][lane] = part;
         __syncthreads();
@@ -82,26 +85,28 @@ __device__ __forceinline__ void apply_reflector(const double *V, int64_t ldv, in
         __syncthreads();  // every wave has read red[] and M[j, c] before row j changes
         if (act) {
             if (w == 0) M[j * ldm + c] -= f;
-            int64_t i = r0;
-            for (; i + U <= r1; i += U) {
+            const double *vp = V + r0 * ldv + j;
+            double *mp = M + r0 * ldm + c;
+            int left = (int)(r1 - r0);
+            for (; left >= U; left -= U, vp += U * ldv, mp += U * ldm) {
                 double v[U], x[U];
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
-                    v[u] = V[(i + u) * ldv + j];
-                    x[u] = M[(i + u) * ldm + c];
+                    v[u] = vp[u * ldv];
+                    x[u] = mp[u * ldm];
                 }
 #pragma unroll
-                for (int u = 0; u < U; ++u) M[(i + u) * ldm + c] = fma(-f, v[u], x[u]);
+                for (int u = 0; u < U; ++u) mp[u * ldm] = fma(-f, v[u], x[u]);
             }
-            for (; i < r1; ++i) M[i * ldm + c] = fma(-f, V[i * ldv + j], M[i * ldm + c]);
+            for (; left > 0; --left, vp += ldv, mp += ldm) *mp = fma(-f, *vp, *mp);
         }
     }
 }
 
 template <int NW, bool IN_LDS>
 __device__ __forceinline__ void qr_one(const syn_qr_item &P, double *lds_w) {
-    __shared__ double red[NW][64];
-    __shared__ double shv[4];
+    constexpr int kTaus = 128;   // reflector scales kept in LDS; the rest is read back
+    __shared__ double red[NW][64], taus[kTaus];
     const int64_t m = P.m, n = P.n, keep = P.keep;
     const int64_t nb = n < keep ? n : keep;
     const int64_t kq = keep < m ? keep : m;
@@ -109,9 +114,16 @@ __device__ __forceinline__ void qr_one(const syn_qr_item &P, double *lds_w) {
     double *W = IN_LDS ? lds_w : P.work;
     const int tid = threadIdx.x;
 
-    for (int64_t e = tid; e < m * nb; e += (64 * NW)) {
-        const int64_t i = e / nb, j = e - i * nb;
-        W[e] = P.a[i * P.rs + j * P.cs];
+    if (m * nb < 0x7fffffff) {
+        for (unsigned e = tid; e < (unsigned)(m * nb); e += 64 * NW) {
+            const unsigned i = e / (unsigned)nb, j = e - i * (unsigned)nb;
+            W[e] = P.a[i * P.rs + j * P.cs];
+        }
+    } else {
+        for (int64_t e = tid; e < m * nb; e += 64 * NW) {
+            const int64_t i = e / nb, j = e - i * nb;
+            W[e] = P.a[i * P.rs + j * P.cs];
+        }
     }
     __syncthreads();
 
@@ -121,29 +133,28 @@ __device__ __forceinline__ void qr_one(const syn_qr_item &P, double *lds_w) {
             const double v = W[i * nb + j];
             part = fma(v, v, part);
         }
-        part = wave_sum(part);
+        part = row_sum(lk_sum(part));   // wave_sum's pairs, without its trips through LDS
         if ((tid & 63) == 0) red[tid >> 6][0] = part;
         __syncthreads();
+        // every thread works out the reflector: no second exchange
+        double xn2 = 0.0;
+#pragma unroll
+        for (int q = 0; q < NW; ++q) xn2 += red[q][0];
+        const double alpha = W[j * nb + j];
+        double tau = 0.0, scal = 0.0, beta = alpha;
+        if (xn2 > 0.0) {
+            beta = -copysign(sqrt(fma(alpha, alpha, xn2)), alpha);
+            tau = (beta - alpha) / beta;
+            scal = 1.0 / (alpha - beta);
+        }
         if (tid == 0) {
-            double xn2 = 0.0;
-            for (int q = 0; q < NW; ++q) xn2 += red[q][0];
-            const double alpha = W[j * nb + j];
-            double tau = 0.0, scal = 0.0;
-            if (xn2 > 0.0) {
-                const double beta = -copysign(sqrt(fma(alpha, alpha, xn2)), alpha);
-                tau = (beta - alpha) / beta;
-                scal = 1.0 / (alpha - beta);
-                W[j * nb + j] = beta;
-            }
-            shv[0] = tau;
-            shv[1] = scal;
+            if (j < kTaus) taus[j] = tau;
             P.tau[j] = tau;
         }
-        __syncthreads();
-        const double tau = shv[0], scal = shv[1];
         if (tau != 0.0) {
             for (int64_t i = j + 1 + tid; i < m; i += (64 * NW)) W[i * nb + j] *= scal;
             __syncthreads();
+            if (tid == 0) W[j * nb + j] = beta;   // all have read alpha
             apply_reflector<NW>(W, nb, j, tau, W, nb, m, j + 1, nb, red);
         }
         __syncthreads();
@@ -159,7 +170,7 @@ __device__ __forceinline__ void qr_one(const syn_qr_item &P, double *lds_w) {
     }
     __syncthreads();
     for (int64_t j = p - 1; j >= 0; --j) {
-        const double tau = P.tau[j];
+        const double tau = j < kTaus ? taus[j] : P.tau[j];
         if (tau != 0.0) apply_reflector<NW>(W, nb, j, tau, Q, ldq, m, j, kq, red);
         __syncthreads();
     }
