@@ -234,12 +234,19 @@ __global__ __launch_bounds__(NT) void jacobi_gram_kernel(Tab tab, int nv_max, do
     // rounding level of forming G (a rank-deficient G has a null space of
     // such entries, which a purely relative test would keep rotating)
     __shared__ double floor_abs;
+    __shared__ int shift;   // power of two the matrix is scaled by
     if (tid < 64) {
         double m = 0.0;
         for (int i = tid; i < g; i += 64) m = fmax(m, fabs(A[i * ld + i]));
         for (int off = 32; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off, 64));
-        if (tid == 0) floor_abs = __DBL_EPSILON__ * m;
+        if (tid == 0) {
+            shift = gram_shift(m);
+            floor_abs = __DBL_EPSILON__ * ldexp(m, shift);
+        }
     }
+    __syncthreads();
+    if (shift)
+        for (int e = tid; e < g * g; e += NT) A[e / g * ld + e % g] = ldexp(A[e / g * ld + e % g], shift);
     const int np = g + (g & 1), half = np / 2;
     int sweep = 0;
     for (; sweep < max_sweeps && g > 1; ++sweep) {
@@ -320,7 +327,7 @@ __global__ __launch_bounds__(NT) void jacobi_gram_kernel(Tab tab, int nv_max, do
             rk += (lj > li) || (lj == li && j < i);
         }
         rank[i] = rk;
-        P.s[rk] = sqrt(fmax(li, 0.0));
+        P.s[rk] = ldexp(sqrt(fmax(li, 0.0)), -shift / 2);
     }
     __syncthreads();
     for (int e = tid; e < g * g; e += NT) {
@@ -385,6 +392,14 @@ __global__ __launch_bounds__(64) void jacobi_gram16_kernel(Tab tab, int nv_max, 
     // absolute rotation floor, as in the other kernel
     double m = diag ? fmax(fabs(a00), fabs(a11)) : 0.0;
     for (int off = 32; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off, 64));
+    const int shift = gram_shift(m);
+    if (shift) {
+        m = ldexp(m, shift);
+        a00 = ldexp(a00, shift);
+        a01 = ldexp(a01, shift);
+        a10 = ldexp(a10, shift);
+        a11 = ldexp(a11, shift);
+    }
     const double floor_abs = __DBL_EPSILON__ * m;
     lds_barrier();
     int sweep = 0;
@@ -457,7 +472,7 @@ __global__ __launch_bounds__(64) void jacobi_gram16_kernel(Tab tab, int nv_max, 
             rk += (lj > li) || (lj == li && j < lane);
         }
         rank[lane] = rk;
-        P.s[rk] = sqrt(fmax(li, 0.0));
+        P.s[rk] = ldexp(sqrt(fmax(li, 0.0)), -shift / 2);
     }
     lds_barrier();
     for (int e = lane; e < g * g; e += 64) {

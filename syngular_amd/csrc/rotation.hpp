@@ -5,10 +5,33 @@
 namespace syn {
 
 // Rotation test of plane (p, q): |G_pq| > max(tol sqrt(|G_pp G_qq|), floor),
-// in squares (no square root on the critical path of a round).
+// in squares (no square root on the critical path of a round), for a matrix
+// whose largest diagonal entry is within 1e-100 .. 1e100: beyond, the squares
+// leave the range of doubles and the test would find nothing to rotate.
 __device__ __forceinline__ bool rotates(double apq, double app, double aqq, double tol, double floor_abs) {
     const double a2 = apq * apq;
     return a2 > tol * tol * fabs(app * aqq) && fabs(apq) > floor_abs;
+}
+
+// The same at any scale, for entries in memory that are not scaled beforehand:
+// floor is eps max G_ii, so it tells whether a power of two has to bring the
+// entries into that range.  The choice is the same for all planes of a matrix.
+// The LDS kernels scale their matrix once instead (an order-16 matrix takes 55 us
+// so, 59 with this form).
+__device__ __forceinline__ bool rotates_any(double apq, double app, double aqq, double tol, double floor_abs) {
+    if (floor_abs < 1e-130 || floor_abs > 1e120) {
+        const double f = floor_abs < 1.0 ? 0x1p700 : 0x1p-700;
+        const double a = f * apq;
+        return a * a > tol * tol * fabs(f * app * (f * aqq)) && fabs(apq) > floor_abs;
+    }
+    return rotates(apq, app, aqq, tol, floor_abs);
+}
+
+// Even power of two that brings a matrix of largest diagonal entry m into the
+// range of `rotates` (0 where it is in it, or zero, or not finite).
+__device__ __forceinline__ int gram_shift(double m) {
+    const bool in = m >= 1e-100 && m <= 1e100;
+    return in || !(m > 0.0) || m > __DBL_MAX__ ? 0 : -(ilogb(m) & ~1);
 }
 
 // Jacobi rotation annihilating G_pq (Rutishauser's angle, Golub & Van Loan

@@ -161,7 +161,7 @@ __device__ __forceinline__ void tj_pair_solve(const syn_gbj_item &P, const TjDim
     const double floor_abs = P.w[tj_floor_off<TB>(D.half)];
     for (int e = tid; e < TP * TP; e += NT) {
         const int i = e / TP, k = e % TP;
-        if (i < k && (!cross || (i < TB && k >= TB)) && rotates(S[i][k], S[i][i], S[k][k], tol, floor_abs))
+        if (i < k && (!cross || (i < TB && k >= TB)) && rotates_any(S[i][k], S[i][i], S[k][k], tol, floor_abs))
             do_rot = 1;
     }
     __syncthreads();
@@ -217,7 +217,7 @@ __device__ __forceinline__ void tj_pair_solve(const syn_gbj_item &P, const TjDim
                 }
                 if (rot_thread) {
                     double c = 1.0, sn = 0.0;
-                    if (rotates(apq, app, aqq, tol, floor_abs)) {
+                    if (rotates_any(apq, app, aqq, tol, floor_abs)) {
                         rotation(apq, app, aqq, c, sn);
                         any_rot = 1;
                     }
@@ -280,7 +280,7 @@ __device__ __forceinline__ void tj_pair_solve(const syn_gbj_item &P, const TjDim
                 const double wy0 = W[wi][wq0], wy1 = W[wi][wq1];
                 if (rot_thread) {
                     double c = 1.0, sn = 0.0;
-                    if (rotates(apq, app, aqq, tol, floor_abs)) {
+                    if (rotates_any(apq, app, aqq, tol, floor_abs)) {
                         rotation(apq, app, aqq, c, sn);
                         any_rot = 1;
                     }
@@ -852,7 +852,7 @@ __global__ __launch_bounds__(256) void tj_check_kernel(const syn_gbj_item *__res
     const int64_t nel = P.nv * P.nv;
     for (int64_t e = (int64_t)blockIdx.y * 256 + threadIdx.x; e < nel && !hit; e += (int64_t)gridDim.y * 256) {
         const int64_t i = e / P.nv, k = e - i * P.nv;
-        if (i != k && rotates(G[i * ld + k], G[i * ld + i], G[k * ld + k], tol, floor_abs)) hit = true;
+        if (i != k && rotates_any(G[i * ld + k], G[i * ld + i], G[k * ld + k], tol, floor_abs)) hit = true;
     }
     if (hit) chk[P.counter - counters] = 1;
 }
