@@ -274,8 +274,9 @@ int syn_jacobi_f64(const syn_jacobi_item *items, int n_items, double tol, int ma
 /* nv <= nv_max <= 64 for every item).  On exit rt rows are the           */
 /* eigenvectors (rt = V^T, G = V diag(lambda) V^T) sorted by decreasing    */
 /* eigenvalue and s[i] = sqrt(max(lambda_i, 0)), the singular values of C */
-/* when G = C^T C.  Items outside the contract get s = NaN.  No reference */
-/* call site (an addition: the SVD form of the rounding, small bonds).  */
+/* when G = C^T C.  Items outside the contract and matrices that are not  */
+/* finite get s = NaN.  No reference call site (an addition: the SVD form */
+/* of the rounding, small bonds).                                         */
 int syn_jacobi_gram_f64(const syn_jacobi_item *items, int n_items, int64_t nv_max, double tol, int max_sweeps,
                         void *stream);
 

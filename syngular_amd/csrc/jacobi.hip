@@ -224,12 +224,15 @@ __global__ __launch_bounds__(NT) void jacobi_gram_kernel(Tab tab, int nv_max, do
     const int g = (int)P.nv, ld = g + 1;
     double *A = lds;
     double *R = lds + g * ld;
+    bool finite = true;
     for (int e = tid; e < g * g; e += NT) {
         const int i = e / g, j = e - i * g;
         A[i * ld + j] = P.x[i * P.ldx + j];
         R[i * ld + j] = (i == j) ? 1.0 : 0.0;
+        finite = finite && fabs(A[i * ld + j]) <= __DBL_MAX__;
     }
-    __syncthreads();
+    // a matrix that is not finite has no eigenvalues to order: s is NaN
+    finite = __syncthreads_and(finite);
     // absolute rotation floor eps * max_i G_ii: entries below it are at the
     // rounding level of forming G (a rank-deficient G has a null space of
     // such entries, which a purely relative test would keep rotating)
@@ -326,8 +329,9 @@ __global__ __launch_bounds__(NT) void jacobi_gram_kernel(Tab tab, int nv_max, do
             const double lj = A[j * ld + j];
             rk += (lj > li) || (lj == li && j < i);
         }
+        if (!finite) rk = i;
         rank[i] = rk;
-        P.s[rk] = ldexp(sqrt(fmax(li, 0.0)), -shift / 2);
+        P.s[rk] = finite ? ldexp(sqrt(fmax(li, 0.0)), -shift / 2) : __builtin_nan("");
     }
     __syncthreads();
     for (int e = tid; e < g * g; e += NT) {
@@ -389,6 +393,8 @@ __global__ __launch_bounds__(64) void jacobi_gram16_kernel(Tab tab, int nv_max, 
     double a00 = at(k, kc), a01 = at(k, h + kc), a10 = at(h + k, kc), a11 = at(h + k, h + kc);
     for (int e = lane; e < kReg * kReg; e += 64) R[e / kReg][e % kReg] = e / kReg == e % kReg ? 1.0 : 0.0;
     const bool diag = k == kc && k < h;
+    const bool finite = !__ballot(!(fabs(a00) <= __DBL_MAX__ && fabs(a01) <= __DBL_MAX__ && fabs(a10) <= __DBL_MAX__ &&
+                                    fabs(a11) <= __DBL_MAX__));
     // absolute rotation floor, as in the other kernel
     double m = diag ? fmax(fabs(a00), fabs(a11)) : 0.0;
     for (int off = 32; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off, 64));
@@ -471,8 +477,9 @@ __global__ __launch_bounds__(64) void jacobi_gram16_kernel(Tab tab, int nv_max, 
             const double lj = lam[j];
             rk += (lj > li) || (lj == li && j < lane);
         }
+        if (!finite) rk = lane;
         rank[lane] = rk;
-        P.s[rk] = ldexp(sqrt(fmax(li, 0.0)), -shift / 2);
+        P.s[rk] = finite ? ldexp(sqrt(fmax(li, 0.0)), -shift / 2) : __builtin_nan("");
     }
     lds_barrier();
     for (int e = lane; e < g * g; e += 64) {

@@ -75,3 +75,32 @@ def test_rounding_of_a_scaled_chain(k):
     assert list(rep0.kept) == list(rep1.kept)
     # orders up to 8: a few dozen rotations and products of a few eps
     assert np.linalg.norm(np.ldexp(got, -k) - want) <= 1000 * EPS * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+@pytest.mark.parametrize("where", [(2, 2), (2, 3), (0, 6)])
+def test_lds_non_finite(value, where):
+    """A matrix that is not finite gives NaN singular values, writes every
+    entry of its results and leaves its neighbours alone."""
+    import torch
+
+    from syngular_amd import batch, ops
+
+    orders = [7, 16, 17, 40, 64]
+    mats = []
+    for g in orders:
+        G = torch.eye(g, dtype=torch.float64) + 0.1
+        bad = G.clone()
+        bad[where] = bad[where[::-1]] = value
+        mats += [bad.cuda(), G.cuda()]
+    rts = [torch.full_like(m, 7.0) for m in mats]
+    ss = [torch.full((m.shape[0],), 7.0, dtype=torch.float64, device="cuda") for m in mats]
+    ptr = lambda ts: np.array([t.data_ptr() for t in ts], np.uint64)   # noqa: E731
+    batch.jacobi_table(ptr(mats), np.array([m.shape[0] for m in mats]), ptr(rts), ptr(ss))
+    for i, (m, rt, s) in enumerate(zip(mats, rts, ss)):
+        assert not (rt == 7.0).any() and not (s == 7.0).any(), (m.shape[0], i)
+        if i % 2 == 0:
+            assert torch.isnan(s).all(), m.shape[0]
+        else:
+            ref = ops.jacobi_gram_many([m])[0]
+            assert torch.equal(rt, ref[0]) and torch.equal(s, ref[1]), m.shape[0]
