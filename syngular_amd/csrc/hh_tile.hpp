@@ -107,6 +107,16 @@ __device__ __forceinline__ void hh_panel_regs(double *A, int64_t lda, int m, int
                 scal = 1.0 / (alpha - beta);
             }
             if (tid == 0) sm.tau[j] = tau;
+            if (tau == 0.0) {
+                // no reflector: a NaN in the column stays in it
+#pragma unroll
+                for (int t = 0; t < RT; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (li == jl && 16 * (wv + NW * t) + lk + 4 * r > j) a[t][ct][r] = 0.0;
+                lds_barrier();   // all have read xs and red
+                continue;
+            }
             double v[RT][4], d0 = 0.0, d1 = 0.0;
 #pragma unroll
             for (int t = 0; t < RT; ++t)
