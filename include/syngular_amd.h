@@ -160,6 +160,7 @@ int syn_direct_sum_f64(const syn_dsum_item *items, int n_items, int64_t total_bl
 /* Replaces numpy.linalg.qr at tensor/matrix_product_state.py:307,332,  */
 /* 443,560,574 and tensor/matrix_product_operator.py:436,555,680,703.     */
 /* ------------------------------------------------------------------ */
+#define SYN_QR_COLUMNS 0x4c4f4351
 typedef struct {
     const double *a;
     int64_t rs, cs;
@@ -167,17 +168,26 @@ typedef struct {
     double *q;
     int64_t ldq;
     int32_t q_trans;  /* 1: store Q^T (kq x m, row-major, ldq) instead of Q */
-    int32_t columns;  /* 1: column by column, in one order of sums whatever the shape */
+    int32_t columns;  /* SYN_QR_COLUMNS: column by column, one order of sums for all shapes;
+                         anything else: the form that suits the shape */
     double *work;
     double *tau;
 } syn_qr_item;
 int syn_qr_f64(const syn_qr_item *items, int n_items, void *stream);
-/* The same with the launch's dynamic LDS sized by the caller: lds_doubles  */
-/* (at most 12288, the 96 KB of syn_qr_f64); a matrix whose leading block  */
-/* m * min(n, keep) fits works in LDS, a larger one in its workspace.  A   */
-/* batch of small matrices launched with a small size keeps more           */
-/* work-groups on each compute unit.                                        */
+/* The same with the LDS of the column-by-column form sized by the caller:  */
+/* lds_doubles (at most 12288, the 96 KB of syn_qr_f64); a matrix of that   */
+/* form whose leading block m * min(n, keep) fits works in LDS, a larger    */
+/* one in its workspace.  One work-group fits a compute unit whatever the   */
+/* size; the two entry points below are for launches of more matrices than  */
+/* the chip has units, and give the same bits.                              */
 int syn_qr_sized_f64(const syn_qr_item *items, int n_items, int64_t lds_doubles, void *stream);
+/* Every matrix in the column-by-column form, with lds_doubles of LDS: a    */
+/* small size keeps more work-groups on each compute unit.                  */
+int syn_qr_columns_f64(const syn_qr_item *items, int n_items, int64_t lds_doubles, void *stream);
+/* Matrices of at most `rows` rows (1..64), by launches of one to four waves */
+/* a matrix.  One with more rows or more than 96 factored columns is taken  */
+/* too, column by column in its workspace.                                  */
+int syn_qr_rows_f64(const syn_qr_item *items, int n_items, int64_t rows, void *stream);
 
 /* Panel of the blocked Householder QR (one work-group of 1024 threads). */
 /* Factors columns [j0, j0+b) of the m-row matrix w (row-major, ldw;     */

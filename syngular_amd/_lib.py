@@ -38,6 +38,7 @@ MPO_MPO_ITEM = np.dtype(
 DSUM_ITEM = np.dtype(
     [("a", _P), ("b", _P), ("out", _P), ("la", _I), ("ra", _I), ("lb", _I), ("rb", _I), ("mid", _I),
      ("lo", _I), ("ro", _I), ("edge", np.int32), ("block_start", _I)], align=True)
+QR_COLUMNS = 0x4c4f4351  # SYN_QR_COLUMNS
 QR_ITEM = np.dtype(
     [("a", _P), ("rs", _I), ("cs", _I), ("m", _I), ("n", _I), ("keep", _I), ("q", _P), ("ldq", _I),
      ("q_trans", np.int32), ("columns", np.int32), ("work", _P), ("tau", _P)], align=True)
@@ -96,6 +97,8 @@ SIGNATURES = {
     "syn_direct_sum_f64": (_I32, [_VP, _I32, _I64, _VP]),
     "syn_qr_f64": (_I32, [_VP, _I32, _VP]),
     "syn_qr_sized_f64": (_I32, [_VP, _I32, _I64, _VP]),
+    "syn_qr_columns_f64": (_I32, [_VP, _I32, _I64, _VP]),
+    "syn_qr_rows_f64": (_I32, [_VP, _I32, _I64, _VP]),
     "syn_lu_sign_leaf_f64": (_I32, [_VP, _I32, _D, _VP]),
     "syn_hh_panel_f64": (_I32, [_VP, _I64, _VP, _I64, _VP, _VP, _I64, _I64, _I64, _I64, _VP]),
     "syn_colscale_f64": (_I32, [_VP, _I32, _I64, _VP]),

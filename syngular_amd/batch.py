@@ -205,33 +205,58 @@ def apply_table(x, o, p, chil, din, chir, dl, dout, dr):
     _launch_blocks("syn_mpo_apply_f64", it, nel)
 
 
-# LDS classes (doubles) of the grouped Householder QR: 16, 48 and 96 KB;
-# matrices above the last work from their workspace
+# LDS classes (doubles) of the column-by-column Householder QR: 16, 48 and 96
+# KB; matrices above the last work from their workspace
 QR_LDS_CLASSES = (2048, 6144, 12288)
+# row classes of the panel form's launches for many small matrices
+QR_ROW_CLASSES = (16, 32, 64)
+# matrices of one launch (the chip has 256 compute units) up to which a
+# work-group per compute unit is no limit and classes would only add launches
+QR_FEW = 256
 
 
 def qr_table(a, m, n, q, work, tau, columns=False):
     """Householder QR of every row-major m x n (m > n) matrix: q (m x n) gets
     the thin orthogonal factor.  columns: column by column, in one order of
     sums (the mixed sweep rounds the factors to FP32, which would turn another
-    order's last bits into differences of an FP32 ulp)."""
+    order's last bits into differences of an FP32 ulp).
+
+    Up to QR_FEW matrices go in one launch.  More of them are limited by how
+    many work-groups a compute unit holds: the column form's launches are by
+    the LDS their matrices need, the panel form's by rows (4096 matrices of
+    16 x 8, 32 x 16 and 64 x 32 in one launch 489, 698 and 1221 us, by rows
+    266, 299 and 545; of 128 x 32 in the column form 3705, by LDS 1629)."""
     it = np.zeros(len(a), dtype=_lib.QR_ITEM)
     it["a"], it["rs"], it["cs"] = a, n, 1
     it["m"], it["n"], it["keep"] = m, n, n
     it["q"], it["ldq"], it["q_trans"] = q, n, 0
-    it["work"], it["tau"], it["columns"] = work, tau, columns
-    # one launch per LDS class of the matrices, each with the dynamic LDS its
-    # largest matrix needs: small matrices do not hold a compute unit's LDS
-    # for the large ones
-    need = np.asarray(m, dtype=np.int64) * np.asarray(n, dtype=np.int64)
-    cls = np.searchsorted(QR_LDS_CLASSES, need, side="left")
-    for c in range(len(QR_LDS_CLASSES) + 1):
+    it["work"], it["tau"], it["columns"] = work, tau, _lib.QR_COLUMNS if columns else 0
+    if len(it) == 0:
+        return
+    need = it["m"] * it["n"]
+    need[need > QR_LDS_CLASSES[-1]] = 0
+
+    def launch(fn, sel, size):
+        dev = ops._device_table(it[sel]) if fn not in _lib.HOST_ENTRIES else ops._upload(it[sel])
+        call(ops.entry(fn, dev), dev.data_ptr(), len(sel), int(size), ops._stream())
+
+    every = np.arange(len(it))
+    if len(it) <= QR_FEW:
+        launch("syn_qr_sized_f64", every, need.max())
+        return
+    if columns:
+        cls = np.where(need > 0, np.searchsorted(QR_LDS_CLASSES, need, side="left"), len(QR_LDS_CLASSES))
+        for c in np.unique(cls):
+            sel = np.nonzero(cls == c)[0]
+            launch("syn_qr_columns_f64", sel, need[sel].max())
+        return
+    cls = np.searchsorted(QR_ROW_CLASSES, it["m"], side="left")
+    for c in np.unique(cls):
         sel = np.nonzero(cls == c)[0]
-        if len(sel) == 0:
-            continue
-        dev = ops._upload(it[sel])
-        lds = int(need[sel].max()) if c < len(QR_LDS_CLASSES) else 0
-        call(ops.entry("syn_qr_sized_f64", dev), dev.data_ptr(), len(sel), lds, ops._stream())
+        if c < len(QR_ROW_CLASSES):
+            launch("syn_qr_rows_f64", sel, QR_ROW_CLASSES[c])
+        else:
+            launch("syn_qr_sized_f64", sel, need[sel].max())
 
 
 # size classes (matrix order) of the LDS Jacobi launches

@@ -50,26 +50,44 @@ __device__ __forceinline__ double row_sum(double v) {
     return v + dpp_f64<0x121>(v);
 }
 
-template <int NW>
+// For a panel of at most ROWS rows.  SMALL: the waves' parts of V^T V take the
+// place of what the columns needed, for a barrier, so that more work-groups fit a
+// compute unit.  A launch of one matrix keeps them apart (a two-site gate at chi =
+// 300 takes 1.60 ms with them together, 1.58 apart).
+template <int NW, int ROWS, bool SMALL = false>
 struct HhSmem {
-    double xs[1024];                     // the column being reflected
+    double xs[ROWS];                     // the column being reflected
     double red[NW];                      // partial squared norms
     double part[NW][kHhCols];            // partial dot products
     double tau[kHhCols];
     double S[3][16][17];                 // V^T V, upper triangle by tiles (0,0), (0,1), (1,1)
     double Sp[NW][3][256];               // each wave's part of it
 };
+template <int NW, int ROWS>
+struct HhSmem<NW, ROWS, true> {
+    union {
+        struct {
+            double xs[ROWS];
+            double red[NW];
+            double part[NW][kHhCols];
+        };
+        double Sp[NW][3][256];
+    };
+    double tau[kHhCols];
+    double S[3][16][17];
+};
 
 // Factors the m x b panel at A (row-major, leading dimension lda; m <= 16 NW
-// RT, b <= 32) in place: R on and above the diagonal, v below (LAPACK dgeqrf:
+// RT <= ROWS, b <= 32) in place: R on and above the diagonal, v below (LAPACK dgeqrf:
 // beta = -sign(alpha) norm, tau = 0 and v = e1 for a column already zero below
 // the diagonal).  T (ld ldt): the upper triangular factor of I - V T V^T,
 // zeros below, tau to tau_out.  Vx, when given (leading dimension ldv), gets
 // V with its unit diagonal and zeros above.  Every thread of the work-group
 // (64 NW) calls it; ends with a barrier.
-template <int RT, int NW>
+template <int RT, int NW, int ROWS, bool SMALL>
 __device__ __forceinline__ void hh_panel_regs(double *A, int64_t lda, int m, int b, double *T, int64_t ldt,
-                                              double *tau_out, double *Vx, int64_t ldv, HhSmem<NW> &sm) {
+                                              double *tau_out, double *Vx, int64_t ldv, HhSmem<NW, ROWS, SMALL> &sm) {
+    static_assert(16 * NW * RT <= ROWS, "rows of the panel");
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lk = lane >> 4;
     double a[RT][2][4];
@@ -141,6 +159,9 @@ __device__ __forceinline__ void hh_panel_regs(double *A, int64_t lda, int m, int
             double f0 = 0.0, f1 = 0.0;
 #pragma unroll
             for (int q = 0; q < NW; q += 4) {
+                if constexpr (NW < 4) {
+                    if (lk >= NW) continue;
+                }
                 f0 += sm.part[q + lk][li];
                 f1 += sm.part[q + lk][16 + li];
             }
@@ -178,6 +199,7 @@ __device__ __forceinline__ void hh_panel_regs(double *A, int64_t lda, int m, int
             s01 = __builtin_amdgcn_mfma_f64_16x16x4f64(v[0], v[1], s01, 0, 0, 0);
             s11 = __builtin_amdgcn_mfma_f64_16x16x4f64(v[1], v[1], s11, 0, 0, 0);
         }
+    if (SMALL) lds_barrier();   // all have read the last column's part
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const int e = (lk + 4 * r) * 16 + li;

@@ -174,7 +174,7 @@ __global__ __launch_bounds__(kPanelThreads) void hh_panel_reg_kernel(double *W, 
                                                                      double *tau, double *T, int64_t ldt, int64_t m,
                                                                      int64_t j0, int b) {
     extern __shared__ double dyn[];
-    HhSmem<kPanelWaves> &sm = *(HhSmem<kPanelWaves> *)dyn;
+    auto &sm = *(HhSmem<kPanelWaves, 1024> *)dyn;
     hh_panel_regs<RT, kPanelWaves>(W + j0 * ldw + j0, ldw, (int)(m - j0), b, T, ldt, tau + j0, V + j0 * ldv + j0, ldv,
                                    sm);
 }
@@ -182,7 +182,7 @@ __global__ __launch_bounds__(kPanelThreads) void hh_panel_reg_kernel(double *W, 
 template <int RT>
 static int panel_regs(double *w, int64_t ldw, double *v, int64_t ldv, double *tau, double *t, int64_t ldt, int64_t m,
                       int64_t j0, int b, hipStream_t s) {
-    constexpr size_t lds = sizeof(HhSmem<kPanelWaves>);
+    constexpr size_t lds = sizeof(HhSmem<kPanelWaves, 1024>);
     static bool attr_set = false;
     if (!attr_set) {
         if (int rc = hip_check(hipFuncSetAttribute((const void *)hh_panel_reg_kernel<RT>,

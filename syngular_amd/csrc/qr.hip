@@ -47,9 +47,9 @@ __device__ __forceinline__ void apply_reflector(const double *V, int64_t ldv, in
                                                 int64_t ldm, int64_t m, int64_t c_lo, int64_t c_hi,
                                                 double (*red)[64]) {
     // rows loaded together: column j is not among those written, but the
-    // compiler cannot know, and row by row each would wait for the last store (a
-    // segment has 30 rows at most where this form is used: 8 x 128 x 64 409 us
-    // by four, 437 by eight, more by sixteen)
+    // compiler cannot know, and row by row each would wait for the last store
+    // (8 matrices of 128 x 64, segments of up to 32 rows: 409 us by four, 437 by
+    // eight, more by sixteen; taller segments not measured)
     constexpr int U = 4;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     int64_t r0, r1;
@@ -191,17 +191,19 @@ __device__ __forceinline__ void qr_one(const syn_qr_item &P, double *lds_w) {
 // 245, 96 x 90 772 / 226, 512 x 24 1086 / 172.
 constexpr int64_t kTileRows = 512, kTileCols = 96;
 constexpr int kTilePanels = (int)kTileCols / kHhCols;
+template <int NW, int ROWS, int PANELS, bool SMALL>
 struct QrTileSmem {
-    HhSmem<kQrWaves> hh;
-    double T[kTilePanels][kHhCols * kHhCols];
+    HhSmem<NW, ROWS, SMALL> hh;
+    double T[PANELS][kHhCols * kHhCols];
 };
 
-template <int RT>
-__device__ __forceinline__ void qr_tile(const syn_qr_item &P, QrTileSmem &sm) {
+template <int RT, int NW, typename Smem>
+__device__ __forceinline__ void qr_tile(const syn_qr_item &P, Smem &sm) {
+    constexpr int NT = 64 * NW;
     const int m = (int)P.m, nb = (int)(P.n < P.keep ? P.n : P.keep), kq = (int)(P.keep < P.m ? P.keep : P.m);
     const int p = m < nb ? m : nb, tid = threadIdx.x, wv = tid >> 6;
     double *W = P.work;
-    for (int e = tid; e < m * nb; e += kQrThreads) {
+    for (int e = tid; e < m * nb; e += NT) {
         const int i = e / nb, j = e - i * nb;
         W[e] = P.a[i * P.rs + j * P.cs];
     }
@@ -209,27 +211,27 @@ __device__ __forceinline__ void qr_tile(const syn_qr_item &P, QrTileSmem &sm) {
     for (int j0 = 0; j0 < p; j0 += kHhCols) {
         const int b = p - j0 < kHhCols ? p - j0 : kHhCols;
         double *Wp = W + (int64_t)j0 * nb + j0, *T = sm.T[j0 / kHhCols];
-        hh_panel_regs<RT, kQrWaves>(Wp, nb, m - j0, b, T, kHhCols, P.tau + j0, nullptr, 0, sm.hh);
-        for (int c = j0 + b + 16 * wv; c < p; c += 16 * kQrWaves)
+        hh_panel_regs<RT, NW>(Wp, nb, m - j0, b, T, kHhCols, P.tau + j0, nullptr, 0, sm.hh);
+        for (int c = j0 + b + 16 * wv; c < p; c += 16 * NW)
             hh_apply_wave(Wp, nb, m - j0, b, T, kHhCols, true, W + (int64_t)j0 * nb + c, nb, p - c < 16 ? p - c : 16);
         __syncthreads();
     }
     double *Q = P.q_trans ? P.work + (int64_t)m * nb : P.q;
     const int64_t ldq = P.q_trans ? kq : P.ldq;
-    for (int e = tid; e < m * kq; e += kQrThreads) {
+    for (int e = tid; e < m * kq; e += NT) {
         const int i = e / kq, c = e - i * kq;
         Q[i * ldq + c] = (i == c) ? 1.0 : 0.0;
     }
     __syncthreads();
     for (int j0 = (p - 1) / kHhCols * kHhCols; j0 >= 0; j0 -= kHhCols) {
         const int b = p - j0 < kHhCols ? p - j0 : kHhCols;
-        for (int c = j0 + 16 * wv; c < kq; c += 16 * kQrWaves)
+        for (int c = j0 + 16 * wv; c < kq; c += 16 * NW)
             hh_apply_wave(W + (int64_t)j0 * nb + j0, nb, m - j0, b, sm.T[j0 / kHhCols], kHhCols, false,
                           Q + j0 * ldq + c, ldq, kq - c < 16 ? kq - c : 16);
         __syncthreads();
     }
     if (P.q_trans) {
-        for (int e = tid; e < m * kq; e += kQrThreads) {
+        for (int e = tid; e < m * kq; e += NT) {
             const int c = e / m, i = e - c * m;
             P.q[c * P.ldq + i] = Q[i * ldq + c];
         }
@@ -238,48 +240,78 @@ __device__ __forceinline__ void qr_tile(const syn_qr_item &P, QrTileSmem &sm) {
 
 // lds_cap: doubles of dynamic LDS the launch holds; a matrix whose leading
 // block fits works in LDS, a larger one in its workspace.
+template <int NW>
+__device__ __forceinline__ void qr_columns(const syn_qr_item &P, double *lds_w, int64_t lds_cap) {
+    const int64_t nb = P.n < P.keep ? P.n : P.keep;
+    if (P.m * nb <= lds_cap)
+        qr_one<NW, true>(P, lds_w);
+    else
+        qr_one<NW, false>(P, lds_w);
+}
+
+// Matrices of any shape and form.  One work-group fits a compute unit (103 KB of
+// LDS with the static part, 200 registers a thread), so a launch of more matrices
+// than the chip has units takes the two kernels below for what they are for.
+typedef QrTileSmem<kQrWaves, kTileRows, kTilePanels, false> QrAnySmem;
 template <typename Tab>
 __global__ __launch_bounds__(kQrThreads) void qr_kernel(Tab tab, int64_t lds_cap) {
     extern __shared__ double lds_w[];
     const syn_qr_item &P = tab.get()[blockIdx.x];
     const int64_t nb = P.n < P.keep ? P.n : P.keep;
-    if (P.columns) {
-        // The column-by-column form by four waves, whatever the shape.  The mixed
-        // sweep asks for it: it rounds its factors to FP32, where another order of
-        // the FP64 sums, no less exact, now and then ends on the neighbouring FP32
-        // number, so this order is part of that form's results.
+    if (P.columns == SYN_QR_COLUMNS) {
         if (threadIdx.x >= 64 * kColWaves) return;   // whole waves: the others' barriers do not wait for them
-        if (P.m * nb <= lds_cap)
-            qr_one<kColWaves, true>(P, lds_w);
-        else
-            qr_one<kColWaves, false>(P, lds_w);
+        qr_columns<kColWaves>(P, lds_w, lds_cap);
     } else if (P.m <= kTileRows && nb <= kTileCols) {
-        QrTileSmem &sm = *(QrTileSmem *)lds_w;
+        QrAnySmem &sm = *(QrAnySmem *)lds_w;
         if (P.m <= 128)
-            qr_tile<1>(P, sm);
+            qr_tile<1, kQrWaves>(P, sm);
         else if (P.m <= 256)
-            qr_tile<2>(P, sm);
+            qr_tile<2, kQrWaves>(P, sm);
         else
-            qr_tile<4>(P, sm);
-    } else if (P.m * nb <= lds_cap)
-        qr_one<kQrWaves, true>(P, lds_w);
-    else
-        qr_one<kQrWaves, false>(P, lds_w);
+            qr_tile<4, kQrWaves>(P, sm);
+    } else
+        qr_columns<kQrWaves>(P, lds_w, lds_cap);
+}
+
+// The column-by-column form by four waves, whatever the shape, with the LDS
+// that the launch's matrices need.  The mixed sweep asks for it: it rounds its
+// factors to FP32, where another order of the FP64 sums, no less exact, now and
+// then ends on the neighbouring FP32 number, so this order is part of that
+// form's results.
+template <typename Tab>
+__global__ __launch_bounds__(64 * kColWaves) void qr_columns_kernel(Tab tab, int64_t lds_cap) {
+    extern __shared__ double lds_w[];
+    qr_columns<kColWaves>(tab.get()[blockIdx.x], lds_w, lds_cap);
+}
+
+// Matrices of up to 16 NW rows (NW 1, 2, 4): the panel form by NW waves, the same
+// bits as by eight, whose other waves hold no rows.
+template <int NW, typename Tab>
+__global__ __launch_bounds__(64 * NW, 3) void qr_rows_kernel(Tab tab) {
+    constexpr int ROWS = 16 * NW, PANELS = (ROWS + kHhCols - 1) / kHhCols;
+    __shared__ QrTileSmem<NW, ROWS, PANELS, true> sm;
+    const syn_qr_item &P = tab.get()[blockIdx.x];
+    if (P.m <= ROWS && (P.n < P.keep ? P.n : P.keep) <= kTileCols)
+        qr_tile<1, NW>(P, sm);
+    else   // not a matrix of the class: right, if slow
+        qr_one<NW, false>(P, nullptr);
+}
+
+template <typename Kernel>
+static int qr_lds(Kernel *kern, size_t most, const char *who) {
+    return hip_check(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)most), who);
 }
 
 // every launch holds what the panel form needs; the other form its lds_cap
 template <typename Tab>
 static int qr_launch(Tab tab, int n_items, int64_t lds_doubles, hipStream_t s) {
     static bool attr_set = false;
-    const size_t most = std::max(sizeof(QrTileSmem), (size_t)kQrLdsDoubles * sizeof(double));
     if (!attr_set) {
-        if (int rc = hip_check(hipFuncSetAttribute((const void *)qr_kernel<Tab>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                   (int)most),
-                               "syn_qr_f64: hipFuncSetAttribute"))
-            return rc;
+        const size_t most = std::max(sizeof(QrAnySmem), (size_t)kQrLdsDoubles * sizeof(double));
+        if (int rc = qr_lds(qr_kernel<Tab>, most, "syn_qr_f64: hipFuncSetAttribute")) return rc;
         attr_set = true;
     }
-    const size_t lds = std::max(sizeof(QrTileSmem), (size_t)lds_doubles * sizeof(double));
+    const size_t lds = std::max(sizeof(QrAnySmem), (size_t)lds_doubles * sizeof(double));
     ProfScope ps(kTagQr, 0.0, s);
     hipLaunchKernelGGL(qr_kernel<Tab>, dim3(n_items), dim3(kQrThreads), lds, s, tab, lds_doubles);
     SYN_LAUNCH_CHECK("syn_qr_f64 launch");
@@ -324,4 +356,49 @@ extern "C" int syn_qr_sized_f64_host(const syn_qr_item *items, int n_items, int6
     if (n_items == 0) return SYN_OK;
     return launch_inline(items, n_items,
                          [&](const auto &tab) { return qr_launch(tab, n_items, lds_doubles, (hipStream_t)stream); });
+}
+
+// tables of many matrices, so from device memory only
+extern "C" int syn_qr_columns_f64(const syn_qr_item *items, int n_items, int64_t lds_doubles, void *stream) {
+    using namespace syn;
+    if (n_items < 0 || (n_items && !items) || lds_doubles < 0 || lds_doubles > kQrLdsDoubles) {
+        set_error("syn_qr_columns_f64: bad item count %d or LDS size %lld (at most %lld doubles)", n_items,
+                  (long long)lds_doubles, (long long)kQrLdsDoubles);
+        return SYN_EINVAL;
+    }
+    if (n_items == 0) return SYN_OK;
+    typedef DeviceTable<syn_qr_item> Tab;
+    static bool attr_set = false;
+    if (!attr_set) {
+        if (int rc = qr_lds(qr_columns_kernel<Tab>, (size_t)kQrLdsDoubles * sizeof(double),
+                            "syn_qr_columns_f64: hipFuncSetAttribute"))
+            return rc;
+        attr_set = true;
+    }
+    hipStream_t s = (hipStream_t)stream;
+    ProfScope ps(kTagQr, 0.0, s);
+    hipLaunchKernelGGL(qr_columns_kernel<Tab>, dim3(n_items), dim3(64 * kColWaves), (size_t)lds_doubles * sizeof(double),
+                       s, Tab{items}, lds_doubles);
+    SYN_LAUNCH_CHECK("syn_qr_columns_f64 launch");
+    return SYN_OK;
+}
+
+extern "C" int syn_qr_rows_f64(const syn_qr_item *items, int n_items, int64_t rows, void *stream) {
+    using namespace syn;
+    if (n_items < 0 || (n_items && !items) || rows < 1 || rows > 64) {
+        set_error("syn_qr_rows_f64: bad item count %d or rows %lld (at most 64)", n_items, (long long)rows);
+        return SYN_EINVAL;
+    }
+    if (n_items == 0) return SYN_OK;
+    typedef DeviceTable<syn_qr_item> Tab;
+    hipStream_t s = (hipStream_t)stream;
+    ProfScope ps(kTagQr, 0.0, s);
+    if (rows <= 16)
+        hipLaunchKernelGGL((qr_rows_kernel<1, Tab>), dim3(n_items), dim3(64), 0, s, Tab{items});
+    else if (rows <= 32)
+        hipLaunchKernelGGL((qr_rows_kernel<2, Tab>), dim3(n_items), dim3(128), 0, s, Tab{items});
+    else
+        hipLaunchKernelGGL((qr_rows_kernel<4, Tab>), dim3(n_items), dim3(256), 0, s, Tab{items});
+    SYN_LAUNCH_CHECK("syn_qr_rows_f64 launch");
+    return SYN_OK;
 }
