@@ -18,6 +18,11 @@ from .. import _lib, linalg, ops
 from ..tensor import MatrixProductOperator, MatrixProductState
 
 
+# bytes of equally shaped outputs of one site that share a buffer: an output
+# that a program keeps holds on to no more than this of the others'
+SHARED_BYTES = 1 << 21
+
+
 def _arena(sizes):
     """One float64 device tensor with a 256-byte aligned sub-buffer per size:
     (tensor, offsets in doubles, addresses)."""
@@ -27,9 +32,21 @@ def _arena(sizes):
     return t, off, np.uint64(t.data_ptr()) + (8 * off).astype(np.uint64)
 
 
+def _outputs(sizes):
+    """As _arena for buffers that are results; a list of tensors in place of
+    the one, with one a result, where they are too large to share."""
+    if 8 * int(sizes.sum()) <= SHARED_BYTES:
+        return _arena(sizes)
+    dev = ops.device()
+    ts = [torch.empty(int(v), dtype=torch.float64, device=dev) for v in sizes]
+    return ts, None, np.array([t.data_ptr() for t in ts], dtype=np.uint64)
+
+
 def _views(t, off, first, count, shape):
     """The tensors of `count` equally shaped neighbours of an arena."""
     l, d, r = (int(v) for v in shape)
+    if off is None:
+        return [v.view(l, d, r) for v in t[first:first + count]]
     step = (l * d * r + 31) // 32 * 32
     return t.as_strided((count, l, d, r), (step, d * r, r, 1), int(off[first])).unbind(0)
 
@@ -142,7 +159,8 @@ def matmul_batch(weight, states):
     rep = np.repeat(np.arange(len(keys)), count)
     hold = [[s.contiguous() for s in states[i].sites] for i in order]     # inputs, alive until the launch
     ws = [w.contiguous() for w in weight.sites]
-    cores = [_arena(P[rep, k].prod(axis=1)) for k in range(n)]
+    new = _arena if cut.all() else _outputs     # product cores that are results
+    cores = [new(P[rep, k].prod(axis=1)) for k in range(n)]
 
     # the tables, one after the other in one buffer
     J = len(order)
@@ -179,7 +197,8 @@ def matmul_batch(weight, states):
             m, r = rows[sel, k], P[sel, k, 2]
             cols = P[sel, k + 1, 1] * P[sel, k + 1, 2]
             nb = np.minimum(r, Dt)
-            Q, S, W = _arena(m * Dt), _arena(Dt * r), _arena(Dt * cols)
+            Q, S = _outputs(m * Dt), _arena(Dt * r)
+            W = (_outputs if k == n - 2 else _arena)(Dt * cols)
             work, tau = _arena(m * nb), _arena(nb)
             oq, it = take(qr, T)
             it["a"], it["rs"], it["cs"], it["m"], it["n"], it["keep"] = core, r, 1, m, r, Dt

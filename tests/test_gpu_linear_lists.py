@@ -36,3 +36,23 @@ def test_lengths(count, wbonds, xbonds, d):
         assert (y.shape, y.bond_shape, y.input_shape, y.parameters_number) == (
             z.shape, z.bond_shape, z.input_shape, z.parameters_number)
         assert all(torch.equal(a, b) for a, b in zip(y.sites, z.sites))
+
+
+@pytest.mark.parametrize("wbonds,xbonds", [((1, 8), (1, 400)), ((12, 12), (20, 20)), ((24, 24), (24, 24))])
+def test_a_kept_output_holds_little_else(wbonds, xbonds):
+    """Results that are product cores (a min bond of one is kept) and truncated
+    ones, small and large."""
+    import torch
+
+    from syngular_amd.core import matmul_batch
+    from syngular_amd.tensor import MatrixProductState
+
+    rng = np.random.default_rng(xbonds[1])
+    W = layer(rng, wbonds, 24)
+    xs = [MatrixProductState.from_sites(chain(rng, xbonds, 24)) for _ in range(24)]
+    ys = matmul_batch(W, xs)
+    alone = matmul_batch(W, xs[3:4])[0]
+    for a, b in zip(ys[3].sites, alone.sites):
+        assert torch.equal(a, b)
+        held = a.untyped_storage().nbytes()
+        assert held <= max(a.numel() * 8, 1 << 21)
