@@ -362,6 +362,16 @@ typedef struct {
 } syn_gbj_item;
 int syn_jacobi_gram_blocked_f64(syn_gbj_item *items, const syn_gbj_item *items_host, int n_items, double *work,
                                 int32_t *counters, double tol, int max_sweeps, int *sweeps, void *stream);
+/* The same with at most `polls` polls in each wait of a work-group for      */
+/* another (0: the bounds of syn_jacobi_gram_blocked_f64, a second or so).   */
+/* A matrix of order 257..2048 is first reduced by several work-groups that  */
+/* exchange their results; one that waits longer gives up, and the matrix    */
+/* takes the Jacobi sweeps from the start: right, but slower and with other  */
+/* rounding.  syn_jacobi_gram_gave_up: how many matrices of this process did. */
+int syn_jacobi_gram_blocked_polls_f64(syn_gbj_item *items, const syn_gbj_item *items_host, int n_items, double *work,
+                                      int32_t *counters, double tol, int max_sweeps, int polls, int *sweeps,
+                                      void *stream);
+int64_t syn_jacobi_gram_gave_up(void);
 int64_t syn_jacobi_gram_blocked_workspace(const int64_t *nv, int n_items);
 
 /* Batched copy: dst[0..n) = src[0..n) for every item (compaction). */

@@ -123,6 +123,9 @@ SIGNATURES = {
     "syn_cholqr_refine_f64": (_I32, [_VP, _I64, _I64, _I64, _VP, _I64, _VP, _I64, _VP, _D, _D, _VP,
                                      ctypes.POINTER(ctypes.c_int), _I32, _VP]),
     "syn_jacobi_gram_blocked_f64": (_I32, [_VP, _VP, _I32, _VP, _VP, _D, _I32, ctypes.POINTER(ctypes.c_int), _VP]),
+    "syn_jacobi_gram_blocked_polls_f64": (_I32, [_VP, _VP, _I32, _VP, _VP, _D, _I32, _I32, ctypes.POINTER(ctypes.c_int),
+                                                 _VP]),
+    "syn_jacobi_gram_gave_up": (_I64, []),
     "syn_jacobi_gram_blocked_workspace": (_I64, [_VP, _I32]),
     "syn_chol_leaf_f64": (_I32, [_VP, _I32, _VP]),
     "syn_prof_begin": (_I32, []),

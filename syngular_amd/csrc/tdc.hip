@@ -34,6 +34,7 @@
 #include "tdc.hpp"
 
 #include <algorithm>
+#include <mutex>
 
 namespace syn {
 
@@ -42,6 +43,7 @@ typedef double v2du __attribute__((ext_vector_type(2), aligned(8)));
 
 // Vector region of a problem (2048 * half >= 64 n doubles, tjacobi.hpp):
 // rows of n doubles, then the 32 x 32 T factors of the reflector blocks.
+constexpr int kGaveUp = 2;     // in Tdc::fail: a work-group waited too long for another
 struct Tdc {
     int n;
     int64_t ldg, ldr;
@@ -55,7 +57,7 @@ struct Tdc {
     int *rp;                   // row pairs of the rotations
     double *rcs;               // their cosines and sines
     double *rho;               // rank-one weight of a node (at its first row)
-    int *fail;                 // the direct phase does not apply to this matrix
+    int *fail;                 // the direct phase does not apply to this matrix, or gave up
     double *tf;                // T factors
 };
 
@@ -478,10 +480,18 @@ __global__ __launch_bounds__(64 * NB) void td_reduce_kernel(const syn_gbj_item *
 // published step j after it), and empties its own words of step j - 1's buffer
 // before it publishes step j + 1, so they are empty when anyone polls them for
 // step j + 2.  For that every work-group publishes in every step: the last S
-// columns, one of each, go on when their rows are dead.  Every wait is
-// bounded: past the limit (another work-group never got a compute unit) the
-// work-group gives up, the matrix counts as failed and the Jacobi sweeps take
-// it.
+// columns, one of each, go on when their rows are dead.
+//
+// A work-group can wait for one that has no compute unit yet only in its first
+// exchange: past it, all of the matrix are running and stay so.  SpinTurn keeps other
+// launches of this kernel from holding the units, and a launch's work-groups start
+// in order, so the first unfinished matrix always gets its units, and that first
+// wait lasts as long as the matrices ahead or another stream's kernels do.  Every wait is
+// bounded all the same, that one by kArrive polls and the others by kSpin: past
+// the limit the work-group gives up, the matrix counts as failed and the Jacobi
+// sweeps take it.  (One limit of kSpin for all waits and launches side by side:
+// 3 matrices of order 1500 in a call 50 ms, now 24; four streams of such calls at
+// once: 5 of 48 calls gave up, up to 230 ms each, now none, up to 81.)
 //
 // Order 2048 (128 work-groups) is bound by the exchange, 128 readers of every
 // word (3.0 of a step's 6.6 us; the vectors 1.5, the pass 0.8), the smaller
@@ -494,7 +504,8 @@ __global__ __launch_bounds__(64 * NB) void td_reduce_kernel(const syn_gbj_item *
 // 1024 and 2048 took 1.31, 2.16, 5.5 and 28.1 ms; now 1.01, 1.7, 4.6, 13.5.
 constexpr int kMultiThreads = 512;
 constexpr int kMultiWaves = kMultiThreads / 64;
-constexpr int kSpin = 1 << 14;   // polls of one step
+constexpr int kSpin = 1 << 14;    // polls of one step
+constexpr int kArrive = 1 << 19;  // polls of the first, a second or so
 constexpr unsigned kGroupedMax = 16;
 constexpr uint64_t kEmpty = ~(uint64_t)0;   // a NaN no operation makes
 
@@ -520,16 +531,17 @@ __host__ __device__ __forceinline__ int multi_groups(int64_t n) {
     return (int)((n + kMultiWaves * Q - 1) / (kMultiWaves * Q));
 }
 
-__global__ __launch_bounds__(256) void td_clear_kernel(const syn_gbj_item *__restrict__ items, int nlo, int nhi) {
+__global__ __launch_bounds__(256) void td_clear_kernel(const syn_gbj_item *__restrict__ items, int nlo, int nhi, int fail) {
     if (items[blockIdx.x].nv <= nlo || items[blockIdx.x].nv > nhi) return;
     const Tdc T = tdc_view(items[blockIdx.x]);
     for (int i = blockIdx.y * 256 + threadIdx.x; i < 6 * T.n; i += gridDim.y * 256) ((uint64_t *)T.x)[i] = kEmpty;
-    if (blockIdx.y == 0 && threadIdx.x == 0) *T.fail = 0;
+    if (blockIdx.y == 0 && threadIdx.x == 0) *T.fail = fail;
 }
 
 template <int P, int Q>
 __global__ __launch_bounds__(kMultiThreads) void td_reduce_multi_kernel(const syn_gbj_item *__restrict__ items,
-                                                                        int n_items, int nlo, int nhi, int S, int grouped) {
+                                                                        int n_items, int nlo, int nhi, int S, int grouped,
+                                                                        int arrive, int spin) {
     constexpr int N = 64 * P, NW = kMultiWaves, E = (N + kMultiThreads - 1) / kMultiThreads;
     __shared__ v2d vw[N];                         // v and w of the step before
     __shared__ double us[N], red[NW], red2[NW], sp, sd, sa;
@@ -590,7 +602,7 @@ __global__ __launch_bounds__(kMultiThreads) void td_reduce_multi_kernel(const sy
                 wp[e] = i < n && (i >= j || i >= tail) ? kEmpty : 0;
                 wc[e] = i < n && i >= j ? kEmpty : 0;
             }
-            for (int left = kSpin;;) {
+            for (int left = j == 1 ? arrive : spin;;) {
                 ok = true;
 #pragma unroll
                 for (int e = 0; e < E; ++e) {
@@ -600,7 +612,8 @@ __global__ __launch_bounds__(kMultiThreads) void td_reduce_multi_kernel(const sy
                 }
 #pragma unroll
                 for (int e = 0; e < E; ++e) ok = ok && wp[e] != kEmpty && wc[e] != kEmpty;
-                if (ok || --left == 0) break;
+                if (ok || --left <= 0) break;
+                if (j == 1) __builtin_amdgcn_s_sleep(8);
             }
 #pragma unroll
             for (int e = 0; e < E; ++e) {
@@ -618,7 +631,7 @@ __global__ __launch_bounds__(kMultiThreads) void td_reduce_multi_kernel(const sy
         if (lane == 0) red[wv] = s;
         lds_barrier();
         if (gone) {
-            if (tid == 0) *T.fail = 1;
+            if (tid == 0) *T.fail = kGaveUp;
             return;
         }
         // all have read step j - 1's words: the wave's own are empty again
@@ -720,9 +733,9 @@ __global__ __launch_bounds__(kMultiThreads) void td_reduce_multi_kernel(const sy
     // and w are zero)
     if (g == 0 && tid == 0) {
         uint64_t u = kEmpty;
-        for (int left = kSpin; u == kEmpty && left > 0; --left) u = peek(xword(T, buf, 1, n - 1));
+        for (int left = spin; u == kEmpty && left > 0; --left) u = peek(xword(T, buf, 1, n - 1));
         T.d[n - 1] = __builtin_bit_cast(double, u);
-        if (u == kEmpty) *T.fail = 1;
+        if (u == kEmpty) *T.fail = kGaveUp;
     }
 }
 
@@ -1010,8 +1023,8 @@ __global__ __launch_bounds__(256) void td_copy_kernel(const syn_gbj_item *__rest
 }
 
 // ---------------------------------------------------------------------------
-// Secular equation 1 + sum_i a_i / (d_i - lambda) = 0, a_i = rho z_i^2, one
-// four lanes per root, poles in LDS.  A root is kept as its distance tau to the
+// Secular equation 1 + sum_i a_i / (d_i - lambda) = 0, a_i = rho z_i^2, four
+// lanes per root, poles in LDS.  A root is kept as its distance tau to the
 // nearer pole (its origin), so d_i - lambda = (d_i - d_origin) - tau has no
 // cancellation.  Iteration: the rational interpolation through the two poles
 // around the root (Li 1993, the middle way), safeguarded by a bracket that
@@ -1460,6 +1473,7 @@ __global__ __launch_bounds__(256) void td_restore_kernel(const syn_gbj_item *__r
     __shared__ double s[32][33];
     const Tdc T = tdc_view(items[blockIdx.x]);
     const int n = T.n, nt = (n + 31) / 32;
+    if (blockIdx.y == 0 && threadIdx.x == 0 && *T.fail == kGaveUp) *items[blockIdx.x].counter = 1;   // in host memory
     int bi = 0, t = blockIdx.y;
     if (t >= nt * (nt + 1) / 2) return;
     while (t > bi) t -= ++bi;   // tile (bi, t), t <= bi
@@ -1479,6 +1493,8 @@ __global__ __launch_bounds__(256) void td_restore_kernel(const syn_gbj_item *__r
     }
 }
 
+constexpr int kSingleMax = 256;   // largest order that one work-group reduces
+
 // largest order of the class (nlo, nhi], 0 if it has none
 static int64_t class_max(const std::vector<syn_gbj_item> &host, int nlo, int nhi) {
     int64_t m = 0;
@@ -1495,20 +1511,136 @@ static int reduce_single(const syn_gbj_item *items, const std::vector<syn_gbj_it
     return SYN_OK;
 }
 
+// work-groups of a matrix, and the kernel's launch: how many one XCD gets, and
+// whether a whole matrix fits the device
+struct MultiPlan {
+    unsigned S = 0;
+    int grouped = 0;
+    bool fits = true, half = true;
+};
+
+// work-groups of the kernel that the device holds at a time
 template <int P, int Q>
-static int reduce_multi(const syn_gbj_item *items, const std::vector<syn_gbj_item> &host, int nlo, hipStream_t st) {
+static int64_t multi_slots() {
+    int dev = 0, cus = 0, per_cu = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, td_reduce_multi_kernel<P, Q>, kMultiThreads, 0) !=
+            hipSuccess)
+        return 0;
+    return (int64_t)cus * per_cu;
+}
+
+template <int P, int Q>
+static MultiPlan multi_plan(const std::vector<syn_gbj_item> &host, int nlo) {
+    MultiPlan m;
+    const int64_t nmax = class_max(host, nlo, 64 * P);
+    if (!nmax) return m;
+    m.S = (unsigned)multi_groups<Q>(nmax);
+    // up to 16 work-groups of a matrix on one XCD, more over all of them
+    m.grouped = m.S <= kGroupedMax;
+    static const int64_t slots = multi_slots<P, Q>();   // a process's devices are alike
+    int64_t xcd[kXcds] = {};
+    for (size_t i = 0; i < host.size(); ++i)
+        if (host[i].nv > nlo && host[i].nv <= 64 * P) {
+            if (m.grouped)
+                xcd[i & (kXcds - 1)] += m.S;
+            else
+                for (int64_t &x : xcd) x += (m.S + kXcds - 1) / kXcds;
+        }
+    m.fits = (int64_t)(m.grouped ? kXcds * m.S : m.S) <= slots;
+    m.half = 2 * kXcds * *std::max_element(xcd, xcd + kXcds) <= slots;
+    return m;
+}
+
+// Launches whose work-groups wait for each other, over all streams of a device:
+// side by side they could each hold units that the other waits for.  Two may run
+// at once if both take no more than half of the work-groups that fit an XCD (the
+// work-groups of one then always find units beside the other's); a larger one runs
+// alone.  A turn waits on the device for the one before it in its place (a larger
+// one for both) and ends with an event; the lock covers the enqueueing alone.
+class SpinTurn {
+  public:
+    SpinTurn(hipStream_t st, bool half) : lock_(mu()), st_(st) {
+        int dev = 0;
+        rc_ = hip_check(hipGetDevice(&dev), "direct phase device");
+        if (rc_) return;
+        auto &all = events();
+        if ((size_t)dev >= all.size()) all.resize((size_t)dev + 1);
+        Places &pl = all[dev];
+        int at = 0;
+        if (half) {
+            // the place that this stream had last, or the one taken longer ago
+            at = pl.last[0] == st ? 0 : pl.last[1] == st ? 1 : pl.next;
+            pl.last[at] = st;
+            pl.next = at ^ 1;
+        }
+        for (int i = 0; i < 2 && !rc_; ++i) {
+            if (half && i != at) continue;
+            hipEvent_t &ev = pl.ev[i];
+            if (ev)
+                rc_ = hip_check(hipStreamWaitEvent(st, ev, 0), "direct phase turn");
+            else
+                rc_ = hip_check(hipEventCreateWithFlags(&ev, hipEventDisableTiming), "direct phase event");
+            end_[i] = rc_ ? nullptr : ev;
+        }
+    }
+    int rc() const { return rc_; }
+    int end() {
+        int rc = SYN_OK;
+        for (hipEvent_t ev : end_)
+            if (ev && !rc) rc = hip_check(hipEventRecord(ev, st_), "direct phase turn");
+        return rc;
+    }
+
+  private:
+    struct Places {
+        hipEvent_t ev[2] = {nullptr, nullptr};
+        hipStream_t last[2] = {(hipStream_t)-1, (hipStream_t)-1};   // a hint, never used as a stream
+        int next = 0;
+    };
+    static std::mutex &mu() {
+        static std::mutex m;
+        return m;
+    }
+    static std::vector<Places> &events() {
+        static std::vector<Places> v;
+        return v;
+    }
+    std::lock_guard<std::mutex> lock_;
+    hipStream_t st_;
+    hipEvent_t end_[2] = {nullptr, nullptr};
+    int rc_ = 0;
+};
+
+template <int P, int Q>
+static int reduce_multi(const syn_gbj_item *items, const std::vector<syn_gbj_item> &host, int nlo, const MultiPlan &m,
+                        int polls, hipStream_t st) {
+    if (!m.S) return SYN_OK;
     const int nhi = 64 * P;
     const int64_t nmax = class_max(host, nlo, nhi);
-    if (!nmax) return SYN_OK;
-    const unsigned ni = (unsigned)host.size(), S = (unsigned)multi_groups<Q>(nmax);
-    hipLaunchKernelGGL(td_clear_kernel, dim3(ni, (unsigned)((6 * nmax + 255) / 256)), dim3(256), 0, st, items, nlo, nhi);
-    // up to 16 work-groups of a matrix on one XCD, more over all of them
-    const int grouped = S <= kGroupedMax;
-    const unsigned grid = (grouped ? (ni + 7) / 8 * 8 : ni) * S;
-    hipLaunchKernelGGL((td_reduce_multi_kernel<P, Q>), dim3(grid), dim3(kMultiThreads), 0, st, items, (int)ni, nlo, nhi,
-                       (int)S, grouped);
+    const unsigned ni = (unsigned)host.size();
+    hipLaunchKernelGGL(td_clear_kernel, dim3(ni, (unsigned)((6 * nmax + 255) / 256)), dim3(256), 0, st, items, nlo, nhi,
+                       m.fits ? 0 : 1);
+    if (m.fits) {
+        const unsigned grid = (m.grouped ? (ni + 7) / 8 * 8 : ni) * m.S;
+        hipLaunchKernelGGL((td_reduce_multi_kernel<P, Q>), dim3(grid), dim3(kMultiThreads), 0, st, items, (int)ni, nlo,
+                           nhi, (int)m.S, m.grouped, polls ? polls : kArrive, polls ? polls : kSpin);
+    }
     SYN_LAUNCH_CHECK("tridiagonal reduction over work-groups");
     return SYN_OK;
+}
+
+static int reduce_multis(const syn_gbj_item *items, const std::vector<syn_gbj_item> &host, int polls, hipStream_t st) {
+    const MultiPlan m8 = multi_plan<8, 4>(host, kSingleMax), m16 = multi_plan<16, 2>(host, 512),
+                    m32 = multi_plan<32, 2>(host, 1024);
+    SpinTurn turn(st, m8.half && m16.half && m32.half);
+    int rc = turn.rc();
+    if (!rc) rc = reduce_multi<8, 4>(items, host, kSingleMax, m8, polls, st);
+    if (!rc) rc = reduce_multi<16, 2>(items, host, 512, m16, polls, st);
+    if (!rc) rc = reduce_multi<32, 2>(items, host, 1024, m32, polls, st);
+    const int ended = turn.end();
+    return rc ? rc : ended;
 }
 
 // The products of a phase; up to 128 tiles as quadrants, the same bits (the
@@ -1523,8 +1655,9 @@ static void td_gemm(const syn_gbj_item *items, unsigned ni, unsigned tiles, unsi
 }
 
 bool tdc_takes(int64_t nv) { return nv >= kTdcMin && nv <= kTdcMax; }
+bool tdc_waits(int64_t nv) { return nv > kSingleMax && nv <= kTdcMax; }
 
-int tdc_launch(const syn_gbj_item *items, const std::vector<syn_gbj_item> &host, hipStream_t st) {
+int tdc_launch(const syn_gbj_item *items, const std::vector<syn_gbj_item> &host, int polls, hipStream_t st) {
     const unsigned ni = (unsigned)host.size();
     int64_t nmax = 0;
     int levels = 0, lmax = 1;
@@ -1538,9 +1671,8 @@ int tdc_launch(const syn_gbj_item *items, const std::vector<syn_gbj_item> &host,
     if (int rc = reduce_single<8>(items, host, 64, st)) return rc;
     if (int rc = reduce_single<12>(items, host, 128, st)) return rc;
     if (int rc = reduce_single<16>(items, host, 192, st)) return rc;
-    if (int rc = reduce_multi<8, 4>(items, host, 256, st)) return rc;
-    if (int rc = reduce_multi<16, 2>(items, host, 512, st)) return rc;
-    if (int rc = reduce_multi<32, 2>(items, host, 1024, st)) return rc;
+    if (tdc_waits(nmax))
+        if (int rc = reduce_multis(items, host, polls, st)) return rc;
     const unsigned nblk = (unsigned)refl_blocks((int)nmax);
     hipLaunchKernelGGL(td_tfac_kernel, dim3(ni, nblk), dim3(256), 0, st, items);
     hipLaunchKernelGGL(td_leaf_kernel, dim3(ni, (unsigned)lmax), dim3(64), 0, st, items);

@@ -35,6 +35,7 @@
 #include "tdc.hpp"
 
 #include <algorithm>
+#include <atomic>
 #include <cstring>
 #include <mutex>
 #include <vector>
@@ -996,23 +997,33 @@ class PinnedLease {
     int rc_ = 0;
 };
 
-// The direct phase (tdc.hip) of the problems it takes.
-static int gram_direct(syn_gbj_item *items, const syn_gbj_item *items_host, int n_items, double *work,
-                       const PinnedLease &pin, hipStream_t st) {
+// Matrices whose direct phase gave up waiting, of this process.
+static std::atomic<int64_t> gram_gave_up{0};
+
+// The direct phase (tdc.hip) of the problems it takes.  gave_up, in pinned
+// memory that the phase writes to, gets 1 for those that gave up waiting when one
+// of them can (returns through `waits`); it and the table's staging are the
+// caller's until its last wait on the stream.
+static int gram_direct(syn_gbj_item *items, const syn_gbj_item *items_host, int n_items, double *work, int polls,
+                       char *staging, int32_t *gave_up, bool &waits, hipStream_t st) {
     std::vector<syn_gbj_item> host;
     int64_t off = 0;
+    waits = false;
     for (int i = 0; i < n_items; ++i) {
+        gave_up[i] = 0;
         if (!tdc_takes(items_host[i].nv)) continue;
         host.push_back(items_host[i]);
         host.back().w = work + off;
+        host.back().counter = gave_up + i;
         off += tj_work<16>(host.back().nv);
+        waits = waits || tdc_waits(items_host[i].nv);
     }
     if (host.empty()) return SYN_OK;
     const size_t bytes = host.size() * sizeof(syn_gbj_item);
-    memcpy(pin.data(), host.data(), bytes);
-    if (int rc = hip_check(hipMemcpyAsync(items, pin.data(), bytes, hipMemcpyHostToDevice, st), "gram direct table"))
+    memcpy(staging, host.data(), bytes);
+    if (int rc = hip_check(hipMemcpyAsync(items, staging, bytes, hipMemcpyHostToDevice, st), "gram direct table"))
         return rc;
-    return tdc_launch(items, host, st);
+    return tdc_launch(items, host, polls, st);
 }
 
 template <int TB>
@@ -1242,8 +1253,16 @@ extern "C" int64_t syn_jacobi_gram_blocked_workspace(const int64_t *nv, int n_it
 extern "C" int syn_jacobi_gram_blocked_f64(syn_gbj_item *items, const syn_gbj_item *items_host, int n_items,
                                            double *work, int32_t *counters, double tol, int max_sweeps, int *sweeps,
                                            void *stream) {
+    return syn_jacobi_gram_blocked_polls_f64(items, items_host, n_items, work, counters, tol, max_sweeps, 0, sweeps, stream);
+}
+
+extern "C" int64_t syn_jacobi_gram_gave_up(void) { return syn::gram_gave_up.load(); }
+
+extern "C" int syn_jacobi_gram_blocked_polls_f64(syn_gbj_item *items, const syn_gbj_item *items_host, int n_items,
+                                                 double *work, int32_t *counters, double tol, int max_sweeps, int polls,
+                                                 int *sweeps, void *stream) {
     using namespace syn;
-    if (n_items < 0 || !items || (n_items && (!items_host || !work || !counters)) || max_sweeps < 0 ||
+    if (n_items < 0 || !items || (n_items && (!items_host || !work || !counters)) || max_sweeps < 0 || polls < 0 ||
         !(tol >= 0.0)) {
         set_error("syn_jacobi_gram_blocked_f64: bad arguments");
         return SYN_EINVAL;
@@ -1274,11 +1293,15 @@ extern "C" int syn_jacobi_gram_blocked_f64(syn_gbj_item *items, const syn_gbj_it
         wide.clear();
     }
     const bool direct = max_sweeps > 0;
-    // its table's staging is held until the sweeps' last wait on the stream
-    PinnedLease pin((size_t)n_items * sizeof(syn_gbj_item), (hipStream_t)stream);
+    // its staging is held until the sweeps' last wait on the stream
+    const size_t tbl = (size_t)n_items * sizeof(syn_gbj_item);
+    PinnedLease pin(tbl + (size_t)n_items * sizeof(int32_t), (hipStream_t)stream);
     if (pin.rc()) return pin.rc();
+    int32_t *gave_up = (int32_t *)(pin.data() + tbl);
+    bool waits = false;
     if (direct)
-        if (int rc = gram_direct(items, items_host, n_items, work, pin, (hipStream_t)stream)) return rc;
+        if (int rc = gram_direct(items, items_host, n_items, work, polls, pin.data(), gave_up, waits, (hipStream_t)stream))
+            return rc;
     int sw_w = 0, sw_n = 0;
     if (!wide.empty())
         if (int rc = gram_blocked<32>(items, wide, (int)wide.size(), work, counters, tol, max_sweeps, &sw_w,
@@ -1288,6 +1311,7 @@ extern "C" int syn_jacobi_gram_blocked_f64(syn_gbj_item *items, const syn_gbj_it
         if (int rc = gram_blocked<16>(items, narrow, (int)narrow.size(), work, counters, tol, max_sweeps, &sw_n,
                                       (hipStream_t)stream, direct))
             return rc;
+    if (waits) gram_gave_up += std::count(gave_up, gave_up + n_items, 1);
     if (sweeps) *sweeps = std::max(sw_w, sw_n);
     return SYN_OK;
 }

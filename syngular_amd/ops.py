@@ -960,3 +960,11 @@ def jacobi_gram_blocked(G, tol=None, max_sweeps=JACOBI_SWEEPS):
     call("syn_jacobi_gram_blocked_f64", _ptr(dev_items), it.ctypes.data_as(ctypes.c_void_p), 1, _ptr(work),
          _ptr(counters), float(tol), int(max_sweeps), ctypes.byref(sweeps), _stream())
     return rt, s, sweeps.value
+
+
+def gram_gave_up():
+    """How many matrices of this process left the direct phase of the blocked
+    Gram eigen-solver because one of their work-groups waited too long for
+    another: their results are right, but came from the Jacobi sweeps, slower
+    and with other rounding."""
+    return int(_lib.load().syn_jacobi_gram_gave_up())
