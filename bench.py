@@ -427,11 +427,13 @@ def chain_form(np, torch, args):
 # shared measurement helpers
 # --------------------------------------------------------------------------
 # Kernels bound by latency (serial rotation rounds in LDS, 64-column
-# Cholesky leaves, one-work-group factorisations): no flop or byte count
+# Cholesky leaves, one-work-group factorisations, the eigen-solver's
+# reduction step by step and its merges): no flop or byte count
 # describes them, so they get no roofline; bench.py names the largest of
 # them beside the roofline when it takes more GPU time than the dominant
 # work kernel.
-LATENCY_KERNELS = ("chol_diag_kernel", "jacobi_kernel", "qr_kernel", "bjacobi_step_kernel")
+LATENCY_KERNELS = ("chol_diag_kernel", "jacobi_kernel", "qr_kernel", "bjacobi_step_kernel", "td_reduce_kernel",
+                   "td_merge_kernels")
 # work figures recorded without launches of their own: the bytes the fused
 # Jacobi step's update work-groups move (counted on the device in the census
 # step only, where every kernel is timed)
@@ -481,7 +483,7 @@ def kernel_roofline(census, timed, dom, steps, traffic_file):
             roof["largest_kernel_by_time"] = {"kernel": lk, "share_of_gpu_time": round(lms / total_ms, 3),
                                               "launches_per_step": ll,
                                               "avg_launch_us": round(1e3 * lms / ll, 2),
-                                              "bound": "latency (serial rounds in LDS; no flop/byte roofline)"}
+                                              "bound": "latency (serial steps; no flop/byte roofline)"}
     return roof
 
 

@@ -558,7 +558,7 @@ int syn_chol_leaf_f64_host(const syn_chol_item *items, int n_items, void *stream
 /* (all by default; kept until changed): two event packets per launch    */
 /* slow a stream of short kernels down by microseconds each.             */
 /* ------------------------------------------------------------------ */
-#define SYN_PROF_NTAGS 20
+#define SYN_PROF_NTAGS 24
 int syn_prof_begin(void);
 int syn_prof_select(uint32_t mask);
 int syn_prof_note_flops(double flops);

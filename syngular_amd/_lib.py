@@ -146,7 +146,7 @@ SIGNATURES.update({host: SIGNATURES[name] for name, host in HOST_ENTRIES.items()
 INLINE_ITEMS = frozenset([GEMM_ITEM, APPLY_ITEM, ROWSCALE_ITEM, EYE_ITEM, COPY_ITEM, VECNORM_ITEM, QR_ITEM, JACOBI_ITEM,
                           TRUNC_ITEM, DIAGMAX_ITEM, CHOL_ITEM])
 
-PROF_NTAGS = 20
+PROF_NTAGS = 24
 PROF_TAGS = {
     0: "gemm_f64_single<64,64>",
     1: "gemm_f64_single<128,128>",
@@ -168,6 +168,10 @@ PROF_TAGS = {
     17: "chol_node_kernel",
     18: "gemm_bf16<64,64>",
     19: "gemm_bf16<128,128>",
+    20: "td_reduce_kernel",
+    21: "td_merge_kernels",
+    22: "td_back_kernel",
+    23: "td_gemm_kernel",
 }
 
 

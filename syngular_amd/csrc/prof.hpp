@@ -26,6 +26,11 @@ enum ProfTag {
     kTagCholNode = 17,
     kTagGemmBf1664 = 18,
     kTagGemmBf16128 = 19,
+    // the direct phase of the Gram eigen-solver (tdc.hip), a scope for each part
+    kTagTdReduce = 20,     // tridiagonal reduction
+    kTagTdMerge = 21,      // leaves and merges of the divide and conquer, with their products
+    kTagTdBack = 22,       // T factors and back-transformation
+    kTagTdGemm = 23,       // the two products that diagonalise G
 };
 
 bool prof_on();

@@ -1667,15 +1667,24 @@ int tdc_launch(const syn_gbj_item *items, const std::vector<syn_gbj_item> &host,
         lmax = std::max(lmax, L);
     }
     while ((1 << levels) < lmax) ++levels;
-    if (int rc = reduce_single<4>(items, host, 0, st)) return rc;
-    if (int rc = reduce_single<8>(items, host, 64, st)) return rc;
-    if (int rc = reduce_single<12>(items, host, 128, st)) return rc;
-    if (int rc = reduce_single<16>(items, host, 192, st)) return rc;
-    if (tdc_waits(nmax))
-        if (int rc = reduce_multis(items, host, polls, st)) return rc;
+    {
+        ProfScope ps(kTagTdReduce, 0.0, st);
+        if (int rc = reduce_single<4>(items, host, 0, st)) return rc;
+        if (int rc = reduce_single<8>(items, host, 64, st)) return rc;
+        if (int rc = reduce_single<12>(items, host, 128, st)) return rc;
+        if (int rc = reduce_single<16>(items, host, 192, st)) return rc;
+        if (tdc_waits(nmax))
+            if (int rc = reduce_multis(items, host, polls, st)) return rc;
+    }
     const unsigned nblk = (unsigned)refl_blocks((int)nmax);
-    hipLaunchKernelGGL(td_tfac_kernel, dim3(ni, nblk), dim3(256), 0, st, items);
-    hipLaunchKernelGGL(td_leaf_kernel, dim3(ni, (unsigned)lmax), dim3(64), 0, st, items);
+    {
+        ProfScope ps(kTagTdBack, 0.0, st);
+        hipLaunchKernelGGL(td_tfac_kernel, dim3(ni, nblk), dim3(256), 0, st, items);
+    }
+    {
+        ProfScope ps(kTagTdMerge, 0.0, st);
+        hipLaunchKernelGGL(td_leaf_kernel, dim3(ni, (unsigned)lmax), dim3(64), 0, st, items);
+    }
     for (int l = 1; l <= levels; ++l) {
         // the largest node of the level and how many the largest problem has
         int64_t k = 0;
@@ -1684,6 +1693,7 @@ int tdc_launch(const syn_gbj_item *items, const std::vector<syn_gbj_item> &host,
             if ((L >> l) > 0) k = std::max(k, ((it.nv << l) + L - 1) / L);
         }
         const unsigned nodes = (unsigned)(lmax >> l), c64 = (unsigned)((k + 63) / 64);
+        ProfScope ps(kTagTdMerge, 0.0, st);
         const size_t plds = (size_t)prep_lds(k) * sizeof(double), slds = (size_t)k * 2 * sizeof(double);
         hipLaunchKernelGGL(td_prep_kernel, dim3(ni, nodes), dim3(kPrepThreads), plds, st, items, l);
         hipLaunchKernelGGL(td_copy_kernel, dim3(ni, c64, nodes), dim3(256), 0, st, items, l);
@@ -1694,13 +1704,22 @@ int tdc_launch(const syn_gbj_item *items, const std::vector<syn_gbj_item> &host,
         SYN_LAUNCH_CHECK("divide and conquer");
     }
     const unsigned t32 = (unsigned)((nmax + 31) / 32), t64 = (unsigned)((nmax + 63) / 64);
-    if ((int64_t)ni * t32 <= kBackFew)
-        hipLaunchKernelGGL((td_back_kernel<1, 8>), dim3(ni, (unsigned)((nmax + 15) / 16)), dim3(512), 0, st, items);
-    else
-        hipLaunchKernelGGL((td_back_kernel<2, 4>), dim3(ni, t32), dim3(256), 0, st, items);
+    double n3 = 0.0;
+    for (const syn_gbj_item &it : host) n3 += (double)it.nv * it.nv * it.nv;
+    {
+        // every reflector meets the columns right of it twice: 2 n^3
+        ProfScope ps(kTagTdBack, 2.0 * n3, st);
+        if ((int64_t)ni * t32 <= kBackFew)
+            hipLaunchKernelGGL((td_back_kernel<1, 8>), dim3(ni, (unsigned)((nmax + 15) / 16)), dim3(512), 0, st, items);
+        else
+            hipLaunchKernelGGL((td_back_kernel<2, 4>), dim3(ni, t32), dim3(256), 0, st, items);
+    }
     hipLaunchKernelGGL(td_restore_kernel, dim3(ni, t32 * (t32 + 1) / 2), dim3(256), 0, st, items);
-    td_gemm(items, ni, t64 * t64, 1, 1, 0, st);
-    td_gemm(items, ni, t64 * t64, 1, 2, 0, st);
+    {
+        ProfScope ps(kTagTdGemm, 4.0 * n3, st);
+        td_gemm(items, ni, t64 * t64, 1, 1, 0, st);
+        td_gemm(items, ni, t64 * t64, 1, 2, 0, st);
+    }
     SYN_LAUNCH_CHECK("direct phase");
     return SYN_OK;
 }
