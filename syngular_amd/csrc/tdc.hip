@@ -31,6 +31,7 @@
 #include "gemm_tile.hpp"
 #include "hh_tile.hpp"
 #include "prof.hpp"
+#include "rotation.hpp"
 #include "tdc.hpp"
 
 #include <algorithm>
@@ -43,7 +44,9 @@ typedef double v2du __attribute__((ext_vector_type(2), aligned(8)));
 
 // Vector region of a problem (2048 * half >= 64 n doubles, tjacobi.hpp):
 // rows of n doubles, then the 32 x 32 T factors of the reflector blocks.
-constexpr int kGaveUp = 2;     // in Tdc::fail: a work-group waited too long for another
+// in Tdc::fail, beside 0 and 1: a work-group waited too long for another; no
+// entry of the matrix passes the rotation test
+constexpr int kGaveUp = 2, kDiagonal = 3;
 struct Tdc {
     int n;
     int64_t ldg, ldr;
@@ -57,7 +60,7 @@ struct Tdc {
     int *rp;                   // row pairs of the rotations
     double *rcs;               // their cosines and sines
     double *rho;               // rank-one weight of a node (at its first row)
-    int *fail;                 // the direct phase does not apply to this matrix, or gave up
+    int *fail;                 // not 0: the direct phase does not apply to this matrix
     double *tf;                // T factors
 };
 
@@ -182,6 +185,14 @@ __device__ __forceinline__ double gram_scale(const Tdc &T) {
     return bad != 0.0 || !(mx > 1e-280) ? 0.0 : ldexp(1.0, -ilogb(mx));
 }
 
+// largest of n entries, in every lane of a wave
+__device__ __forceinline__ double gram_top(const double *d, int n) {
+    double mx = 0.0;
+    for (int i = threadIdx.x & 63; i < n; i += 64) mx = fmax(mx, fabs(d[i]));
+    for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off, 64));
+    return mx;
+}
+
 // Orders up to 16 NB, one work-group of NB waves per matrix.  The matrix is
 // symmetric: of its NB x NB tiles of 16 x 16, wave I keeps the diagonal one,
 // those an even distance left of it and those an odd distance right of it, so
@@ -255,7 +266,8 @@ __device__ __forceinline__ double row_sum4(double s0, double s1, double s2, doub
 }
 
 template <int NB>
-__global__ __launch_bounds__(64 * NB) void td_reduce_kernel(const syn_gbj_item *__restrict__ items, int nlo, int nhi) {
+__global__ __launch_bounds__(64 * NB) void td_reduce_kernel(const syn_gbj_item *__restrict__ items, int nlo, int nhi,
+                                                              double tol) {
     typedef TdTiles<NB> Tl;
     constexpr int N = 16 * NB, KT = Tl::KT, KS = Tl::KS, KG = Tl::KG, E = N / 64;
     __shared__ v2d vw[N + 16];                  // v and w of the step before
@@ -268,6 +280,7 @@ __global__ __launch_bounds__(64 * NB) void td_reduce_kernel(const syn_gbj_item *
     const double sc = gram_scale(T);
     if (tid == 0) *T.fail = sc == 0.0;
     if (sc == 0.0) return;
+    for (int i = tid; i < N; i += 64 * NB) rowp[i] = i < n ? T.g[i * T.ldg + i] * sc : 0.0;
     double a[KT][4];
 #pragma unroll
     for (int k = 0; k < KT; ++k) {
@@ -277,6 +290,23 @@ __global__ __launch_bounds__(64 * NB) void td_reduce_kernel(const syn_gbj_item *
             const int i = 16 * I + lk + 4 * r, c = 16 * J + li;
             a[k][r] = (J < NB && i < n && c < n) ? T.g[i * T.ldg + c] * sc : 0.0;
         }
+    }
+    // nothing to rotate: the matrix stays as it is (below)
+    __syncthreads();
+    const double floor_abs = __DBL_EPSILON__ * gram_top(rowp, N);
+    bool hit = false;
+#pragma unroll
+    for (int k = 0; k < KT; ++k) {
+        const int J = Tl::block(I, k);
+        if (J >= NB) continue;
+        const double dc = rowp[16 * J + li];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            hit = hit || ((k > 0 || lk + 4 * r != li) && rotates(a[k][r], rowp[16 * I + lk + 4 * r], dc, tol, floor_abs));
+    }
+    if (!__syncthreads_or(hit)) {
+        if (tid == 0) *T.fail = kDiagonal;
+        return;
     }
     for (int i = tid; i < N + 16; i += 64 * NB) {
         vw[i] = v2d{0.0, 0.0};
@@ -532,10 +562,33 @@ __host__ __device__ __forceinline__ int multi_groups(int64_t n) {
 }
 
 __global__ __launch_bounds__(256) void td_clear_kernel(const syn_gbj_item *__restrict__ items, int nlo, int nhi, int fail) {
+    // fail: kDiagonal until td_test_kernel finds an entry to rotate
     if (items[blockIdx.x].nv <= nlo || items[blockIdx.x].nv > nhi) return;
     const Tdc T = tdc_view(items[blockIdx.x]);
     for (int i = blockIdx.y * 256 + threadIdx.x; i < 6 * T.n; i += gridDim.y * 256) ((uint64_t *)T.x)[i] = kEmpty;
     if (blockIdx.y == 0 && threadIdx.x == 0) *T.fail = fail;
+}
+
+// The rotation test of the sweeps (tj_check_kernel), rows dealt to grid.y.  A
+// matrix without an entry to rotate, as at a bond that no gate has touched, is left
+// to them as it is: through the whole phase one of order 130 took 538 us and one of
+// 300 1463, by the sweeps alone 184 and 338, and with this test 215 and 252.  (The
+// reductions in one work-group test their registers, for about a microsecond.)
+__global__ __launch_bounds__(256) void td_test_kernel(const syn_gbj_item *__restrict__ items, int nlo, int nhi, double tol) {
+    __shared__ double d[kTdcMax];
+    if (items[blockIdx.x].nv <= nlo || items[blockIdx.x].nv > nhi) return;
+    const Tdc T = tdc_view(items[blockIdx.x]);
+    const int n = T.n;
+    for (int i = threadIdx.x; i < n; i += 256) d[i] = T.g[i * T.ldg + i];
+    __syncthreads();
+    const double floor_abs = __DBL_EPSILON__ * gram_top(d, n);
+    for (int i = blockIdx.y; i < n; i += gridDim.y) {
+        bool hit = false;
+        for (int k = threadIdx.x; k < n; k += 256)
+            hit = hit || (i != k && rotates_any(T.g[i * T.ldg + k], d[i], d[k], tol, floor_abs));
+        if (hit) *T.fail = 0;
+        if (__syncthreads_or(hit)) return;
+    }
 }
 
 template <int P, int Q>
@@ -556,6 +609,7 @@ __global__ __launch_bounds__(kMultiThreads) void td_reduce_multi_kernel(const sy
     const int n = T.n;
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int tail = n - S;   // the columns that are published to the end
+    if (*T.fail == kDiagonal) return;
     const double sc = gram_scale(T);
     if (sc == 0.0) {
         if (g == 0 && tid == 0) *T.fail = 1;
@@ -1477,15 +1531,17 @@ __global__ __launch_bounds__(256) void td_restore_kernel(const syn_gbj_item *__r
     int bi = 0, t = blockIdx.y;
     if (t >= nt * (nt + 1) / 2) return;
     while (t > bi) t -= ++bi;   // tile (bi, t), t <= bi
-    const int r0 = 32 * bi, c0 = 32 * t, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-    for (int i = ty; i < 32; i += 8)
-        s[i][tx] = (r0 + i < n && c0 + tx < n) ? T.g[(int64_t)(r0 + i) * T.ldg + c0 + tx] : 0.0;
-    __syncthreads();
-    for (int i = ty; i < 32; i += 8) {
-        const int r = c0 + i, c = r0 + tx;
-        if (r < n && c < n && c > r) T.g[(int64_t)r * T.ldg + c] = s[tx][i];
+    const int r0 = 32 * bi, c0 = 32 * t, tx = threadIdx.x & 31, ty = threadIdx.x >> 5, fail = *T.fail;
+    if (fail != kDiagonal) {
+        for (int i = ty; i < 32; i += 8)
+            s[i][tx] = (r0 + i < n && c0 + tx < n) ? T.g[(int64_t)(r0 + i) * T.ldg + c0 + tx] : 0.0;
+        __syncthreads();
+        for (int i = ty; i < 32; i += 8) {
+            const int r = c0 + i, c = r0 + tx;
+            if (r < n && c < n && c > r) T.g[(int64_t)r * T.ldg + c] = s[tx][i];
+        }
     }
-    if (*T.fail) {
+    if (fail) {
         for (int i = ty; i < 32; i += 8) {
             if (r0 + i < n && c0 + tx < n) T.rt[(int64_t)(r0 + i) * T.ldr + c0 + tx] = (r0 + i == c0 + tx) ? 1.0 : 0.0;
             if (c0 + i < n && r0 + tx < n) T.rt[(int64_t)(c0 + i) * T.ldr + r0 + tx] = (c0 + i == r0 + tx) ? 1.0 : 0.0;
@@ -1504,9 +1560,10 @@ static int64_t class_max(const std::vector<syn_gbj_item> &host, int nlo, int nhi
 }
 
 template <int NB>
-static int reduce_single(const syn_gbj_item *items, const std::vector<syn_gbj_item> &host, int nlo, hipStream_t st) {
+static int reduce_single(const syn_gbj_item *items, const std::vector<syn_gbj_item> &host, int nlo, double tol, hipStream_t st) {
     if (!class_max(host, nlo, 16 * NB)) return SYN_OK;
-    hipLaunchKernelGGL(td_reduce_kernel<NB>, dim3((unsigned)host.size()), dim3(64 * NB), 0, st, items, nlo, 16 * NB);
+    hipLaunchKernelGGL(td_reduce_kernel<NB>, dim3((unsigned)host.size()), dim3(64 * NB), 0, st, items, nlo, 16 * NB,
+                       tol);
     SYN_LAUNCH_CHECK("tridiagonal reduction");
     return SYN_OK;
 }
@@ -1615,14 +1672,15 @@ class SpinTurn {
 
 template <int P, int Q>
 static int reduce_multi(const syn_gbj_item *items, const std::vector<syn_gbj_item> &host, int nlo, const MultiPlan &m,
-                        int polls, hipStream_t st) {
+                        int polls, double tol, hipStream_t st) {
     if (!m.S) return SYN_OK;
     const int nhi = 64 * P;
     const int64_t nmax = class_max(host, nlo, nhi);
     const unsigned ni = (unsigned)host.size();
     hipLaunchKernelGGL(td_clear_kernel, dim3(ni, (unsigned)((6 * nmax + 255) / 256)), dim3(256), 0, st, items, nlo, nhi,
-                       m.fits ? 0 : 1);
+                       m.fits ? kDiagonal : 1);
     if (m.fits) {
+        hipLaunchKernelGGL(td_test_kernel, dim3(ni, 64), dim3(256), 0, st, items, nlo, nhi, tol);
         const unsigned grid = (m.grouped ? (ni + 7) / 8 * 8 : ni) * m.S;
         hipLaunchKernelGGL((td_reduce_multi_kernel<P, Q>), dim3(grid), dim3(kMultiThreads), 0, st, items, (int)ni, nlo,
                            nhi, (int)m.S, m.grouped, polls ? polls : kArrive, polls ? polls : kSpin);
@@ -1631,14 +1689,15 @@ static int reduce_multi(const syn_gbj_item *items, const std::vector<syn_gbj_ite
     return SYN_OK;
 }
 
-static int reduce_multis(const syn_gbj_item *items, const std::vector<syn_gbj_item> &host, int polls, hipStream_t st) {
+static int reduce_multis(const syn_gbj_item *items, const std::vector<syn_gbj_item> &host, int polls, double tol,
+                         hipStream_t st) {
     const MultiPlan m8 = multi_plan<8, 4>(host, kSingleMax), m16 = multi_plan<16, 2>(host, 512),
                     m32 = multi_plan<32, 2>(host, 1024);
     SpinTurn turn(st, m8.half && m16.half && m32.half);
     int rc = turn.rc();
-    if (!rc) rc = reduce_multi<8, 4>(items, host, kSingleMax, m8, polls, st);
-    if (!rc) rc = reduce_multi<16, 2>(items, host, 512, m16, polls, st);
-    if (!rc) rc = reduce_multi<32, 2>(items, host, 1024, m32, polls, st);
+    if (!rc) rc = reduce_multi<8, 4>(items, host, kSingleMax, m8, polls, tol, st);
+    if (!rc) rc = reduce_multi<16, 2>(items, host, 512, m16, polls, tol, st);
+    if (!rc) rc = reduce_multi<32, 2>(items, host, 1024, m32, polls, tol, st);
     const int ended = turn.end();
     return rc ? rc : ended;
 }
@@ -1657,7 +1716,7 @@ static void td_gemm(const syn_gbj_item *items, unsigned ni, unsigned tiles, unsi
 bool tdc_takes(int64_t nv) { return nv >= kTdcMin && nv <= kTdcMax; }
 bool tdc_waits(int64_t nv) { return nv > kSingleMax && nv <= kTdcMax; }
 
-int tdc_launch(const syn_gbj_item *items, const std::vector<syn_gbj_item> &host, int polls, hipStream_t st) {
+int tdc_launch(const syn_gbj_item *items, const std::vector<syn_gbj_item> &host, int polls, double tol, hipStream_t st) {
     const unsigned ni = (unsigned)host.size();
     int64_t nmax = 0;
     int levels = 0, lmax = 1;
@@ -1669,12 +1728,12 @@ int tdc_launch(const syn_gbj_item *items, const std::vector<syn_gbj_item> &host,
     while ((1 << levels) < lmax) ++levels;
     {
         ProfScope ps(kTagTdReduce, 0.0, st);
-        if (int rc = reduce_single<4>(items, host, 0, st)) return rc;
-        if (int rc = reduce_single<8>(items, host, 64, st)) return rc;
-        if (int rc = reduce_single<12>(items, host, 128, st)) return rc;
-        if (int rc = reduce_single<16>(items, host, 192, st)) return rc;
+        if (int rc = reduce_single<4>(items, host, 0, tol, st)) return rc;
+        if (int rc = reduce_single<8>(items, host, 64, tol, st)) return rc;
+        if (int rc = reduce_single<12>(items, host, 128, tol, st)) return rc;
+        if (int rc = reduce_single<16>(items, host, 192, tol, st)) return rc;
         if (tdc_waits(nmax))
-            if (int rc = reduce_multis(items, host, polls, st)) return rc;
+            if (int rc = reduce_multis(items, host, polls, tol, st)) return rc;
     }
     const unsigned nblk = (unsigned)refl_blocks((int)nmax);
     {

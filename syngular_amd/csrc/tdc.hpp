@@ -18,8 +18,10 @@ bool tdc_waits(int64_t nv);
 // tj_work<16>(nv) doubles and counter to an entry each, cleared.  polls bounds
 // every wait of a work-group for another (0: the phase's own bounds).  On return
 // (stream order) g is rt g rt^T and rt the eigenvector rows, or g as it was and rt
-// the identity for a matrix the phase cannot take (zero, not finite, far out of
-// range) or whose reduction gave up waiting; counter is set to 1 for the latter.
-int tdc_launch(const syn_gbj_item *items, const std::vector<syn_gbj_item> &host, int polls, hipStream_t st);
+// the identity for a matrix with no entry that passes the sweeps' rotation test
+// (threshold tol), one that the phase cannot take (zero, not finite, far out of
+// range) or whose reduction gave up waiting; counter is set to 1 for the last.
+int tdc_launch(const syn_gbj_item *items, const std::vector<syn_gbj_item> &host, int polls, double tol,
+               hipStream_t st);
 
 }  // namespace syn

@@ -1005,7 +1005,7 @@ static std::atomic<int64_t> gram_gave_up{0};
 // of them can (returns through `waits`); it and the table's staging are the
 // caller's until its last wait on the stream.
 static int gram_direct(syn_gbj_item *items, const syn_gbj_item *items_host, int n_items, double *work, int polls,
-                       char *staging, int32_t *gave_up, bool &waits, hipStream_t st) {
+                       double tol, char *staging, int32_t *gave_up, bool &waits, hipStream_t st) {
     std::vector<syn_gbj_item> host;
     int64_t off = 0;
     waits = false;
@@ -1023,7 +1023,7 @@ static int gram_direct(syn_gbj_item *items, const syn_gbj_item *items_host, int 
     memcpy(staging, host.data(), bytes);
     if (int rc = hip_check(hipMemcpyAsync(items, staging, bytes, hipMemcpyHostToDevice, st), "gram direct table"))
         return rc;
-    return tdc_launch(items, host, polls, st);
+    return tdc_launch(items, host, polls, tol, st);
 }
 
 template <int TB>
@@ -1300,7 +1300,7 @@ extern "C" int syn_jacobi_gram_blocked_polls_f64(syn_gbj_item *items, const syn_
     int32_t *gave_up = (int32_t *)(pin.data() + tbl);
     bool waits = false;
     if (direct)
-        if (int rc = gram_direct(items, items_host, n_items, work, polls, pin.data(), gave_up, waits, (hipStream_t)stream))
+        if (int rc = gram_direct(items, items_host, n_items, work, polls, tol, pin.data(), gave_up, waits, (hipStream_t)stream))
             return rc;
     int sw_w = 0, sw_n = 0;
     if (!wide.empty())
