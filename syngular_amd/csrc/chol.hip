@@ -296,9 +296,9 @@ __global__ __launch_bounds__(kCholThreads) void chol_diag_kernel(const double *G
 
 // One leaf (n <= 64) per work-group, for many problems at once.
 template <typename Tab>
-__global__ __launch_bounds__(kCholThreads) void chol_leaf_many_kernel(Tab tab) {
+__global__ __launch_bounds__(kCholThreads) void chol_leaf_many_kernel(KernelTable<Tab> tab) {
     __shared__ double a[kNb][kNb + 1], lo[kNb][kNb + 1];
-    const syn_chol_item &P = tab.get()[blockIdx.x];
+    const syn_chol_item &P = items_of(tab)[blockIdx.x];
     chol_diag_body<kCholTG>(P.g, P.ldg, P.l, P.ldl, P.n, 0, P.x, P.ldx, P.maxdiag, P.tolrel, P.dropped, a, lo);
 }
 
@@ -398,8 +398,8 @@ __global__ __launch_bounds__(kCholThreads) void chol_node_kernel(double *G, int6
 }
 
 template <typename Tab>
-__global__ __launch_bounds__(256) void diagmax_many_kernel(Tab tab) {
-    const syn_diagmax_item &P = tab.get()[blockIdx.x];
+__global__ __launch_bounds__(256) void diagmax_many_kernel(KernelTable<Tab> tab) {
+    const syn_diagmax_item &P = items_of(tab)[blockIdx.x];
     __shared__ double red[4];
     double m = 0.0;
     for (int64_t i = threadIdx.x; i < P.n; i += 256) m = fmax(m, P.g[i * P.ld + i]);

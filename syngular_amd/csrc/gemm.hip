@@ -26,8 +26,8 @@ __device__ __forceinline__ int64_t tile_of_block(int64_t bid, int64_t total, int
 }
 
 template <int BM, int BN, int BK, int WM, int WN, typename CT, typename Tab>
-__global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, 2) void gemm_f64_grouped(Tab tab, int n_items, int64_t total) {
-    const syn_gemm_item *__restrict__ items = tab.get();
+__global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, 2) void gemm_f64_grouped(KernelTable<Tab> tab, int n_items, int64_t total) {
+    const syn_gemm_item *__restrict__ items = items_of(tab);
     if (n_items == 1) {
         gemm_f64_tile<BM, BN, BK, WM, WN, CT>(items[0],
                                               tile_of_block(blockIdx.x, total, items[0].tiles_n, items[0].tri));
@@ -85,8 +85,8 @@ constexpr int kQuadK = 32;
 constexpr int64_t kQuadMax = 128;
 
 template <typename CT, typename Tab>
-__global__ __launch_bounds__(256, 2) void gemm_quad_grouped(Tab tab, int n_items, int64_t total) {
-    const syn_gemm_item *__restrict__ items = tab.get();
+__global__ __launch_bounds__(256, 2) void gemm_quad_grouped(KernelTable<Tab> tab, int n_items, int64_t total) {
+    const syn_gemm_item *__restrict__ items = items_of(tab);
     const int64_t b = xcd_remap(blockIdx.x, 4 * total), t = b >> 2;
     const syn_gemm_item &P = items[find_item(items, n_items, t)];
     gemm_f64_quad<kQuadK, CT>(P, t - P.block_start, (int)(b & 3));
@@ -329,10 +329,10 @@ static int launch_grouped(Tab tab, int n_items, int64_t total, int tile, hipStre
     if constexpr (kDevice) {
         if (pers && tile == 0)
             hipLaunchKernelGGL((gemm_f64_grouped_persistent<64, 64, 16, 32, 32, CT>), dim3(grid), dim3(256), 0, s,
-                               tab.p, n_items, total);
+                               tab, n_items, total);
         else if (pers)
             hipLaunchKernelGGL((gemm_f64_grouped_persistent<128, 128, 16, 64, 64, CT>), dim3(grid), dim3(256), 0, s,
-                               tab.p, n_items, total);
+                               tab, n_items, total);
     }
     if (!pers && !quad) {
         if (tile == 0)

@@ -177,9 +177,9 @@ __device__ void jacobi_one(const syn_jacobi_item &P, double *lds, double tol, in
 }
 
 template <typename Tab>
-__global__ __launch_bounds__(kJacThreads) void jacobi_kernel(Tab tab, double tol, int max_sweeps) {
+__global__ __launch_bounds__(kJacThreads) void jacobi_kernel(KernelTable<Tab> tab, double tol, int max_sweeps) {
     extern __shared__ double lds[];
-    const syn_jacobi_item &P = tab.get()[blockIdx.x];
+    const syn_jacobi_item &P = items_of(tab)[blockIdx.x];
     if (P.nv * P.len + P.nv * P.nv <= kJacLdsDoubles)
         jacobi_one<true>(P, lds, tol, max_sweeps);
     else
@@ -208,13 +208,13 @@ constexpr int kGramThreads = 256;
 constexpr int kGramMax = 64;
 
 template <int NT, typename Tab>
-__global__ __launch_bounds__(NT) void jacobi_gram_kernel(Tab tab, int nv_max, double tol, int max_sweeps) {
+__global__ __launch_bounds__(NT) void jacobi_gram_kernel(KernelTable<Tab> tab, int nv_max, double tol, int max_sweeps) {
     extern __shared__ double lds[];
     __shared__ double cs[kGramMax / 2][2];
     __shared__ int pp[kGramMax / 2], qq[kGramMax / 2];
     __shared__ int rank[kGramMax];
     __shared__ int rotated;
-    const syn_jacobi_item &P = tab.get()[blockIdx.x];
+    const syn_jacobi_item &P = items_of(tab)[blockIdx.x];
     const int tid = threadIdx.x;
     if (P.nv < 1 || P.nv > nv_max || P.len != P.nv) {
         // not a problem this kernel takes: flag it in s and leave the rest
@@ -375,12 +375,12 @@ __device__ __forceinline__ double from_lane(double v, int lane) {
 }
 
 template <typename Tab>
-__global__ __launch_bounds__(64) void jacobi_gram16_kernel(Tab tab, int nv_max, double tol, int max_sweeps) {
+__global__ __launch_bounds__(64) void jacobi_gram16_kernel(KernelTable<Tab> tab, int nv_max, double tol, int max_sweeps) {
     __shared__ __attribute__((aligned(16))) double R[kReg][kReg + 2];
     __shared__ jv2d cs[8];
     __shared__ double lam[kReg];
     __shared__ int rank[kReg];
-    const syn_jacobi_item &P = tab.get()[blockIdx.x];
+    const syn_jacobi_item &P = items_of(tab)[blockIdx.x];
     const int lane = threadIdx.x;
     if (P.nv < 1 || P.nv > nv_max || P.len != P.nv) {
         // not a problem this kernel takes: flag it in s and leave the rest

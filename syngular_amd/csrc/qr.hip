@@ -254,9 +254,9 @@ __device__ __forceinline__ void qr_columns(const syn_qr_item &P, double *lds_w, 
 // than the chip has units takes the two kernels below for what they are for.
 typedef QrTileSmem<kQrWaves, kTileRows, kTilePanels, false> QrAnySmem;
 template <typename Tab>
-__global__ __launch_bounds__(kQrThreads) void qr_kernel(Tab tab, int64_t lds_cap) {
+__global__ __launch_bounds__(kQrThreads) void qr_kernel(KernelTable<Tab> tab, int64_t lds_cap) {
     extern __shared__ double lds_w[];
-    const syn_qr_item &P = tab.get()[blockIdx.x];
+    const syn_qr_item &P = items_of(tab)[blockIdx.x];
     const int64_t nb = P.n < P.keep ? P.n : P.keep;
     if (P.columns == SYN_QR_COLUMNS) {
         if (threadIdx.x >= 64 * kColWaves) return;   // whole waves: the others' barriers do not wait for them
@@ -279,18 +279,18 @@ __global__ __launch_bounds__(kQrThreads) void qr_kernel(Tab tab, int64_t lds_cap
 // then ends on the neighbouring FP32 number, so this order is part of that
 // form's results.
 template <typename Tab>
-__global__ __launch_bounds__(64 * kColWaves) void qr_columns_kernel(Tab tab, int64_t lds_cap) {
+__global__ __launch_bounds__(64 * kColWaves) void qr_columns_kernel(KernelTable<Tab> tab, int64_t lds_cap) {
     extern __shared__ double lds_w[];
-    qr_columns<kColWaves>(tab.get()[blockIdx.x], lds_w, lds_cap);
+    qr_columns<kColWaves>(items_of(tab)[blockIdx.x], lds_w, lds_cap);
 }
 
 // Matrices of up to 16 NW rows (NW 1, 2, 4): the panel form by NW waves, the same
 // bits as by eight, whose other waves hold no rows.
 template <int NW, typename Tab>
-__global__ __launch_bounds__(64 * NW, 3) void qr_rows_kernel(Tab tab) {
+__global__ __launch_bounds__(64 * NW, 3) void qr_rows_kernel(KernelTable<Tab> tab) {
     constexpr int ROWS = 16 * NW, PANELS = (ROWS + kHhCols - 1) / kHhCols;
     __shared__ QrTileSmem<NW, ROWS, PANELS, true> sm;
-    const syn_qr_item &P = tab.get()[blockIdx.x];
+    const syn_qr_item &P = items_of(tab)[blockIdx.x];
     if (P.m <= ROWS && (P.n < P.keep ? P.n : P.keep) <= kTileCols)
         qr_tile<1, NW>(P, sm);
     else   // not a matrix of the class: right, if slow

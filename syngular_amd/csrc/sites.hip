@@ -40,8 +40,8 @@ __device__ __forceinline__ void apply_block(const syn_apply_item &P, int64_t loc
 }
 
 template <typename Tab>
-__global__ __launch_bounds__(kSiteThreads) void apply_kernel(Tab tab, int n) {
-    const syn_apply_item *__restrict__ items = tab.get();
+__global__ __launch_bounds__(kSiteThreads) void apply_kernel(KernelTable<Tab> tab, int n) {
+    const syn_apply_item *__restrict__ items = items_of(tab);
     const int64_t bid = blockIdx.x;
     const syn_apply_item &P = items[find_item(items, n, bid)];
     const int64_t nel = P.chil * P.dl * P.dout * P.chir * P.dr;
@@ -137,8 +137,8 @@ __global__ __launch_bounds__(kSiteThreads) void dsum_kernel(const syn_dsum_item 
 }
 
 template <typename Tab>
-__global__ __launch_bounds__(kSiteThreads) void rowscale_kernel(Tab tab, int n) {
-    const syn_rowscale_item *__restrict__ items = tab.get();
+__global__ __launch_bounds__(kSiteThreads) void rowscale_kernel(KernelTable<Tab> tab, int n) {
+    const syn_rowscale_item *__restrict__ items = items_of(tab);
     const int64_t bid = blockIdx.x;
     const syn_rowscale_item &P = items[find_item(items, n, bid)];
     const int64_t nel = P.rows * P.cols;
@@ -157,8 +157,8 @@ __global__ __launch_bounds__(kSiteThreads) void rowscale_kernel(Tab tab, int n) 
 }
 
 template <typename Tab>
-__global__ __launch_bounds__(kSiteThreads) void eye_kernel(Tab tab, int n) {
-    const syn_eye_item *__restrict__ items = tab.get();
+__global__ __launch_bounds__(kSiteThreads) void eye_kernel(KernelTable<Tab> tab, int n) {
+    const syn_eye_item *__restrict__ items = items_of(tab);
     const int64_t bid = blockIdx.x;
     const syn_eye_item &P = items[find_item(items, n, bid)];
     const int64_t nel = P.n * P.n;
@@ -172,8 +172,8 @@ __global__ __launch_bounds__(kSiteThreads) void eye_kernel(Tab tab, int n) {
 }
 
 template <typename Tab>
-__global__ __launch_bounds__(kSiteThreads) void copy_kernel(Tab tab, int n) {
-    const syn_copy_item *__restrict__ items = tab.get();
+__global__ __launch_bounds__(kSiteThreads) void copy_kernel(KernelTable<Tab> tab, int n) {
+    const syn_copy_item *__restrict__ items = items_of(tab);
     const int64_t bid = blockIdx.x;
     const syn_copy_item &P = items[find_item(items, n, bid)];
     const int64_t base = (bid - P.block_start) * SYN_APPLY_BLOCK + threadIdx.x;

@@ -19,8 +19,8 @@ __device__ __forceinline__ double wave_suffix_incl(double v, int lane) {
 }
 
 template <typename Tab>
-__global__ __launch_bounds__(64) void trunc_kernel(Tab tab) {
-    const syn_trunc_item &P = tab.get()[blockIdx.x];
+__global__ __launch_bounds__(64) void trunc_kernel(KernelTable<Tab> tab) {
+    const syn_trunc_item &P = items_of(tab)[blockIdx.x];
     const int lane = threadIdx.x;
     const int64_t n = P.n;
     const double *s = P.s;
@@ -99,8 +99,8 @@ namespace syn {
 constexpr int kNormThreads = 256;
 
 template <typename Tab>
-__global__ __launch_bounds__(kNormThreads) void vecnorm_kernel(Tab tab, int n) {
-    const syn_vecnorm_item *__restrict__ items = tab.get();
+__global__ __launch_bounds__(kNormThreads) void vecnorm_kernel(KernelTable<Tab> tab, int n) {
+    const syn_vecnorm_item *__restrict__ items = items_of(tab);
     __shared__ double part[kNormThreads];
     const int64_t bid = blockIdx.x;
     const syn_vecnorm_item &P = items[find_item(items, n, bid)];
