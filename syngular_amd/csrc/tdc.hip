@@ -535,7 +535,7 @@ __global__ __launch_bounds__(64 * NB) void td_reduce_kernel(const syn_gbj_item *
 constexpr int kMultiThreads = 512;
 constexpr int kMultiWaves = kMultiThreads / 64;
 constexpr int kSpin = 1 << 14;    // polls of one step
-constexpr int kArrive = 1 << 19;  // polls of the first, a second or so
+constexpr int kArrive = 1 << 21;  // of the first, a second or so
 constexpr unsigned kGroupedMax = 16;
 constexpr uint64_t kEmpty = ~(uint64_t)0;   // a NaN no operation makes
 
@@ -656,7 +656,15 @@ __global__ __launch_bounds__(kMultiThreads) void td_reduce_multi_kernel(const sy
                 wp[e] = i < n && (i >= j || i >= tail) ? kEmpty : 0;
                 wc[e] = i < n && i >= j ? kEmpty : 0;
             }
-            for (int left = j == 1 ? arrive : spin;;) {
+            // the first time once they are all there: a loop of its own
+            for (int left = j == 1 ? arrive : 0; left > 0; --left) {
+                bool there = true;
+                for (int i = me ? me : kMultiThreads; i < n; i += kMultiThreads)   // nothing comes for row 0
+                    there = there && peek(xword(T, buf, 0, i)) != kEmpty && peek(xword(T, buf, 1, i)) != kEmpty;
+                if (there) break;
+                __builtin_amdgcn_s_sleep(8);
+            }
+            for (int left = spin;;) {
                 ok = true;
 #pragma unroll
                 for (int e = 0; e < E; ++e) {
@@ -667,7 +675,6 @@ __global__ __launch_bounds__(kMultiThreads) void td_reduce_multi_kernel(const sy
 #pragma unroll
                 for (int e = 0; e < E; ++e) ok = ok && wp[e] != kEmpty && wc[e] != kEmpty;
                 if (ok || --left <= 0) break;
-                if (j == 1) __builtin_amdgcn_s_sleep(8);
             }
 #pragma unroll
             for (int e = 0; e < E; ++e) {
