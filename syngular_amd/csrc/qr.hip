@@ -249,10 +249,12 @@ __device__ __forceinline__ void qr_columns(const syn_qr_item &P, double *lds_w, 
         qr_one<NW, false>(P, lds_w);
 }
 
-// Matrices of any shape and form.  One work-group fits a compute unit (103 KB of
+// Matrices of any shape and form.  One work-group fits a compute unit (107 KB of
 // LDS with the static part, 200 registers a thread), so a launch of more matrices
 // than the chip has units takes the two kernels below for what they are for.
-typedef QrTileSmem<kQrWaves, kTileRows, kTilePanels, false> QrAnySmem;
+// (Rows as in the blocked QR's panels: with the 512 that it needs, the other
+// places in LDS cost a two-site gate at chi = 64 3 of 247 us.)
+typedef QrTileSmem<kQrWaves, 1024, kTilePanels, false> QrAnySmem;
 template <typename Tab>
 __global__ __launch_bounds__(kQrThreads) void qr_kernel(KernelTable<Tab> tab, int64_t lds_cap) {
     extern __shared__ double lds_w[];
