@@ -513,7 +513,7 @@ def roofline(census, timed, dom, steps, ms_per_step, census_ms, W, n, chi, dw, d
 
 # committed rocprofv3 --pmc summaries, per workload (a kernel's bytes per
 # launch depend on the problems its launches carry)
-BATCH_TRAFFIC = os.path.join(ROOT, "profiles", "batch4096_jacobi_step_traffic.json")
+BATCH_TRAFFIC = os.path.join(ROOT, "profiles", "batch4096_back_transform_traffic.json")
 CHAIN_TRAFFIC = os.path.join(ROOT, "profiles", "cholqr_8192x4096_gemm_traffic.json")
 
 

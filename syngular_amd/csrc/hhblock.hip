@@ -4,11 +4,12 @@
 // reflectors as the one-work-group kernel of qr.hip, but only a panel of at
 // most 32 columns is factored column by column; the rest of the matrix is
 // updated with the compact WY form H_j0 ... H_{j0+b-1} = I - V T V^T on the
-// MFMA GEMM, and Q is accumulated panel by panel the same way.  This kernel
-// factors one panel in place (one work-group of 1024 threads, rows spread
-// over the threads, the panel in L2) and writes the explicit V (unit
-// diagonal, zeros above) and T (LAPACK dlarft, forward, columnwise:
-// T[0:j, j] = -tau_j T[0:j, 0:j] V[:, 0:j]^T v_j, T[j, j] = tau_j).
+// MFMA GEMM, and Q is accumulated panel by panel the same way.  These kernels
+// factor one panel in place (one work-group of 1024 threads) and write the
+// explicit V (unit diagonal, zeros above) and T (LAPACK dlarft, forward,
+// columnwise: T[0:j, j] = -tau_j T[0:j, 0:j] V[:, 0:j]^T v_j, T[j, j] = tau_j):
+// up to 1024 rows in the waves' registers (hh_panel_reg_kernel), taller ones
+// streamed from L2, three passes a column (hh_panel_kernel).
 #include "common.hpp"
 #include "hh_tile.hpp"
 #include "prof.hpp"

@@ -27,9 +27,9 @@ enum ProfTag {
     kTagGemmBf1664 = 18,
     kTagGemmBf16128 = 19,
     // the direct phase of the Gram eigen-solver (tdc.hip), a scope for each part
-    kTagTdReduce = 20,     // tridiagonal reduction
+    kTagTdReduce = 20,     // tridiagonal reduction and T factors
     kTagTdMerge = 21,      // leaves and merges of the divide and conquer, with their products
-    kTagTdBack = 22,       // T factors and back-transformation
+    kTagTdBack = 22,       // back-transformation
     kTagTdGemm = 23,       // the two products that diagonalise G
 };
 

@@ -16,10 +16,9 @@
 // steps and a call takes 7..14 sweeps, about 4 n^3 flops each; the reduction
 // costs 4/3 n^3, the divide and conquer 8/3 n^3 at most and the products
 // 6 n^3, once.  Calls measured with the sweeps alone and with this phase, in
-// ms: one matrix of order 64 0.78 / 0.39, 128 1.5 / 0.60, 256 3.3 / 1.25, 512
-// 7.1 / 2.7, 1024 21 / 6.7, 2048 80 / 19; before the reductions below had their
-// present form, 8 of order 512 9.6 / 4.1; 2000 of order 64 5.3 / 2.0, 1000 of
-// 128 15.5 / 3.2, 800 of 256 88 / 12.1.
+// ms: one matrix of order 64 0.78 / 0.33, 128 1.5 / 0.54, 256 3.3 / 1.19, 512
+// 7.1 / 2.5, 1024 21 / 6.2, 2048 80 / 17.9; 2000 of order 64 5.3 / 1.6, 1000 of
+// 128 15.5 / 2.7, 800 of 256 88 / 10.3, 8 of 512 9.6 / 2.7.
 // Residuals fall with the number of rotations: rt^T diag(s^2) rt - G from
 // 1e-13 to 1e-15 of the largest eigenvalue.
 //
@@ -513,15 +512,16 @@ __global__ __launch_bounds__(64 * NB) void td_reduce_kernel(const syn_gbj_item *
 // columns, one of each, go on when their rows are dead.
 //
 // A work-group can wait for one that has no compute unit yet only in its first
-// exchange: past it, all of the matrix are running and stay so.  SpinTurn keeps other
-// launches of this kernel from holding the units, and a launch's work-groups start
-// in order, so the first unfinished matrix always gets its units, and that first
-// wait lasts as long as the matrices ahead or another stream's kernels do.  Every wait is
-// bounded all the same, that one by kArrive polls and the others by kSpin: past
-// the limit the work-group gives up, the matrix counts as failed and the Jacobi
-// sweeps take it.  (One limit of kSpin for all waits and launches side by side:
-// 3 matrices of order 1500 in a call 50 ms, now 24; four streams of such calls at
-// once: 5 of 48 calls gave up, up to 230 ms each, now none, up to 81.)
+// exchange: past it, all of the matrix are running and stay so.  SpinTurn keeps
+// other launches of this kernel from holding the units, and a launch's
+// work-groups start in order, so the first unfinished matrix always gets its
+// units, and that first wait lasts as long as the matrices ahead or another
+// stream's kernels do.  Every wait is bounded all the same, that one by kArrive
+// polls and the others by kSpin: past the limit the work-group gives up, the
+// matrix counts as failed and the Jacobi sweeps take it.  (One limit of kSpin for
+// all waits and launches side by side: 3 matrices of order 1500 in a call 50 ms,
+// now 24; four streams of such calls at once: 5 of 48 calls gave up, up to 230 ms
+// each, now none, up to 81.)
 //
 // Order 2048 (128 work-groups) is bound by the exchange, 128 readers of every
 // word (3.0 of a step's 6.6 us; the vectors 1.5, the pass 0.8), the smaller
@@ -1741,10 +1741,7 @@ int tdc_launch(const syn_gbj_item *items, const std::vector<syn_gbj_item> &host,
         if (int rc = reduce_single<16>(items, host, 192, tol, st)) return rc;
         if (tdc_waits(nmax))
             if (int rc = reduce_multis(items, host, polls, tol, st)) return rc;
-    }
-    const unsigned nblk = (unsigned)refl_blocks((int)nmax);
-    {
-        ProfScope ps(kTagTdBack, 0.0, st);
+        const unsigned nblk = (unsigned)refl_blocks((int)nmax);
         hipLaunchKernelGGL(td_tfac_kernel, dim3(ni, nblk), dim3(256), 0, st, items);
     }
     {
